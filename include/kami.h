@@ -3,7 +3,7 @@
  *
  * Three entry-point families, all device-pointer based and caller-owned:
  *   block GEMM      kami_block_gemm            one problem per workgroup, fixed shape
- *   batched GEMM    kami_batched_plan_*        uneven shapes, persistent kernel + queue
+ *   batched GEMM    kami_batched_plan_*        uneven shapes, one launch over a work queue
  *   block SpGEMM    kami_bsr_spgemm_*          symbolic (count/scan/fill) + numeric
  *
  * Conventions shared by every entry point:
@@ -124,7 +124,8 @@ typedef struct kami_batched_opts {
     int32_t b_layout;  /* kami_b_layout */
     int32_t autotune;  /* 1 = time the candidate tile variants on the device at plan
                           creation; 0 = use the built-in priors */
-    int32_t use_graph; /* 1 = execute through a captured hipGraph */
+    int32_t use_graph; /* accepted; an execution is one kernel launch either way, which costs
+                          a caller less than replaying a captured hipGraph of it */
     int32_t reserved;
     double alpha, beta;
 } kami_batched_opts;
@@ -135,7 +136,7 @@ typedef struct kami_plan_info {
     int64_t problems;
     int64_t work_items;     /* queue entries (output tiles) of one execution */
     int32_t buckets;        /* size buckets the autotuner decided */
-    int32_t workgroups;     /* persistent grid size */
+    int32_t workgroups;     /* workgroups of one execution (four wave tiles each) */
     double flops;           /* 2*sum(M*N*K) of one execution */
     int32_t variant_of_bucket[16]; /* chosen tile variant per bucket (first 16) */
 } kami_plan_info;
@@ -195,11 +196,9 @@ kami_status kami_split_gemm(const kami_gemm_desc* d, const void* A, const void* 
 kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count,
                                      int32_t precision, const kami_batched_opts* opts,
                                      void* stream, kami_batched_plan** out);
-/* One persistent launch (through the plan's hipGraph when use_graph is set).
- * A plan owns one device queue counter that every execution resets and then draws
- * from, so a plan allows one execution in flight: serialise its executions on one
- * stream (a second stream, or two replays of a captured graph running at once, would
- * race on the counter and skip or repeat tiles).  Distinct plans run concurrently. */
+/* One kernel launch.  A plan's executions share nothing but its read-only queue and the
+ * problems' C: executions that may overlap write the same C values (with beta = 0), so
+ * order them when beta != 0.  Distinct plans run concurrently. */
 kami_status kami_batched_execute(kami_batched_plan* plan, void* stream);
 kami_status kami_batched_plan_info(const kami_batched_plan* plan, kami_plan_info* out);
 kami_status kami_batched_plan_destroy(kami_batched_plan* plan);
@@ -209,8 +208,8 @@ kami_status kami_batched_plan_destroy(kami_batched_plan* plan);
  * problems, precision and options mean what they mean for kami_batched_plan_create and
  * the result equals that of a plan created with the same arguments and executed once;
  * autotune and use_graph must be 0 (KAMI_EINVAL otherwise: both need memory of their
- * own), tile variants come from the tuning cache or the priors.  The work queue and its
- * counter live in a fixed device array of 2 MiB per device (held until the process ends):
+ * own), tile variants come from the tuning cache or the priors.  The work queue lives in
+ * a fixed device array of 6 MiB per device (held until the process ends):
  * at most 32768 queue entries (output tiles of 64 x 64, 32 x 32 or 128 x 64 by size
  * bucket), KAMI_ENOSPC beyond, checked before any device call.  The entries are built on
  * the host in static arrays and copied to the device on `stream`; the call allocates no

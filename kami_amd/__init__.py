@@ -240,8 +240,8 @@ class BatchedPlan:
 
     problems: sequence of (A, B, C) contiguous 2-D device tensors, A (M, K), B (N, K)
     ("nk") or (K, N) ("kn"), C (M, N); M, N, K multiples of 16.  The tensors must stay
-    alive while the plan exists.  execute() is one persistent launch, replayed through a
-    hipGraph when use_graph is set.
+    alive while the plan exists.  execute() is one kernel launch (use_graph is accepted;
+    replaying a captured graph of that launch costs a caller more than the launch).
     """
 
     def __init__(self, problems, *, precision=None, b_layout="nk", autotune=False,

@@ -1,5 +1,5 @@
-// Batched GEMM over problems of uneven size: one persistent launch, a device work queue,
-// per-size-bucket tile variants chosen by an autotuner, optional hipGraph execution.
+// Batched GEMM over problems of uneven size: one launch over a device queue of wave tiles,
+// per-size-bucket tile variants chosen by an autotuner.
 //
 // Reference: batched_gemm_{1d,2d,3d}_double_mma (src/batched_gemm/KAMI/1d/
 // batched_gemm_1d_double_mma.cu:59-218) runs one uniform-size problem per CTA at fixed
@@ -8,18 +8,27 @@
 //   * problems carry their own {m, n, k, lda, ldb, ldc, A, B, C} (the kami_problem array);
 //   * every problem is cut into output tiles; a tile is one 64-byte queue entry holding
 //     its own operand pointers, strides, extents and variant (WorkItem);
-//   * a persistent grid (CUs x resident workgroups) pops a batch of up to kQueueBatch
-//     entries per atomic add (fewer when the queue is short, so that every workgroup
-//     gets work), in descending-cost order (longest first), until the queue is empty;
-//     the next batch is fetched while the current one's tiles compute;
+//   * an entry is cut into wave tiles of up to 32 x 32 (WaveUnit, 8 bytes each).  A wave
+//     computes one of them alone, staged through LDS of its own, so there is no barrier
+//     and no shared counter: the hardware's dispatcher hands out the workgroups, longest
+//     problems first, and one wave's loads hide behind the products of the others;
+//   * units are laid out so that neighbouring tiles run on one XCD at the same time;
 //   * the variant of a tile is the tile shape and wave partition of its size bucket,
 //     picked by timing candidates on the device at plan creation (or from priors);
-//   * one execution is [reset the queue counter] -> [persistent kernel], captured once
-//     into a hipGraph and replayed.  The counter is cleared by a one-thread kernel,
-//     never by a memset node.
+//   * one execution is one kernel launch, also for plans made with use_graph: replaying a
+//     captured graph of that one kernel took 18.5 us of a caller's loop where the launch
+//     takes 8.9 us (100 FP64 problems of 16 to 256).
 // M, N and K must be multiples of 16.
+//
+// What bounds it: 20000 problems of 16 to 256 (3.58 GB FP64, 1.19 GB FP16 with FP32 C) run
+// in 801 us and 293 us, 4.5 and 4.1 TB/s of the algorithmic bytes; the matrix pipes are
+// 57 % busy in FP64.  The persistent form this replaced (workgroups popping tiles of up to
+// 128 x 128 from an atomic counter, LDS stages shared by four waves, one barrier a stage, a
+// one-thread kernel to clear the counter) took 1023 us and 388 us: two workgroups a CU and
+// their barriers left too little in flight.
 #include <algorithm>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -40,565 +49,288 @@ struct WorkItem {
 };
 static_assert(sizeof(WorkItem) == 64, "queue entry layout");
 
-// Queue entries popped per atomic add: a power of two from 2 to kQueueBatch (the LDS
-// record size); the plan picks fewer for short queues.  Fetching a batch takes three
-// tile boundaries (atomic add, entry loads, LDS write), so the next batch is requested
-// when the workgroup starts the tile kFetchAhead before the end of its current batch,
-// and never at the batch's first tile: a workgroup that starts early cannot take a
-// second batch before the others have taken their first.
-constexpr int kQueueShift = 3, kQueueBatch = 1 << kQueueShift;
-constexpr int kFetchAhead = 3;
-
-// Staging shared by every tile variant: a stage holds up to TMAX rows of A and TNMAX rows
-// of B (or KC rows of TNMAX columns when B is K x N), KC elements of K each, in LDS rows
-// padded to the conflict-free stride.  Pieces are 16 bytes; a thread owns pieces tid + i * NT.
-template <class AT>
-struct StreamGeom {
-    static constexpr int NT = 256;
-    static constexpr int ELT = (int)sizeof(typename AT::in_t), VE = 16 / ELT;
-    // FP64 stages 8-wide K chunks of tiles up to 128 x 128 (96-byte rows, 48 KB of LDS
-    // for the two stage buffers), FP16/BF16 64-wide chunks of tiles up to 128 x 64
-    // (160-byte rows, 60 KB); two workgroups per CU either way.  FP64 offers the 128-wide
-    // tiles because its batches are bound by HBM: a problem cut into 64 x 64 tiles reads
-    // each row of A once per 64 columns of C and each row of B once per 64 rows, and
-    // across the thousands of tiles in flight L2 keeps none of those rows for the next
-    // tile that needs them
-    static constexpr int KC = ELT == 8 ? 8 : 64;
-    static constexpr int TMAX = 128, TNMAX = ELT == 8 ? 128 : 64;
-    static constexpr int ROWB = lds_row_bytes(KC * ELT, AT::FRAG_BYTES);
-    static constexpr int A_REGION = TMAX * ROWB;
-    static constexpr int STAGE = (TMAX + TNMAX) * ROWB;
-    static constexpr int LDS = 2 * STAGE;
-    static constexpr int CPR = KC / VE;  // pieces per staged row
-    static constexpr int NP = ((TMAX + TNMAX) * CPR + NT - 1) / NT;
-    static_assert((KC * TNMAX) / VE <= TNMAX * CPR, "K x N staging fits the B region");
-    static_assert((TMAX * CPR) % NT == 0 && (TNMAX * CPR) % NT == 0, "whole piece groups");
-};
-
-// Tile geometry of a variant: TM x TN output tile, WM x WN waves (4 waves).
-template <class AT, int TM_, int TN_, int WM_, int WN_>
-struct TileGeom {
-    using SG = StreamGeom<AT>;
-    static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_;
-    static_assert(WM * WN * 64 == SG::NT, "four waves");
-    static_assert(TM <= SG::TMAX && TN <= SG::TNMAX, "tile fits the stage");
-    static constexpr int SUBM = TM / WM, SUBN = TN / WN, IM = SUBM / 16, JN = SUBN / 16;
-    static_assert(SUBM % 16 == 0 && SUBN % 16 == 0 && SG::KC % AT::KSTEP == 0, "tile");
-};
+// Consecutive queue entries dealt to one XCD at a time: a power of two up to
+// 1 << kQueueShift.
+constexpr int kQueueShift = 3;
 
 // Tile variants.  Index = variant id stored in the work items.
-//   0: 64 x 64 tile, 2 x 2 waves (2D)       1: 32 x 32 tile, 2 x 2 waves (2D)
-//   2: 64 x 64 tile, 4 x 1 waves (1D)       3: 128 x 64 tile, 2 x 2 waves (2D)
-//   4: 128 x 128 tile, 2 x 2 waves (FP64)   5: 64 x 128 tile, 2 x 2 waves (FP64)
+//   0: 64 x 64 tile      1: 32 x 32 tile      2: 64 x 64 tile, wave tiles of 16 x 32
+//   3: 128 x 64 tile     4: 128 x 128 tile (FP64)     5: 64 x 128 tile (FP64)
+// Wave tiles are 32 x 32 except where noted.
 constexpr int kVariants = 6;
 static_assert(kVariants == kBatchedVariants, "tuning-cache variant range");
 static const int kVariantTM[kVariants] = {64, 32, 64, 128, 128, 64};
 static const int kVariantTN[kVariants] = {64, 32, 64, 64, 128, 128};
+static const int kVariantSM[kVariants] = {2, 2, 1, 2, 2, 2};  // atoms of a wave tile
+static const int kVariantSN[kVariants] = {2, 2, 2, 2, 2, 2};
 
-template <class AT>
-struct Variants {
-    using V0 = TileGeom<AT, 64, 64, 2, 2>;
-    using V1 = TileGeom<AT, 32, 32, 2, 2>;
-    using V2 = TileGeom<AT, 64, 64, 4, 1>;
-    using V3 = TileGeom<AT, 128, 64, 2, 2>;
-    using V4 = TileGeom<AT, 128, 128, 2, 2>;
-    using V5 = TileGeom<AT, 64, 128, 2, 2>;
-};
-
-// Variants a precision offers: FP16/BF16 stage 64 columns of B, so not 4 and 5.
+// Variants a precision offers: 4 and 5 are FP64's.
 inline int variants_of(int prec) { return prec == KAMI_PREC_F64 ? kVariants : 4; }
 
-__device__ inline int variant_tm(int v) { return v == 1 ? 32 : (v == 3 || v == 4 ? 128 : 64); }
-__device__ inline int variant_tn(int v) { return v == 1 ? 32 : (v == 4 || v == 5 ? 128 : 64); }
+// One wave's share of a queue entry: the im x jn atoms (16 x 16) of C whose first atom is
+// (ra, ca), counted in atoms from the entry's origin.  im = 0: nothing to do.
+struct WaveUnit {
+    uint32_t item;
+    uint8_t ra, ca, im, jn;
+};
+static_assert(sizeof(WaveUnit) == 8, "wave unit layout");
+constexpr int kWaveAtoms = 2;  // atoms of a wave tile per dimension, at most
+constexpr int kWavesPerGroup = 4;
+constexpr int kXcds = 8;  // workgroup L runs on XCD L mod 8
 
 struct BatchArgs {
     const WorkItem* items;
-    unsigned int* counter;
-    int64_t n_items;
+    const WaveUnit* units;
+    int64_t n_units;  // a multiple of kWavesPerGroup
     double alpha, beta;
-    int32_t b_kn;
-    int32_t qshift;  // entries per pop = 1 << qshift, at most kQueueBatch
 };
 
-// A tile as the kernel holds it: wave-uniform values (in scalar registers).
-struct Tile {
-    const unsigned char* A;
-    const unsigned char* B;
-    unsigned char* C;
-    int64_t lda, ldb, ldc;
-    int mlim, nlim, k, variant, nch;
-    bool valid;
-};
+// The queue is read through scalar loads (constant address space, wave-uniform index).
+template <class T>
+__device__ __forceinline__ T load_uniform(const T* p) {
+    static_assert(sizeof(T) % 8 == 0, "whole 8-byte words");
+    typedef const __attribute__((address_space(4))) uint64_t* cptr;
+    struct words {
+        uint64_t w[sizeof(T) / 8];
+    } x;
+    const cptr q = (cptr)(uintptr_t)p;
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T) / 8; ++i) x.w[i] = q[i];
+    return __builtin_bit_cast(T, x);
+}
 
 __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
-__device__ __forceinline__ int64_t uni64(int64_t x) {
-    const uint64_t u = (uint64_t)x;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
-    return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-template <class P>
-__device__ __forceinline__ P* uniptr(P* p) {
-    return reinterpret_cast<P*>(uni64((int64_t)reinterpret_cast<uintptr_t>(p)));
-}
 
-template <class AT>
-__device__ __forceinline__ Tile read_tile(const WorkItem* rec, bool valid) {
-    Tile t;
-    t.valid = valid;
-    if (!valid) {
-        t.A = t.B = t.C = nullptr;
-        t.lda = t.ldb = t.ldc = 0;
-        t.mlim = t.nlim = t.k = t.variant = t.nch = 0;
-        return t;
-    }
-    const WorkItem w = *rec;
-    t.A = uniptr(reinterpret_cast<const unsigned char*>(w.A));
-    t.B = uniptr(reinterpret_cast<const unsigned char*>(w.B));
-    t.C = uniptr(reinterpret_cast<unsigned char*>(w.C));
-    t.lda = uni64(w.lda);
-    t.ldb = uni64(w.ldb);
-    t.ldc = uni64(w.ldc);
-    t.mlim = uni(w.mlim);
-    t.nlim = uni(w.nlim);
-    t.k = uni(w.k);
-    t.variant = uni(w.variant);
-    t.nch = (t.k + StreamGeom<AT>::KC - 1) / StreamGeom<AT>::KC;
-    return t;
-}
-
-// Raw buffer descriptors over a tile's operands.  An offset at or past kBufferRange reads
-// as zero, so pieces outside C or past K need no branch.
+// Raw buffer descriptors over a wave tile's operands.  A lane offset at or past
+// kBufferRange reads as zero, so pieces past K need no branch.
 constexpr int kBufferRange = 0x7FFFFFF0;
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const unsigned char* base) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(base), (short)0,
-                                             kBufferRange, 0x00020000);
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const void* base) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, kBufferRange,
+                                             0x00020000);
 }
-__device__ __forceinline__ u4_t buffer_load16(__amdgpu_buffer_rsrc_t r, int off) {
-    return __builtin_bit_cast(u4_t, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+__device__ __forceinline__ u4_t buffer_load16(__amdgpu_buffer_rsrc_t r, int off, int soff) {
+    return __builtin_bit_cast(u4_t, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0));
 }
-
-// Loads the pieces of stage (tile t, K chunk c) into registers.  Every stage covers the
-// full staging area (TMAX rows of A, TNMAX rows of B, or KC rows of TNMAX columns when B
-// is K x N) with a fixed piece-to-thread mapping; rows outside the tile or C and K past
-// the problem read as zero (no memory traffic), so the code is the same for every tile
-// variant and free of branches.
-template <class AT, bool KN>
-__device__ __forceinline__ void stream_load(const Tile& t, int c, u4_t (&r)[StreamGeom<AT>::NP]) {
-    using SG = StreamGeom<AT>;
-    constexpr int CA = SG::TMAX * SG::CPR, CB = SG::TNMAX * SG::CPR;
-    const int k0 = c * SG::KC;
-    const int mrows = min(variant_tm(t.variant), t.mlim);
-    const int ncols = min(variant_tn(t.variant), t.nlim);
-    const __amdgpu_buffer_rsrc_t ra = tile_rsrc(t.A), rb = tile_rsrc(t.B);
-    const int lda = (int)t.lda, ldb = (int)t.ldb;
-#pragma unroll
-    for (int i = 0; i < SG::NP; ++i) {
-        const int idx = threadIdx.x + i * SG::NT;
-        if (i * SG::NT < CA) {  // compile-time: the group is all A
-            const int row = idx / SG::CPR, kc = (idx % SG::CPR) * SG::VE;
-            const bool ok = row < mrows && k0 + kc < t.k;
-            r[i] = buffer_load16(ra, ok ? (row * lda + k0 + kc) * SG::ELT : kBufferRange);
-        } else if (i * SG::NT < CA + CB) {  // all B
-            const int j = idx - CA;
-            int off;
-            if constexpr (!KN) {
-                const int row = j / SG::CPR, kc = (j % SG::CPR) * SG::VE;
-                off = (row < ncols && k0 + kc < t.k) ? (row * ldb + k0 + kc) * SG::ELT : kBufferRange;
-            } else {
-                constexpr int PPR = SG::TNMAX / SG::VE;  // pieces per K row
-                const int kr = j / PPR, jc = (j % PPR) * SG::VE;
-                off = (jc < ncols && k0 + kr < t.k) ? ((k0 + kr) * ldb + jc) * SG::ELT : kBufferRange;
-            }
-            r[i] = buffer_load16(rb, off);
-        } else {
-            r[i] = u4_t{0, 0, 0, 0};
-        }
-    }
+__device__ __forceinline__ double buffer_load8(__amdgpu_buffer_rsrc_t r, int off, int soff) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0));
 }
 
-template <class AT, bool KN>
-__device__ __forceinline__ void stream_write(const u4_t (&r)[StreamGeom<AT>::NP], unsigned char* buf) {
-    using SG = StreamGeom<AT>;
-    using in_t = typename AT::in_t;
-    constexpr int CA = SG::TMAX * SG::CPR, CB = SG::TNMAX * SG::CPR;
-#pragma unroll
-    for (int i = 0; i < SG::NP; ++i) {
-        const int idx = threadIdx.x + i * SG::NT;
-        if (i * SG::NT < CA) {
-            store_raw<16>(buf + (idx / SG::CPR) * SG::ROWB + (idx % SG::CPR) * 16, r[i]);
-        } else if (i * SG::NT < CA + CB) {
-            const int j = idx - CA;
-            if constexpr (!KN) {
-                store_raw<16>(buf + SG::A_REGION + (j / SG::CPR) * SG::ROWB + (j % SG::CPR) * 16, r[i]);
-            } else {
-                constexpr int PPR = SG::TNMAX / SG::VE;
-                const int kr = j / PPR, jc = (j % PPR) * SG::VE;
-                const in_t* e = reinterpret_cast<const in_t*>(&r[i]);
-#pragma unroll
-                for (int q = 0; q < SG::VE; ++q)
-                    *reinterpret_cast<in_t*>(buf + SG::A_REGION + (jc + q) * SG::ROWB + kr * SG::ELT) = e[q];
-            }
-        }
-    }
+// Transposing LDS read of 2-byte values (gfx950): each group of 16 lanes reads four rows
+// of 16 values, lane l of the group the four at row l / 4, columns 4 (l mod 4) .. + 3, and
+// receives column l of the four rows (layout checked with an in-bounds probe).
+__device__ __forceinline__ u2_t lds_read_turned(const unsigned char* p) {
+    return __builtin_bit_cast(
+        u2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                  (__attribute__((address_space(3))) s4_t*)(const_cast<unsigned char*>(p))));
 }
 
-// Shared state of a workgroup's stream of (tile, K chunk) stages.
-//   * The queue is popped Q = qb = 1 << qs entries at a time into one of two LDS record
-//     buffers; stream tile s lives in buffer (s / Q) % 2, slot s % Q.  The next batch
-//     is fetched in steps taken at tile boundaries (atomic add; entry loads; LDS write),
-//     so its latency hides behind whole tiles.
-//   * Stage x of the stream (x counts (tile, chunk) pairs) is loaded into register slot
-//     x % 2 and computed from LDS buffer x % 2.  While stage x is computed, slot
-//     (x + 1) % 2 holds stage x + 1 and slot x % 2 holds stage x + 2.  The stage loop is
-//     unrolled in pairs so both slot indices are compile-time, and it issues no memory
-//     operation other than the stage loads: the compiler then waits only for the slot
-//     it writes, never for the loads still in flight.
-//   * The cursor (tile tc, chunk cc) is the next stage to load.  It stops ("blocked")
-//     at a tile whose record has not been fetched yet; tile boundaries unblock it and
-//     load any stage that is missing.
-template <class AT>
-struct Stream {
-    Tile cur;            // tile being computed (stream index t0)
-    Tile ct;             // tile at the cursor (stream index tc)
-    int64_t t0, tc;
-    int cc;              // chunk of the cursor
-    bool blocked;
-    int64_t x;           // stage being computed
-    int64_t loaded;      // stages loaded so far
-    int64_t fetched;     // stream tiles whose records are in LDS (whole batches)
-    int qb, qs, lead;    // entries per batch (1 << qs); tile of a batch that requests the next
-    int phase;           // next batch fetch: -1 idle, 0 start, 1 atomic issued,
-                         // 2 entries loaded, 3 records written
-    u4_t slot0[StreamGeom<AT>::NP], slot1[StreamGeom<AT>::NP];
-    int sv0, sv1;        // variant of the stage in each slot, -1 = empty
-    // wave 0 only: batch fetch in flight
-    unsigned fbase;
-    u4_t fpiece;         // lane l < 4 Q: 16-byte piece l % 4 of entry l / 4
-    bool fvalid;
-};
+#define KAMI_GLOBAL __attribute__((address_space(1)))
 
-struct QueueLds {
-    alignas(16) WorkItem rec[2][kQueueBatch];
-    int valid[2][kQueueBatch];
-};
-
-template <class AT>
-__device__ __forceinline__ Tile stream_tile(const QueueLds& q, int64_t s, int qs) {
-    const int b = (int)((s >> qs) & 1), slot = (int)(s & ((1 << qs) - 1));
-    return read_tile<AT>(&q.rec[b][slot], uni(q.valid[b][slot]) != 0);
-}
-
-// One step of the batch fetch (every thread, uniform); the caller puts a barrier after
-// it and then calls fetch_commit.
-template <class AT>
-__device__ __forceinline__ void fetch_step(const BatchArgs& a, Stream<AT>& st, QueueLds& q) {
-    st.phase = uni(st.phase);
-    if (st.phase == 0) {
-        // pop the queue range of stream tiles [fetched, fetched + Q)
-        if (threadIdx.x == 0) st.fbase = atomicAdd(a.counter, (unsigned)st.qb);
-        st.phase = 1;
-    } else if (st.phase == 1) {
-        if (threadIdx.x < 64) {
-            const unsigned base = __shfl(st.fbase, 0);
-            const int lane = threadIdx.x, e = lane >> 2;
-            st.fvalid = e < st.qb && (int64_t)base + e < a.n_items;
-            if (st.fvalid)
-                st.fpiece = load_raw<16>(reinterpret_cast<const unsigned char*>(a.items + base + e) +
-                                         16 * (lane & 3));
-        }
-        st.phase = 2;
-    } else {
-        const int b = (int)((st.fetched >> st.qs) & 1);
-        if (threadIdx.x < 4 * st.qb) {
-            const int e = threadIdx.x >> 2;
-            if (st.fvalid)
-                store_raw<16>(reinterpret_cast<unsigned char*>(&q.rec[b][e]) + 16 * (threadIdx.x & 3),
-                              st.fpiece);
-            if ((threadIdx.x & 3) == 0) q.valid[b][e] = st.fvalid ? 1 : 0;
-        }
-        st.phase = 3;
-    }
-}
-
-template <class AT>
-__device__ __forceinline__ void fetch_commit(Stream<AT>& st) {
-    if (st.phase == 3) {
-        st.fetched += st.qb;
-        st.phase = -1;  // idle until the next batch is started
-    }
-}
-
-// Makes the record of stream tile s available (uniform; synchronous).  The batch
-// fetched here goes to the LDS buffer of the batch two before it, which the current
-// tile and the cursor have both left.
-template <class AT>
-__device__ __forceinline__ void ensure_ready(const BatchArgs& a, Stream<AT>& st, QueueLds& q, int64_t s) {
-    while (st.fetched <= s) {
-        if (st.phase < 0) st.phase = 0;
-        fetch_step(a, st, q);
-        __syncthreads();
-        fetch_commit(st);
-    }
-}
-
-// Load the stage at the cursor into `dst` and advance the cursor.  Returns the stage's
-// variant, or -1 when the cursor is at the end of the stream or blocked.  Only LDS is
-// read besides the stage itself.
-template <class AT, bool KN>
-__device__ __forceinline__ int load_at_cursor(Stream<AT>& st, const QueueLds& q,
-                                              u4_t (&dst)[StreamGeom<AT>::NP]) {
-    if (!st.ct.valid || st.blocked) return -1;
-    stream_load<AT, KN>(st.ct, st.cc, dst);
-    const int v = st.ct.variant;
-    ++st.loaded;
-    if (++st.cc >= st.ct.nch) {
-        st.cc = 0;
-        ++st.tc;
-        if (st.tc < st.fetched)
-            st.ct = stream_tile<AT>(q, st.tc, st.qs);
-        else
-            st.blocked = true;
-    }
-    return v;
-}
-
-// Slot S holds the stage after the one being computed: write it to LDS buffer S and
-// load the stage at the cursor into it.
-template <class AT, bool KN, int S>
-__device__ __forceinline__ void advance_slot(Stream<AT>& st, const QueueLds& q, unsigned char* smem) {
-    using SG = StreamGeom<AT>;
-    auto& slot = S ? st.slot1 : st.slot0;
-    int& sv = S ? st.sv1 : st.sv0;
-    if (sv >= 0) stream_write<AT, KN>(slot, smem + S * SG::STAGE);
-    sv = load_at_cursor<AT, KN>(st, q, slot);
-}
-
-// Loads stage `loaded` into its slot (runtime parity; tile-boundary use only).
-template <class AT, bool KN>
-__device__ __forceinline__ void load_next_into_slot(Stream<AT>& st, const QueueLds& q) {
-    if (st.loaded & 1)
-        st.sv1 = load_at_cursor<AT, KN>(st, q, st.slot1);
-    else
-        st.sv0 = load_at_cursor<AT, KN>(st, q, st.slot0);
-}
-
-template <class AT, bool KN, class V>
-__device__ __forceinline__ void run_tile(const BatchArgs& a, Stream<AT>& st, const QueueLds& q,
-                                         unsigned char* smem) {
-    using SG = StreamGeom<AT>;
+// A wave tile of IM x JN atoms computed by one wave on its own: no barrier, so the waves of a
+// CU run apart and one wave's loads hide behind the others' products.  A stage is one
+// 128-byte line of every row of the tile (16 FP64 or 64 FP16 / BF16 values of K, two
+// fragments).  Loading fragments straight from memory would put 16 rows under 16
+// consecutive lanes, which the address unit takes 4 lanes a clock (64 clocks an
+// instruction); so eight lanes load a row's line (16 clocks) and the lines are turned into
+// fragments through LDS of the wave's own.
+template <class AT, bool KN, int IM, int JN>
+struct WaveTile {
+    using frag_t = typename AT::frag_t;
     using acc_t = typename AT::acc_t;
     using out_t = typename AT::out_t;
-    using frag_t = typename AT::frag_t;
     using accv_t = typename AT::accv_t;
-    constexpr int FB = AT::FRAG_BYTES;
-    const int lane = threadIdx.x & 63;
-    const int wave = uni(threadIdx.x >> 6);
-    const int wm = wave / V::WN, wn = wave % V::WN;
-    const Tile cur = st.cur;
-    // wave-uniform bounds
-    const int mlim = uni(cur.mlim), nlim = uni(cur.nlim), nch = uni(cur.nch);
+    static constexpr int ELT = (int)sizeof(typename AT::in_t);
+    static constexpr bool F64 = ELT == 8;
+    static constexpr int VE = 16 / ELT;
+    static constexpr int KS = 128 / ELT, NF = KS / AT::KSTEP;
+    static_assert(NF == 2 && AT::FRAG_BYTES == 16, "a stage row is two 64-byte fragment groups");
+    // K x N operands: FP64 fragments are loaded straight (16 lanes read 16 consecutive
+    // columns); rows of 2-byte values are turned by transposing LDS reads
+    static constexpr bool TURN = KN && !F64;
+    static constexpr int TROW = JN * 32 + 16;  // bytes of a staged K row
+    static constexpr int PPR = JN * 2;         // 16-byte pieces of a K row
+    static constexpr int NA = IM * 2, NB = JN * 2;  // 16-byte pieces of a lane
+    static constexpr int A_LDS = IM * 16 * 128;
+    static constexpr int LDS = A_LDS + (!KN ? JN * 16 * 128 : TURN ? KS * TROW : 0);
 
-    accv_t acc[V::IM][V::JN];
-#pragma unroll
-    for (int i = 0; i < V::IM; ++i)
-#pragma unroll
-        for (int j = 0; j < V::JN; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[i][j][v] = 0;
+    struct Stage {
+        u4_t a[NA], b[NB];
+    };
 
-    // Every atom of a live wave is computed: staged rows and columns outside C are zero,
-    // and a guard per atom would make the compiler copy the accumulators around each
-    // MFMA.  Waves whose whole sub-tile lies outside C skip the products.
-    const bool wave_live = wm * V::SUBM < mlim && wn * V::SUBN < nlim;  // wave-uniform
-    // atoms of the wave's sub-tile inside C (wave-uniform)
-    const int im_live = uni(min(V::IM, (mlim - wm * V::SUBM + 15) / 16));
-    const int jn_live = uni(min(V::JN, (nlim - wn * V::SUBN + 15) / 16));
-    auto compute = [&](const unsigned char* base) {
-        const unsigned char* bb = base + SG::A_REGION;
-        if (!wave_live) return;
+    const __amdgpu_buffer_rsrc_t ra, rb;
+    const int lane, grp, lda, ldb, k;
+    unsigned char* const lds;
+    int aoff, boff;  // the lane's byte offsets in the first stage
+    // LDS offsets.  Piece p of row r lies in slot p ^ 2 ((r / 4) mod 4) of the row's eight, so
+    // that the 32 lanes of a read pass (16 rows, two neighbouring pieces) and the rows of a
+    // write fall on different banks.
+    int woff, roff;
+
+    __device__ __forceinline__ WaveTile(const WorkItem& w, const WaveUnit& u, unsigned char* lds_)
+        : ra(tile_rsrc(static_cast<const char*>(w.A) + (int64_t)u.ra * 16 * w.lda * ELT)),
+          rb(tile_rsrc(static_cast<const char*>(w.B) + (int64_t)u.ca * 16 * (KN ? 1 : w.ldb) * ELT)),
+          lane(threadIdx.x & 63), grp(lane >> 4), lda((int)w.lda), ldb((int)w.ldb), k(w.k), lds(lds_) {
+        aoff = ((lane >> 3) * lda + (lane & 7) * VE) * ELT;
+        if constexpr (!KN)
+            boff = ((lane >> 3) * ldb + (lane & 7) * VE) * ELT;
+        else if constexpr (F64)
+            boff = (2 * grp * ldb + (lane & 15)) * ELT;  // sub-step e takes row k = 2 grp + e
+        else
+            boff = (lane / PPR * ldb + (lane % PPR) * 8) * ELT;
+        woff = (lane >> 3) * 128 + (((lane & 7) ^ ((lane >> 5) << 1)) << 4);
+        roff = (lane & 15) * 128 + ((grp ^ (((lane >> 2) & 3) << 1)) << 4);
+    }
+
+    __device__ __forceinline__ void load(Stage& s, int c) const {
+        // pieces past K lie out of the descriptor's range; the scalar offsets stay inside
+        // the operand
+        const int k0 = c * KS, kb = k0 < k ? k0 : 0;
+        const bool ok = F64 ? k0 < k : k0 + (lane & 7) * VE < k;  // K is a multiple of 16
+        const int ao = ok ? aoff : kBufferRange, bo = ok ? boff : kBufferRange;
 #pragma unroll
-        for (int ks = 0; ks < SG::KC / AT::KSTEP; ++ks) {
-            const int kk = (ks * AT::KSTEP + AT::KV * (lane >> 4)) * SG::ELT;
-            frag_t bf[V::JN];
+        for (int i = 0; i < NA; ++i) s.a[i] = buffer_load16(ra, ao, (i * 8 * lda + kb) * ELT);
+        if constexpr (!KN) {
 #pragma unroll
-            for (int jn = 0; jn < V::JN; ++jn)
-                bf[jn] = bitcast<frag_t>(load_raw<FB>(
-                    bb + (wn * V::SUBN + jn * 16 + (lane & 15)) * SG::ROWB + kk));
-            auto a_frag = [&](int im) {
-                return bitcast<frag_t>(load_raw<FB>(
-                    base + (wm * V::SUBM + im * 16 + (lane & 15)) * SG::ROWB + kk));
-            };
-            if constexpr (V::IM * V::JN >= 16) {
-                // the 128 x 128 FP64 tile: its 128 accumulator VGPRs leave room for one
-                // A fragment at a time; the JN products of a fragment's sub-step separate
-                // the two sub-steps of one accumulator.  Row and column atoms past the
-                // problem's edge are skipped (wave-uniform branches): M and N are
-                // multiples of 16, so no product is wasted
+            for (int j = 0; j < NB; ++j) s.b[j] = buffer_load16(rb, bo, (j * 8 * ldb + kb) * ELT);
+        } else if constexpr (F64) {
 #pragma unroll
-                for (int im = 0; im < V::IM; ++im) {
-                    if (im >= im_live) break;
-                    const frag_t af = a_frag(im);
+            for (int t = 0; t < NF; ++t)
 #pragma unroll
-                    for (int e = 0; e < AT::NSUB; ++e)
-#pragma unroll
-                        for (int jn = 0; jn < V::JN; ++jn)
-                            if (jn < jn_live) AT::mma_sub(acc[im][jn], af, bf[jn], e);
+                for (int j = 0; j < JN; ++j) {
+                    const int so = ((kb + t * AT::KSTEP) * ldb + j * 16) * ELT;
+                    const d2_t x = {buffer_load8(rb, bo, so), buffer_load8(rb, bo, so + ldb * ELT)};
+                    s.b[j * NF + t] = bitcast<u4_t>(x);
                 }
-            } else {
-                frag_t af[V::IM];
+        } else {
+            constexpr int RPL = 64 / PPR;  // K rows of one load instruction
 #pragma unroll
-                for (int im = 0; im < V::IM; ++im) af[im] = a_frag(im);
-                // sub-steps of a fragment (FP64: two 16x16x4 instructions) interleaved
-                // across the accumulators, so no instruction waits on the one just issued
-#pragma unroll
-                for (int e = 0; e < AT::NSUB; ++e)
-#pragma unroll
-                    for (int jn = 0; jn < V::JN; ++jn)
-#pragma unroll
-                        for (int im = 0; im < V::IM; ++im)
-                            AT::mma_sub(acc[im][jn], af[im], bf[jn], e);
+            for (int i = 0; i < NB; ++i) {
+                const int r = k0 + i * RPL;
+                s.b[i] = buffer_load16(rb, r + lane / PPR < k ? boff : kBufferRange,
+                                       (r < k ? r : 0) * ldb * ELT);
             }
         }
-    };
-    // stage of parity P: products from LDS buffer P, then the next stage (slot 1 - P) to
-    // LDS buffer 1 - P and the cursor's stage into that slot
-    auto stage0 = [&]() {
-        compute(smem);
-        advance_slot<AT, KN, 1>(st, q, smem);
-        __syncthreads();
-        ++st.x;
-    };
-    auto stage1 = [&]() {
-        compute(smem + SG::STAGE);
-        advance_slot<AT, KN, 0>(st, q, smem);
-        __syncthreads();
-        ++st.x;
-    };
-    int c = 0;
-    if ((st.x & 1) && c < nch) {
-        stage1();
-        ++c;
     }
-    for (; c + 1 < nch; c += 2) {
-        stage0();
-        stage1();
-    }
-    if (c < nch) stage0();
 
-    const acc_t alpha = (acc_t)a.alpha, beta = (acc_t)a.beta;
-    out_t* C = reinterpret_cast<out_t*>(cur.C);
+    // Stage registers to LDS (a wave's LDS accesses complete in order: no wait between the
+    // reads of one stage and the writes of the next)
+    __device__ __forceinline__ void write(const Stage& s) const {
 #pragma unroll
-    for (int im = 0; im < V::IM; ++im)
+        for (int i = 0; i < NA; ++i) store_raw<16>(lds + (woff ^ ((i & 1) * 64)) + i * 1024, s.a[i]);
+        if constexpr (!KN) {
 #pragma unroll
-        for (int jn = 0; jn < V::JN; ++jn) {
-            const int rb = wm * V::SUBM + im * 16, cb = wn * V::SUBN + jn * 16;
-            if (rb >= mlim || cb >= nlim) continue;
-            const int col = cb + (lane & 15);
+            for (int j = 0; j < NB; ++j)
+                store_raw<16>(lds + A_LDS + (woff ^ ((j & 1) * 64)) + j * 1024, s.b[j]);
+        } else if constexpr (TURN) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int row = rb + AT::out_row(lane, v);
-                out_t* dst = C + (int64_t)row * cur.ldc + col;
-                acc_t val = alpha * acc[im][jn][v];
-                if (beta != (acc_t)0) val += beta * (acc_t)(*dst);
-                *dst = (out_t)val;
-            }
+            for (int i = 0; i < NB; ++i)
+                store_raw<16>(lds + A_LDS + (i * (64 / PPR) + lane / PPR) * TROW + (lane % PPR) * 16, s.b[i]);
         }
-}
+    }
 
-// Two workgroups per CU: the 128 x 128 FP64 tile holds 128 accumulator VGPRs per lane,
-// and FP16/BF16 staging takes 60 KB of LDS.
+    struct Frags {
+        frag_t a[IM][NF], b[JN][NF];
+    };
+    // Fragments of the stage in LDS (FP64 K x N: `s`, which holds B's as loaded)
+    __device__ __forceinline__ void read(const Stage& s, Frags& f) const {
+#pragma unroll
+        for (int i = 0; i < IM; ++i)
+#pragma unroll
+            for (int t = 0; t < NF; ++t)
+                f.a[i][t] = bitcast<frag_t>(load_raw<16>(lds + (roff ^ (t * 64)) + i * 2048));
+        if constexpr (TURN) {
+            const unsigned char* p = lds + A_LDS + (8 * grp + ((lane & 15) >> 2)) * TROW + 8 * (lane & 3);
+#pragma unroll
+            for (int j = 0; j < JN; ++j)
+#pragma unroll
+                for (int t = 0; t < NF; ++t) {
+                    const u2_t lo = lds_read_turned(p + t * 32 * TROW + j * 32);
+                    const u2_t hi = lds_read_turned(p + (t * 32 + 4) * TROW + j * 32);
+                    f.b[j][t] = bitcast<frag_t>(u4_t{lo[0], lo[1], hi[0], hi[1]});
+                }
+        } else {
+#pragma unroll
+            for (int j = 0; j < JN; ++j)
+#pragma unroll
+                for (int t = 0; t < NF; ++t)
+                    f.b[j][t] = KN ? bitcast<frag_t>(s.b[j * NF + t])
+                                   : bitcast<frag_t>(load_raw<16>(lds + A_LDS + (roff ^ (t * 64)) + j * 2048));
+        }
+    }
+
+    __device__ __forceinline__ void mma(const Frags& f, accv_t (&acc)[IM][JN]) const {
+#pragma unroll
+        for (int t = 0; t < NF; ++t)
+#pragma unroll
+            for (int e = 0; e < AT::NSUB; ++e)
+#pragma unroll
+                for (int j = 0; j < JN; ++j)
+#pragma unroll
+                    for (int i = 0; i < IM; ++i) AT::mma_sub(acc[i][j], f.a[i][t], f.b[j][t], e);
+    }
+
+    __device__ __forceinline__ void run(const WorkItem& w, const WaveUnit& u, double alpha_d,
+                                        double beta_d) const {
+        accv_t acc[IM][JN];
+#pragma unroll
+        for (int i = 0; i < IM; ++i)
+#pragma unroll
+            for (int j = 0; j < JN; ++j) acc[i][j] = accv_t{0, 0, 0, 0};
+        // Stage c in LDS, stage c + 1 in registers or on its way.  Straight-line stages: a
+        // branch around a load would make the compiler wait for every load in flight where
+        // the paths meet, so the stage past the last one is loaded too, out of range (no
+        // memory traffic).
+        Stage s;
+        Frags f;
+        const int n = (k + KS - 1) / KS;
+        load(s, 0);
+        for (int c = 1; c < n; ++c) {
+            write(s);
+            read(s, f);
+            load(s, c);
+            __builtin_amdgcn_sched_barrier(0);
+            mma(f, acc);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        write(s);
+        read(s, f);
+        mma(f, acc);
+        const acc_t alpha = (acc_t)alpha_d, beta = (acc_t)beta_d;
+        KAMI_GLOBAL out_t* C = (KAMI_GLOBAL out_t*)w.C + ((int64_t)u.ra * 16 * w.ldc + u.ca * 16);
+#pragma unroll
+        for (int i = 0; i < IM; ++i)
+#pragma unroll
+            for (int j = 0; j < JN; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    KAMI_GLOBAL out_t* dst = C + (int64_t)(i * 16 + AT::out_row(lane, v)) * w.ldc + j * 16 + (lane & 15);
+                    acc_t val = alpha * acc[i][j][v];
+                    if (beta != (acc_t)0) val += beta * (acc_t)(*dst);
+                    *dst = (out_t)val;
+                }
+    }
+};
+
+// One wave per unit; a workgroup is four consecutive units (neighbouring wave tiles of
+// one problem share its lines of A and B in the CU's L1).
 template <class AT, bool KN>
 __global__ void __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(2)))
-batched_persistent_kernel(BatchArgs args) {
-    using SG = StreamGeom<AT>;
-    using VS = Variants<AT>;
-    __shared__ __attribute__((aligned(16))) unsigned char smem[SG::LDS];
-    __shared__ QueueLds q;
-    Stream<AT> st;
-    st.t0 = st.tc = 0;
-    st.cc = 0;
-    st.blocked = false;
-    st.x = st.loaded = 0;
-    st.fetched = 0;
-    st.phase = -1;
-    st.fvalid = false;
-    st.sv0 = st.sv1 = -1;
-    st.qs = min(kQueueShift, max(1, uni(args.qshift)));
-    st.qb = 1 << st.qs;
-    st.lead = max(1, st.qb - kFetchAhead);
-    // prologue: the first batch synchronously
-    ensure_ready(args, st, q, 0);
-    st.cur = stream_tile<AT>(q, 0, st.qs);
-    if (!st.cur.valid) return;  // uniform: the queue is empty
-    st.ct = st.cur;
-    // stage 0 into LDS buffer 0, stage 1 into slot 1, stage 2 into slot 0
-    load_at_cursor<AT, KN>(st, q, st.slot0);
-    stream_write<AT, KN>(st.slot0, smem);
-    st.sv1 = load_at_cursor<AT, KN>(st, q, st.slot1);
-    st.sv0 = load_at_cursor<AT, KN>(st, q, st.slot0);
-    __syncthreads();
-    while (true) {
-        switch (st.cur.variant) {
-            case 0: run_tile<AT, KN, typename VS::V0>(args, st, q, smem); break;
-            case 1: run_tile<AT, KN, typename VS::V1>(args, st, q, smem); break;
-            case 2: run_tile<AT, KN, typename VS::V2>(args, st, q, smem); break;
-            case 3: run_tile<AT, KN, typename VS::V3>(args, st, q, smem); break;
-            default:  // 4 and 5 exist where B is staged 128 columns wide
-                if constexpr (SG::TNMAX >= 128) {
-                    if (st.cur.variant == 4)
-                        run_tile<AT, KN, typename VS::V4>(args, st, q, smem);
-                    else
-                        run_tile<AT, KN, typename VS::V5>(args, st, q, smem);
-                }
-                break;
-        }
-        // ---- tile boundary ----
-        ++st.t0;
-        // the next batch is requested at tile `lead` (at least 1) of the current one,
-        // which is then fetched; a fetch in flight takes one step per tile boundary (the
-        // buffer it fills is the one of the batch before the current one, which the
-        // tile and the cursor have left)
-        if (st.phase < 0 && (int)(st.t0 & (st.qb - 1)) == st.lead &&
-            st.fetched == st.t0 - st.lead + st.qb)
-            st.phase = 0;
-        if (st.phase >= 0) {
-            fetch_step(args, st, q);
-            __syncthreads();
-            fetch_commit(st);
-        }
-        ensure_ready(args, st, q, st.t0);  // uniform; normally already done
-        st.cur = stream_tile<AT>(q, st.t0, st.qs);
-        if (!st.cur.valid) break;  // uniform
-        // a blocked cursor resumes; stages that could not be loaded are loaded now
-        if (st.blocked) {
-            ensure_ready(args, st, q, st.tc);
-            st.ct = stream_tile<AT>(q, st.tc, st.qs);
-            st.blocked = false;
-            if (st.loaded == st.x) {
-                // the new tile's first stage: through its slot straight to its LDS buffer
-                load_next_into_slot<AT, KN>(st, q);
-                if (st.x & 1) {
-                    stream_write<AT, KN>(st.slot1, smem + SG::STAGE);
-                    st.sv1 = -1;
-                } else {
-                    stream_write<AT, KN>(st.slot0, smem);
-                    st.sv0 = -1;
-                }
-            }
-            // then stages x + 1 and x + 2 into their slots, as far as the fetched tiles
-            // reach: a cursor that blocks again (the batch just fetched holds fewer
-            // stages than that) stays blocked until the next tile boundary repairs it
-            while (st.loaded < st.x + 3 && st.ct.valid && !st.blocked)
-                load_next_into_slot<AT, KN>(st, q);
-            __syncthreads();
-        }
+__attribute__((amdgpu_waves_per_eu(4)))
+batched_wave_kernel(BatchArgs args) {
+    constexpr int LDS_WAVE = WaveTile<AT, KN, kWaveAtoms, kWaveAtoms>::LDS;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[kWavesPerGroup * LDS_WAVE];
+    const int wave = uni(threadIdx.x >> 6);
+    unsigned char* const lds = smem + wave * LDS_WAVE;
+    const WaveUnit u = load_uniform(args.units + ((int64_t)blockIdx.x * kWavesPerGroup + wave));
+    if (u.im == 0) return;
+    const WorkItem w = load_uniform(args.items + u.item);
+    const int shape = u.im * kWaveAtoms + u.jn - kWaveAtoms - 1;
+    switch (shape) {
+        case 0: WaveTile<AT, KN, 1, 1>(w, u, lds).run(w, u, args.alpha, args.beta); break;
+        case 1: WaveTile<AT, KN, 1, 2>(w, u, lds).run(w, u, args.alpha, args.beta); break;
+        case 2: WaveTile<AT, KN, 2, 1>(w, u, lds).run(w, u, args.alpha, args.beta); break;
+        default: WaveTile<AT, KN, 2, 2>(w, u, lds).run(w, u, args.alpha, args.beta); break;
     }
-}
-
-__global__ void reset_counter_kernel(unsigned int* counter) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *counter = 0u;
 }
 
 static int size_class(int x) { return x <= 32 ? 0 : x <= 64 ? 1 : x <= 128 ? 2 : x <= 256 ? 3 : 4; }
@@ -608,9 +340,8 @@ static int bucket_of(const kami_problem& p) {
 
 // Prior variant of a bucket: the largest tile that the problem fills, following the
 // reference's choice of fewer, larger warps for larger sizes
-// (scripts/fp64_batched_GH200.sh:7-14).  FP64 takes 128 rows or columns wherever the
-// problem has more than 64 of them (its batches are bound by HBM, and the wider tile
-// halves the re-reads of the other operand).
+// (scripts/fp64_batched_GH200.sh:7-14).  The tile is what the queue counts and deals out;
+// every prior's wave tiles are 32 x 32.
 static int prior_variant(int prec, int bucket) {
     const int cm = bucket / 25, cn = (bucket / 5) % 5;
     if (cm == 0 && cn == 0) return 1;
@@ -632,78 +363,154 @@ struct kami_batched_plan {
     int prec = 0;
     int64_t problems = 0;
     int64_t n_items = 0;
-    int grid = 0;
+    int64_t n_units = 0;
     double flops = 0;
     int b_kn = 0;
     double alpha = 1.0, beta = 0.0;
     WorkItem* d_items = nullptr;
-    unsigned int* d_counter = nullptr;
-    bool use_graph = false;
-    hipStream_t cap_stream = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
+    WaveUnit* d_units = nullptr;
     std::vector<int> bucket_ids;      // non-empty buckets, ascending
     std::vector<int> bucket_variant;  // chosen variant per non-empty bucket
 };
 
 namespace kami {
 
+// Workgroups of one execution: one per kWavesPerGroup units.
+static int64_t batched_groups(int64_t n_units) { return n_units / kWavesPerGroup; }
+
+// A dispatch holds fewer than 2^32 work-items; longer queues take several.
+constexpr int64_t kMaxGroups = (int64_t)1 << 23;
+
 template <class AT>
-static hipError_t launch_for(const BatchArgs& a, int grid, hipStream_t s) {
-    if (a.b_kn)
-        hipLaunchKernelGGL((batched_persistent_kernel<AT, true>), dim3(grid), dim3(256), 0, s, a);
-    else
-        hipLaunchKernelGGL((batched_persistent_kernel<AT, false>), dim3(grid), dim3(256), 0, s, a);
-    return hipGetLastError();
+static hipError_t launch_for(BatchArgs a, bool kn, hipStream_t s) {
+    hipError_t e = hipSuccess;
+    for (int64_t left = batched_groups(a.n_units); left > 0 && e == hipSuccess; left -= kMaxGroups) {
+        const dim3 grid((unsigned)std::min(left, kMaxGroups));
+        if (kn)
+            hipLaunchKernelGGL((batched_wave_kernel<AT, true>), grid, dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL((batched_wave_kernel<AT, false>), grid, dim3(256), 0, s, a);
+        e = hipGetLastError();
+        a.units += kMaxGroups * kWavesPerGroup;
+    }
+    return e;
 }
 
-// log2 of the entries per pop: kQueueBatch when every workgroup gets three batches or
-// more, fewer for a short queue (4096 tiles over 768 workgroups: two entries per pop).
-static int32_t queue_shift(int64_t n_items, int grid) {
-    const int64_t per = n_items / (3 * (int64_t)std::max(grid, 1));
+// log2 of the entries dealt to one of `takers` XCDs at a time: as many as leave every XCD
+// three deals or more, from 2 to 1 << kQueueShift.
+static int32_t queue_shift(int64_t n_items, int takers) {
+    const int64_t per = n_items / (3 * (int64_t)std::max(takers, 1));
     int32_t sh = 1;
     while (sh < kQueueShift && (int64_t(2) << sh) <= per) ++sh;
     return sh;
 }
 
-static hipError_t launch_batched(int prec, const BatchArgs& a, int grid, hipStream_t s) {
-    hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(64), 0, s, a.counter);
-    if (prec == KAMI_PREC_F64) return launch_for<AtomF64>(a, grid, s);
-    if (prec == KAMI_PREC_F16_F32) return launch_for<AtomF16x32>(a, grid, s);
-    return launch_for<AtomBF16x32>(a, grid, s);
+static hipError_t launch_batched(int prec, const BatchArgs& a, bool kn, hipStream_t s) {
+    if (prec == KAMI_PREC_F64) return launch_for<AtomF64>(a, kn, s);
+    if (prec == KAMI_PREC_F16_F32) return launch_for<AtomF16x32>(a, kn, s);
+    return launch_for<AtomBF16x32>(a, kn, s);
 }
 
-template <class AT>
-static hipError_t occupancy_for(bool kn, int* per_cu) {
-    if (kn)
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, batched_persistent_kernel<AT, true>, 256, 0);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, batched_persistent_kernel<AT, false>, 256, 0);
+// The wave tiles of one queue entry, two by two so that four consecutive ones form a
+// square (they share lines of A and B).
+struct UnitCursor {
+    int rows = 0, cols = 0;  // wave tiles of the entry
+    int r = 0, c = 0;        // next one
+    int am = 0, an = 0;      // atoms of the entry
+    int sm = 1, sn = 1;      // atoms of a wave tile
+    bool done = true;
+    void start(const WorkItem& w, int cap) {
+        am = std::min(w.mlim, kVariantTM[w.variant]) / 16;
+        an = std::min(w.nlim, kVariantTN[w.variant]) / 16;
+        sm = std::min(cap >> 1 ? 2 : 1, kVariantSM[w.variant]);
+        sn = std::min(cap & 1 ? 2 : 1, kVariantSN[w.variant]);
+        rows = (am + sm - 1) / sm;
+        cols = (an + sn - 1) / sn;
+        r = c = 0;
+        done = false;
+    }
+    WaveUnit take(uint32_t item) {
+        const WaveUnit u{item, (uint8_t)(r * sm), (uint8_t)(c * sn),
+                         (uint8_t)std::min(sm, am - r * sm), (uint8_t)std::min(sn, an - c * sn)};
+        if ((c & 1) == 0 && c + 1 < cols) {
+            ++c;
+        } else if ((r & 1) == 0 && r + 1 < rows) {
+            ++r;
+            c &= ~1;
+        } else if ((c | 1) + 1 < cols) {
+            c = (c | 1) + 1;
+            r &= ~1;
+        } else {
+            r = (r | 1) + 1;
+            c = 0;
+            done = r >= rows;
+        }
+        return u;
+    }
+};
+
+// Wave tiles of all entries for wave tiles of up to (cap >> 1 ? 2 : 1) x (cap & 1 ? 2 : 1)
+// atoms, rounded up to whole workgroups.
+static int64_t count_units(const WorkItem* items, int64_t n_items, int cap) {
+    int64_t n = 0;
+    UnitCursor u;
+    for (int64_t i = 0; i < n_items; ++i) {
+        u.start(items[i], cap);
+        n += (int64_t)u.rows * u.cols;
+    }
+    return (n + kWavesPerGroup - 1) / kWavesPerGroup * kWavesPerGroup;
 }
 
-static hipError_t persistent_grid(int prec, bool kn, int* grid) {
-    int dev = 0, cus = 0, per_cu = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e != hipSuccess) return e;
-    if (prec == KAMI_PREC_F64)
-        e = occupancy_for<AtomF64>(kn, &per_cu);
-    else if (prec == KAMI_PREC_F16_F32)
-        e = occupancy_for<AtomF16x32>(kn, &per_cu);
-    else
-        e = occupancy_for<AtomBF16x32>(kn, &per_cu);
-    if (e != hipSuccess) return e;
-    *grid = std::max(1, cus * std::max(1, per_cu));
-    return hipSuccess;
+// Fewest wave tiles that fill the chip (four a SIMD); below that the wave tiles are made
+// smaller, 16 x 32 and then 16 x 16, until there are as many.  FP64, problems of 16 to 256:
+// 8 of them 6.0 us against 9.9 with 32 x 32 tiles, 100 9.1 against 13.5, 300 14.7 against
+// 17.2 (and 17.2 with 2048 here); FP16 is bound by the launch itself there.
+constexpr int64_t kFullUnits = 4096;
+
+static int wave_cap(const WorkItem* items, int64_t n_items, int64_t* n_units) {
+    int cap = 3;
+    while ((*n_units = count_units(items, n_items, cap)) < kFullUnits && cap > 0) cap = cap == 3 ? 1 : 0;
+    return cap;
+}
+
+// The wave units in launch order.  Workgroup L runs on XCD L mod kXcds; every XCD takes
+// deals of consecutive entries (neighbouring tiles of a problem, or problems of nearly
+// equal cost), so the tiles that share rows of A or columns of B run on one XCD at the
+// same time and its L2 serves all but the first reader.
+static void build_units(const WorkItem* items, int64_t n_items, int cap, int64_t n_units, WaveUnit* out) {
+    struct {
+        int64_t item = 0, end = 0;
+        UnitCursor u;
+    } x[kXcds];
+    const int64_t deal = (int64_t)1 << queue_shift(n_items, kXcds);
+    int64_t next = 0;
+    auto more = [&](int q) {  // the next unit of XCD q's stream, dealing again when needed
+        if (!x[q].u.done) return true;
+        if (++x[q].item >= x[q].end) {
+            if (next >= n_items) {
+                x[q].item = x[q].end;
+                return false;
+            }
+            x[q].item = next;
+            x[q].end = next = std::min(n_items, next + deal);
+        }
+        x[q].u.start(items[x[q].item], cap);
+        return true;
+    };
+    for (int64_t i = 0; i < n_units; ++i) {
+        const int q = (int)(i / kWavesPerGroup % kXcds);
+        int t = 0;
+        while (t < kXcds && !more((q + t) % kXcds)) ++t;  // an empty stream takes from another
+        out[i] = t < kXcds ? x[(q + t) % kXcds].u.take((uint32_t)x[(q + t) % kXcds].item)
+                           : WaveUnit{0, 0, 0, 0, 0};
+    }
 }
 
 // Queue entries of the problems: every problem cut into tiles of its bucket's variant,
 // each entry carrying the tile's own operand pointers.  Problems are ordered longest
 // first (by m n k) so the tail of the queue holds the cheapest work, and a problem's tiles
-// stay consecutive in row-major order: a workgroup pops a batch of neighbouring tiles at
-// once, so tiles that share rows of A or columns of B run on one CU, back to back, and
-// find those operands in its L2 instead of fetching them again (ordering by tile cost
-// scattered them over all XCDs and read A and B 1.8 times over).
+// stay consecutive in row-major order, so that build_units can put the tiles that share
+// rows of A or columns of B on one XCD together.
 // Queue entries of `count` problems (bucket[p] their size bucket), written to out[];
 // `order` is room for `count` indices.  Equal-cost problems keep their input order
 // (an index tie-break instead of a stable sort, which may allocate).
@@ -808,17 +615,35 @@ static kami_status upload(const void* host, size_t bytes, void** dev) {
     return KAMI_OK;
 }
 
+// The entries and their wave units on the device.
+static kami_status upload_queue(const std::vector<WorkItem>& items, WorkItem** d_items,
+                                WaveUnit** d_units, int64_t* n_units) {
+    const int64_t n = (int64_t)items.size();
+    if (n > UINT32_MAX) return KAMI_ENOMEM;  // 256 GiB of entries
+    const int cap = wave_cap(items.data(), n, n_units);
+    std::unique_ptr<WaveUnit[]> units(new (std::nothrow) WaveUnit[(size_t)*n_units]);
+    if (!units) return KAMI_ENOMEM;
+    build_units(items.data(), n, cap, *n_units, units.get());
+    kami_status st = upload(items.data(), items.size() * sizeof(WorkItem), (void**)d_items);
+    if (st == KAMI_OK) st = upload(units.get(), (size_t)*n_units * sizeof(WaveUnit), (void**)d_units);
+    return st;
+}
+
 // ---- one-shot execution without allocation ----
-// The queue and its counter of kami_batched_gemm_static live in `scratch`, a file-scope
-// device array (each device holds its own copy until the process ends): the counter in its
-// first 256 bytes, then up to kStaticItems queue entries.  Host code reaches a device's
-// copy only through the address hipGetSymbolAddress returns with that device current (the
-// array's name is a host-side stand-in, not a device address).  The host side stages the
-// problems, their order and the entries in static arrays, so the call makes no allocation
-// of device or host memory; a mutex keeps two host threads from sharing the staging.
+// The queue of kami_batched_gemm_static lives in `scratch`, a file-scope device array
+// (each device holds its own copy until the process ends): up to kStaticItems queue
+// entries, and behind them their wave units, at most kStaticUnits (16 wave tiles of
+// 32 x 32 in an entry of 128 x 128; smaller wave tiles only while there are fewer than
+// kFullUnits).  Host code reaches a device's copy only through the address
+// hipGetSymbolAddress returns with that device current (the array's name is a host-side
+// stand-in, not a device address).  The host side stages the problems, their order and
+// the queue in static arrays, so the call makes no allocation of device or host memory; a
+// mutex keeps two host threads from sharing the staging.
 constexpr int64_t kStaticItems = 32768;  // 2 MiB of queue entries
-constexpr size_t kStaticCounterBytes = 256;
-static __device__ __align__(256) unsigned char scratch[kStaticCounterBytes + kStaticItems * sizeof(WorkItem)];
+constexpr int64_t kStaticUnits = 16 * kStaticItems;
+constexpr size_t kStaticBytes = kStaticItems * sizeof(WorkItem) + kStaticUnits * sizeof(WaveUnit);
+static_assert(4 * kFullUnits + kWavesPerGroup <= kStaticUnits, "small wave tiles fit");
+static __device__ __align__(256) unsigned char scratch[kStaticBytes];
 
 struct StaticStaging {
     std::mutex mu;
@@ -826,7 +651,7 @@ struct StaticStaging {
     kami_problem probs[kStaticItems];  // a problem holds at least one entry
     int bucket[kStaticItems];
     int64_t order[kStaticItems];
-    WorkItem items[kStaticItems];
+    alignas(16) unsigned char queue[kStaticBytes];  // entries, then units
 };
 static StaticStaging g_static;
 
@@ -848,11 +673,8 @@ static kami_status static_scratch(unsigned char** out) {
 
 static void free_plan(kami_batched_plan* p) {
     if (!p) return;
-    if (p->exec) (void)hipGraphExecDestroy(p->exec);
-    if (p->graph) (void)hipGraphDestroy(p->graph);
-    if (p->cap_stream) (void)hipStreamDestroy(p->cap_stream);
     if (p->d_items) (void)hipFree(p->d_items);
-    if (p->d_counter) (void)hipFree(p->d_counter);
+    if (p->d_units) (void)hipFree(p->d_units);
     delete p;
 }
 
@@ -893,7 +715,6 @@ kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count, i
     plan->b_kn = o.b_layout == KAMI_B_KN;
     plan->alpha = o.alpha;
     plan->beta = o.beta;
-    plan->use_graph = o.use_graph != 0;
 
     std::vector<int> bucket(hp.size());
     int variant_of_bucket[125];
@@ -904,17 +725,7 @@ kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count, i
     }
     untimed_variants(precision, variant_of_bucket);
 
-    hipError_t e = persistent_grid(precision, plan->b_kn, &plan->grid);
-    if (e != hipSuccess) {
-        free_plan(plan);
-        return hip_fail(e);
-    }
-    st = upload(nullptr, 0, (void**)&plan->d_counter);
-    if (st != KAMI_OK) {
-        free_plan(plan);
-        return st;
-    }
-
+    hipError_t e = hipSuccess;
     if (o.autotune) {
         // time every variant on up to 256 problems of each bucket, keep the fastest.  The
         // sample is repeated until it carries at least kTuneProblems problems so that every
@@ -949,19 +760,25 @@ kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count, i
                 std::vector<WorkItem> items;
                 build_items(sample, sb, vb, ei, eo, plan->b_kn, items);
                 WorkItem* d_it = nullptr;
-                st = upload(items.data(), items.size() * sizeof(WorkItem), (void**)&d_it);
-                if (st != KAMI_OK) break;
-                BatchArgs a{d_it, plan->d_counter, (int64_t)items.size(), o.alpha, 0.0, plan->b_kn,
-                            queue_shift((int64_t)items.size(), plan->grid)};
-                e = launch_batched(precision, a, plan->grid, s);  // warm-up
+                WaveUnit* d_un = nullptr;
+                int64_t n_units = 0;
+                st = upload_queue(items, &d_it, &d_un, &n_units);
+                if (st != KAMI_OK) {
+                    if (d_it) (void)hipFree(d_it);
+                    if (d_un) (void)hipFree(d_un);
+                    break;
+                }
+                BatchArgs a{d_it, d_un, n_units, o.alpha, 0.0};
+                e = launch_batched(precision, a, plan->b_kn, s);  // warm-up
                 if (e == hipSuccess) e = hipEventRecord(e0, s);
                 for (int rep = 0; rep < 3 && e == hipSuccess; ++rep)
-                    e = launch_batched(precision, a, plan->grid, s);
+                    e = launch_batched(precision, a, plan->b_kn, s);
                 if (e == hipSuccess) e = hipEventRecord(e1, s);
                 if (e == hipSuccess) e = hipEventSynchronize(e1);
                 float ms = 0;
                 if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
                 (void)hipFree(d_it);
+                (void)hipFree(d_un);
                 if (e != hipSuccess) {
                     st = hip_fail(e);
                     break;
@@ -984,7 +801,7 @@ kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count, i
     std::vector<WorkItem> items;
     build_items(hp, bucket, variant_of_bucket, ei, eo, plan->b_kn, items);
     plan->n_items = (int64_t)items.size();
-    st = upload(items.data(), items.size() * sizeof(WorkItem), (void**)&plan->d_items);
+    st = upload_queue(items, &plan->d_items, &plan->d_units, &plan->n_units);
     if (st != KAMI_OK) {
         free_plan(plan);
         return st;
@@ -995,22 +812,6 @@ kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count, i
             plan->bucket_variant.push_back(variant_of_bucket[b]);
         }
 
-    if (plan->use_graph) {
-        e = hipStreamCreateWithFlags(&plan->cap_stream, hipStreamNonBlocking);
-        if (e == hipSuccess) e = hipStreamBeginCapture(plan->cap_stream, hipStreamCaptureModeThreadLocal);
-        if (e == hipSuccess) {
-            BatchArgs a{plan->d_items, plan->d_counter, plan->n_items, plan->alpha,
-                        plan->beta, plan->b_kn, queue_shift(plan->n_items, plan->grid)};
-            hipError_t le = launch_batched(precision, a, plan->grid, plan->cap_stream);
-            e = hipStreamEndCapture(plan->cap_stream, &plan->graph);
-            if (le != hipSuccess) e = le;
-        }
-        if (e == hipSuccess) e = hipGraphInstantiate(&plan->exec, plan->graph, nullptr, nullptr, 0);
-        if (e != hipSuccess) {
-            free_plan(plan);
-            return hip_fail(e);
-        }
-    }
     *out = plan;
     return KAMI_OK;
 }
@@ -1018,14 +819,8 @@ kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count, i
 kami_status kami_batched_execute(kami_batched_plan* plan, void* stream) {
     if (!plan) return KAMI_EINVAL;
     hipStream_t s = (hipStream_t)stream;
-    hipError_t e;
-    if (plan->use_graph) {
-        e = hipGraphLaunch(plan->exec, s);
-    } else {
-        BatchArgs a{plan->d_items, plan->d_counter, plan->n_items, plan->alpha,
-                    plan->beta, plan->b_kn, queue_shift(plan->n_items, plan->grid)};
-        e = launch_batched(plan->prec, a, plan->grid, s);
-    }
+    const BatchArgs a{plan->d_items, plan->d_units, plan->n_units, plan->alpha, plan->beta};
+    const hipError_t e = launch_batched(plan->prec, a, plan->b_kn, s);
     if (e != hipSuccess) return hip_fail(e);
     return KAMI_OK;
 }
@@ -1036,7 +831,7 @@ kami_status kami_batched_plan_info(const kami_batched_plan* plan, kami_plan_info
     out->problems = plan->problems;
     out->work_items = plan->n_items;
     out->buckets = (int32_t)plan->bucket_ids.size();
-    out->workgroups = plan->grid;
+    out->workgroups = (int32_t)std::min<int64_t>(batched_groups(plan->n_units), INT32_MAX);
     out->flops = plan->flops;
     for (size_t i = 0; i < plan->bucket_variant.size() && i < 16; ++i)
         out->variant_of_bucket[i] = plan->bucket_variant[i];
@@ -1081,22 +876,23 @@ kami_status kami_batched_gemm_static(const kami_problem* probs, int64_t count, i
     unsigned char* base = nullptr;
     st = static_scratch(&base);
     if (st != KAMI_OK) return st;
-    int grid = 0;
-    hipError_t e = persistent_grid(precision, b_kn, &grid);
-    if (e != hipSuccess) return hip_fail(e);
+    WorkItem* const items = reinterpret_cast<WorkItem*>(g_static.queue);
+    WaveUnit* const units = reinterpret_cast<WaveUnit*>(items + n_items);
     build_items(g_static.probs, count, g_static.bucket, variant_of_bucket, ei, eo, b_kn,
-                g_static.order, g_static.items);
+                g_static.order, items);
+    int64_t n_units = 0;
+    const int cap = wave_cap(items, n_items, &n_units);
+    build_units(items, n_items, cap, n_units, units);
     hipStream_t s = (hipStream_t)stream;
     // From pageable memory the copy has consumed the staging array when the call returns,
     // so the next call may refill it.
-    WorkItem* d_items = reinterpret_cast<WorkItem*>(base + kStaticCounterBytes);
-    e = hipMemcpyAsync(d_items, g_static.items, (size_t)n_items * sizeof(WorkItem),
-                       hipMemcpyHostToDevice, s);
+    hipError_t e = hipMemcpyAsync(base, g_static.queue,
+                                  (size_t)n_items * sizeof(WorkItem) + (size_t)n_units * sizeof(WaveUnit),
+                                  hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return hip_fail(e);
-    // launch_batched resets the counter with a kernel before the persistent launch
-    BatchArgs a{d_items, reinterpret_cast<unsigned int*>(base), n_items, o.alpha, o.beta,
-                (int32_t)b_kn, queue_shift(n_items, grid)};
-    e = launch_batched(precision, a, grid, s);
+    const WorkItem* d_items = reinterpret_cast<const WorkItem*>(base);
+    BatchArgs a{d_items, reinterpret_cast<const WaveUnit*>(d_items + n_items), n_units, o.alpha, o.beta};
+    e = launch_batched(precision, a, b_kn, s);
     if (e != hipSuccess) return hip_fail(e);
     return KAMI_OK;
 }

@@ -8,8 +8,8 @@ on the device):
   w3  FP64 through int8 / FP16 digits, M = N = K = 128, 4096 problems, sign-random
       entries with log10|x| ~ U[-4, 4], against native FP64 (timed by bench.py);
   w4  batched uneven sizes: 20000 problems, M, N, K log-uniform in [16, 256] rounded to
-      multiples of 16, U[-1, 1], FP16->FP32 and FP64, one persistent launch per
-      execution in a hipGraph, autotuned per size bucket;
+      multiples of 16, U[-1, 1], FP16->FP32 and FP64, one launch per
+      execution, autotuned per size bucket;
   w5  block SpGEMM C = A * A, 8192 x 8192 with 32 x 32 blocks at 2 % block density,
       N(0, 1) values in FP16, FP32 accumulation.
 Timing: inputs resident in HBM, warm-up calls, then torch.cuda events on the stream the
