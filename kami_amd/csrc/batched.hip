@@ -85,20 +85,6 @@ struct BatchArgs {
     double alpha, beta;
 };
 
-// The queue is read through scalar loads (constant address space, wave-uniform index).
-template <class T>
-__device__ __forceinline__ T load_uniform(const T* p) {
-    static_assert(sizeof(T) % 8 == 0, "whole 8-byte words");
-    typedef const __attribute__((address_space(4))) uint64_t* cptr;
-    struct words {
-        uint64_t w[sizeof(T) / 8];
-    } x;
-    const cptr q = (cptr)(uintptr_t)p;
-#pragma unroll
-    for (size_t i = 0; i < sizeof(T) / 8; ++i) x.w[i] = q[i];
-    return __builtin_bit_cast(T, x);
-}
-
 __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 // Raw buffer descriptors over a wave tile's operands.  A lane offset at or past
@@ -113,15 +99,6 @@ __device__ __forceinline__ u4_t buffer_load16(__amdgpu_buffer_rsrc_t r, int off,
 }
 __device__ __forceinline__ double buffer_load8(__amdgpu_buffer_rsrc_t r, int off, int soff) {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0));
-}
-
-// Transposing LDS read of 2-byte values (gfx950): each group of 16 lanes reads four rows
-// of 16 values, lane l of the group the four at row l / 4, columns 4 (l mod 4) .. + 3, and
-// receives column l of the four rows (layout checked with an in-bounds probe).
-__device__ __forceinline__ u2_t lds_read_turned(const unsigned char* p) {
-    return __builtin_bit_cast(
-        u2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                  (__attribute__((address_space(3))) s4_t*)(const_cast<unsigned char*>(p))));
 }
 
 #define KAMI_GLOBAL __attribute__((address_space(1)))
@@ -286,13 +263,16 @@ struct WaveTile {
         load(s, 0);
         for (int c = 1; c < n; ++c) {
             write(s);
+            wave_lds_order();
             read(s, f);
+            wave_lds_order();
             load(s, c);
             __builtin_amdgcn_sched_barrier(0);
             mma(f, acc);
             __builtin_amdgcn_sched_barrier(0);
         }
         write(s);
+        wave_lds_order();
         read(s, f);
         mma(f, acc);
         const acc_t alpha = (acc_t)alpha_d, beta = (acc_t)beta_d;

@@ -258,4 +258,37 @@ __device__ inline void store_raw(void* p, const typename Raw<BYTES>::type& v) {
     *reinterpret_cast<typename Raw<BYTES>::type*>(p) = v;
 }
 
+// Wave-uniform read-only data through scalar loads (constant address space): shorter than a
+// vector load, and the values are known to be uniform.
+template <class T>
+__device__ inline T load_uniform(const T* p) {
+    using word = typename std::conditional<sizeof(T) % 8 == 0, uint64_t, uint32_t>::type;
+    static_assert(sizeof(T) % sizeof(word) == 0, "whole words");
+    typedef const __attribute__((address_space(4))) word* cptr;
+    struct words {
+        word w[sizeof(T) / sizeof(word)];
+    } x;
+    const cptr q = (cptr)(uintptr_t)p;
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T) / sizeof(word); ++i) x.w[i] = q[i];
+    return __builtin_bit_cast(T, x);
+}
+
+// Orders a wave's own LDS accesses across its lanes: the hardware completes them in order, so
+// this only keeps the compiler from moving one lane's access past another's.
+__device__ inline void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Transposing LDS read of 2-byte values (gfx950): each group of 16 lanes reads four rows
+// of 16 values, lane l of the group the four at row l / 4, columns 4 (l mod 4) .. + 3, and
+// receives column l of the four rows (layout checked with an in-bounds probe).
+__device__ inline u2_t lds_read_turned(const unsigned char* p) {
+    return __builtin_bit_cast(
+        u2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                  (__attribute__((address_space(3))) s4_t*)(const_cast<unsigned char*>(p))));
+}
+
 }  // namespace kami

@@ -5,21 +5,15 @@
 // N x K, so C(i, j) = sum_k A(i, k) B[j * K + k] (check loop :378-403).  Here A stays in
 // plain BSR (the same format the SpGEMM entry points take) and the product is spread
 // over workgroups:
-//   * one workgroup per (block row i, 64-column tile of C).  FP16 / BF16 (split form,
-//     spmm_split_kernel): the row's blocks are shared out over the four waves, each wave
-//     computing all 64 columns of its blocks from fragments loaded straight from memory,
-//     and the four partial tiles are summed through LDS in a fixed order.  FP64
-//     (spmm_kernel): wave w owns the 16 columns [16 w, 16 w + 16) of the tile and all of
-//     the row's blocks, as below;
-//   * only the A block is shared by the four waves, so only it is staged in LDS (rows
-//     padded to the conflict-free stride, double-buffered, one barrier per block); each
-//     lane loads its own B values straight into MFMA fragments, in the fragment layout of
-//     the MFMA atom (for column c, k-step t and lane group g the KV values from
-//     t KSTEP + g KV), so one load instruction reads four consecutive fragments (64 bytes
-//     with 16-byte fragments) of every column it touches;
-//   * the next block's A piece and B fragments are loaded while the current block is
-//     multiplied; the column indices of a row are read 64 at a time into a register and
-//     taken out with readlane, so no scalar load waits in the loop;
+//   * one workgroup per (block row i, column tile of C).  The row's blocks are cut into
+//     stages of one line of K (up to 128 bytes) per row of A and column of B; the stages
+//     are shared out over the workgroup's K groups of waves, which sum their partial tiles
+//     through LDS in a fixed order;
+//   * a wave stages lines through LDS of its own (no barrier in its loop): loading MFMA
+//     fragments straight from memory puts 16 lines under 16 consecutive lanes, which the
+//     address unit takes four lanes a clock, four times as long as whole lines;
+//   * the next stage's lines are loaded while the current one is multiplied; column
+//     indices come through scalar loads, two stages ahead;
 //   * workgroups are numbered so that each XCD (workgroup L runs on XCD L mod 8) takes a
 //     contiguous run of (column tile, block row) pairs: its L2 sees the B columns of few
 //     tiles;
@@ -30,23 +24,6 @@
 #include "kami_internal.hpp"
 
 namespace kami {
-
-template <int BS, class AT>
-struct SpmmGeom {
-    using in_t = typename AT::in_t;
-    static constexpr int NT = 256, TN = 64;  // C tile: BS rows x TN columns, 4 waves
-    static constexpr int ELT = (int)sizeof(in_t), VE = 16 / ELT;
-    static constexpr int FB = AT::FRAG_BYTES;
-    static constexpr int ROWB = lds_row_bytes(BS * ELT, FB);
-    static constexpr int STAGE = BS * ROWB;  // one A block
-    static constexpr int CPR = BS / VE;      // 16-byte pieces per A row
-    static constexpr int NA = BS * CPR;      // pieces of an A block
-    static constexpr int NPA = (NA + NT - 1) / NT;
-    static constexpr int IM = BS / 16;
-    static constexpr int NKS = BS / AT::KSTEP;  // MFMA k-steps per block
-    static_assert(BS % AT::KSTEP == 0 && BS % 16 == 0, "block size");
-    static_assert(TN == 16 * (NT / 64), "one 16-column atom per wave");
-};
 
 struct SpmmArgs {
     int32_t mb, nb, n, b_kn;
@@ -59,310 +36,313 @@ struct SpmmArgs {
     double alpha, beta;
 };
 
-template <int BS, class AT>
-__global__ void __launch_bounds__(256) spmm_kernel(SpmmArgs a) {
-    using G = SpmmGeom<BS, AT>;
+// One workgroup per (block row i, tile of WN x 16 CT columns of C): wave (wk, wn) multiplies
+// the row's stages wk, wk + WK, ... with its 16 CT columns, so the longest row's chain of
+// load-multiply steps is 1 / WK as long.  The partial tiles are summed through LDS in the
+// order of wk (the same order every run), then C = alpha sum + beta C.
+// What bounds it: 8192^2, 2 % of 32 x 32 blocks, n = 256.  FP64 23.5 us (the earlier kernel,
+// fragments of B straight from memory and a barrier per block: 30.4): 89 MB of A and B
+// reach the XCDs' L2s and MFMA pipes are 44 % busy; the longest rows (13 blocks against a
+// mean of 5) end last.  FP16 6.4 us replayed from a graph (8.3): the chain row pointers ->
+// column indices -> lines -> LDS -> sum -> store, once.
+template <int BS, class AT, bool KN, int WK_, int WN_, int CT>
+struct SpmmGeom {
     using in_t = typename AT::in_t;
     using acc_t = typename AT::acc_t;
-    using out_t = typename AT::out_t;
-    using frag_t = typename AT::frag_t;
-    using accv_t = typename AT::accv_t;
-    constexpr int FB = AT::FRAG_BYTES, KV = AT::KV;
-    struct elems_t {
-        in_t v[KV];
-    };
-    __shared__ __attribute__((aligned(16))) unsigned char smem[2 * G::STAGE];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, grp = lane >> 4;
-    // XCD x = L mod 8 takes the contiguous run [x q + min(x, r), ...) of the tile-major
-    // order, q = total / 8, r = total mod 8 (a bijection of [0, total)).
-    const uint32_t L = blockIdx.x, total = gridDim.x;
-    const uint32_t x = L % 8, q8 = total / 8, r8 = total % 8;
-    const uint32_t P = x * q8 + (x < r8 ? x : r8) + L / 8;
-    const int i = (int)(P % (uint32_t)a.mb);      // block row of A and C
-    const int n0 = (int)(P / (uint32_t)a.mb) * G::TN;  // first column of the C tile
-    const int col = n0 + wave * 16 + (lane & 15);
-    const bool wave_live = n0 + wave * 16 < a.n;  // wave-uniform; n is a multiple of 16
-    const in_t* __restrict__ vals = reinterpret_cast<const in_t*>(a.vals);
-    const in_t* __restrict__ B = reinterpret_cast<const in_t*>(a.B);
-    // stored blocks of row i (clamped to the arrays the caller described)
-    const int64_t rb = a.rowptr[i], re = a.rowptr[i + 1];
-    const int64_t beg = rb < 0 ? 0 : rb;
-    const int64_t end = re > a.nnzb ? a.nnzb : re;
-
-    // column indices [cbase, cbase + 64) of the row, one per lane
-    int64_t cbase = beg;
-    int cvec = beg + lane < end ? a.colidx[beg + lane] : -1;
-    auto block_col = [&](int64_t q) {  // q uniform, called with q = beg, beg + 1, ...
-        if (q - cbase >= 64) {
-            cbase += 64;
-            cvec = cbase + lane < end ? a.colidx[cbase + lane] : -1;
-        }
-        return __builtin_amdgcn_readlane(cvec, (int)(q - cbase));
-    };
-
-    u4_t ra[G::NPA];
-    auto load_a = [&](int64_t q) {
-#pragma unroll
-        for (int p = 0; p < G::NPA; ++p) {
-            const int idx = tid + p * G::NT;
-            if (idx < G::NA)
-                ra[p] = load_raw<16>(vals + q * BS * BS + (idx / G::CPR) * BS + (idx % G::CPR) * G::VE);
-        }
-    };
-    auto write_a = [&](int buf) {
-        unsigned char* base = smem + buf * G::STAGE;
-#pragma unroll
-        for (int p = 0; p < G::NPA; ++p) {
-            const int idx = tid + p * G::NT;
-            if (idx < G::NA)
-                store_raw<16>(base + (idx / G::CPR) * G::ROWB + (idx % G::CPR) * 16, ra[p]);
-        }
-    };
-    // B fragments of block column kb for this lane: step t holds k = kb bs + t KSTEP + g KV + v
-    auto load_b = [&](int kb, frag_t (&f)[G::NKS]) {
-        elems_t z;
-#pragma unroll
-        for (int v = 0; v < KV; ++v) z.v[v] = in_t(0);
-#pragma unroll
-        for (int t = 0; t < G::NKS; ++t) f[t] = bitcast<frag_t>(z);
-        if (!wave_live || kb < 0 || kb >= a.nb) return;  // wave-uniform
-        const int64_t k0 = (int64_t)kb * BS + grp * KV;
-        if (!a.b_kn) {
-            const in_t* p = B + (int64_t)col * a.ldb + k0;
-#pragma unroll
-            for (int t = 0; t < G::NKS; ++t) f[t] = bitcast<frag_t>(load_raw<FB>(p + t * AT::KSTEP));
-        } else {
-            const in_t* p = B + k0 * a.ldb + col;
-#pragma unroll
-            for (int t = 0; t < G::NKS; ++t) {
-                elems_t e;
-#pragma unroll
-                for (int v = 0; v < KV; ++v) e.v[v] = p[(int64_t)(t * AT::KSTEP + v) * a.ldb];
-                f[t] = bitcast<frag_t>(e);
-            }
-        }
-    };
-
-    accv_t acc[G::IM];
-#pragma unroll
-    for (int im = 0; im < G::IM; ++im)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[im][v] = 0;
-
-    if (beg < end) {
-        frag_t bc[G::NKS], bn[G::NKS];
-        load_a(beg);
-        load_b(block_col(beg), bc);
-        write_a(0);
-        __syncthreads();
-        int buf = 0;
-        for (int64_t q = beg; q < end; ++q) {
-            const bool next = q + 1 < end;
-            if (next) {
-                load_a(q + 1);
-                load_b(block_col(q + 1), bn);
-            }
-            if (wave_live) {
-                const unsigned char* base = smem + buf * G::STAGE;
-#pragma unroll
-                for (int ks = 0; ks < G::NKS; ++ks) {
-                    const int kk = (ks * AT::KSTEP + KV * grp) * G::ELT;
-                    frag_t af[G::IM];
-#pragma unroll
-                    for (int im = 0; im < G::IM; ++im)
-                        af[im] = bitcast<frag_t>(load_raw<FB>(base + (im * 16 + (lane & 15)) * G::ROWB + kk));
-#pragma unroll
-                    for (int e = 0; e < AT::NSUB; ++e)
-#pragma unroll
-                        for (int im = 0; im < G::IM; ++im) AT::mma_sub(acc[im], af[im], bc[ks], e);
-                }
-            }
-            if (next) write_a(buf ^ 1);
-            __syncthreads();
-            buf ^= 1;
-#pragma unroll
-            for (int t = 0; t < G::NKS; ++t) bc[t] = bn[t];
-        }
+    static constexpr int WK = WK_, WN = WN_, WAVES = WK * WN, NT = 64 * WAVES, IM = BS / 16;
+    static constexpr int WTN = 16 * CT, TN = WTN * WN;  // columns of a wave, of the workgroup
+    static constexpr int ELT = (int)sizeof(in_t), VE = 16 / ELT;
+    static constexpr bool F64 = ELT == 8;
+    static constexpr int RB = BS * ELT < 128 ? BS * ELT : 128;
+    static constexpr int HS = BS * ELT / RB;     // stages per block
+    static constexpr int KS = RB / ELT;          // K of a stage
+    static constexpr int NF = KS / AT::KSTEP;    // fragments per stage
+    static constexpr int PPR = RB / 16;          // 16-byte pieces of a line
+    static constexpr int RPI = 64 / PPR;         // lines of one load instruction
+    static constexpr int NA = (BS + RPI - 1) / RPI;
+    // K x N operands: FP64 fragments straight from memory (16 lanes read 16 consecutive
+    // columns), rows of 2-byte values turned by transposing LDS reads
+    static constexpr bool TURN = KN && !F64;
+    static constexpr int TROW = CT * 32 + 16;    // bytes of a turned K row in LDS
+    static constexpr int TPR = CT * 2;           // its 16-byte pieces
+    static constexpr int NB = !KN ? (WTN + RPI - 1) / RPI : TURN ? (KS * TPR + 63) / 64 : CT * NF;
+    static constexpr int A_LDS = BS * RB;
+    static constexpr int B_LDS = !KN ? WTN * RB : TURN ? KS * TROW : 0;
+    // a wave's partial tile: FP64 as the accumulators lie; FP32 in rows, padded so that the
+    // four rows of one store fall on different banks
+    static constexpr int CROW = WTN * 4 + 16;
+    static constexpr int PART = F64 ? IM * CT * 4 * 64 * 8 : BS * CROW;
+    static constexpr int WAVE_LDS = A_LDS + B_LDS > PART ? A_LDS + B_LDS : PART;
+    // slot of piece p of line r: p ^ swz(r), so that the 32 lanes of a fragment read (16
+    // lines, two neighbouring pieces) fall on different banks of the 512-byte window
+    static constexpr __device__ int swz(int r) {
+        return RB == 128 ? ((r >> 2) & 3) << 1 : RB == 64 ? ((r >> 3) & 1) << 1 : 0;
     }
-
-    if (!wave_live) return;
-    out_t* __restrict__ C = reinterpret_cast<out_t*>(a.C);
-    const acc_t alpha = (acc_t)a.alpha, beta = (acc_t)a.beta;
-#pragma unroll
-    for (int im = 0; im < G::IM; ++im)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int64_t row = (int64_t)i * BS + im * 16 + AT::out_row(lane, v);
-            out_t* dst = C + row * a.ldc + col;
-            acc_t val = alpha * acc[im][v];
-            if (beta != (acc_t)0) val += beta * (acc_t)(*dst);
-            *dst = (out_t)val;
-        }
-}
-
-// ---- split form: the blocks of a row shared by the workgroup's four waves ----
-//
-// One workgroup per (block row i, tile of TN = 16 CT columns of C).  Wave w takes the
-// row's blocks w, w + 4, w + 8, ..., so the longest row's chain of load-multiply steps
-// is a quarter as long; each wave loads the A block's and B's MFMA fragments straight
-// from memory (no LDS staging, no barrier in the loop), the next block's while the
-// current one is multiplied.  The four partial tiles are summed through LDS in wave
-// order 0, 1, 2, 3 (the same order every run), then C = alpha sum + beta C.
-template <int BS, class AT, int CT>
-struct SpmmSplitGeom {
-    using in_t = typename AT::in_t;
-    using acc_t = typename AT::acc_t;
-    static constexpr int NT = 256, WAVES = 4, TN = 16 * CT;
-    static constexpr int IM = BS / 16;
-    static constexpr int NKS = BS / AT::KSTEP;  // MFMA k-steps per block
-    static constexpr int NE = IM * CT * 4;      // accumulator values per lane
-    static constexpr int LDS = WAVES * NE * 64 * (int)sizeof(acc_t);
-    static_assert(BS % AT::KSTEP == 0 && BS % 16 == 0, "block size");
-    static_assert(LDS <= 64 * 1024, "partial tiles");
+    static_assert(BS % AT::KSTEP == 0 && BS % 16 == 0 && KS % AT::KSTEP == 0, "block size");
+    static_assert(WAVES * WAVE_LDS <= 160 * 1024 && NT <= 1024, "workgroup");
 };
 
-template <int BS, class AT, int CT>
-__global__ void __launch_bounds__(256) spmm_split_kernel(SpmmArgs a) {
-    using G = SpmmSplitGeom<BS, AT, CT>;
+template <int BS, class AT, bool KN, int WK_, int WN_, int CT>
+__global__ void __launch_bounds__(64 * WK_ * WN_) __attribute__((amdgpu_waves_per_eu(4)))
+spmm_kernel(SpmmArgs a) {
+    using G = SpmmGeom<BS, AT, KN, WK_, WN_, CT>;
     using in_t = typename AT::in_t;
     using acc_t = typename AT::acc_t;
     using out_t = typename AT::out_t;
     using frag_t = typename AT::frag_t;
     using accv_t = typename AT::accv_t;
-    constexpr int FB = AT::FRAG_BYTES, KV = AT::KV;
-    struct elems_t {
-        in_t v[KV];
-    };
-    __shared__ __attribute__((aligned(16))) acc_t part[G::WAVES * G::NE * 64];
+    constexpr int FB = AT::FRAG_BYTES, NF = G::NF, IM = G::IM;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[G::WAVES * G::WAVE_LDS];
 
     const int tid = threadIdx.x, lane = tid & 63, grp = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    unsigned char* const lds = smem + wave * G::WAVE_LDS;
     // XCD x = L mod 8 takes the contiguous run [x q + min(x, r), ...) of the tile-major
     // order, q = total / 8, r = total mod 8 (a bijection of [0, total)).
     const uint32_t L = blockIdx.x, total = gridDim.x;
     const uint32_t x = L % 8, q8 = total / 8, r8 = total % 8;
     const uint32_t P = x * q8 + (x < r8 ? x : r8) + L / 8;
-    const int i = (int)(P % (uint32_t)a.mb);           // block row of A and C
-    const int n0 = (int)(P / (uint32_t)a.mb) * G::TN;  // first column of the C tile
+    const int i = (int)(P % (uint32_t)a.mb);             // block row of A and C
+    const int nt = (int)(P / (uint32_t)a.mb) * G::TN;    // first column of the C tile
+    const int wk = wave / G::WN, wn = wave % G::WN;
+    const int n0 = nt + wn * G::WTN;                     // first column of the wave
     const in_t* __restrict__ vals = reinterpret_cast<const in_t*>(a.vals);
     const in_t* __restrict__ B = reinterpret_cast<const in_t*>(a.B);
-    const int64_t rb = a.rowptr[i], re = a.rowptr[i + 1];
+    // stored blocks of row i (clamped to the arrays the caller described)
+    const int64_t rb = load_uniform(a.rowptr + i), re = load_uniform(a.rowptr + i + 1);
     const int64_t beg = rb < 0 ? 0 : rb;
     const int64_t end = re > a.nnzb ? a.nnzb : re;
 
-    // the row's column indices [cbase, cbase + 64), one per lane, taken out with readlane
-    // (q grows with each call of a wave, so the window only moves forward)
-    int64_t cbase = beg;
-    int cvec = beg + lane < end ? a.colidx[beg + lane] : -1;
-    auto block_col = [&](int64_t q) {
-        if (q - cbase >= 64) {
-            cbase += (q - cbase) / 64 * 64;
-            cvec = cbase + lane < end ? a.colidx[cbase + lane] : -1;
+    const int64_t n_st = (end > beg ? end - beg : 0) * G::HS;
+    // block column of stage st (of the row's last block past the end)
+    auto block_col = [&](int64_t st) {
+        return load_uniform(a.colidx + (st < n_st ? beg + st / G::HS : end - 1));
+    };
+
+    // Lines of A and of B (N x K) are loaded by PPR lanes each (a load of fragments would
+    // put 16 lines under 16 consecutive lanes, four times the address unit's clocks) and
+    // turned into fragments through the wave's own LDS.  Columns past n repeat the last.
+    const int lrow = lane / G::PPR, lpiece = lane % G::PPR;
+    const in_t* const pa = vals + (lrow % BS) * BS + lpiece * G::VE;
+    const in_t* pb[G::NB];
+#pragma unroll
+    for (int j = 0; j < G::NB; ++j) {
+        if constexpr (!KN) {
+            const int col = min(n0 + (lrow % G::WTN) + j * G::RPI, a.n - 1);
+            pb[j] = B + (int64_t)col * a.ldb + lpiece * G::VE;
+        } else if constexpr (G::TURN) {
+            const int p = (lane + 64 * j) % (G::KS * G::TPR);
+            const int col = min(n0 + (p % G::TPR) * 8, a.n - 8);
+            pb[j] = B + (int64_t)(p / G::TPR) * a.ldb + col;
+        } else {
+            const int col = min(n0 + (j / NF) * 16 + (lane & 15), a.n - 1);
+            pb[j] = B + (int64_t)((j % NF) * AT::KSTEP + 2 * grp) * a.ldb + col;
         }
-        return __builtin_amdgcn_readlane(cvec, (int)(q - cbase));
+    }
+    struct Stage {
+        u4_t a[G::NA], b[G::NB];
     };
-    // fragments of one block: A (IM atom rows x NKS k-steps) and B (CT atoms x NKS)
+    // stage st of the row: block beg + st / HS, columns h KS .. of it, h = st mod HS
+    auto load_a = [&](int64_t st, Stage& s) {
+        const int64_t ao = (beg + st / G::HS) * BS * BS + st % G::HS * G::KS;
+#pragma unroll
+        for (int t = 0; t < G::NA; ++t) s.a[t] = load_raw<16>(pa + ao + t * G::RPI * BS);
+    };
+    auto valid = [&](int kb) { return kb >= 0 && kb < a.nb; };  // wave-uniform
+    auto load_b = [&](int64_t st, int kb, Stage& s) {
+        const int64_t k0 = (int64_t)(valid(kb) ? kb : 0) * BS + st % G::HS * G::KS;
+        const int64_t bo = KN ? k0 * a.ldb : k0;
+#pragma unroll
+        for (int j = 0; j < G::NB; ++j) {
+            if constexpr (KN && G::F64) {
+                const in_t* p = pb[j] + bo;
+                const d2_t v = {p[0], p[a.ldb]};
+                s.b[j] = bitcast<u4_t>(v);
+            } else {
+                s.b[j] = load_raw<16>(pb[j] + bo);
+            }
+        }
+    };
+    auto write = [&](const Stage& s) {
+#pragma unroll
+        for (int t = 0; t < G::NA; ++t) {
+            const int r = lrow % BS + t * G::RPI;
+            store_raw<16>(lds + r * G::RB + ((lpiece ^ G::swz(r)) << 4), s.a[t]);
+        }
+#pragma unroll
+        for (int j = 0; j < G::NB; ++j) {
+            if constexpr (!KN) {
+                const int r = lrow % G::WTN + j * G::RPI;
+                store_raw<16>(lds + G::A_LDS + r * G::RB + ((lpiece ^ G::swz(r)) << 4), s.b[j]);
+            } else if constexpr (G::TURN) {
+                const int p = (lane + 64 * j) % (G::KS * G::TPR);
+                store_raw<16>(lds + G::A_LDS + (p / G::TPR) * G::TROW + (p % G::TPR) * 16, s.b[j]);
+            }
+        }
+    };
     struct Frags {
-        frag_t a[G::IM][G::NKS];
-        frag_t b[CT][G::NKS];
+        frag_t a[IM][NF], b[CT][NF];
     };
-    auto load = [&](int64_t q, Frags& f) {
-        const int kb = block_col(q);
-        const in_t* ab = vals + q * BS * BS + (lane & 15) * BS + grp * KV;
+    auto read = [&](const Stage& s, Frags& f) {
+        const int r = lane & 15;
+        auto line_frag = [&](const unsigned char* base, int t) {
+            if constexpr (FB == 16)
+                return bitcast<frag_t>(load_raw<FB>(base + r * G::RB + (((4 * t + grp) ^ G::swz(r)) << 4)));
+            else
+                return bitcast<frag_t>(load_raw<FB>(base + r * G::RB + grp * FB));
+        };
 #pragma unroll
-        for (int im = 0; im < G::IM; ++im)
+        for (int t = 0; t < NF; ++t) {
 #pragma unroll
-            for (int t = 0; t < G::NKS; ++t)
-                f.a[im][t] = bitcast<frag_t>(load_raw<FB>(ab + im * 16 * BS + t * AT::KSTEP));
-        const int64_t k0 = (int64_t)kb * BS + grp * KV;
-        const bool kb_ok = kb >= 0 && kb < a.nb;  // wave-uniform
+            for (int im = 0; im < IM; ++im) f.a[im][t] = line_frag(lds + im * 16 * G::RB, t);
 #pragma unroll
-        for (int jn = 0; jn < CT; ++jn) {
-            const int col = n0 + jn * 16 + (lane & 15);
-            const bool live = kb_ok && n0 + jn * 16 < a.n;  // wave-uniform (n % 16 == 0)
-#pragma unroll
-            for (int t = 0; t < G::NKS; ++t) {
-                elems_t e;
-                if (!live) {
-#pragma unroll
-                    for (int v = 0; v < KV; ++v) e.v[v] = in_t(0);
-                    f.b[jn][t] = bitcast<frag_t>(e);
-                } else if (!a.b_kn) {
-                    f.b[jn][t] = bitcast<frag_t>(
-                        load_raw<FB>(B + (int64_t)col * a.ldb + k0 + t * AT::KSTEP));
+            for (int jn = 0; jn < CT; ++jn) {
+                if constexpr (!KN) {
+                    f.b[jn][t] = line_frag(lds + G::A_LDS + jn * 16 * G::RB, t);
+                } else if constexpr (G::TURN) {
+                    const unsigned char* p = lds + G::A_LDS + (t * AT::KSTEP + AT::KV * grp + (r >> 2)) * G::TROW +
+                                             jn * 32 + 8 * (lane & 3);
+                    if constexpr (FB == 16) {
+                        const u2_t lo = lds_read_turned(p), hi = lds_read_turned(p + 4 * G::TROW);
+                        f.b[jn][t] = bitcast<frag_t>(u4_t{lo[0], lo[1], hi[0], hi[1]});
+                    } else {
+                        f.b[jn][t] = bitcast<frag_t>(lds_read_turned(p));
+                    }
                 } else {
-                    const in_t* p = B + k0 * a.ldb + col;
-#pragma unroll
-                    for (int v = 0; v < KV; ++v) e.v[v] = p[(int64_t)(t * AT::KSTEP + v) * a.ldb];
-                    f.b[jn][t] = bitcast<frag_t>(e);
+                    f.b[jn][t] = bitcast<frag_t>(s.b[jn * NF + t]);
                 }
             }
         }
     };
 
-    accv_t acc[G::IM][CT];
+    accv_t acc[IM][CT];
 #pragma unroll
-    for (int im = 0; im < G::IM; ++im)
+    for (int im = 0; im < IM; ++im)
 #pragma unroll
-        for (int jn = 0; jn < CT; ++jn)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[im][jn][v] = 0;
+        for (int jn = 0; jn < CT; ++jn) acc[im][jn] = accv_t{0, 0, 0, 0};
 
-    int64_t q = beg + wave;
-    if (q < end) {
-        Frags cur, nxt;
-        load(q, cur);
-        for (; q < end; q += G::WAVES) {
-            const bool more = q + G::WAVES < end;  // wave-uniform
-            if (more) load(q + G::WAVES, nxt);
+    // stage in LDS, the next one in registers or on its way
+    if (wk < n_st && n0 < a.n) {  // wave-uniform
+        Stage s;
+        Frags f;
+        int kb = block_col(wk), kb_next = block_col(wk + G::WK);
+        load_a(wk, s);
+        load_b(wk, kb, s);
+        for (int64_t st = wk; st < n_st; st += G::WK) {
+            const bool ok = valid(kb);
+            write(s);
+            wave_lds_order();
+            read(s, f);
+            wave_lds_order();
+            if (st + G::WK < n_st) {
+                kb = kb_next;
+                load_a(st + G::WK, s);
+                load_b(st + G::WK, kb, s);
+                kb_next = block_col(st + 2 * G::WK);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (ok) {
 #pragma unroll
-            for (int t = 0; t < G::NKS; ++t)
+                for (int t = 0; t < NF; ++t)
 #pragma unroll
-                for (int e = 0; e < AT::NSUB; ++e)
+                    for (int e = 0; e < AT::NSUB; ++e)
 #pragma unroll
-                    for (int jn = 0; jn < CT; ++jn)
+                        for (int jn = 0; jn < CT; ++jn)
 #pragma unroll
-                        for (int im = 0; im < G::IM; ++im) AT::mma_sub(acc[im][jn], cur.a[im][t], cur.b[jn][t], e);
-            if (more) cur = nxt;
+                            for (int im = 0; im < IM; ++im) AT::mma_sub(acc[im][jn], f.a[im][t], f.b[jn][t], e);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
 
-    // partial tiles: value (im, jn, v) of lane l of wave w at ((w NE + (im CT + jn) 4 + v) 64 + l)
-#pragma unroll
-    for (int im = 0; im < G::IM; ++im)
-#pragma unroll
-        for (int jn = 0; jn < CT; ++jn)
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-                part[((wave * G::NE + (im * CT + jn) * 4 + v) << 6) + lane] = acc[im][jn][v];
-    __syncthreads();
+    // the wave's partial tile over its own stages, which it has left
     out_t* __restrict__ C = reinterpret_cast<out_t*>(a.C);
     const acc_t alpha = (acc_t)a.alpha, beta = (acc_t)a.beta;
 #pragma unroll
-    for (int s = 0; s < G::NE / 4; ++s) {
-        const int e = tid + G::NT * s;  // element (im, jn, v) = e / 64, lane e % 64
-        acc_t sum = part[e];
+    for (int im = 0; im < IM; ++im)
 #pragma unroll
-        for (int w = 1; w < G::WAVES; ++w) sum += part[w * G::NE * 64 + e];
-        const int iv = e >> 6, l = e & 63;
-        const int im = iv / (CT * 4), jn = (iv / 4) % CT, v = iv % 4;
-        const int col = n0 + jn * 16 + (l & 15);
-        if (col >= a.n) continue;
-        const int64_t row = (int64_t)i * BS + im * 16 + AT::out_row(l, v);
-        out_t* dst = C + row * a.ldc + col;
-        acc_t val = alpha * sum;
-        if (beta != (acc_t)0) val += beta * (acc_t)(*dst);
-        *dst = (out_t)val;
+        for (int jn = 0; jn < CT; ++jn)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int at = G::F64 ? (((im * CT + jn) * 4 + v) * 64 + lane) * 8
+                                      : (im * 16 + AT::out_row(lane, v)) * G::CROW + (jn * 16 + (lane & 15)) * 4;
+                *reinterpret_cast<acc_t*>(lds + at) = acc[im][jn][v];
+            }
+    __syncthreads();
+    // wave (wk, wn)'s partial tile lies in region wk WN + wn
+    if constexpr (G::F64) {
+        constexpr int NE = IM * CT * 4 * 64;  // values of a wave tile
+#pragma unroll
+        for (int s = 0; s < (G::WN * NE + G::NT - 1) / G::NT; ++s) {
+            const int g = tid + G::NT * s, e = g % NE, cn = g / NE;
+            if (G::WN * NE % G::NT != 0 && cn >= G::WN) break;
+            const unsigned char* at = smem + cn * G::WAVE_LDS + e * 8;
+            acc_t sum = *reinterpret_cast<const acc_t*>(at);
+#pragma unroll
+            for (int w = 1; w < G::WK; ++w)
+                sum += *reinterpret_cast<const acc_t*>(at + w * G::WN * G::WAVE_LDS);
+            const int iv = e >> 6, l = e & 63;  // (im, jn, v) and lane
+            const int im = iv / (CT * 4), jn = (iv / 4) % CT, v = iv % 4;
+            const int col = nt + cn * G::WTN + jn * 16 + (l & 15);
+            if (col >= a.n) continue;
+            out_t* dst = C + ((int64_t)i * BS + im * 16 + AT::out_row(l, v)) * a.ldc + col;
+            acc_t val = alpha * sum;
+            if (beta != (acc_t)0) val += beta * (acc_t)(*dst);
+            *dst = (out_t)val;
+        }
+    } else {
+        typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));  // C: 4-byte aligned
+        constexpr int QR = G::TN / 4;  // 16-byte pieces of a C row
+#pragma unroll
+        for (int s = 0; s < (BS * QR + G::NT - 1) / G::NT; ++s) {
+            const int e = tid + G::NT * s, row = e / QR, c4 = (e % QR) * 4;
+            if (BS * QR % G::NT != 0 && row >= BS) break;
+            const unsigned char* at = smem + c4 / G::WTN * G::WAVE_LDS + row * G::CROW + c4 % G::WTN * 4;
+            f4_t sum = *reinterpret_cast<const f4_t*>(at);
+#pragma unroll
+            for (int w = 1; w < G::WK; ++w)
+                sum += *reinterpret_cast<const f4_t*>(at + w * G::WN * G::WAVE_LDS);
+            if (nt + c4 >= a.n) continue;
+            f4u_t* dst = reinterpret_cast<f4u_t*>(C + ((int64_t)i * BS + row) * a.ldc + nt + c4);
+            f4u_t val = alpha * sum;
+            if (beta != (acc_t)0) val += beta * *dst;
+            *dst = val;
+        }
     }
 }
 
-// The split form serves FP16 / BF16 (64-column tiles, 88 VGPRs: every workgroup of the
-// w6 product resident at once; kernel 10.6 -> 9.2 µs).  FP64 keeps the one-wave-per-16-
-// columns form: its split tiles need 198 VGPRs (two waves per SIMD), and the 2048
-// workgroups then run in four rounds (33.7 -> 39.8 µs); with 16-column split tiles (144
-// VGPRs, every column tile loading the row's A blocks again) it ran 42.3-42.6 µs.
-constexpr int kSpmmSplitAtoms = 4;
+template <int BS, class AT, int WK, int WN, int CT>
+static hipError_t launch_form(const SpmmArgs& a, hipStream_t s) {
+    using G = SpmmGeom<BS, AT, false, WK, WN, CT>;
+    const int64_t total = (int64_t)a.mb * (((int64_t)a.n + G::TN - 1) / G::TN);
+    const dim3 grid((unsigned)total), block(G::NT);
+    if (a.b_kn)
+        hipLaunchKernelGGL((spmm_kernel<BS, AT, true, WK, WN, CT>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((spmm_kernel<BS, AT, false, WK, WN, CT>), grid, block, 0, s, a);
+    return hipGetLastError();
+}
+
+// Which form: enough workgroups share a row's stages among four waves; FP64 blocks of 32 as
+// two K groups x two column groups (a row's two stages per block go to one wave each, and
+// the column groups read A's lines together: 23.5 us against 26.2 for four K groups at
+// 8192^2, 2 % of 32 x 32 blocks, n = 256), the others as four K groups (FP64 blocks of 16
+// at 4800^2, 20 %, n = 128: 31.7 us against 36.3).  Where the tiles leave the chip idle
+// and the rows are long, one row's stages go to 16 or 8 waves: 20 block rows of 80 blocks of
+// 32, n = 48: FP64 28.6 us against 43.5 with four (and 135 with the earlier kernel), FP16
+// 11.2 against 13.6; 100 rows of 20, n = 64: FP64 15.1 against 17.0.
+template <int BS, class AT, int CT>
+static hipError_t launch_spmm(const SpmmArgs& a, hipStream_t s) {
+    using G = SpmmGeom<BS, AT, false, 4, 1, CT>;
+    const int64_t tiles = (int64_t)a.mb * ((a.n + G::WTN - 1) / G::WTN);
+    const int64_t stages = a.nnzb * G::HS / a.mb;  // of an average row
+    if (tiles <= 256 && stages >= 32) return launch_form<BS, AT, 16, 1, CT>(a, s);
+    if (tiles <= 512 && stages >= 16) return launch_form<BS, AT, 8, 1, CT>(a, s);
+    if constexpr (G::F64 && BS == 32)
+        return launch_form<BS, AT, 2, 2, CT>(a, s);
+    else
+        return launch_form<BS, AT, 4, 1, CT>(a, s);
+}
 
 }  // namespace kami
 
@@ -398,9 +378,7 @@ kami_status kami_bsr_spmm(const kami_bsr* A, const void* B, int32_t n, int64_t l
         return KAMI_EINVAL;
     if ((ldb * ei) % 16 || ((uintptr_t)B % 16) || ((uintptr_t)C % eo)) return KAMI_EINVAL;
     if (A->nnzb > 0 && ((uintptr_t)A->vals % 16)) return KAMI_EINVAL;
-    // workgroups: one per (block row, 64-column tile of C) in both forms
-    const int64_t wgs = (int64_t)A->mb * (((int64_t)n + 63) / 64);
-    if (wgs >= ((int64_t)1 << 24)) return KAMI_ENOTSUP;  // work-items of one dispatch < 2^32
+    if ((int64_t)A->mb * (((int64_t)n + 63) / 64) >= ((int64_t)1 << 24)) return KAMI_ENOTSUP;
     kami_status st = device_check();
     if (st != KAMI_OK) return st;
     SpmmArgs a;
@@ -418,21 +396,14 @@ kami_status kami_bsr_spmm(const kami_bsr* A, const void* B, int32_t n, int64_t l
     a.C = C;
     a.alpha = alpha;
     a.beta = beta;
-    const dim3 grid((unsigned)wgs);
     hipStream_t s = (hipStream_t)stream;
-#define KAMI_SPMM_SPLIT(BS, AT) \
-    hipLaunchKernelGGL((spmm_split_kernel<BS, AT, kSpmmSplitAtoms>), grid, dim3(256), 0, s, a)
-#define KAMI_SPMM(BS, AT) hipLaunchKernelGGL((spmm_kernel<BS, AT>), grid, dim3(256), 0, s, a)
-    if (precision == KAMI_PREC_F16_F32) {
-        if (A->bs == 16) KAMI_SPMM_SPLIT(16, AtomF16x16); else KAMI_SPMM_SPLIT(32, AtomF16x32);
-    } else if (precision == KAMI_PREC_BF16_F32) {
-        if (A->bs == 16) KAMI_SPMM_SPLIT(16, AtomBF16x16); else KAMI_SPMM_SPLIT(32, AtomBF16x32);
-    } else {
-        if (A->bs == 16) KAMI_SPMM(16, AtomF64); else KAMI_SPMM(32, AtomF64);
-    }
-#undef KAMI_SPMM
-#undef KAMI_SPMM_SPLIT
-    hipError_t e = hipGetLastError();
+    hipError_t e;
+    if (precision == KAMI_PREC_F16_F32)
+        e = A->bs == 16 ? launch_spmm<16, AtomF16x16, 4>(a, s) : launch_spmm<32, AtomF16x32, 4>(a, s);
+    else if (precision == KAMI_PREC_BF16_F32)
+        e = A->bs == 16 ? launch_spmm<16, AtomBF16x16, 4>(a, s) : launch_spmm<32, AtomBF16x32, 4>(a, s);
+    else
+        e = A->bs == 16 ? launch_spmm<16, AtomF64, 2>(a, s) : launch_spmm<32, AtomF64, 2>(a, s);
     if (e != hipSuccess) return hip_fail(e);
     return KAMI_OK;
 }
