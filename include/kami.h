@@ -180,9 +180,9 @@ kami_status kami_block_gemm_autotune(const kami_gemm_desc* d, const void* A, con
 
 /* FP64 GEMM through FP16 / BF16 slices at sizes beyond the block instances: same
  * arguments as kami_block_gemm with precision KAMI_PREC_F64_SPLIT_F16 or _BF16, B stored
- * N x K, iters = 1, partition AUTO or 2D; M and N multiples of 128 (or of 64), K a
- * multiple of 32.  Each problem is cut into 128 x 128 (64 x 64) tiles of C; persistent
- * workgroups walk the tiles of all problems.  Error bound as for the block form, with
+ * N x K, iters = 1, partition AUTO or 2D; M and N multiples of 64, K a
+ * multiple of 32.  Each problem is cut into tiles of C, 32 to 128 wide by how many fill
+ * the chip; persistent workgroups walk the tiles of all problems.  Error bound as for the block form, with
  * digit exponents per row and 32-wide chunk of K.  No counterpart in the reference (it
  * has no split-precision path); it widens the split-precision block GEMM to any size. */
 kami_status kami_split_gemm(const kami_gemm_desc* d, const void* A, const void* B, void* C,

@@ -321,17 +321,360 @@ split_gemm_kernel(SplitArgs args) {
         }
 }
 
+// Digits of two values at once, packed as the planes hold them, by integer fields instead of
+// a rounding, a conversion and a rescaling per digit (v_rndne, v_cvt and v_ldexp on FP64 run
+// below the rate of FP64 add and FMA; 64 x 64 tiles at 1024^3 took 87 us with them).  Adding
+// 1.5 2^52 rounds to nearest even and leaves the integer in the low word, so three digits
+// come from one addition; a bias in the constant makes every field but the first digit's
+// unsigned, d = field - 2^(BETA-1), so the digits stay within +-2^(BETA-1) and the first
+// within +-2^BETA, and the remainder after the last digit is at most half of one.
+// `a`, `b`: the values times 2^(3 BETA - e).
+constexpr double kRound = 6755399441055744.0;  // 1.5 2^52
+
+__device__ inline uint32_t low_word(double t) { return (uint32_t)__builtin_bit_cast(uint64_t, t); }
+__device__ inline uint32_t low_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
+__device__ inline uint32_t high_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+
+// 1024 + field per binary16 half: a 10-bit field under the exponent of 1024 (and 2048 for the
+// field 1024, by the carry); subtracting 1024 + bias leaves the digit, exactly.
+__device__ inline uint32_t half_digits(uint32_t fields, float bias) {
+    typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+    const _Float16 off = (_Float16)(-1024.0f - bias);
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2_t, fields) + h2_t{off, off});
+}
+
+template <class SAT, int BETA, int S>
+struct PairDigits;
+
+template <int S>
+struct PairDigits<AtomF16x32, 9, S> {
+    static_assert(S == 6 || S == 7, "two triples and at most one digit more");
+    __device__ static inline void triple(uint32_t ua, uint32_t ub, uint32_t* d) {
+        typedef uint16_t us2_t __attribute__((ext_vector_type(2)));
+        const us2_t hi = __builtin_bit_cast(us2_t, high_halves(ua, ub)) >> (uint16_t)2;
+        d[0] = half_digits(__builtin_bit_cast(uint32_t, hi) + 0x64006400u, 512.0f);
+        d[1] = half_digits((low_halves(ua >> 9, ub >> 9) & 0x01FF01FFu) | 0x64006400u, 256.0f);
+        d[2] = half_digits((low_halves(ua, ub) & 0x01FF01FFu) | 0x64006400u, 256.0f);
+    }
+    __device__ static inline void make(double a, double b, uint32_t (&d)[S]) {
+        constexpr double M = kRound + (double)((512 << 18) + (256 << 9) + 256);
+        const double ta = a + M, tb = b + M;
+        triple(low_word(ta), low_word(tb), d);
+        const double ra = a - (ta - M), rb = b - (tb - M);  // exact
+        constexpr double W = 134217728.0;  // 2^27
+        const double sa = __builtin_fma(ra, W, M), sb = __builtin_fma(rb, W, M);
+        triple(low_word(sa), low_word(sb), d + 3);
+        if constexpr (S == 7) {
+            constexpr double M1 = kRound + 512.0;
+            const double qa = __builtin_fma(ra, W, -(sa - M)), qb = __builtin_fma(rb, W, -(sb - M));
+            const uint32_t f = low_halves(low_word(__builtin_fma(qa, 512.0, M1)), low_word(__builtin_fma(qb, 512.0, M1)));
+            d[6] = half_digits(f + 0x64006400u, 512.0f);
+        }
+    }
+};
+
+template <>
+struct PairDigits<AtomBF16x32, 8, 7> {
+    // |digit| <= 256 is exact in bfloat16: the upper half of its float
+    __device__ static inline uint32_t pack(float a, float b) {
+        return high_halves(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
+    }
+    __device__ static inline void triple(uint32_t ua, uint32_t ub, uint32_t* d) {
+        d[0] = pack((float)((int32_t)ua >> 16), (float)((int32_t)ub >> 16));
+        d[1] = pack((float)((ua >> 8) & 255u) - 128.0f, (float)((ub >> 8) & 255u) - 128.0f);
+        d[2] = pack((float)(ua & 255u) - 128.0f, (float)(ub & 255u) - 128.0f);
+    }
+    __device__ static inline void make(double a, double b, uint32_t (&d)[7]) {
+        constexpr double M = kRound + (double)((128 << 8) + 128);
+        const double ta = a + M, tb = b + M;
+        triple(low_word(ta), low_word(tb), d);
+        const double ra = a - (ta - M), rb = b - (tb - M);  // exact
+        constexpr double W = 16777216.0;  // 2^24
+        const double sa = __builtin_fma(ra, W, M), sb = __builtin_fma(rb, W, M);
+        triple(low_word(sa), low_word(sb), d + 3);
+        const double qa = __builtin_fma(ra, W, -(sa - M)), qb = __builtin_fma(rb, W, -(sb - M));
+        d[6] = pack((float)(int32_t)low_word(__builtin_fma(qa, 256.0, kRound)),
+                    (float)(int32_t)low_word(__builtin_fma(qb, 256.0, kRound)));
+    }
+};
+
+// Geometry of the persistent form: BT x BT tiles of C (BT = 64 or 32), BT / 8 waves on a
+// (BT / 16) x 2 grid, each 16 rows by one or two 16-column atoms.
+template <class SAT, int BT_, int BETA_, int S_, int G_>
+struct SplitStreamGeom {
+    static constexpr int BT = BT_, BETA = BETA_, S = S_, G = G_;
+    static constexpr int KC = 32;                    // K of a chunk
+    static constexpr int NT = 8 * BT;                // four threads per row of A and of B
+    static constexpr int PM = BT / 16, PN = 2, JN = BT / 32;
+    static constexpr int ROWS = 2 * BT;              // rows of A, then rows of B
+    static constexpr int PLANE = ROWS * KC * 2;      // one digit plane: 64-byte rows
+    static constexpr int EXP_OFF = S * PLANE;
+    static constexpr int BUF = EXP_OFF + ROWS * 4;   // digit planes and row exponents of a chunk
+    static constexpr int LDS = 2 * BUF;
+    // 16-byte piece p of row r lies in slot p ^ swz(r) of the row's four: the 32 lanes of a
+    // fragment read (16 rows, two neighbouring pieces) fall on different banks
+    static constexpr __device__ int swz(int r) { return ((r >> 3) & 1) << 1; }
+    static_assert(PM * PN * kWave == NT && JN * PN * 16 == BT, "wave grid");
+    static_assert(BUF % 16 == 0 && LDS <= 160 * 1024, "LDS budget");
+    static_assert(levels_exact(BETA, S, G, KC), "slice digits would not sum exactly in FP32");
+    // the two smallest levels are added in FP32 before they are converted
+    static_assert(G >= 3 && level_bound(BETA, S, G - 1, KC) * pow2(-24 - BETA * (G - 1)) <= pow2(-50),
+                  "the two smallest levels are combined in FP32");
+};
+
 // Persistent form.  A workgroup walks work units blockIdx.x, + gridDim.x, ... -- one unit
-// is a BM x BN tile of C of one problem (the whole problem for a block GEMM; a tile of a
-// larger GEMM for kami_split_gemm, with K any multiple of 32) -- and reads every operand
-// once: the exponents are taken per row and per 32-wide K chunk (so no
-// separate exponent pass over K is needed), the chunk is sliced from registers, and the
-// next chunk -- chunk 0 of the next problem after the last one -- is loaded while the
-// MFMAs of the current chunk run.  A chunk's level sums are combined in FP64 with the
-// weights 2^(-BETA g) and then scaled by 2^(e_i + f_j) of that chunk into the
+// is a BT x BT tile of C of one problem, K any multiple of 32 -- as one stream of 32-wide
+// K chunks.  The exponents are taken per row and per chunk, from the registers that hold
+// it, so no exponent pass over K is needed.  A chunk's level sums are combined in FP64 with
+// the weights 2^(-BETA g) and then scaled by 2^(e_i + f_j) of that chunk into the
 // accumulator, which holds C in absolute units.  Per-chunk exponents bound each chunk's
 // digits by the chunk's own row maximum, so the truncation error is no larger than
 // with exponents over the full K.
+//
+// Chunk s is multiplied from LDS buffer s mod 2 while chunk s + 1 is sliced into the other
+// one and chunk s + 2 is on its way in registers: one barrier a chunk.  Slicing is VALU work
+// and the products are matrix work; they are independent here, and the block is scheduled
+// as one matrix instruction and six VALU ones by turns, so both pipes run.
+// What bounds it: VALU issue (about 330 instructions a wave and chunk, two waves a SIMD,
+// beside 56 matrix instructions).  1024^3 with seven FP16 digits: 217 us with 128 x 128
+// tiles (64 of them on 256 CUs, slicing and products across barriers), 87 with 64 x 64
+// tiles and two buffers, 78 with PairDigits, 73 with the schedule.
+// Digit products of levels g <= G with S digits per operand
+constexpr int products_of(int S, int G) {
+    int n = 0;
+    for (int s = 1; s <= S; ++s)
+        for (int t = 1; t <= S; ++t) n += s + t <= G;
+    return n;
+}
+
+template <class SAT, class G>
+__global__ void __launch_bounds__(G::NT)
+split_stream_kernel(SplitArgs args, int64_t count) {
+    using frag_t = typename SAT::frag_t;
+    using accv_t = typename SAT::accv_t;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[G::LDS];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int pm = wave % G::PM, pn = wave / G::PM;
+    const int64_t grid = gridDim.x;
+    const int64_t lda = args.lda, ldb = args.ldb, ldc = args.ldc;
+    const int nch = args.nch;
+    // Unit u is tile u mod tiles of problem u / tiles, the column tile fastest.  Consecutive
+    // units go to one XCD (workgroup L runs on XCD L mod 8), whose L2 then serves the tiles
+    // that share rows of A or B.
+    const int64_t tiles = (int64_t)args.tiles_m * args.tiles_n;
+    const int64_t first = grid % 8 == 0 ? blockIdx.x % 8 * (grid / 8) + blockIdx.x / 8 : blockIdx.x;
+    struct Unit {
+        int64_t prob, tm, tn;
+    };
+    auto unit_at = [&](int64_t u) {
+        const int64_t prob = u / tiles, t = u - prob * tiles, tm = t / args.tiles_n;
+        return Unit{prob, tm, t - tm * args.tiles_n};
+    };
+    const Unit start = unit_at(first), step = unit_at(grid);
+    auto advance = [&](Unit& n) {  // to the workgroup's next unit, without a division
+        n.prob += step.prob;
+        n.tm += step.tm;
+        n.tn += step.tn;
+        if (n.tn >= args.tiles_n) {
+            n.tn -= args.tiles_n;
+            ++n.tm;
+        }
+        if (n.tm >= args.tiles_m) {
+            n.tm -= args.tiles_m;
+            ++n.prob;
+        }
+    };
+
+    // Slicing: thread t owns row t / 4 of the unit's rows of A and B and four 16-byte pieces
+    // of the chunk's 16, t mod 4 + 4 i: four lanes read 64 consecutive bytes.  The k values
+    // of a row thus lie permuted in LDS, the same way for A and B.
+    const int srow = tid >> 2, sq = tid & 3;
+    const bool row_a = wave < G::NT / 128;  // the first half of the waves slices A
+    auto unit_ptr = [&](const Unit& n) {
+        return row_a ? args.A + n.prob * args.sa + (n.tm * G::BT + srow) * lda + 2 * sq
+                     : args.B + n.prob * args.sb + (n.tn * G::BT + srow - G::BT) * ldb + 2 * sq;
+    };
+    Unit ln = start;                  // unit and chunk of the next load
+    int64_t lu = first;
+    int lc = 0;
+    const double* px = unit_ptr(ln);  // the thread's first piece of the chunk loaded last
+    // moves on to the next chunk; after the last one it stays there (loaded again, unused)
+    auto next_chunk = [&]() {
+        if (lc + 1 < nch) {
+            ++lc;
+            px += G::KC;
+        } else if (lu + grid < count) {
+            lu += grid;
+            lc = 0;
+            advance(ln);
+            px = unit_ptr(ln);
+        }
+    };
+    u4_t x[4];
+    auto load = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = load_raw<16>(px + 8 * i);
+    };
+    // Exponent e with |x| < 2^e over the row's 32 values of the chunk: the largest upper
+    // word of |x| (monotonic in |x|) over the thread's 8 values and the row's 4 threads (one
+    // DPP quad), completed with all-ones lower bits, so frexp also covers subnormal rows.
+    auto chunk_exp = [&]() {
+        uint32_t h = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h = max(h, max(x[i][1] & 0x7fffffffu, x[i][3] & 0x7fffffffu));
+        h = max(h, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h, 0xB1, 0xF, 0xF, false));  // quad_perm 1,0,3,2
+        h = max(h, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h, 0x4E, 0xF, 0xF, false));  // quad_perm 2,3,0,1
+        return __builtin_amdgcn_frexp_exp(__builtin_bit_cast(double, ((uint64_t)h << 32) | 0xffffffffu));
+    };
+    int e;      // row exponent of the chunk taken from x
+    d2_t v[4];  // its values, scaled
+    auto scale = [&]() {
+        e = chunk_exp();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const d2_t d = bitcast<d2_t>(x[i]);
+            v[i] = d2_t{__builtin_amdgcn_ldexp(d[0], 3 * G::BETA - e), __builtin_amdgcn_ldexp(d[1], 3 * G::BETA - e)};
+        }
+    };
+    u4_t plane[G::S];  // the scaled chunk's digits
+    auto slice = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t d[G::S];
+            PairDigits<SAT, G::BETA, G::S>::make(v[i][0], v[i][1], d);
+#pragma unroll
+            for (int s = 0; s < G::S; ++s) plane[s][i] = d[s];
+        }
+    };
+    auto write = [&](unsigned char* buf) {
+        // (by all four lanes of the row: a branch here would end the block that is scheduled)
+        reinterpret_cast<int*>(buf + G::EXP_OFF)[srow] = e;
+        unsigned char* const dst = buf + srow * 64 + ((sq ^ G::swz(srow)) << 4);
+#pragma unroll
+        for (int s = 0; s < G::S; ++s) store_raw<16>(dst + s * G::PLANE, plane[s]);
+    };
+
+    double acc[G::JN][4];
+    const int fr = lane & 15, slot = ((lane >> 4) ^ G::swz(fr)) << 4;
+    frag_t af[G::S], bf[G::S];
+    int erow[4], ecol[G::JN];
+    auto read_a = [&](const unsigned char* buf) {
+#pragma unroll
+        for (int s = 0; s < G::S; ++s)
+            af[s] = bitcast<frag_t>(load_raw<16>(buf + s * G::PLANE + (pm * 16 + fr) * 64 + slot));
+        const int* const expo = reinterpret_cast<const int*>(buf + G::EXP_OFF);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) erow[q] = expo[pm * 16 + 4 * (lane >> 4) + q];
+#pragma unroll
+        for (int jn = 0; jn < G::JN; ++jn) ecol[jn] = expo[G::BT + (pn * G::JN + jn) * 16 + fr];
+    };
+    auto read_b = [&](const unsigned char* buf, int jn) {
+#pragma unroll
+        for (int t = 0; t < G::S; ++t)
+            bf[t] = bitcast<frag_t>(load_raw<16>(buf + t * G::PLANE + (G::BT + (pn * G::JN + jn) * 16 + fr) * 64 + slot));
+    };
+    // Level sums of one 16 x 16 atom over the chunk: level g in T[g - 2]
+    struct Levels {
+        accv_t T[G::G - 1];
+    };
+    auto products = [&](Levels& l) {
+#pragma unroll
+        for (int g = 0; g < G::G - 1; ++g) l.T[g] = accv_t{0, 0, 0, 0};
+#pragma unroll
+        for (int t = 1; t <= G::S; ++t)
+#pragma unroll
+            for (int s = 1; s <= G::S; ++s)
+                if (s + t <= G::G) SAT::mma(l.T[s + t - 2], af[s - 1], bf[t - 1]);
+    };
+    auto combine = [&](const Levels& l, int jn) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            // Horner from the smallest weight, in units of level 2; the two
+            // smallest levels are added in FP32 first (rounding below 2^-50)
+            double cs = (double)__builtin_fmaf(l.T[G::G - 2][q], (float)pow2(-G::BETA), l.T[G::G - 3][q]);
+#pragma unroll
+            for (int g = G::G - 2; g >= 2; --g)
+                cs = __builtin_fma(cs, pow2(-G::BETA), (double)l.T[g - 2][q]);
+            acc[jn][q] += __builtin_amdgcn_ldexp(cs, erow[q] + ecol[jn] - 2 * G::BETA);
+        }
+    };
+    // one matrix instruction, then VALU others, `n` times (scheduling of the block so far)
+    constexpr int NP = products_of(G::S, G::G);
+
+    load();
+    scale();
+    next_chunk();
+    load();
+    slice();
+    write(smem);
+    __syncthreads();
+    int cur = 0;  // offset of the buffer being multiplied
+    Unit un = start;
+    for (int64_t u = first; u < count; u += grid) {
+#pragma unroll
+        for (int jn = 0; jn < G::JN; ++jn)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc[jn][q] = 0.0;
+        for (int c = 0; c < nch; ++c) {
+            scale();
+            next_chunk();
+            load();
+            unsigned char* const buf = smem + cur;
+            Levels l0, l1;
+            read_a(buf);
+            read_b(buf, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            products(l0);
+            slice();
+#pragma unroll
+            for (int i = 0; i < NP; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (G::JN == 2) read_b(buf, 1);
+            write(smem + (G::BUF - cur));
+            if constexpr (G::JN == 2) {
+                __builtin_amdgcn_sched_barrier(0);
+                products(l1);
+                combine(l0, 0);
+#pragma unroll
+                for (int i = 0; i < NP; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                combine(l1, 1);
+            } else {
+                combine(l0, 0);
+            }
+            __syncthreads();
+            cur = G::BUF - cur;
+        }
+
+        // ---- store ----
+        double* __restrict__ C = args.C + un.prob * args.sc + (un.tm * G::BT + pm * 16) * ldc +
+                                 un.tn * G::BT + pn * 16 * G::JN;
+#pragma unroll
+        for (int jn = 0; jn < G::JN; ++jn)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                double* dst = C + (int64_t)(4 * (lane >> 4) + v) * ldc + jn * 16 + (lane & 15);
+                double val = acc[jn][v] * args.alpha;
+                if (args.beta != 0.0) val += args.beta * (*dst);
+                *dst = val;
+            }
+        advance(un);
+    }
+}
+
+// Persistent form with 128 x 128 tiles of C: half the slicing per output of the 64 x 64 form,
+// but the digit planes of a chunk fill LDS, so slicing and products alternate across
+// barriers.  Same chunks, exponents and combination as split_stream_kernel; a workgroup of
+// eight waves (4 x 2) walks units blockIdx.x, + gridDim.x, ... and loads the next chunk while
+// the current one is multiplied.
 template <class SAT, class G>
 __global__ void __launch_bounds__(G::NT)
 split_pipe_kernel(SplitArgs args, int64_t count) {
@@ -725,6 +1068,9 @@ split_resident_kernel(SplitArgs args) {
         }
 }
 
+// Fewest 64 x 64 tiles that take the 64-wide form; below, 32 x 32 tiles use more of the chip.
+constexpr int64_t kSmallTileUnits = 128;
+
 template <class SAT, class G>
 hipError_t launch_split(const SplitArgs& a, int64_t count, hipStream_t s) {
     hipLaunchKernelGGL((split_gemm_kernel<SAT, G>), dim3((unsigned)count), dim3(G::NT), 0, s, a);
@@ -732,17 +1078,53 @@ hipError_t launch_split(const SplitArgs& a, int64_t count, hipStream_t s) {
 }
 
 // Persistent grid: every CU filled to the kernel's occupancy, never more workgroups
-// than problems.
+// than units.
 template <class SAT, class G>
-hipError_t launch_split_pipe(const SplitArgs& a, int64_t count, hipStream_t s) {
+static hipError_t launch_stream_tiles(const SplitArgs& a, int64_t units, hipStream_t s) {
+    static std::atomic<int> cache[kMaxCachedDevices];
+    int slots = 0;
+    const hipError_t e = resident_workgroups(split_stream_kernel<SAT, G>, G::NT, cache, &slots);
+    if (e != hipSuccess) return e;
+    const int64_t grid = std::min<int64_t>(units, (int64_t)slots);
+    hipLaunchKernelGGL((split_stream_kernel<SAT, G>), dim3((unsigned)grid), dim3(G::NT), 0, s, a,
+                       units);
+    return hipGetLastError();
+}
+
+template <class SAT, class G>
+static hipError_t launch_pipe_tiles(const SplitArgs& a, int64_t units, hipStream_t s) {
     static std::atomic<int> cache[kMaxCachedDevices];
     int slots = 0;
     const hipError_t e = resident_workgroups(split_pipe_kernel<SAT, G>, G::NT, cache, &slots);
     if (e != hipSuccess) return e;
-    const int64_t grid = std::min<int64_t>(count, (int64_t)slots);
+    const int64_t grid = std::min<int64_t>(units, (int64_t)slots);
     hipLaunchKernelGGL((split_pipe_kernel<SAT, G>), dim3((unsigned)grid), dim3(G::NT), 0, s, a,
-                       count);
+                       units);
     return hipGetLastError();
+}
+
+// a.tiles_m x a.tiles_n counts 64 x 64 tiles of C per problem.  A tile and chunk takes a CU
+// 2.3-2.7 us in the 64-wide form, 6.8-8.9 us in the 128-wide one (four times the outputs), so
+// the wide form is taken where its rounds over the chip, at three times the price, are
+// fewer: 128^3 x 4096 568 us against 676, but 1024^3 (64 wide tiles) 217 against 73 and
+// 1536^3 (144) 325 against 300.
+template <class SAT, int BETA, int S, int G>
+hipError_t launch_split_stream(const SplitArgs& a, int64_t count, hipStream_t s) {
+    const int64_t units = count * a.tiles_m * a.tiles_n;
+    auto rounds = [](int64_t n) { return (n + 255) / 256; };
+    if (a.tiles_m % 2 == 0 && a.tiles_n % 2 == 0 && 3 * rounds(units / 4) < rounds(units)) {
+        SplitArgs t = a;
+        t.tiles_m /= 2;
+        t.tiles_n /= 2;
+        using Geo = SplitGeom<SAT, 128, 128, 128, 4, 2, BETA, S, G>;
+        return launch_pipe_tiles<SAT, Geo>(t, units / 4, s);
+    }
+    if (units >= kSmallTileUnits)
+        return launch_stream_tiles<SAT, SplitStreamGeom<SAT, 64, BETA, S, G>>(a, units, s);
+    SplitArgs t = a;
+    t.tiles_m *= 2;
+    t.tiles_n *= 2;
+    return launch_stream_tiles<SAT, SplitStreamGeom<SAT, 32, BETA, S, G>>(t, 4 * units, s);
 }
 
 template <class SAT, class G>
@@ -757,8 +1139,10 @@ static void add_split(std::vector<SplitInstance>& v) {
     using Geo = SplitGeom<SAT, BM, BN, BK, PM, PN, BETA, S, G>;
     v.push_back(SplitInstance{PREC, BM, BN, BK, S, PM, PN, Geo::NT, Geo::LDS,
                               &launch_split<SAT, Geo>, 1, 0});
-    v.push_back(SplitInstance{PREC, BM, BN, BK, S, PM, PN, Geo::NT, Geo::LDS,
-                              &launch_split_pipe<SAT, Geo>, 2, 0});
+    using Str = SplitStreamGeom<SAT, 64, BETA, S, G>;
+    static_assert(BM % 64 == 0 && BN % 64 == 0, "64 x 64 tiles of C");
+    v.push_back(SplitInstance{PREC, BM, BN, BK, S, Str::PM, Str::PN, Str::NT, Str::LDS,
+                              &launch_split_stream<SAT, BETA, S, G>, 2, 0});
 }
 
 template <class SAT, int PREC, int BM, int BN, int BK, int PM, int PN, int BETA, int S, int G,
@@ -873,8 +1257,8 @@ kami_status split_launch(const kami_gemm_desc* d, const BlockArgs& b, int64_t co
     a.alpha = b.alpha;
     a.beta = b.beta;
     a.nch = d->k / 32;
-    a.tiles_m = 1;
-    a.tiles_n = 1;
+    a.tiles_m = d->m / 64;
+    a.tiles_n = d->n / 64;
     a.iters = b.iters;
     hipError_t e = in->launch(a, count, stream);
     if (e != hipSuccess) return hip_fail(e);
@@ -890,16 +1274,14 @@ kami_status split_gemm_tiled(const kami_gemm_desc* d, const BlockArgs& b, int64_
     if (d->b_layout != KAMI_B_NK || d->iters != 1) return KAMI_ENOTSUP;
     if (d->partition != KAMI_PART_AUTO && d->partition != KAMI_PART_2D) return KAMI_ENOTSUP;
     if (d->k % 32 != 0) return KAMI_ENOTSUP;
-    const int tile = (d->m % 128 == 0 && d->n % 128 == 0) ? 128
-                     : (d->m % 64 == 0 && d->n % 64 == 0) ? 64 : 0;
-    if (!tile) return KAMI_ENOTSUP;
+    if (d->m % 64 != 0 || d->n % 64 != 0) return KAMI_ENOTSUP;
     kami_gemm_desc t = *d;
-    t.m = t.n = t.k = tile;
+    t.m = t.n = t.k = 64;
     t.pipeline = 2;
     const SplitInstance* in = resolve_split(&t);
     if (!in) return KAMI_ENOTSUP;
-    const int64_t tiles = (int64_t)(d->m / tile) * (d->n / tile);
-    if (count > INT64_MAX / tiles) return KAMI_EINVAL;
+    const int64_t tiles = (int64_t)(d->m / 64) * (d->n / 64);
+    if (count > INT64_MAX / 4 / tiles) return KAMI_EINVAL;
     SplitArgs a;
     a.A = reinterpret_cast<const double*>(b.A);
     a.B = reinterpret_cast<const double*>(b.B);
@@ -913,12 +1295,12 @@ kami_status split_gemm_tiled(const kami_gemm_desc* d, const BlockArgs& b, int64_
     a.alpha = b.alpha;
     a.beta = b.beta;
     a.nch = d->k / 32;
-    a.tiles_m = d->m / tile;
-    a.tiles_n = d->n / tile;
+    a.tiles_m = d->m / 64;
+    a.tiles_n = d->n / 64;
     a.iters = 1;
     kami_status st = device_check();
     if (st != KAMI_OK) return st;
-    hipError_t e = in->launch(a, count * tiles, stream);
+    hipError_t e = in->launch(a, count, stream);
     if (e != hipSuccess) return hip_fail(e);
     return KAMI_OK;
 }
