@@ -282,6 +282,17 @@ __device__ inline void wave_lds_order() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Slot of 16-byte piece p of row r in LDS rows of RB bytes without padding: the 32 lanes of one
+// pass of a fragment read (16 rows, two neighbouring pieces) fall on different banks of the
+// 512-byte window.
+template <int RB>
+__device__ inline constexpr int line_slot(int r, int p) {
+    static_assert(RB == 32 || RB == 64 || RB == 128 || RB == 256, "line");
+    return RB == 256 ? p ^ (((r >> 1) & 7) << 1)
+           : RB == 128 ? p ^ (((r >> 2) & 3) << 1)
+           : RB == 64 ? p ^ (((r >> 3) & 1) << 1) : p;
+}
+
 // Transposing LDS read of 2-byte values (gfx950): each group of 16 lanes reads four rows
 // of 16 values, lane l of the group the four at row l / 4, columns 4 (l mod 4) .. + 3, and
 // receives column l of the four rows (layout checked with an in-bounds probe).

@@ -15,11 +15,10 @@
 //   fill   -- the stored bitmap (without a workspace: a rebuilt one) has its set bits
 //             written in ascending order, each thread placing the bits of one 32-bit word
 //             after the prefix popcount of the words before it;
-//   numeric -- one wave per output block (i, j): the row i comes from a 64-way search
-//             of rowptrC; the lanes binary-search B's sorted rows k of all blocks (i, k)
-//             of A at once for column j; A fragments are loaded straight into
-//             registers, B blocks (row-major K x N) are transposed through the wave's LDS
-//             into the K-contiguous MFMA layout.
+//   numeric -- one wave per output block (i, j): the row i comes from a 256-way search of
+//             rowptrC; the lanes binary-search B's sorted rows k of all blocks (i, k) of A
+//             at once for column j; both blocks are loaded by whole lines and turned into
+//             MFMA fragments in the wave's own LDS.
 // All integer phases are exact and deterministic.  B may have at most 491520 block
 // columns (a 60 KiB bitmap).
 #include <algorithm>
@@ -219,25 +218,36 @@ spgemm_fill_kernel(int mb, int nwords, const int32_t* rpA, const int32_t* ciA,
 }
 
 // ---- numeric: one wave per output block ----
-
+//
+// What bounds it: 6606 output blocks of 32 x 32 (8192^2, 2 %, FP16) are one round of waves on
+// the chip: 9.7 us replayed from a graph (10.1 with fragments of A straight from memory and B
+// turned by 2-byte LDS writes), of which the launch and the searches take 3.6, the products
+// 1.7 and the 27 MB of C 4.4, near the rate at which the card writes.  Where a row has many
+// products, their operands from L2 bound it: 8 % of 512 x 512 blocks of 32, FP16 517 -> 396 us;
+// FP64 2 % of 256 x 256 34.2 -> 23.0 us.  Comparing all (A entry, B entry) pairs of a short row
+// at once instead of searching took as long (9.6) or longer (16 x 16 blocks: 35.0 against 30.3).
 template <int BS, class AT>
 struct SpNumGeom {
     static constexpr int IM = BS / 16;                 // atom rows (= atom cols)
     static constexpr int KSTEPS = BS / AT::KSTEP;
-    static constexpr int ELT = (int)sizeof(typename AT::in_t);
-    static constexpr int ROWB = lds_row_bytes(BS * ELT, AT::FRAG_BYTES);  // transposed B row
-    static constexpr int LDS = BS * ROWB;
-    static constexpr int CHUNKS = BS * BS * ELT / 16;   // 16-byte pieces of a block
-    static constexpr int PER_LANE = (CHUNKS + 63) / 64;
+    static constexpr int ELT = (int)sizeof(typename AT::in_t), VE = 16 / ELT;
+    static constexpr bool F64 = ELT == 8;
+    // A block: rows of RB bytes, loaded PPR lanes a row and turned into fragments through
+    // LDS (a load of fragments puts 16 rows under 16 consecutive lanes, which the address
+    // unit takes four lanes a clock).  B block: FP64 fragments straight from memory (16 lanes
+    // read 16 consecutive columns); 2-byte rows are staged as they lie and turned by
+    // transposing LDS reads.  A 2-byte block of 16 x 16 is 512 consecutive bytes, which one
+    // load of its fragments reads whole: no staging of A.
+    static constexpr int RB = BS * ELT, PPR = RB / 16, PIECES = BS * PPR;
+    static constexpr int NP = (PIECES + 63) / 64;      // 16-byte pieces of a lane
+    static constexpr int TROW = RB + 16;               // bytes of a staged row of B
+    static constexpr int NB = F64 ? IM * KSTEPS : NP;
+    static constexpr bool A_LINES = RB > 32;
+    static constexpr int A_LDS = A_LINES ? BS * RB : 0;
+    static constexpr int LDS = A_LDS + (F64 ? 0 : BS * TROW);
 };
 
-// The numeric kernel's workgroup is one wave: its LDS accesses complete in order, so
-// sB needs no workgroup barrier, only this wave's LDS operations finished and a
-// compiler fence.  (__syncthreads() would also wait for every global load in flight.)
-__device__ inline void wave_lds_sync() {
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0); vmcnt and expcnt left at their maxima
-    __builtin_amdgcn_wave_barrier();
-}
+constexpr int kNumWaves = 4;  // waves (output blocks) of a workgroup
 
 __device__ inline int find_col(const int32_t* ci, int lo, int hi, int j) {
     // index in [lo, hi) with ci[idx] == j, or -1 (ci ascending within the row)
@@ -249,8 +259,30 @@ __device__ inline int find_col(const int32_t* ci, int lo, int hi, int j) {
     return (lo < end && ci[lo] == j) ? lo : -1;
 }
 
+// Block row of output block cb: the last row with rpC[row] <= cb, found by a 256-way search
+// (each round a lane probes four of 256 evenly spaced row pointers).
+__device__ inline int row_of(const int32_t* rpC, int mb, int64_t cb, int lane) {
+    int lo = 0, hi = mb;
+    while (hi - lo > 1) {
+        const int64_t step = ((int64_t)hi - lo + 255) / 256;
+        int c = 0;
+        bool le[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t idx = lo + (lane + 64 * q + 1) * step;
+            le[q] = idx < hi && (int64_t)rpC[idx] <= cb;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) c += __popcll(__ballot(le[q]));  // probes are monotone
+        const int64_t nlo = lo + c * step;
+        hi = (int)min((int64_t)hi, nlo + step);
+        lo = (int)nlo;
+    }
+    return __builtin_amdgcn_readfirstlane(lo);
+}
+
 template <int BS, class AT>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(64 * kNumWaves)
 spgemm_numeric_kernel(int mb, int64_t nnzc, const int32_t* rpA, const int32_t* ciA,
                       const void* vA_, const int32_t* rpB, const int32_t* ciB, const void* vB_,
                       const int32_t* rpC, const int32_t* ciC, void* vC_, double alpha_d,
@@ -261,107 +293,117 @@ spgemm_numeric_kernel(int mb, int64_t nnzc, const int32_t* rpA, const int32_t* c
     using out_t = typename AT::out_t;
     using frag_t = typename AT::frag_t;
     using accv_t = typename AT::accv_t;
-    constexpr int FB = AT::FRAG_BYTES;
-    __shared__ __attribute__((aligned(16))) unsigned char sB[G::LDS];
+    constexpr int FB = AT::FRAG_BYTES, IM = G::IM, KSTEPS = G::KSTEPS;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[kNumWaves * G::LDS];
     const in_t* vA = reinterpret_cast<const in_t*>(vA_);
     const in_t* vB = reinterpret_cast<const in_t*>(vB_);
     out_t* vC = reinterpret_cast<out_t*>(vC_);
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63, grp = lane >> 4, r16 = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    unsigned char* const lds = smem + wave * G::LDS;
     const acc_t alpha = (acc_t)alpha_d;
+    // XCD x = L mod 8 takes a contiguous run of output blocks, so that a row of A is read by
+    // one XCD: a bijection of [0, gridDim.x), as in spmm.hip
+    const uint32_t L = blockIdx.x, x8 = L % 8, q8 = gridDim.x / 8, r8 = gridDim.x % 8;
+    const int64_t P = x8 * q8 + (x8 < r8 ? x8 : r8) + L / 8;
 
-    for (int64_t cb = blockIdx.x; cb < nnzc; cb += gridDim.x) {
-        const int j = ciC[cb];  // issued before the row search, which does not need it
-        // block row of output block cb: the last row with rpC[row] <= cb, found by a
-        // 64-way search (each round the lanes probe 64 evenly spaced row pointers)
-        int lo = 0, hi = mb;
-        while (hi - lo > 1) {
-            const int step = (hi - lo + 63) / 64;
-            const int idx = lo + (lane + 1) * step;
-            const bool le = idx < hi && (int64_t)rpC[idx] <= cb;
-            const int c = __popcll(__ballot(le));  // probes are monotone: a prefix is set
-            const int nlo = lo + c * step;
-            hi = min(hi, nlo + step);
-            lo = nlo;
-        }
-        const int i = lo;
-        accv_t acc[G::IM][G::IM];
+    for (int64_t cb = P * kNumWaves + wave; cb < nnzc; cb += (int64_t)gridDim.x * kNumWaves) {
+        const int j = load_uniform(ciC + cb);
+        const int i = row_of(rpC, mb, cb, lane);
+        accv_t acc[IM][IM];
 #pragma unroll
-        for (int a = 0; a < G::IM; ++a)
+        for (int a = 0; a < IM; ++a)
 #pragma unroll
-            for (int b = 0; b < G::IM; ++b)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc[a][b][v] = 0;
+            for (int b = 0; b < IM; ++b) acc[a][b] = accv_t{0, 0, 0, 0};
 
-        // every lane searches the B row of one block of A's row i for column j; the
-        // matches are then multiplied in ascending order of A's blocks
-        const int a0 = rpA[i], a1 = rpA[i + 1];
-        for (int base = a0; base < a1; base += 64) {
-          const int tl = base + lane;
-          int lmatch = -1;
-          if (tl < a1) {
-              const int k = ciA[tl];
-              lmatch = find_col(ciB, rpB[k], rpB[k + 1], j);
-          }
-          uint64_t todo = __ballot(lmatch >= 0);
-          while (todo) {
-            const int src = __ffsll((unsigned long long)todo) - 1;
-            todo &= todo - 1;
-            const int t = base + src;
-            const int l = __shfl(lmatch, src);
+        // products of A block t and B block l
+        auto product = [&](int t, int l) {
             const in_t* Ablk = vA + (int64_t)t * BS * BS;
             const in_t* Bblk = vB + (int64_t)l * BS * BS;
-            // A fragments straight to registers, issued with the B block's loads
-            frag_t af[G::KSTEPS][G::IM], bf[G::KSTEPS][G::IM];
+            u4_t pa[G::NP], pb[G::NB];
+            frag_t af[KSTEPS][IM], bf[KSTEPS][IM];
+            if constexpr (!G::A_LINES) af[0][0] = bitcast<frag_t>(load_raw<FB>(Ablk + r16 * BS + AT::KV * grp));
 #pragma unroll
-            for (int ks = 0; ks < G::KSTEPS; ++ks) {
-                const int kk = ks * AT::KSTEP + AT::KV * (lane >> 4);
-#pragma unroll
-                for (int x = 0; x < G::IM; ++x)
-                    af[ks][x] = bitcast<frag_t>(load_raw<FB>(Ablk + (x * 16 + (lane & 15)) * BS + kk));
+            for (int q = 0; q < G::NP; ++q) {
+                const int c = (lane + 64 * q) % G::PIECES;  // a short block's pieces repeat
+                if constexpr (G::A_LINES) pa[q] = load_raw<16>(Ablk + c * G::VE);
+                if constexpr (!G::F64) pb[q] = load_raw<16>(Bblk + c * G::VE);
             }
-            // B block (row-major K x N) -> LDS as N rows of K (transposed)
+            if constexpr (G::F64) {
 #pragma unroll
-            for (int q = 0; q < G::PER_LANE; ++q) {
-                const int c = lane + 64 * q;
-                if (c >= G::CHUNKS) break;
-                constexpr int CPR = BS * G::ELT / 16;   // pieces per block row
-                const int kr = c / CPR, jc = (c % CPR) * (16 / G::ELT);
-                const u4_t raw = load_raw<16>(Bblk + kr * BS + jc);
-                const in_t* e = reinterpret_cast<const in_t*>(&raw);
+                for (int ks = 0; ks < KSTEPS; ++ks)
 #pragma unroll
-                for (int x = 0; x < 16 / G::ELT; ++x)
-                    *reinterpret_cast<in_t*>(sB + (jc + x) * G::ROWB + kr * G::ELT) = e[x];
+                    for (int x = 0; x < IM; ++x) {
+                        const in_t* p = Bblk + (ks * AT::KSTEP + 2 * grp) * BS + x * 16 + r16;
+                        pb[ks * IM + x] = bitcast<u4_t>(d2_t{p[0], p[BS]});
+                    }
             }
-            wave_lds_sync();
+            wave_lds_order();  // the previous product's fragments are read
+#pragma unroll
+            for (int q = 0; q < G::NP; ++q) {
+                const int c = (lane + 64 * q) % G::PIECES, row = c / G::PPR, piece = c % G::PPR;
+                if constexpr (G::A_LINES)
+                    store_raw<16>(lds + row * G::RB + (line_slot<G::RB>(row, piece) << 4), pa[q]);
+                if constexpr (!G::F64)
+                    store_raw<16>(lds + G::A_LDS + row * G::TROW + piece * 16, pb[q]);
+            }
+            wave_lds_order();
             // both blocks' fragments in registers; `iters` > 1 repeats the products on them
             // (the reference's in-kernel NUM_ITER repeat), iters = 1 is the plain product
 #pragma unroll
-            for (int ks = 0; ks < G::KSTEPS; ++ks) {
-                const int kk = ks * AT::KSTEP + AT::KV * (lane >> 4);
+            for (int ks = 0; ks < KSTEPS; ++ks)
 #pragma unroll
-                for (int x = 0; x < G::IM; ++x)
-                    bf[ks][x] = bitcast<frag_t>(
-                        load_raw<FB>(sB + (x * 16 + (lane & 15)) * G::ROWB + kk * G::ELT));
-            }
-            wave_lds_sync();  // the fragments are read before the next match rewrites sB
+                for (int x = 0; x < IM; ++x) {
+                    const unsigned char* line = lds + (x * 16 + r16) * G::RB;
+                    if constexpr (G::A_LINES)
+                        af[ks][x] = bitcast<frag_t>(load_raw<FB>(line + (line_slot<G::RB>(r16, 4 * ks + grp) << 4)));
+                    if constexpr (G::F64) {
+                        bf[ks][x] = bitcast<frag_t>(pb[ks * IM + x]);
+                    } else {
+                        const unsigned char* p = lds + G::A_LDS +
+                                                 (ks * AT::KSTEP + AT::KV * grp + (r16 >> 2)) * G::TROW +
+                                                 x * 32 + 8 * (lane & 3);
+                        if constexpr (FB == 16) {
+                            const u2_t lo = lds_read_turned(p), hi = lds_read_turned(p + 4 * G::TROW);
+                            bf[ks][x] = bitcast<frag_t>(u4_t{lo[0], lo[1], hi[0], hi[1]});
+                        } else {
+                            bf[ks][x] = bitcast<frag_t>(lds_read_turned(p));
+                        }
+                    }
+                }
             for (int it = 0; it < iters; ++it)
 #pragma unroll
-                for (int ks = 0; ks < G::KSTEPS; ++ks)
+                for (int ks = 0; ks < KSTEPS; ++ks)
 #pragma unroll
-                    for (int jn = 0; jn < G::IM; ++jn)
+                    for (int jn = 0; jn < IM; ++jn)
 #pragma unroll
-                        for (int im = 0; im < G::IM; ++im) AT::mma(acc[im][jn], af[ks][im], bf[ks][jn]);
-          }
+                        for (int im = 0; im < IM; ++im) AT::mma(acc[im][jn], af[ks][im], bf[ks][jn]);
+        };
+
+        // A's row i, 64 entries at a time, one per lane: its blocks (i, k) whose B row k holds
+        // column j are multiplied in ascending order
+        const int a0 = load_uniform(rpA + i), a1 = load_uniform(rpA + i + 1);
+        for (int base = a0; base < a1; base += 64) {
+            int match = -1;
+            if (base + lane < a1) {
+                const int k = ciA[base + lane];
+                match = find_col(ciB, rpB[k], rpB[k + 1], j);
+            }
+            uint64_t todo = __ballot(match >= 0);
+            while (todo) {
+                const int src = __ffsll((unsigned long long)todo) - 1;
+                todo &= todo - 1;
+                product(base + src, __builtin_amdgcn_readlane(match, src));
+            }
         }
         out_t* Cblk = vC + cb * BS * BS;
 #pragma unroll
-        for (int im = 0; im < G::IM; ++im)
+        for (int im = 0; im < IM; ++im)
 #pragma unroll
-            for (int jn = 0; jn < G::IM; ++jn)
+            for (int jn = 0; jn < IM; ++jn)
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    Cblk[(im * 16 + AT::out_row(lane, v)) * BS + jn * 16 + (lane & 15)] =
-                        (out_t)(alpha * acc[im][jn][v]);
+                    Cblk[(im * 16 + AT::out_row(lane, v)) * BS + jn * 16 + r16] = (out_t)(alpha * acc[im][jn][v]);
     }
 }
 
@@ -522,9 +564,9 @@ kami_status kami_bsr_spgemm_numeric_repeat(const kami_bsr* A, const kami_bsr* B,
     st = device_check();
     if (st != KAMI_OK) return st;
     hipStream_t s = (hipStream_t)stream;
-    const unsigned grid = (unsigned)std::min<int64_t>(nnzbC, 1 << 20);
+    const unsigned grid = (unsigned)std::min<int64_t>((nnzbC + kNumWaves - 1) / kNumWaves, 1 << 20);
 #define KAMI_SPNUM(BS, AT)                                                                      \
-    hipLaunchKernelGGL((spgemm_numeric_kernel<BS, AT>), dim3(grid), dim3(64), 0, s, A->mb,       \
+    hipLaunchKernelGGL((spgemm_numeric_kernel<BS, AT>), dim3(grid), dim3(64 * kNumWaves), 0, s, A->mb,       \
                        nnzbC, A->rowptr, A->colidx, A->vals, B->rowptr, B->colidx, B->vals,      \
                        rowptrC, colidxC, valC, alpha, (int)iters)
     if (precision == KAMI_PREC_F16_F32) {

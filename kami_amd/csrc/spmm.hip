@@ -73,11 +73,6 @@ struct SpmmGeom {
     static constexpr int CROW = WTN * 4 + 16;
     static constexpr int PART = F64 ? IM * CT * 4 * 64 * 8 : BS * CROW;
     static constexpr int WAVE_LDS = A_LDS + B_LDS > PART ? A_LDS + B_LDS : PART;
-    // slot of piece p of line r: p ^ swz(r), so that the 32 lanes of a fragment read (16
-    // lines, two neighbouring pieces) fall on different banks of the 512-byte window
-    static constexpr __device__ int swz(int r) {
-        return RB == 128 ? ((r >> 2) & 3) << 1 : RB == 64 ? ((r >> 3) & 1) << 1 : 0;
-    }
     static_assert(BS % AT::KSTEP == 0 && BS % 16 == 0 && KS % AT::KSTEP == 0, "block size");
     static_assert(WAVES * WAVE_LDS <= 160 * 1024 && NT <= 1024, "workgroup");
 };
@@ -167,13 +162,13 @@ spmm_kernel(SpmmArgs a) {
 #pragma unroll
         for (int t = 0; t < G::NA; ++t) {
             const int r = lrow % BS + t * G::RPI;
-            store_raw<16>(lds + r * G::RB + ((lpiece ^ G::swz(r)) << 4), s.a[t]);
+            store_raw<16>(lds + r * G::RB + (line_slot<G::RB>(r, lpiece) << 4), s.a[t]);
         }
 #pragma unroll
         for (int j = 0; j < G::NB; ++j) {
             if constexpr (!KN) {
                 const int r = lrow % G::WTN + j * G::RPI;
-                store_raw<16>(lds + G::A_LDS + r * G::RB + ((lpiece ^ G::swz(r)) << 4), s.b[j]);
+                store_raw<16>(lds + G::A_LDS + r * G::RB + (line_slot<G::RB>(r, lpiece) << 4), s.b[j]);
             } else if constexpr (G::TURN) {
                 const int p = (lane + 64 * j) % (G::KS * G::TPR);
                 store_raw<16>(lds + G::A_LDS + (p / G::TPR) * G::TROW + (p % G::TPR) * 16, s.b[j]);
@@ -187,7 +182,7 @@ spmm_kernel(SpmmArgs a) {
         const int r = lane & 15;
         auto line_frag = [&](const unsigned char* base, int t) {
             if constexpr (FB == 16)
-                return bitcast<frag_t>(load_raw<FB>(base + r * G::RB + (((4 * t + grp) ^ G::swz(r)) << 4)));
+                return bitcast<frag_t>(load_raw<FB>(base + r * G::RB + (line_slot<G::RB>(r, 4 * t + grp) << 4)));
             else
                 return bitcast<frag_t>(load_raw<FB>(base + r * G::RB + grp * FB));
         };
