@@ -127,6 +127,28 @@ def _stream_ptr(stream):
     return ctypes.c_void_p(stream.cuda_stream)
 
 
+_FAST = None
+
+
+def _fast():
+    """The native call path (host/fast_calls.cpp), bound to the loaded library.  Its functions
+    answer None to any call that is not plain, and the wrapper then checks and calls itself."""
+    global _FAST
+    if _FAST is None:
+        path = os.path.join(_abi.HERE, "_fast_calls.so")
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is missing: build it with `make -C kami_amd/csrc` "
+                               "(or __graft_entry__.build())")
+        import torch  # noqa: F401  (the extension links against it)
+        from . import _fast_calls
+        L = lib()
+        _fast_calls.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (
+            L.kami_block_gemm, L.kami_split_gemm, L.kami_batched_execute, L.kami_bsr_spgemm_symbolic,
+            L.kami_bsr_spgemm_fill, L.kami_bsr_spgemm_numeric, L.kami_bsr_spmm)))
+        _FAST = _fast_calls
+    return _FAST
+
+
 def block_gemm(A, B, C=None, *, precision=None, partition="auto", ranks=0, b_layout="nk",
                iters=1, alpha=1.0, beta=0.0, slices=0, pipeline=0, stream=None):
     """C = alpha * A @ op(B) + beta * C for a batch of problems, one per workgroup.
@@ -135,6 +157,12 @@ def block_gemm(A, B, C=None, *, precision=None, partition="auto", ranks=0, b_lay
     (count, K, N) ("kn"); C: (count, M, N), float64 for FP64 and split precision,
     float32 for FP16/BF16 inputs.  Tensors must be contiguous device tensors.
     """
+    if stream is None:
+        out = (_FAST or _fast()).block_gemm(
+            A, B, C, -1 if precision is None else precision, _part(partition), ranks,
+            _layout(b_layout), iters, alpha, beta, slices, pipeline, 0)
+        if out is not None:
+            return out
     import torch
     squeeze = A.dim() == 2
     if squeeze:
@@ -169,6 +197,11 @@ def split_gemm(A, B, C=None, *, precision=PREC_F64_SPLIT_F16, slices=0, alpha=1.
 
     A: (count, M, K) or (M, K) float64; B: (count, N, K) or (N, K); C like A @ B^T.
     """
+    if stream is None:
+        out = (_FAST or _fast()).block_gemm(A, B, C, precision, PART_AUTO, 0, B_NK, 1, alpha, beta,
+                                            slices, 0, 1)
+        if out is not None:
+            return out
     import torch
     squeeze = A.dim() == 2
     if squeeze:
@@ -275,10 +308,13 @@ class BatchedPlan:
                                              _stream_ptr(stream), ctypes.byref(handle)),
               "kami_batched_plan_create")
         self._h = handle
+        self._plan = handle.value
         self._keep = problems
         self.precision = prec
 
     def execute(self, stream=None):
+        if stream is None and self._plan and (_FAST or _fast()).batched_execute(self._plan):
+            return
         check(lib().kami_batched_execute(self._h, _stream_ptr(stream)), "kami_batched_execute")
 
     def info(self) -> dict:
@@ -291,7 +327,7 @@ class BatchedPlan:
     def close(self):
         if getattr(self, "_h", None):
             lib().kami_batched_plan_destroy(self._h)
-            self._h = None
+            self._h = self._plan = None
 
     def __del__(self):
         try:
@@ -477,6 +513,12 @@ def spgemm_numeric(A: BsrMatrix, B: BsrMatrix, rowptrC, colidxC, *, precision=No
 
 def bsr_spgemm(A: BsrMatrix, B: BsrMatrix, *, precision=None, alpha=1.0, stream=None):
     """C = alpha * A * B as a BsrMatrix (symbolic, fill and numeric phases)."""
+    if stream is None and type(A) is BsrMatrix and type(B) is BsrMatrix:
+        out = (_FAST or _fast()).bsr_spgemm(
+            A.mb, A.nb, A.bs, A.rowptr, A.colidx, A.vals, B.mb, B.nb, B.bs, B.rowptr, B.colidx,
+            B.vals, -1 if precision is None else precision, alpha)
+        if out is not None:
+            return BsrMatrix(A.mb, B.nb, A.bs, *out)
     ws = spgemm_workspace(A, B)
     rowptr, nnz = spgemm_symbolic(A, B, stream, workspace=ws)
     colidx = spgemm_fill(A, B, rowptr, nnz, stream, workspace=ws)
@@ -491,6 +533,12 @@ def bsr_spmm(A: BsrMatrix, B, C=None, *, b_layout="nk", precision=None, alpha=1.
     b_layout "nk": B is (n, K) row-major and C(i, j) = sum_k A(i, k) B[j, k] (the
     reference's layout); "kn": B is (K, n).  K = A.nb * A.bs.  C is (A.mb * A.bs, n),
     float32 for FP16/BF16 inputs, float64 for FP64."""
+    if stream is None and type(A) is BsrMatrix:
+        out = (_FAST or _fast()).bsr_spmm(
+            A.mb, A.nb, A.bs, A.rowptr, A.colidx, A.vals, B, C, B_KN if b_layout == "kn" else B_NK,
+            -1 if precision is None else precision, alpha, beta)
+        if out is not None:
+            return out
     import torch
     A.check("A")
     prec = _precision_of(A.vals if A.nnzb else B, precision)
