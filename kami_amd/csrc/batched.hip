@@ -8,7 +8,8 @@
 //   * problems carry their own {m, n, k, lda, ldb, ldc, A, B, C} (the kami_problem array);
 //   * every problem is cut into output tiles; a tile is one 64-byte queue entry holding
 //     its own operand pointers, strides, extents and variant (WorkItem);
-//   * an entry is cut into wave tiles of up to 32 x 32 (WaveUnit, 8 bytes each).  A wave
+//   * an entry is cut into wave tiles of up to 32 x 32 (2-byte inputs: 64 x 32; WaveUnit, 8
+//     bytes each).  A wave
 //     computes one of them alone, staged through LDS of its own, so there is no barrier
 //     and no shared counter: the hardware's dispatcher hands out the workgroups, longest
 //     problems first, and one wave's loads hide behind the products of the others;
@@ -21,10 +22,10 @@
 // M, N and K must be multiples of 16.
 //
 // What bounds it: 20000 problems of 16 to 256 (3.58 GB FP64, 1.19 GB FP16 with FP32 C) run
-// in 801 us and 293 us, 4.5 and 4.1 TB/s of the algorithmic bytes; the matrix pipes are
-// 57 % busy in FP64.  The persistent form this replaced (workgroups popping tiles of up to
+// in 810 us and 290 us, 4.4 and 4.1 TB/s of the algorithmic bytes; the matrix pipes are
+// 57 % busy in FP64, and L1 takes 10 TB/s of lines from L2 in either.  The persistent form this replaced (workgroups popping tiles of up to
 // 128 x 128 from an atomic counter, LDS stages shared by four waves, one barrier a stage, a
-// one-thread kernel to clear the counter) took 1023 us and 388 us: two workgroups a CU and
+// one-thread kernel to clear the counter) took 1027 us and 398 us: two workgroups a CU and
 // their barriers left too little in flight.
 #include <algorithm>
 #include <cstring>
@@ -61,7 +62,7 @@ constexpr int kVariants = 6;
 static_assert(kVariants == kBatchedVariants, "tuning-cache variant range");
 static const int kVariantTM[kVariants] = {64, 32, 64, 128, 128, 64};
 static const int kVariantTN[kVariants] = {64, 32, 64, 64, 128, 128};
-static const int kVariantSM[kVariants] = {2, 2, 1, 2, 2, 2};  // atoms of a wave tile
+static const int kVariantSM[kVariants] = {4, 4, 1, 4, 4, 4};  // atoms of a wave tile, at most
 static const int kVariantSN[kVariants] = {2, 2, 2, 2, 2, 2};
 
 // Variants a precision offers: 4 and 5 are FP64's.
@@ -74,15 +75,30 @@ struct WaveUnit {
     uint8_t ra, ca, im, jn;
 };
 static_assert(sizeof(WaveUnit) == 8, "wave unit layout");
-constexpr int kWaveAtoms = 2;  // atoms of a wave tile per dimension, at most
+// Wave tiles in atoms, largest first; a precision starts at first_cap.  2-byte inputs take
+// 64 x 32: the rate at which a CU's L1 takes lines bounds them, and a taller tile reads B's
+// half as often (20000 problems of 16 to 256: 284 us against 304 with 32 x 32; 64 x 64 tiles, at
+// two waves a SIMD, 273, but 109 against 102 at 128^3 x 4096 and 23.8 against 21.7 for problems
+// of 16 to 64).  FP64 takes 32 x 32: 64 x 32 at two waves a SIMD, 789 us against 808, leaves
+// 60 against 59 for problems of 16 to 64 and twice the registers.
+constexpr int kCaps = 4;
+static const int kCapM[kCaps] = {4, 2, 1, 1}, kCapN[kCaps] = {2, 2, 2, 1};
+constexpr int kMostN = 2;
+constexpr int first_cap(int elt) { return elt == 8 ? 1 : 0; }
 constexpr int kWavesPerGroup = 4;
 constexpr int kXcds = 8;  // workgroup L runs on XCD L mod 8
+
+// Where the unit of wave w of workgroup L of `groups` lies
+__host__ __device__ inline int64_t unit_at(int64_t L, int64_t groups, int w) {
+    return (L % kXcds * (groups / kXcds) + L / kXcds) * kWavesPerGroup + w;
+}
 
 struct BatchArgs {
     const WorkItem* items;
     const WaveUnit* units;
-    int64_t n_units;  // a multiple of kWavesPerGroup
+    int64_t n_units;  // a multiple of kWavesPerGroup x kXcds
     double alpha, beta;
+    int tall;  // 1: wave tiles may be four atoms high (cap 0)
 };
 
 __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
@@ -205,45 +221,48 @@ struct WaveTile {
         }
     }
 
-    struct Frags {
-        frag_t a[IM][NF], b[JN][NF];
+    // FP64 K x N: B's fragments as loaded, kept while the stage's registers are loaded again
+    struct Held {
+        u4_t b[KN && F64 ? NB : 1];
+        __device__ __forceinline__ explicit Held(const Stage& s) {
+            if constexpr (KN && F64)
+#pragma unroll
+                for (int j = 0; j < NB; ++j) b[j] = s.b[j];
+        }
     };
-    // Fragments of the stage in LDS (FP64 K x N: `s`, which holds B's as loaded)
-    __device__ __forceinline__ void read(const Stage& s, Frags& f) const {
+
+    // Products of the stage in LDS, one fragment (half a line) at a time
+    __device__ __forceinline__ void mma(const Held& held, accv_t (&acc)[IM][JN]) const {
 #pragma unroll
-        for (int i = 0; i < IM; ++i)
+        for (int t = 0; t < NF; ++t) {
+            frag_t a[IM], b[JN];
 #pragma unroll
-            for (int t = 0; t < NF; ++t)
-                f.a[i][t] = bitcast<frag_t>(load_raw<16>(lds + (roff ^ (t * 64)) + i * 2048));
-        if constexpr (TURN) {
-            const unsigned char* p = lds + A_LDS + (8 * grp + ((lane & 15) >> 2)) * TROW + 8 * (lane & 3);
+            for (int i = 0; i < IM; ++i)
+                a[i] = bitcast<frag_t>(load_raw<16>(lds + (roff ^ (t * 64)) + i * 2048));
+            if constexpr (TURN) {
+                const unsigned char* p = lds + A_LDS + (8 * grp + ((lane & 15) >> 2)) * TROW + 8 * (lane & 3);
 #pragma unroll
-            for (int j = 0; j < JN; ++j)
-#pragma unroll
-                for (int t = 0; t < NF; ++t) {
+                for (int j = 0; j < JN; ++j) {
                     const u2_t lo = lds_read_turned(p + t * 32 * TROW + j * 32);
                     const u2_t hi = lds_read_turned(p + (t * 32 + 4) * TROW + j * 32);
-                    f.b[j][t] = bitcast<frag_t>(u4_t{lo[0], lo[1], hi[0], hi[1]});
+                    b[j] = bitcast<frag_t>(u4_t{lo[0], lo[1], hi[0], hi[1]});
                 }
-        } else {
+            } else {
 #pragma unroll
-            for (int j = 0; j < JN; ++j)
-#pragma unroll
-                for (int t = 0; t < NF; ++t)
-                    f.b[j][t] = KN ? bitcast<frag_t>(s.b[j * NF + t])
-                                   : bitcast<frag_t>(load_raw<16>(lds + A_LDS + (roff ^ (t * 64)) + j * 2048));
-        }
-    }
-
-    __device__ __forceinline__ void mma(const Frags& f, accv_t (&acc)[IM][JN]) const {
-#pragma unroll
-        for (int t = 0; t < NF; ++t)
+                for (int j = 0; j < JN; ++j) {
+                    if constexpr (KN)
+                        b[j] = bitcast<frag_t>(held.b[j * NF + t]);
+                    else
+                        b[j] = bitcast<frag_t>(load_raw<16>(lds + A_LDS + (roff ^ (t * 64)) + j * 2048));
+                }
+            }
 #pragma unroll
             for (int e = 0; e < AT::NSUB; ++e)
 #pragma unroll
                 for (int j = 0; j < JN; ++j)
 #pragma unroll
-                    for (int i = 0; i < IM; ++i) AT::mma_sub(acc[i][j], f.a[i][t], f.b[j][t], e);
+                    for (int i = 0; i < IM; ++i) AT::mma_sub(acc[i][j], a[i], b[j], e);
+        }
     }
 
     __device__ __forceinline__ void run(const WorkItem& w, const WaveUnit& u, double alpha_d,
@@ -258,23 +277,21 @@ struct WaveTile {
         // the paths meet, so the stage past the last one is loaded too, out of range (no
         // memory traffic).
         Stage s;
-        Frags f;
         const int n = (k + KS - 1) / KS;
         load(s, 0);
         for (int c = 1; c < n; ++c) {
             write(s);
             wave_lds_order();
-            read(s, f);
-            wave_lds_order();
+            const Held held(s);
             load(s, c);
             __builtin_amdgcn_sched_barrier(0);
-            mma(f, acc);
+            mma(held, acc);
+            wave_lds_order();
             __builtin_amdgcn_sched_barrier(0);
         }
         write(s);
         wave_lds_order();
-        read(s, f);
-        mma(f, acc);
+        mma(Held(s), acc);
         const acc_t alpha = (acc_t)alpha_d, beta = (acc_t)beta_d;
         KAMI_GLOBAL out_t* C = (KAMI_GLOBAL out_t*)w.C + ((int64_t)u.ra * 16 * w.ldc + u.ca * 16);
 #pragma unroll
@@ -291,25 +308,34 @@ struct WaveTile {
     }
 };
 
-// One wave per unit; a workgroup is four consecutive units (neighbouring wave tiles of
+// MM: atoms of a wave tile's height, at most (a queue without taller ones keeps the smaller
+// kernel, four waves a SIMD).  One wave per unit; a workgroup is four consecutive units (neighbouring wave tiles of
 // one problem share its lines of A and B in the CU's L1).
-template <class AT, bool KN>
+template <class AT, bool KN, int MM>
 __global__ void __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(4)))
+__attribute__((amdgpu_waves_per_eu(MM == 2 ? 4 : 3)))
 batched_wave_kernel(BatchArgs args) {
-    constexpr int LDS_WAVE = WaveTile<AT, KN, kWaveAtoms, kWaveAtoms>::LDS;
+    constexpr int LDS_WAVE = WaveTile<AT, KN, MM, kMostN>::LDS;
     __shared__ __attribute__((aligned(16))) unsigned char smem[kWavesPerGroup * LDS_WAVE];
     const int wave = uni(threadIdx.x >> 6);
     unsigned char* const lds = smem + wave * LDS_WAVE;
-    const WaveUnit u = load_uniform(args.units + ((int64_t)blockIdx.x * kWavesPerGroup + wave));
+    const WaveUnit u = load_uniform(args.units + unit_at(blockIdx.x, gridDim.x, wave));
     if (u.im == 0) return;
     const WorkItem w = load_uniform(args.items + u.item);
-    const int shape = u.im * kWaveAtoms + u.jn - kWaveAtoms - 1;
-    switch (shape) {
-        case 0: WaveTile<AT, KN, 1, 1>(w, u, lds).run(w, u, args.alpha, args.beta); break;
-        case 1: WaveTile<AT, KN, 1, 2>(w, u, lds).run(w, u, args.alpha, args.beta); break;
-        case 2: WaveTile<AT, KN, 2, 1>(w, u, lds).run(w, u, args.alpha, args.beta); break;
-        default: WaveTile<AT, KN, 2, 2>(w, u, lds).run(w, u, args.alpha, args.beta); break;
+    auto run = [&](auto im, auto jn) {
+        WaveTile<AT, KN, decltype(im)::value, decltype(jn)::value>(w, u, lds).run(w, u, args.alpha, args.beta);
+    };
+    auto run_rows = [&](auto im) {
+        if (u.jn == 1)
+            run(im, std::integral_constant<int, 1>{});
+        else
+            run(im, std::integral_constant<int, 2>{});
+    };
+    if (u.im == 1) return run_rows(std::integral_constant<int, 1>{});
+    if (u.im == 2) return run_rows(std::integral_constant<int, 2>{});
+    if constexpr (MM > 2) {
+        if (u.im == 3) return run_rows(std::integral_constant<int, 3>{});
+        return run_rows(std::integral_constant<int, 4>{});
     }
 }
 
@@ -335,25 +361,6 @@ static int prior_variant(int prec, int bucket) {
     return 0;
 }
 
-}  // namespace kami
-
-using namespace kami;
-
-struct kami_batched_plan {
-    int prec = 0;
-    int64_t problems = 0;
-    int64_t n_items = 0;
-    int64_t n_units = 0;
-    double flops = 0;
-    int b_kn = 0;
-    double alpha = 1.0, beta = 0.0;
-    WorkItem* d_items = nullptr;
-    WaveUnit* d_units = nullptr;
-    std::vector<int> bucket_ids;      // non-empty buckets, ascending
-    std::vector<int> bucket_variant;  // chosen variant per non-empty bucket
-};
-
-namespace kami {
 
 // Workgroups of one execution: one per kWavesPerGroup units.
 static int64_t batched_groups(int64_t n_units) { return n_units / kWavesPerGroup; }
@@ -361,15 +368,27 @@ static int64_t batched_groups(int64_t n_units) { return n_units / kWavesPerGroup
 // A dispatch holds fewer than 2^32 work-items; longer queues take several.
 constexpr int64_t kMaxGroups = (int64_t)1 << 23;
 
+template <class AT, int MM>
+static void launch_kernel(const BatchArgs& a, bool kn, dim3 grid, hipStream_t s) {
+    if (kn)
+        hipLaunchKernelGGL((batched_wave_kernel<AT, true, MM>), grid, dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((batched_wave_kernel<AT, false, MM>), grid, dim3(256), 0, s, a);
+}
+
 template <class AT>
 static hipError_t launch_for(BatchArgs a, bool kn, hipStream_t s) {
     hipError_t e = hipSuccess;
     for (int64_t left = batched_groups(a.n_units); left > 0 && e == hipSuccess; left -= kMaxGroups) {
         const dim3 grid((unsigned)std::min(left, kMaxGroups));
-        if (kn)
-            hipLaunchKernelGGL((batched_wave_kernel<AT, true>), grid, dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL((batched_wave_kernel<AT, false>), grid, dim3(256), 0, s, a);
+        if constexpr (sizeof(typename AT::in_t) == 2) {
+            if (a.tall)
+                launch_kernel<AT, 4>(a, kn, grid, s);
+            else
+                launch_kernel<AT, 2>(a, kn, grid, s);
+        } else {
+            launch_kernel<AT, 2>(a, kn, grid, s);
+        }
         e = hipGetLastError();
         a.units += kMaxGroups * kWavesPerGroup;
     }
@@ -399,13 +418,15 @@ struct UnitCursor {
     int am = 0, an = 0;      // atoms of the entry
     int sm = 1, sn = 1;      // atoms of a wave tile
     bool done = true;
+    static int strips(int atoms, int most) { return (atoms + most - 1) / most; }
     void start(const WorkItem& w, int cap) {
         am = std::min(w.mlim, kVariantTM[w.variant]) / 16;
         an = std::min(w.nlim, kVariantTN[w.variant]) / 16;
-        sm = std::min(cap >> 1 ? 2 : 1, kVariantSM[w.variant]);
-        sn = std::min(cap & 1 ? 2 : 1, kVariantSN[w.variant]);
-        rows = (am + sm - 1) / sm;
-        cols = (an + sn - 1) / sn;
+        // as few strips as the cap allows, of nearly equal height
+        rows = strips(am, std::min(kCapM[cap], kVariantSM[w.variant]));
+        cols = strips(an, std::min(kCapN[cap], kVariantSN[w.variant]));
+        sm = strips(am, rows);
+        sn = strips(an, cols);
         r = c = 0;
         done = false;
     }
@@ -429,8 +450,7 @@ struct UnitCursor {
     }
 };
 
-// Wave tiles of all entries for wave tiles of up to (cap >> 1 ? 2 : 1) x (cap & 1 ? 2 : 1)
-// atoms, rounded up to whole workgroups.
+// Wave tiles of all entries for the cap, rounded up to a workgroup for every XCD.
 static int64_t count_units(const WorkItem* items, int64_t n_items, int cap) {
     int64_t n = 0;
     UnitCursor u;
@@ -438,25 +458,28 @@ static int64_t count_units(const WorkItem* items, int64_t n_items, int cap) {
         u.start(items[i], cap);
         n += (int64_t)u.rows * u.cols;
     }
-    return (n + kWavesPerGroup - 1) / kWavesPerGroup * kWavesPerGroup;
+    constexpr int64_t kRound = kWavesPerGroup * kXcds;
+    return (n + kRound - 1) / kRound * kRound;
 }
 
 // Fewest wave tiles that fill the chip (four a SIMD); below that the wave tiles are made
-// smaller, 16 x 32 and then 16 x 16, until there are as many.  FP64, problems of 16 to 256:
+// smaller, down to 16 x 16, until there are as many.  FP64, problems of 16 to 256:
 // 8 of them 6.0 us against 9.9 with 32 x 32 tiles, 100 9.1 against 13.5, 300 14.7 against
 // 17.2 (and 17.2 with 2048 here); FP16 is bound by the launch itself there.
 constexpr int64_t kFullUnits = 4096;
 
-static int wave_cap(const WorkItem* items, int64_t n_items, int64_t* n_units) {
-    int cap = 3;
-    while ((*n_units = count_units(items, n_items, cap)) < kFullUnits && cap > 0) cap = cap == 3 ? 1 : 0;
+static int wave_cap(const WorkItem* items, int64_t n_items, int elt, int64_t* n_units) {
+    int cap = first_cap(elt);
+    while ((*n_units = count_units(items, n_items, cap)) < kFullUnits && cap + 1 < kCaps) ++cap;
     return cap;
 }
 
-// The wave units in launch order.  Workgroup L runs on XCD L mod kXcds; every XCD takes
+// The wave units of a launch.  Workgroup L runs on XCD L mod kXcds; every XCD takes
 // deals of consecutive entries (neighbouring tiles of a problem, or problems of nearly
 // equal cost), so the tiles that share rows of A or columns of B run on one XCD at the
-// same time and its L2 serves all but the first reader.
+// same time and its L2 serves all but the first reader.  An XCD's units lie together, in
+// the order of its workgroups (unit_at), so the line one workgroup reads its units from
+// serves the next three as well.
 static void build_units(const WorkItem* items, int64_t n_items, int cap, int64_t n_units, WaveUnit* out) {
     struct {
         int64_t item = 0, end = 0;
@@ -477,12 +500,19 @@ static void build_units(const WorkItem* items, int64_t n_items, int cap, int64_t
         x[q].u.start(items[x[q].item], cap);
         return true;
     };
-    for (int64_t i = 0; i < n_units; ++i) {
-        const int q = (int)(i / kWavesPerGroup % kXcds);
-        int t = 0;
-        while (t < kXcds && !more((q + t) % kXcds)) ++t;  // an empty stream takes from another
-        out[i] = t < kXcds ? x[(q + t) % kXcds].u.take((uint32_t)x[(q + t) % kXcds].item)
-                           : WaveUnit{0, 0, 0, 0, 0};
+    const int64_t groups = batched_groups(n_units);
+    for (int64_t first = 0; first < groups; first += kMaxGroups) {  // dispatch by dispatch
+        const int64_t here = std::min(groups - first, kMaxGroups);
+        WaveUnit* const base = out + first * kWavesPerGroup;
+        for (int64_t L = 0; L < here; ++L) {
+            const int q = (int)(L % kXcds);
+            for (int w = 0; w < kWavesPerGroup; ++w) {
+                int t = 0;
+                while (t < kXcds && !more((q + t) % kXcds)) ++t;  // an empty stream takes from another
+                base[unit_at(L, here, w)] = t < kXcds ? x[(q + t) % kXcds].u.take((uint32_t)x[(q + t) % kXcds].item)
+                                                      : WaveUnit{0, 0, 0, 0, 0};
+            }
+        }
     }
 }
 
@@ -595,18 +625,29 @@ static kami_status upload(const void* host, size_t bytes, void** dev) {
     return KAMI_OK;
 }
 
-// The entries and their wave units on the device.
-static kami_status upload_queue(const std::vector<WorkItem>& items, WorkItem** d_items,
-                                WaveUnit** d_units, int64_t* n_units) {
+// A queue on the device: the entries, and behind them their wave units.
+struct DeviceQueue {
+    void* mem = nullptr;
+    int64_t n_items = 0, n_units = 0;
+    int tall = 0;
+    const WorkItem* items() const { return static_cast<const WorkItem*>(mem); }
+    const WaveUnit* units() const { return reinterpret_cast<const WaveUnit*>(items() + n_items); }
+};
+
+static kami_status upload_queue(const std::vector<WorkItem>& items, int elt, DeviceQueue* q) {
     const int64_t n = (int64_t)items.size();
     if (n > UINT32_MAX) return KAMI_ENOMEM;  // 256 GiB of entries
-    const int cap = wave_cap(items.data(), n, n_units);
-    std::unique_ptr<WaveUnit[]> units(new (std::nothrow) WaveUnit[(size_t)*n_units]);
-    if (!units) return KAMI_ENOMEM;
-    build_units(items.data(), n, cap, *n_units, units.get());
-    kami_status st = upload(items.data(), items.size() * sizeof(WorkItem), (void**)d_items);
-    if (st == KAMI_OK) st = upload(units.get(), (size_t)*n_units * sizeof(WaveUnit), (void**)d_units);
-    return st;
+    int64_t n_units = 0;
+    const int cap = wave_cap(items.data(), n, elt, &n_units);
+    const size_t item_bytes = (size_t)n * sizeof(WorkItem), bytes = item_bytes + (size_t)n_units * sizeof(WaveUnit);
+    std::unique_ptr<unsigned char[]> host(new (std::nothrow) unsigned char[bytes]);
+    if (!host) return KAMI_ENOMEM;
+    std::memcpy(host.get(), items.data(), item_bytes);
+    build_units(items.data(), n, cap, n_units, reinterpret_cast<WaveUnit*>(host.get() + item_bytes));
+    q->n_items = n;
+    q->n_units = n_units;
+    q->tall = cap == 0;
+    return upload(host.get(), bytes, &q->mem);
 }
 
 // ---- one-shot execution without allocation ----
@@ -622,7 +663,7 @@ static kami_status upload_queue(const std::vector<WorkItem>& items, WorkItem** d
 constexpr int64_t kStaticItems = 32768;  // 2 MiB of queue entries
 constexpr int64_t kStaticUnits = 16 * kStaticItems;
 constexpr size_t kStaticBytes = kStaticItems * sizeof(WorkItem) + kStaticUnits * sizeof(WaveUnit);
-static_assert(4 * kFullUnits + kWavesPerGroup <= kStaticUnits, "small wave tiles fit");
+static_assert(4 * kFullUnits + kWavesPerGroup * kXcds <= kStaticUnits, "small wave tiles fit");
 static __device__ __align__(256) unsigned char scratch[kStaticBytes];
 
 struct StaticStaging {
@@ -651,14 +692,31 @@ static kami_status static_scratch(unsigned char** out) {
     return KAMI_OK;
 }
 
+}  // namespace kami
+
+struct kami_batched_plan {
+    int prec = 0;
+    int64_t problems = 0;
+    int64_t n_items = 0;
+    double flops = 0;
+    int b_kn = 0;
+    double alpha = 1.0, beta = 0.0;
+    kami::DeviceQueue queue;
+    std::vector<int> bucket_ids;      // non-empty buckets, ascending
+    std::vector<int> bucket_variant;  // chosen variant per non-empty bucket
+};
+
+namespace kami {
+
 static void free_plan(kami_batched_plan* p) {
     if (!p) return;
-    if (p->d_items) (void)hipFree(p->d_items);
-    if (p->d_units) (void)hipFree(p->d_units);
+    if (p->queue.mem) (void)hipFree(p->queue.mem);
     delete p;
 }
 
 }  // namespace kami
+
+using namespace kami;
 
 extern "C" {
 
@@ -739,16 +797,13 @@ kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count, i
                 int vb[1] = {v};
                 std::vector<WorkItem> items;
                 build_items(sample, sb, vb, ei, eo, plan->b_kn, items);
-                WorkItem* d_it = nullptr;
-                WaveUnit* d_un = nullptr;
-                int64_t n_units = 0;
-                st = upload_queue(items, &d_it, &d_un, &n_units);
+                DeviceQueue q;
+                st = upload_queue(items, ei, &q);
                 if (st != KAMI_OK) {
-                    if (d_it) (void)hipFree(d_it);
-                    if (d_un) (void)hipFree(d_un);
+                    if (q.mem) (void)hipFree(q.mem);
                     break;
                 }
-                BatchArgs a{d_it, d_un, n_units, o.alpha, 0.0};
+                BatchArgs a{q.items(), q.units(), q.n_units, o.alpha, 0.0, q.tall};
                 e = launch_batched(precision, a, plan->b_kn, s);  // warm-up
                 if (e == hipSuccess) e = hipEventRecord(e0, s);
                 for (int rep = 0; rep < 3 && e == hipSuccess; ++rep)
@@ -757,8 +812,7 @@ kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count, i
                 if (e == hipSuccess) e = hipEventSynchronize(e1);
                 float ms = 0;
                 if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
-                (void)hipFree(d_it);
-                (void)hipFree(d_un);
+                (void)hipFree(q.mem);
                 if (e != hipSuccess) {
                     st = hip_fail(e);
                     break;
@@ -781,7 +835,7 @@ kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count, i
     std::vector<WorkItem> items;
     build_items(hp, bucket, variant_of_bucket, ei, eo, plan->b_kn, items);
     plan->n_items = (int64_t)items.size();
-    st = upload_queue(items, &plan->d_items, &plan->d_units, &plan->n_units);
+    st = upload_queue(items, ei, &plan->queue);
     if (st != KAMI_OK) {
         free_plan(plan);
         return st;
@@ -799,7 +853,8 @@ kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count, i
 kami_status kami_batched_execute(kami_batched_plan* plan, void* stream) {
     if (!plan) return KAMI_EINVAL;
     hipStream_t s = (hipStream_t)stream;
-    const BatchArgs a{plan->d_items, plan->d_units, plan->n_units, plan->alpha, plan->beta};
+    const BatchArgs a{plan->queue.items(), plan->queue.units(), plan->queue.n_units, plan->alpha, plan->beta,
+                      plan->queue.tall};
     const hipError_t e = launch_batched(plan->prec, a, plan->b_kn, s);
     if (e != hipSuccess) return hip_fail(e);
     return KAMI_OK;
@@ -811,7 +866,7 @@ kami_status kami_batched_plan_info(const kami_batched_plan* plan, kami_plan_info
     out->problems = plan->problems;
     out->work_items = plan->n_items;
     out->buckets = (int32_t)plan->bucket_ids.size();
-    out->workgroups = (int32_t)std::min<int64_t>(batched_groups(plan->n_units), INT32_MAX);
+    out->workgroups = (int32_t)std::min<int64_t>(batched_groups(plan->queue.n_units), INT32_MAX);
     out->flops = plan->flops;
     for (size_t i = 0; i < plan->bucket_variant.size() && i < 16; ++i)
         out->variant_of_bucket[i] = plan->bucket_variant[i];
@@ -861,7 +916,7 @@ kami_status kami_batched_gemm_static(const kami_problem* probs, int64_t count, i
     build_items(g_static.probs, count, g_static.bucket, variant_of_bucket, ei, eo, b_kn,
                 g_static.order, items);
     int64_t n_units = 0;
-    const int cap = wave_cap(items, n_items, &n_units);
+    const int cap = wave_cap(items, n_items, ei, &n_units);
     build_units(items, n_items, cap, n_units, units);
     hipStream_t s = (hipStream_t)stream;
     // From pageable memory the copy has consumed the staging array when the call returns,
@@ -871,7 +926,7 @@ kami_status kami_batched_gemm_static(const kami_problem* probs, int64_t count, i
                                   hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return hip_fail(e);
     const WorkItem* d_items = reinterpret_cast<const WorkItem*>(base);
-    BatchArgs a{d_items, reinterpret_cast<const WaveUnit*>(d_items + n_items), n_units, o.alpha, o.beta};
+    BatchArgs a{d_items, reinterpret_cast<const WaveUnit*>(d_items + n_items), n_units, o.alpha, o.beta, cap == 0};
     e = launch_batched(precision, a, b_kn, s);
     if (e != hipSuccess) return hip_fail(e);
     return KAMI_OK;
