@@ -144,7 +144,8 @@ def _fast():
         L = lib()
         _fast_calls.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (
             L.kami_block_gemm, L.kami_split_gemm, L.kami_batched_execute, L.kami_bsr_spgemm_symbolic,
-            L.kami_bsr_spgemm_fill, L.kami_bsr_spgemm_numeric, L.kami_bsr_spmm)))
+            L.kami_bsr_spgemm_fill, L.kami_bsr_spgemm_numeric, L.kami_bsr_spmm,
+            L.kami_bsr_spgemm_structure)))
         _FAST = _fast_calls
     return _FAST
 

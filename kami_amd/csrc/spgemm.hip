@@ -15,6 +15,7 @@
 //   fill   -- the stored bitmap (without a workspace: a rebuilt one) has its set bits
 //             written in ascending order, each thread placing the bits of one 32-bit word
 //             after the prefix popcount of the words before it;
+//   (the last two are one kernel where the caller has room for every column C could have);
 //   numeric -- one wave per output block (i, j): the row i comes from a 256-way search of
 //             rowptrC; the lanes binary-search B's sorted rows k of all blocks (i, k) of A
 //             at once for column j; both blocks are loaded by whole lines and turned into
@@ -25,6 +26,7 @@
 #include <chrono>
 
 #include "kami_internal.hpp"
+#include "spgemm_internal.hpp"
 
 namespace kami {
 
@@ -170,6 +172,36 @@ __global__ void __launch_bounds__(1024) spgemm_scan_kernel(int32_t* x, int n, in
     }
 }
 
+// Writes the columns whose bits are set in the LDS bitmap, ascending, from ciC[out] on: each
+// thread places the bits of one word after the popcount of the words before it.
+__device__ inline void expand_row(const unsigned* bitmap, int nwords, int out, int32_t* ciC, int* s_wave) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int base = 0; base < nwords; base += 256) {
+        const int w = base + tid;
+        const unsigned bits = w < nwords ? bitmap[w] : 0u;
+        const int v = __popc(bits);
+        int incl = v;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int y = __shfl_up(incl, off);
+            if (lane >= off) incl += y;
+        }
+        if (lane == 63) s_wave[wave] = incl;
+        __syncthreads();
+        int before = incl - v;
+        for (int q = 0; q < wave; ++q) before += s_wave[q];
+        int pos = out + before;
+        unsigned b = bits;
+        while (b) {
+            const int bit = __ffs(b) - 1;
+            ciC[pos++] = (w << 5) + bit;
+            b &= b - 1;
+        }
+        out += s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+        __syncthreads();
+    }
+}
+
 __global__ void __launch_bounds__(256)
 spgemm_fill_kernel(int mb, int nwords, const int32_t* rpA, const int32_t* ciA,
                    const int32_t* rpB, const int32_t* ciB, const int32_t* rpC, int32_t* ciC,
@@ -177,7 +209,7 @@ spgemm_fill_kernel(int mb, int nwords, const int32_t* rpA, const int32_t* ciA,
     extern __shared__ unsigned bitmap[];
     __shared__ MarkLds s;
     __shared__ int s_wave[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x;
     for (int row = blockIdx.x; row < mb; row += gridDim.x) {
         if (bitmaps) {  // the count kernel's bitmap of the row
             for (int w = tid; w < nwords; w += blockDim.x) bitmap[w] = bitmaps[(int64_t)row * nwords + w];
@@ -187,32 +219,56 @@ spgemm_fill_kernel(int mb, int nwords, const int32_t* rpA, const int32_t* ciA,
             mark_row(row, rpA, ciA, rpB, ciB, bitmap, s);
         }
         __syncthreads();
-        int out = rpC[row];
-        for (int base = 0; base < nwords; base += 256) {
-            const int w = base + tid;
-            const unsigned bits = w < nwords ? bitmap[w] : 0u;
-            const int v = __popc(bits);
-            int incl = v;
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const int y = __shfl_up(incl, off);
-                if (lane >= off) incl += y;
-            }
-            if (lane == 63) s_wave[wave] = incl;
-            __syncthreads();
-            int before = incl - v;
-            for (int q = 0; q < wave; ++q) before += s_wave[q];
-            int pos = out + before;
-            unsigned b = bits;
-            while (b) {
-                const int bit = __ffs(b) - 1;
-                ciC[pos++] = (w << 5) + bit;
-                b &= b - 1;
-            }
-            const int tot = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
-            __syncthreads();
-            out += tot;
+        expand_row(bitmap, nwords, rpC[row], ciC, s_wave);
+        __syncthreads();
+    }
+}
+
+// Scan and fill in one: the workgroup of a row sums the counts before it (and all of them),
+// stores its row pointer and expands its bitmap, unless C has more than `capacity` blocks.
+// The workgroup of row 0 stores the total, saturated at INT32_MAX, and passes it to the host
+// as spgemm_scan_kernel does.  Launches and the dependent loads bound it, so one kernel less
+// counts: 3.9 us for 256 rows against 2.6 (scan) + 3.5 (fill); the whole bsr_spgemm of 16-blocks
+// 21.7 -> 19.3 us at 256 x 256 blocks and 50.9 -> 48.5 us with 4096 rows, the most it takes.
+__global__ void __launch_bounds__(256)
+spgemm_scan_fill_kernel(int mb, int nwords, const int32_t* counts, const unsigned* bitmaps,
+                        int32_t* rpC, int32_t* ciC, int64_t capacity, int32_t* done, int32_t seq) {
+    extern __shared__ unsigned bitmap[];
+    __shared__ long long s_before[4], s_total[4];
+    __shared__ int s_wave[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int row = blockIdx.x; row < mb; row += gridDim.x) {
+        for (int w = tid; w < nwords; w += 256) bitmap[w] = bitmaps[(int64_t)row * nwords + w];
+        long long before = 0, total = 0;
+        for (int i = tid; i < mb; i += 256) {
+            const int v = counts[i];
+            total += v;
+            if (i < row) before += v;
         }
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) {
+            before += __shfl_xor(before, off);
+            total += __shfl_xor(total, off);
+        }
+        if (lane == 0) {
+            s_before[wave] = before;
+            s_total[wave] = total;
+        }
+        __syncthreads();
+        before = s_before[0] + s_before[1] + s_before[2] + s_before[3];
+        total = s_total[0] + s_total[1] + s_total[2] + s_total[3];
+        if (tid == 0) {
+            rpC[row] = (int32_t)min(before, (long long)INT32_MAX);
+            if (row == 0) {
+                const int32_t sat = (int32_t)min(total, (long long)INT32_MAX);
+                rpC[mb] = sat;
+                if (done) {
+                    __hip_atomic_store(&done[0], sat, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    __hip_atomic_store(&done[1], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+                }
+            }
+        }
+        if (total <= capacity) expand_row(bitmap, nwords, (int)before, ciC, s_wave);  // uniform
         __syncthreads();
     }
 }
@@ -470,6 +526,38 @@ static hipError_t wait_for_word(const int32_t* word, int32_t seq, hipStream_t s)
     return hipSuccess;
 }
 
+// Number of this host thread's next wait on its pinned words: one count for every kernel that
+// writes them, as the host takes the total once the number it waits for is there.
+static int32_t next_seq() {
+    thread_local int32_t seq = 0;
+    return seq = seq == INT32_MAX ? 1 : seq + 1;
+}
+
+// Launches the kernel that forms C's total (`launch(words, seq)`: it stores the total and
+// then seq in the pinned pair) and waits for it on the host; `dev_total` is where it also
+// leaves the total on the device, for a host without pinned memory.
+template <class F>
+static kami_status total_of(const int32_t* dev_total, int64_t* nnzbC, hipStream_t s, F launch) {
+    int32_t* words = pinned_total();
+    const int32_t seq = next_seq();
+    launch(words ? pinned_device(words) : nullptr, seq);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return hip_fail(e);
+    int32_t total = 0;
+    if (words) {
+        e = wait_for_word(words + 1, seq, s);
+        if (e != hipSuccess) return hip_fail(e);
+        total = __atomic_load_n(words, __ATOMIC_ACQUIRE);
+    } else {  // no pinned words: copy the total back
+        e = hipMemcpyAsync(&total, dev_total, sizeof(int32_t), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return hip_fail(e);
+    }
+    if (total == INT32_MAX) return KAMI_ENOTSUP;  // more blocks than int32 row pointers hold
+    *nnzbC = total;
+    return KAMI_OK;
+}
+
 static int sym_grid(int mb) {
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess)
@@ -499,28 +587,36 @@ kami_status kami_bsr_spgemm_symbolic(const kami_bsr* A, const kami_bsr* B, int32
     hipStream_t s = (hipStream_t)stream;
     const int nwords = (B->nb + 31) / 32;
     unsigned* bitmaps = ws && ws_bytes >= bitmap_bytes(A->mb, B->nb) ? static_cast<unsigned*>(ws) : nullptr;
-    int32_t* words = pinned_total();
-    thread_local int32_t seq = 0;
-    seq = seq == INT32_MAX ? 1 : seq + 1;
     hipLaunchKernelGGL(spgemm_count_kernel, dim3(sym_grid(A->mb)), dim3(256), nwords * 4, s, A->mb,
                        nwords, A->rowptr, A->colidx, B->rowptr, B->colidx, rowptrC, bitmaps);
-    hipLaunchKernelGGL(spgemm_scan_kernel, dim3(1), dim3(1024), 0, s, rowptrC, A->mb + 1,
-                       words ? pinned_device(words) : nullptr, seq);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return hip_fail(e);
-    int32_t total = 0;
-    if (words) {
-        e = wait_for_word(words + 1, seq, s);
-        if (e != hipSuccess) return hip_fail(e);
-        total = __atomic_load_n(words, __ATOMIC_ACQUIRE);
-    } else {  // no pinned words: copy the total back
-        e = hipMemcpyAsync(&total, rowptrC + A->mb, sizeof(int32_t), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) return hip_fail(e);
-    }
-    if (total == INT32_MAX) return KAMI_ENOTSUP;  // more blocks than int32 row pointers hold
-    *nnzbC = total;
-    return KAMI_OK;
+    return total_of(rowptrC + A->mb, nnzbC, s, [&](int32_t* words, int32_t seq) {
+        hipLaunchKernelGGL(spgemm_scan_kernel, dim3(1), dim3(1024), 0, s, rowptrC, A->mb + 1, words, seq);
+    });
+}
+
+// Row pointer, columns and nnzb(C) with one wait and no scan launch (spgemm_internal.hpp).
+kami_status kami_bsr_spgemm_structure(const kami_bsr* A, const kami_bsr* B, int32_t* rowptrC,
+                                      int32_t* colidxC, int64_t capacity, int64_t* nnzbC, void* ws,
+                                      size_t ws_bytes, void* stream) {
+    kami_status st = check_pair(A, B);
+    if (st != KAMI_OK) return st;
+    if (!rowptrC || !nnzbC || !ws || capacity < 0 || (capacity > 0 && !colidxC)) return KAMI_EINVAL;
+    const size_t bitmap = bitmap_bytes(A->mb, B->nb);
+    if (ws_bytes < bitmap + (size_t)A->mb * sizeof(int32_t)) return KAMI_ENOSPC;
+    if (A->mb > kStructureRows) return KAMI_ENOTSUP;
+    st = device_check();
+    if (st != KAMI_OK) return st;
+    hipStream_t s = (hipStream_t)stream;
+    const int nwords = (B->nb + 31) / 32;
+    unsigned* const bitmaps = static_cast<unsigned*>(ws);
+    int32_t* const counts = reinterpret_cast<int32_t*>(static_cast<unsigned char*>(ws) + bitmap);
+    const dim3 grid(sym_grid(A->mb));
+    hipLaunchKernelGGL(spgemm_count_kernel, grid, dim3(256), nwords * 4, s, A->mb, nwords, A->rowptr,
+                       A->colidx, B->rowptr, B->colidx, counts, bitmaps);
+    return total_of(rowptrC + A->mb, nnzbC, s, [&](int32_t* words, int32_t seq) {
+        hipLaunchKernelGGL(spgemm_scan_fill_kernel, grid, dim3(256), nwords * 4, s, A->mb, nwords, counts,
+                           bitmaps, rowptrC, colidxC, capacity, words, seq);
+    });
 }
 
 kami_status kami_bsr_spgemm_fill(const kami_bsr* A, const kami_bsr* B, const int32_t* rowptrC,

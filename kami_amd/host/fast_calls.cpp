@@ -12,6 +12,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include "../../include/kami.h"
+#include "../csrc/spgemm_internal.hpp"
 
 namespace {
 
@@ -24,6 +25,7 @@ struct Lib {
     decltype(&kami_bsr_spgemm_fill) fill;
     decltype(&kami_bsr_spgemm_numeric) numeric;
     decltype(&kami_bsr_spmm) spmm;
+    decltype(&kami_bsr_spgemm_structure) structure;
 } g_lib;
 bool g_bound = false;
 
@@ -217,6 +219,11 @@ PyObject* bsr_spgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
             return nullptr;
         if (A.nb != B.mb || A.bs != B.bs || !is(*ta[2], in, *ta[0]) || !is(*tb[2], in, *ta[0])) return nullptr;
         size_t ws_bytes = (size_t)A.mb * (((size_t)B.nb + 31) / 32) * 4;
+        // Up to 1 MiB for every block C could have: the columns are written before the count is
+        // known here, and the scan is not a launch of its own.
+        const int64_t most = (int64_t)A.mb * B.nb;
+        const bool fused = A.mb <= kStructureRows && most <= (1 << 18);
+        if (fused) ws_bytes += (size_t)A.mb * 4;
         const auto ints = ta[0]->options();
         at::Tensor ws = at::empty({(int64_t)ws_bytes / 4}, ints);
         at::Tensor rowptr = at::empty({(int64_t)A.mb + 1}, ints);
@@ -224,13 +231,22 @@ PyObject* bsr_spgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         void* const stream = current_stream();
         int64_t nnz = 0;
         kami_status st;
+        at::Tensor colidx;
+        if (fused) colidx = at::empty({most}, ints);
         Py_BEGIN_ALLOW_THREADS  // waits for the device
-        st = g_lib.symbolic(&A, &B, rp, &nnz, ws.data_ptr(), ws_bytes, stream);
+        st = fused ? g_lib.structure(&A, &B, rp, static_cast<int32_t*>(colidx.data_ptr()), most, &nnz,
+                                     ws.data_ptr(), ws_bytes, stream)
+                   : g_lib.symbolic(&A, &B, rp, &nnz, ws.data_ptr(), ws_bytes, stream);
         Py_END_ALLOW_THREADS
         if (st != KAMI_OK) return nullptr;
-        at::Tensor colidx = at::empty({nnz > 0 ? nnz : 1}, ints);
+        if (fused) {  // the storage's size too, so that a saved C holds its own blocks only
+            colidx.unsafeGetTensorImpl()->set_sizes_contiguous({nnz > 0 ? nnz : 1});
+            colidx.storage().unsafeGetStorageImpl()->set_nbytes((size_t)(nnz > 0 ? nnz : 1) * 4);
+        } else {
+            colidx = at::empty({nnz > 0 ? nnz : 1}, ints);
+        }
         int32_t* const ci = static_cast<int32_t*>(colidx.data_ptr());
-        if (g_lib.fill(&A, &B, rp, ci, ws.data_ptr(), ws_bytes, stream) != KAMI_OK) return nullptr;
+        if (!fused && g_lib.fill(&A, &B, rp, ci, ws.data_ptr(), ws_bytes, stream) != KAMI_OK) return nullptr;
         at::Tensor vals = at::empty({nnz > 0 ? nnz : 1, A.bs, A.bs}, ta[2]->options().dtype(out));
         if (nnz > 0 && g_lib.numeric(&A, &B, rp, ci, nnz, vals.data_ptr(), prec, alpha, stream) != KAMI_OK)
             return nullptr;
@@ -247,14 +263,14 @@ PyObject* bsr_spgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
-// bind(addresses of the seven entry points, in Lib's order)
+// bind(addresses of the eight entry points, in Lib's order)
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    void* p[7];
-    if (n != 7) {
-        PyErr_SetString(PyExc_TypeError, "bind expects seven addresses");
+    void* p[8];
+    if (n != 8) {
+        PyErr_SetString(PyExc_TypeError, "bind expects eight addresses");
         return nullptr;
     }
-    for (int i = 0; i < 7; ++i) {
+    for (int i = 0; i < 8; ++i) {
         p[i] = PyLong_AsVoidPtr(a[i]);
         if (!p[i]) {
             if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "null entry point");
@@ -263,7 +279,8 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     g_lib = Lib{(decltype(Lib::block_gemm))p[0], (decltype(Lib::split_gemm))p[1],
                 (decltype(Lib::batched_execute))p[2], (decltype(Lib::symbolic))p[3],
-                (decltype(Lib::fill))p[4], (decltype(Lib::numeric))p[5], (decltype(Lib::spmm))p[6]};
+                (decltype(Lib::fill))p[4], (decltype(Lib::numeric))p[5], (decltype(Lib::spmm))p[6],
+                (decltype(Lib::structure))p[7]};
     g_bound = true;
     Py_RETURN_NONE;
 }
