@@ -29,8 +29,14 @@ namespace kami {
 constexpr int cmin(int a, int b) { return a < b ? a : b; }
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
-template <class AT, int BM_, int BN_, int BK_, int PM_, int PN_, int PK_, int KS_>
+// KN_: B is stored K x N.  Its K rows go to LDS as they are and the reads turn them.  (Turning
+// them in the writes instead cost eight 2-byte or two 8-byte conflicting stores a piece:
+// FP16 256^3 x 1024 183 us against 114.5, 224^3 x 2048 246 against 177, FP64 128^3 x 4096 431
+// against 376, 64 x 64 x 512 x 2048 273 against 226; N x K 111, 187, 335 and 209.)
+template <class AT, int BM_, int BN_, int BK_, int PM_, int PN_, int PK_, int KS_, bool KN_ = false>
 struct BlockGeom {
+    static constexpr bool KN = KN_;
+    using AsKN = BlockGeom<AT, BM_, BN_, BK_, PM_, PN_, PK_, KS_, true>;
     static constexpr int BM = BM_, BN = BN_, BK = BK_;
     static constexpr int PM = PM_, PN = PN_, PK = PK_, KS = KS_;
     static constexpr int WAVES = PM * PN * PK;
@@ -48,7 +54,15 @@ struct BlockGeom {
     static constexpr int NBUF = (NS == 1) ? 1 : 2;
     static constexpr int ROWB = lds_row_bytes(KS * ELT, AT::FRAG_BYTES);  // conflict-free reads
     static constexpr int A_LDS = A_PRIV ? 0 : BM * ROWB;
-    static constexpr int B_LDS = BN * ROWB;
+    // K x N: bytes between staged K rows, and the extra bytes after every eight of 2-byte
+    // values.  FP64 reads 8 bytes a lane, 16 columns of rows 2 g + e by lane group g: a row of
+    // 64 mod 128 bytes puts two groups on different banks.  2-byte values are read by
+    // transposing reads, four rows of 32 bytes by lane group g: rows 32 mod 64 bytes apart, and
+    // the groups' rows half the banks apart.
+    static constexpr int KROW = BN * ELT + (ELT == 8 ? 64 : BN * ELT % 64 == 0 ? 32 : 0);
+    static constexpr int KGAP = ELT == 8 ? 0 : 128;
+    static constexpr int B_LDS = KN ? KS * KROW + KS / 8 * KGAP : BN * ROWB;
+    __device__ static constexpr int krow(int k) { return k * KROW + (k >> 3) * KGAP; }
     static constexpr int STAGE_LDS = A_LDS + B_LDS;
     static constexpr int STAGING = NBUF * STAGE_LDS;
     static constexpr int ACC_ELT = (int)sizeof(typename AT::acc_t);
@@ -78,8 +92,53 @@ struct BlockArgs {
     int64_t lda, ldb, ldc;    // leading dimensions (elements)
     double alpha, beta;
     int32_t iters;
-    int32_t b_kn;             // 1: B stored K x N
+    int32_t b_kn;             // 1: B stored K x N (the launcher picks the kernel)
 };
+
+// B fragment of column atom jn at K step ks of the K slice of wave (pn, pk), from the stage at
+// bb.  K x N: a lane's values are AT::KV rows of one column.  K step 8: the upper lane groups'
+// values are not used, and they read the lower groups' rows so as to stay in the stage.
+template <class AT, class G>
+__device__ __forceinline__ typename AT::frag_t stage_b_fragment(const unsigned char* bb, int lane, int pn,
+                                                                int pk, int jn, int ks) {
+    using frag_t = typename AT::frag_t;
+    const int col = pn * G::TN + lane % G::DIM, grp = lane / G::DIM;
+    if constexpr (!G::KN) {
+        const int kk = (pk * G::KSW + AT::KV * grp + ks * AT::KSTEP) * G::ELT;
+        return bitcast<frag_t>(load_raw<AT::FRAG_BYTES>(bb + (col + jn * G::DIM) * G::ROWB + kk));
+    } else {
+        constexpr int GROUPS = cmin(64 / G::DIM, AT::KSTEP / AT::KV);
+        const unsigned char* q = bb + G::krow(pk * G::KSW + AT::KV * (grp % GROUPS));
+        const int step = G::krow(ks * AT::KSTEP) + jn * G::DIM * G::ELT;
+        if constexpr (G::ELT == 8) {
+            q += col * 8 + step;
+            return frag_t{*reinterpret_cast<const double*>(q), *reinterpret_cast<const double*>(q + G::KROW)};
+        } else {
+            const int l = lane & 15;
+            q += (l >> 2) * G::KROW + (col - l) * 2 + 8 * (l & 3) + step;
+            const u2_t lo = lds_read_turned(q);
+            if constexpr (AT::KV == 4) {
+                return bitcast<frag_t>(lo);
+            } else {
+                const u2_t hi = lds_read_turned(q + 4 * G::KROW);
+                return bitcast<frag_t>(u4_t{lo[0], lo[1], hi[0], hi[1]});
+            }
+        }
+    }
+}
+
+// Waves a SIMD is to hold, at most.  1D instances of 2-byte values write more than they read,
+// and with fewer problems in flight and the registers spent on longer runs of loads the writes
+// go faster: 64 x 64 x 32 x 8192 43.5 us uncapped, 39.6 with 3 waves; 128 x 128 x 32 x 8192
+// 131 (K x N 145), 124.5; 64 x 64 x 16 39.2, 37.1; 64^3 49.0, 47.6; 192 x 192 x 32 x 2048
+// 141 (K x N 145) and 141 with 2.  Smaller problems want all the waves they can have (16^3
+// 4.2 us, 4.5 with 3), and so do the 2D instances (BF16 64^3 51 us, 58).
+template <class AT, class G>
+constexpr int waves_per_simd() {
+    if (G::ELT == 8 || G::PN > 1 || G::PK > 1 || G::BM < 64) return 8;
+    const int want = G::IM * G::JN * G::NACC >= 128 ? 2 : 3, own = (G::WAVES + 3) / 4;
+    return (want + own - 1) / own * own;  // whole workgroups
+}
 
 // KFENCE > 0: a scheduling fence after every KFENCE K steps of a stage, so the
 // compiler does not hoist the B fragment loads of a whole long stage ahead of the MFMAs
@@ -90,6 +149,7 @@ struct BlockArgs {
 // C columns of pass sp start at sp * G::BN); A is read again in every pass.
 template <class AT, class G, int KFENCE = 0, int SP = 1>
 __global__ void __launch_bounds__(G::NT)
+__attribute__((amdgpu_waves_per_eu((G::WAVES + 3) / 4, waves_per_simd<AT, G>())))
 block_gemm_kernel(BlockArgs args) {
     using in_t = typename AT::in_t;
     using acc_t = typename AT::acc_t;
@@ -110,13 +170,12 @@ block_gemm_kernel(BlockArgs args) {
 
     const int64_t prob = blockIdx.x;
     const int64_t lda = args.lda, ldb = args.ldb, ldc = args.ldc;
-    const bool b_kn = args.b_kn != 0;
     const in_t* __restrict__ A = reinterpret_cast<const in_t*>(args.A) + prob * args.sa;
 #pragma unroll 1
     for (int sp = 0; sp < SP; ++sp) {
     if (sp > 0) __syncthreads();  // the previous pass is done with LDS
     const in_t* __restrict__ B = reinterpret_cast<const in_t*>(args.B) + prob * args.sb +
-                                 (int64_t)sp * G::BN * (b_kn ? 1 : ldb);
+                                 (int64_t)sp * G::BN * (G::KN ? 1 : ldb);
     out_t* __restrict__ C = reinterpret_cast<out_t*>(args.C) + prob * args.sc + sp * G::BN;
 
     accv_t acc[G::IM][G::JN];
@@ -143,7 +202,7 @@ block_gemm_kernel(BlockArgs args) {
                 }
             }
         }
-        if (!b_kn) {
+        if constexpr (!G::KN) {
             constexpr int CPR = G::KS / G::VE;
 #pragma unroll
             for (int i = 0; i < G::NBC; ++i) {
@@ -179,29 +238,13 @@ block_gemm_kernel(BlockArgs args) {
             }
         }
         unsigned char* bb = base + G::A_LDS;
-        if (!b_kn) {
-            constexpr int CPR = G::KS / G::VE;
+        constexpr int CPR = (G::KN ? G::BN : G::KS) / G::VE;
 #pragma unroll
-            for (int i = 0; i < G::NBC; ++i) {
-                const int c = tid + i * G::NT;
-                if (c < G::CB) {
-                    const int r = c / CPR, cc = c % CPR;
-                    store_raw<16>(bb + r * G::ROWB + cc * 16, stB[i]);
-                }
-            }
-        } else {
-            // transpose K x N chunks into the N-major LDS layout
-            constexpr int CPR = G::BN / G::VE;
-#pragma unroll
-            for (int i = 0; i < G::NBC; ++i) {
-                const int c = tid + i * G::NT;
-                if (c < G::CB) {
-                    const int kr = c / CPR, jc = c % CPR;
-                    const in_t* e = reinterpret_cast<const in_t*>(&stB[i]);
-#pragma unroll
-                    for (int q = 0; q < G::VE; ++q)
-                        *reinterpret_cast<in_t*>(bb + (jc * G::VE + q) * G::ROWB + kr * G::ELT) = e[q];
-                }
+        for (int i = 0; i < G::NBC; ++i) {
+            const int c = tid + i * G::NT;
+            if (c < G::CB) {
+                const int r = c / CPR, cc = c % CPR;
+                store_raw<16>(bb + (G::KN ? G::krow(r) : r * G::ROWB) + cc * 16, stB[i]);
             }
         }
     };
@@ -246,8 +289,7 @@ block_gemm_kernel(BlockArgs args) {
             if constexpr (AT::NSUB == 1) {
 #pragma unroll
                 for (int jn = 0; jn < G::JN; ++jn) {
-                    const frag_t bf = bitcast<frag_t>(
-                        load_raw<FB>(bb + (pn * G::TN + jn * G::DIM + (lane % G::DIM)) * G::ROWB + kk));
+                    const frag_t bf = stage_b_fragment<AT, G>(bb, lane, pn, pk, jn, ks);
 #pragma unroll
                     for (int im = 0; im < G::IM; ++im) AT::mma(acc[im][jn], af[im], bf);
                 }
@@ -257,8 +299,7 @@ block_gemm_kernel(BlockArgs args) {
                 frag_t bf[G::JN];
 #pragma unroll
                 for (int jn = 0; jn < G::JN; ++jn)
-                    bf[jn] = bitcast<frag_t>(
-                        load_raw<FB>(bb + (pn * G::TN + jn * G::DIM + (lane % G::DIM)) * G::ROWB + kk));
+                    bf[jn] = stage_b_fragment<AT, G>(bb, lane, pn, pk, jn, ks);
 #pragma unroll
                 for (int e = 0; e < AT::NSUB; ++e)
 #pragma unroll
@@ -375,8 +416,12 @@ block_gemm_kernel(BlockArgs args) {
 
 template <class AT, class G, int KFENCE = 0, int SP = 1>
 hipError_t launch_block_gemm(const BlockArgs& args, int64_t count, hipStream_t stream) {
-    hipLaunchKernelGGL((block_gemm_kernel<AT, G, KFENCE, SP>), dim3((unsigned)count), dim3(G::NT),
-                       0, stream, args);
+    if (args.b_kn)
+        hipLaunchKernelGGL((block_gemm_kernel<AT, typename G::AsKN, KFENCE, SP>), dim3((unsigned)count),
+                           dim3(G::NT), 0, stream, args);
+    else
+        hipLaunchKernelGGL((block_gemm_kernel<AT, G, KFENCE, SP>), dim3((unsigned)count), dim3(G::NT), 0,
+                           stream, args);
     return hipGetLastError();
 }
 

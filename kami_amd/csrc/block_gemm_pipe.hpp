@@ -29,6 +29,7 @@ block_gemm_pipe_kernel(BlockArgs args, int64_t count) {
     using accv_t = typename AT::accv_t;
     constexpr int FB = AT::FRAG_BYTES;
     constexpr int CPR = G::KS / G::VE;  // 16-byte pieces per staged row
+    constexpr int CPRB = (G::KN ? G::BN : G::KS) / G::VE;
 
     __shared__ __attribute__((aligned(16))) unsigned char smem[2 * G::STAGE_LDS];
 
@@ -55,7 +56,11 @@ block_gemm_pipe_kernel(BlockArgs args, int64_t count) {
 #pragma unroll
         for (int i = 0; i < G::NBC; ++i) {
             const int c = tid + i * G::NT;
-            if (c < G::CB) rb[i] = load_raw<16>(B + (c / CPR) * ldb + k0 + (c % CPR) * G::VE);
+            if (c >= G::CB) continue;
+            if constexpr (G::KN)
+                rb[i] = load_raw<16>(B + (k0 + c / CPRB) * ldb + (c % CPRB) * G::VE);
+            else
+                rb[i] = load_raw<16>(B + (c / CPRB) * ldb + k0 + (c % CPRB) * G::VE);
         }
     };
     auto write = [&](int buf, const u4_t (&ra)[G::NA], const u4_t (&rb)[G::NBC]) {
@@ -69,7 +74,8 @@ block_gemm_pipe_kernel(BlockArgs args, int64_t count) {
         for (int i = 0; i < G::NBC; ++i) {
             const int c = tid + i * G::NT;
             if (c < G::CB)
-                store_raw<16>(base + G::A_LDS + (c / CPR) * G::ROWB + (c % CPR) * 16, rb[i]);
+                store_raw<16>(base + G::A_LDS + (G::KN ? G::krow(c / CPRB) : c / CPRB * G::ROWB) +
+                                  (c % CPRB) * 16, rb[i]);
         }
     };
 
@@ -88,8 +94,7 @@ block_gemm_pipe_kernel(BlockArgs args, int64_t count) {
             frag_t bf[G::JN];
 #pragma unroll
             for (int jn = 0; jn < G::JN; ++jn)
-                bf[jn] = bitcast<frag_t>(
-                    load_raw<FB>(bb + (pn * G::TN + jn * 16 + (lane & 15)) * G::ROWB + kk));
+                bf[jn] = stage_b_fragment<AT, G>(bb, lane, pn, 0, jn, ks);
 #pragma unroll
             for (int e = 0; e < AT::NSUB; ++e)
 #pragma unroll
@@ -184,7 +189,7 @@ hipError_t resident_workgroups(F kernel, int threads,
 // Persistent grid: every CU filled to the kernel's occupancy, never more workgroups than
 // problems.
 template <class AT, class G, int PD>
-hipError_t launch_block_gemm_pipe(const BlockArgs& args, int64_t count, hipStream_t stream) {
+hipError_t launch_block_gemm_pipe_as(const BlockArgs& args, int64_t count, hipStream_t stream) {
     static std::atomic<int> cache[kMaxCachedDevices];
     int slots = 0;
     const hipError_t e =
@@ -194,6 +199,14 @@ hipError_t launch_block_gemm_pipe(const BlockArgs& args, int64_t count, hipStrea
     hipLaunchKernelGGL((block_gemm_pipe_kernel<AT, G, PD>), dim3((unsigned)grid), dim3(G::NT), 0,
                        stream, args, count);
     return hipGetLastError();
+}
+
+// Only FP64 is run with B stored K x N (resolved in kami_block_gemm).
+template <class AT, class G, int PD>
+hipError_t launch_block_gemm_pipe(const BlockArgs& args, int64_t count, hipStream_t stream) {
+    if constexpr (G::ELT == 8)
+        if (args.b_kn) return launch_block_gemm_pipe_as<AT, typename G::AsKN, PD>(args, count, stream);
+    return launch_block_gemm_pipe_as<AT, G, PD>(args, count, stream);
 }
 
 }  // namespace kami

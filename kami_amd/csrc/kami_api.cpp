@@ -408,6 +408,17 @@ kami_status kami_block_gemm(const kami_gemm_desc* d, const void* A, const void* 
         return KAMI_ENOTSUP;
     st = device_check();
     if (st != KAMI_OK) return st;
+    // FP64 with B stored K x N and no form asked for: the partition's persistent form, where one
+    // is compiled and the problem is not small (128^3 x 4096 346 us against 380, 64^3 x 1024
+    // 20.6 against 27.0; but 32^3 x 4096 19.3 against 18.1, x 64 4.4 against 3.9).  The query goes
+    // on reporting the partition's plain form.
+    if (args.b_kn && d->precision == KAMI_PREC_F64 && d->pipeline == 0 && d->iters == 1 && in->m >= 64)
+        for (const auto& o : registry())
+            if (o.pipe == 2 && o.prec == in->prec && o.m == in->m && o.n == in->n && o.k == in->k &&
+                o.part == in->part && o.ranks == in->ranks) {
+                in = &o;
+                break;
+            }
     hipError_t e = in->launch(args, count, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e);
     return KAMI_OK;
