@@ -92,10 +92,12 @@ void register_bf16_instances(std::vector<BlockInstance>& v) {
 
     // 208^3 and 224^3 (the reference's FP16 square sweep reaches 224,
     // logs/block_gemm/square/H200/fp16_block_square_1d_H200.csv:13-14): 1D, 13 and 14
-    // waves of 16 rows; B's whole K (90-107 KB) exceeds the stage budget, so K is staged
-    // 16 (208) or 32 (224) wide through double-buffered LDS
-    add_instance<H, F, 208, 208, 208, 13, 1, 1, 2>(v, 1, 13);  // K step 16: 208 = 6.5 x 32
-    add_instance<A, F, 224, 224, 224, 14, 1, 1, 2>(v, 1, 14);
+    // waves of 16 rows.  Such a workgroup has a CU to itself, so B's whole K is one stage
+    // (90 and 108 KB): all of a problem's loads are in flight at once instead of a stage 16
+    // or 32 wide (208^3 x 2048 236 -> 151 us, x 64 19.3 -> 13.2; 224^3 x 2048 186 -> 166,
+    // x 512 51.8 -> 52.4).  The fences are after every K step: with two the fragments spill.
+    add_instance<H, F, 208, 208, 208, 13, 1, 1, 1, kWholeBudget>(v, 1, 13);  // K step 16: 208 = 6.5 x 32
+    add_instance<A, F, 224, 224, 224, 14, 1, 1, 1, kWholeBudget>(v, 1, 14);
     // K = 512 folded into LDS stages (src/batched_gemm/KAMI/1d/batched_gemm_1d_double_mma_128.cu:100-205)
     add_instance<A, F, 128, 128, 512, 8, 1, 1>(v, 1, 8);
     add_instance<A, F, 128, 128, 512, 4, 4, 1>(v, 2, 4);

@@ -50,11 +50,13 @@ constexpr int choose_ks(int budget) {
 }
 
 constexpr int kStageBudget = 80 * 1024;
+constexpr int kWholeBudget = 160 * 1024;  // one workgroup a CU
 
 // KFENCE: see block_gemm_kernel (for stages of many K steps).
-template <class AT, int PREC, int BM, int BN, int BK, int PM, int PN, int PK, int KFENCE = 0>
+template <class AT, int PREC, int BM, int BN, int BK, int PM, int PN, int PK, int KFENCE = 0,
+          int BUDGET = kStageBudget>
 void add_instance(std::vector<BlockInstance>& v, int part, int ranks) {
-    constexpr int KS = choose_ks<AT, BM, BN, BK, PM, PN, PK>(kStageBudget);
+    constexpr int KS = choose_ks<AT, BM, BN, BK, PM, PN, PK>(BUDGET);
     using G = BlockGeom<AT, BM, BN, BK, PM, PN, PK, KS>;
     v.push_back(BlockInstance{PREC, BM, BN, BK, part, ranks, PM, PN, PK, KS, G::NT, G::LDS,
                               AT::KSTEP, &launch_block_gemm<AT, G, KFENCE>, 1, 1});

@@ -170,28 +170,36 @@ kami_status validate_desc(const kami_gemm_desc* d) {
     return KAMI_OK;
 }
 
-// Streaming-mode winners of the instance sweep on MI355X (4096 FP64 / 8192 FP16 problems;
-// for FP64 the persistent 2D form, pipe = 2, wins at 32^3..128^3: 15.5 / 27.2 / 52.1
-// TFLOPS); used for KAMI_PART_AUTO until kami_block_gemm_autotune has measured the shape
+// Streaming-mode winners of the instance sweep on MI355X, 64 to 8192 problems.  FP64: the
+// persistent 2D form, pipe = 2, from 64^3 up for 512 problems and more (64^3 x 1024 21.5 us
+// against 23.5; with 64 problems 5.1 against 4.6), at 32^3 the plain one (x 512 3.7 us against
+// 4.2, x 4096 18.2, 19.0); 128 x 128 x 512 2D 4 x 4 317 us x 1024 against 345 for 1D.  BF16 64^3
+// 1D like FP16 (x 4096 25.7 us against 29.0 for 2D 4 x 4).  Low rank: more, thinner waves hide
+// a small batch's loads (256 x 256 x 32 x 512 1D 8 waves 28.2 us, 16 33.0; 192 x 192 x 32 x 64
+// 12 waves 4.8, 4 6.2, x 1024 34.4 and 33.6; 128 x 128 x 32 x 4096 8 waves 63.2, 4 67.9).
+// Used for KAMI_PART_AUTO until kami_block_gemm_autotune has measured the shape
 // in this process (or a tuning file has been loaded).
 struct Prior {
     int prec, m, n, k, part, ranks, pipe = 1;
 };
 static const Prior kPriors[] = {
     {KAMI_PREC_F64, 16, 16, 16, KAMI_PART_2D, 1},
-    {KAMI_PREC_F64, 32, 32, 32, KAMI_PART_2D, 2, 2},
+    {KAMI_PREC_F64, 32, 32, 32, KAMI_PART_2D, 2},
     {KAMI_PREC_F64, 64, 64, 64, KAMI_PART_2D, 4, 2},
     {KAMI_PREC_F64, 128, 128, 128, KAMI_PART_2D, 4, 2},
+    {KAMI_PREC_F64, 128, 128, 512, KAMI_PART_2D, 4},
     {KAMI_PREC_F16_F32, 32, 32, 32, KAMI_PART_2D, 1}, {KAMI_PREC_F16_F32, 64, 64, 64, KAMI_PART_1D, 4},
     {KAMI_PREC_F16_F32, 128, 128, 128, KAMI_PART_2D, 4},
     {KAMI_PREC_F16_F32, 256, 256, 256, KAMI_PART_1D, 16},
-    {KAMI_PREC_F16_F32, 256, 256, 16, KAMI_PART_1D, 16},
-    {KAMI_PREC_F16_F32, 256, 256, 32, KAMI_PART_1D, 16},
-    {KAMI_PREC_BF16_F32, 32, 32, 32, KAMI_PART_2D, 1}, {KAMI_PREC_BF16_F32, 64, 64, 64, KAMI_PART_2D, 4},
+    {KAMI_PREC_F16_F32, 128, 128, 32, KAMI_PART_1D, 8},
+    {KAMI_PREC_F16_F32, 192, 192, 16, KAMI_PART_1D, 12}, {KAMI_PREC_F16_F32, 192, 192, 32, KAMI_PART_1D, 12},
+    {KAMI_PREC_F16_F32, 256, 256, 16, KAMI_PART_1D, 16}, {KAMI_PREC_F16_F32, 256, 256, 32, KAMI_PART_1D, 8},
+    {KAMI_PREC_BF16_F32, 32, 32, 32, KAMI_PART_2D, 1}, {KAMI_PREC_BF16_F32, 64, 64, 64, KAMI_PART_1D, 4},
     {KAMI_PREC_BF16_F32, 128, 128, 128, KAMI_PART_1D, 4},
     {KAMI_PREC_BF16_F32, 256, 256, 256, KAMI_PART_1D, 16},
-    {KAMI_PREC_BF16_F32, 256, 256, 16, KAMI_PART_1D, 16},
-    {KAMI_PREC_BF16_F32, 256, 256, 32, KAMI_PART_1D, 16},
+    {KAMI_PREC_BF16_F32, 128, 128, 32, KAMI_PART_1D, 8},
+    {KAMI_PREC_BF16_F32, 192, 192, 16, KAMI_PART_1D, 12}, {KAMI_PREC_BF16_F32, 192, 192, 32, KAMI_PART_1D, 12},
+    {KAMI_PREC_BF16_F32, 256, 256, 16, KAMI_PART_1D, 16}, {KAMI_PREC_BF16_F32, 256, 256, 32, KAMI_PART_1D, 8},
 };
 
 // The persistent form handles the 2D partition with B stored N x K and iters = 1.
