@@ -11,14 +11,14 @@
 // Per problem:
 //   1. e_i with |A(i,k)| < 2^e_i over the full row of A (f_j for rows of B, B stored
 //      N x K);
-//   2. X(i,k) = trunc(|A(i,k)| 2^(62 - e_i)) sign(A(i,k)) is a 63-bit signed integer,
+//   2. X(i,k) = A(i,k) 2^(62 - e_i) rounded to an integer is a 63-bit signed integer,
 //      written as eight balanced byte digits X = sum_{p=0..7} d_p 2^(8 (7 - p)),
 //      d_p in [-128, 127] (p = 0 the most significant);
 //   3. level sums T_l = sum_{p + q = l} d_p(A) d_q(B)^T over the whole K on int8 MFMA:
 //      |T_l| <= 8 K 2^14 < 2^31, so every level is exact in int32 in any order;
 //   4. levels l < L are kept (L = 8: 36 digit products) and combined in FP64 by
 //      Horner's rule, C(i,j) = alpha 2^(e_i + f_j - 12) sum_l T_l 2^(-8 l) + beta C(i,j).
-// Truncating each operand costs at most 2^(e - 62) per element; the dropped levels
+// Rounding each operand costs at most 2^(e - 63) per element; the dropped levels
 // l >= L weigh at most 2^(-8 L) each against the kept ones.  Finite inputs are required.
 //
 // Work layout (the reference's 1D partition: A private per wave, B broadcast, F64-1D:73-
@@ -80,24 +80,39 @@ struct I8Geom {
     }
 };
 
-// The eight balanced byte digits of X = trunc(|x| 2^(62 - E)) sign(x), for |x| < 2^E,
-// packed in one word: byte b is the digit of weight 2^(8b), in [-128, 127], and
-// X = sum_b d_b 2^(8b) exactly.  With c_e = 1023 + E: the 53-bit significand of x with its
-// leading bit placed at bit 62 is shifted right by min(c_e - exponent field, 63) (63
-// gives 0: bit 63 is clear).  A zero or subnormal x (exponent field 0) is then 0, which
-// is exact when E >= -960 (|x| < 2^-1022 <= 2^(E - 62)); rows with smaller E are scaled
-// by 2^1000 first (slice_step).  Adding 0x80 to every byte with carries and flipping each
-// byte's top bit back turns the two's complement value into balanced digits.
-__device__ inline uint64_t digit_word(double x, uint32_t c_e) {
-    const uint64_t bits = __builtin_bit_cast(uint64_t, x);
-    const uint32_t h = (uint32_t)(bits >> 32), l = (uint32_t)bits;
-    const uint32_t r = min(c_e - ((h >> 20) & 0x7ffu), 63u);
-    const uint64_t M = ((uint64_t)((h & 0xfffffu) | 0x100000u) << 32 | l) << 10;
-    const uint64_t X = M >> r;
-    const int32_t s = (int32_t)h >> 31;  // 0 or -1
-    const uint64_t s64 = (uint64_t)(int64_t)s;
-    // -X = ~X + 1: the +1 rides in the low word of the byte-wise 0x80 offset
-    const uint64_t Y = (X ^ s64) + ((uint64_t)0x80808080u << 32 | (uint32_t)(0x80808080u - s));
+// Rows whose exponent lies outside this range are scaled by 2^1000 or 2^-1000 (exact down to
+// 2^(E - 62)) before they are sliced, so that the constants of RowCut are normal.
+constexpr int kLowRowExp = -960, kHighRowExp = 960;
+__device__ inline int row_scale(int E) { return E < kLowRowExp ? 1000 : E > kHighRowExp ? -1000 : 0; }
+
+// Constants that cut the elements of a row with |x| < 2^E (E already scaled): 1.5 x 2^(E + 22)
+// has units of 2^(E - 30), 1.5 x 2^(E - 10) units of 2^(E - 62).
+struct RowCut {
+    double high, low;
+    uint32_t fix;  // 0x80808080 less the high word of `low`
+    __device__ explicit RowCut(int E) {
+        const uint32_t h = (uint32_t)(1023 + 22 + E) << 20 | 0x80000u, l = h - (32u << 20);
+        high = __builtin_bit_cast(double, (uint64_t)h << 32);
+        low = __builtin_bit_cast(double, (uint64_t)l << 32);
+        fix = 0x80808080u - l;
+    }
+};
+
+// The eight balanced byte digits of X = x 2^(62 - E) rounded to an integer, packed in one word:
+// byte b is the digit of weight 2^(8b), in [-128, 127], and X = sum_b d_b 2^(8b) exactly.
+// Adding `high` leaves the multiple of 2^32 nearest to X in the low word of the sum (two's
+// complement, as the sum's unit is 2^(E - 30)); what is left is exact, and adding `low` rounds
+// it to units of 2^(E - 62): the low word of that sum is X's, the high word's change the carry
+// into X's high word.  Adding 0x80 to every byte with carries and flipping each byte's top bit
+// back turns the two's complement value into balanced digits.  Four FP64 additions and five
+// integer operations; shifting the significand took sixteen, two of them 64-bit shifts.  The
+// streaming kernel's waves issue VALU work in about as many cycles as products: 128^3 x 4096
+// 377 -> 366 us, x 256 32.5 -> 31.0, 64^3 x 8192 156.5 -> 153.
+__device__ inline uint64_t digit_word(double x, const RowCut& cut) {
+    const double t1 = x + cut.high;
+    const double t2 = (x - (t1 - cut.high)) + cut.low;
+    const uint64_t b1 = __builtin_bit_cast(uint64_t, t1), b2 = __builtin_bit_cast(uint64_t, t2);
+    const uint64_t Y = b2 + ((uint64_t)((uint32_t)b1 + cut.fix) << 32 | 0x80808080u);
     return Y ^ 0x8080808080808080ull;
 }
 
@@ -134,29 +149,24 @@ __device__ inline void lds_barrier() {
     __builtin_amdgcn_s_barrier();
 }
 
-// Rows whose exponent is below this take the scaled path of slice_step.
-constexpr int kTinyRowExp = -960;
-
 // Digit fragments of one 64-wide K step from the lane's eight 16-byte pieces x[i]
 // (doubles k(i, 0), k(i, 1)): frag[p] is the 16-byte MFMA fragment of plane p (p = 0 the
-// most significant digit), slot j = 2 i + q.  `tiny`: some row of the wave has
-// E < -960; its elements are scaled by 2^1000 (exact) so that their subnormals are
-// normal, with E raised by the same amount.
-__device__ inline void slice_step(const u4_t (&x)[8], int E, bool tiny, u4_t (&frag)[8]) {
-    const int sc = (tiny && E < kTinyRowExp) ? 1000 : 0;
-    const uint32_t c_e = (uint32_t)(1023 + E + sc);
+// most significant digit), slot j = 2 i + q.  `sc`: the row's scale, where `scaled` says that
+// some row of the wave has one; E counts it.
+__device__ inline void slice_step(const u4_t (&x)[8], const RowCut& cut, int sc, bool scaled,
+                                  u4_t (&frag)[8]) {
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
         d2_t x0 = bitcast<d2_t>(x[2 * m]), x1 = bitcast<d2_t>(x[2 * m + 1]);
-        if (tiny) {
+        if (scaled) {
             x0[0] = __builtin_amdgcn_ldexp(x0[0], sc);
             x0[1] = __builtin_amdgcn_ldexp(x0[1], sc);
             x1[0] = __builtin_amdgcn_ldexp(x1[0], sc);
             x1[1] = __builtin_amdgcn_ldexp(x1[1], sc);
         }
         uint32_t out[8];
-        transpose4(digit_word(x0[0], c_e), digit_word(x0[1], c_e), digit_word(x1[0], c_e),
-                   digit_word(x1[1], c_e), out);
+        transpose4(digit_word(x0[0], cut), digit_word(x0[1], cut), digit_word(x1[0], cut),
+                   digit_word(x1[1], cut), out);
 #pragma unroll
         for (int b = 0; b < 8; ++b) frag[7 - b][m] = out[b];
     }
@@ -274,11 +284,13 @@ split_i8_kernel(SplitArgs args, int64_t count) {
         {
             const int ea = row_exponent<G::KS>(xa);
             expo[row] = ea;  // the row's four lane groups write the same value
-            const bool tiny = __builtin_amdgcn_ballot_w64(ea < kTinyRowExp) != 0;
+            const int sc = row_scale(ea);
+            const bool scaled = __builtin_amdgcn_ballot_w64(sc != 0) != 0;
+            const RowCut cut(ea + sc);
 #pragma unroll
             for (int h = 0; h < G::KS; ++h) {
                 u4_t f[8];
-                slice_step(xa[h], ea, tiny, f);
+                slice_step(xa[h], cut, sc, scaled, f);
 #pragma unroll
                 for (int q = 0; q < G::S; ++q) ad[q][h] = f[q];
                 __builtin_amdgcn_sched_barrier(0);
@@ -296,11 +308,13 @@ split_i8_kernel(SplitArgs args, int64_t count) {
                 for (int q = 0; q < 8; ++q) xb[h][q] = load_raw<16>(region + (8 * h + q) * G::FRAG + 16 * lane);
             const int eb = row_exponent<G::KS>(xb);
             expo[G::BM + row] = eb;
-            const bool tiny = __builtin_amdgcn_ballot_w64(eb < kTinyRowExp) != 0;
+            const int sc = row_scale(eb);
+            const bool scaled = __builtin_amdgcn_ballot_w64(sc != 0) != 0;
+            const RowCut cut(eb + sc);
 #pragma unroll
             for (int h = 0; h < G::KS; ++h) {
                 u4_t f[8];
-                slice_step(xb[h], eb, tiny, f);
+                slice_step(xb[h], cut, sc, scaled, f);
 #pragma unroll
                 for (int q = 0; q < G::S; ++q)
                     store_raw<16>(region + (q * G::KS + h) * G::FRAG + 16 * lane, f[q]);
@@ -529,15 +543,15 @@ split_i8_stream_kernel(SplitArgs args, int64_t count) {
         for (int w = 1; w < G::WAVES; ++w) E = max(E, pm[w * 16]);
         if (wave == 0 && grp == 0) expb[(int)(reg & 1) * 16 + r] = E;
         d2_t x0 = bitcast<d2_t>(x[0]), x1 = bitcast<d2_t>(x[1]);
-        const int sc = E < kTinyRowExp ? 1000 : 0;  // tiny rows: scaled by 2^1000
+        const int sc = row_scale(E);
         x0[0] = __builtin_amdgcn_ldexp(x0[0], sc);
         x0[1] = __builtin_amdgcn_ldexp(x0[1], sc);
         x1[0] = __builtin_amdgcn_ldexp(x1[0], sc);
         x1[1] = __builtin_amdgcn_ldexp(x1[1], sc);
-        const uint32_t c_e = (uint32_t)(1023 + E + sc);
+        const RowCut cut(E + sc);
         uint32_t out[8];
-        transpose4(digit_word(x0[0], c_e), digit_word(x0[1], c_e), digit_word(x1[0], c_e),
-                   digit_word(x1[1], c_e), out);
+        transpose4(digit_word(x0[0], cut), digit_word(x0[1], cut), digit_word(x1[0], cut),
+                   digit_word(x1[1], cut), out);
         unsigned char* dst = smem + St::PLN_OFF + (int)(reg & 1) * G::REGION + sh * G::FRAG +
                              16 * lane + 4 * (si >> 1);
 #pragma unroll
@@ -581,11 +595,13 @@ split_i8_stream_kernel(SplitArgs args, int64_t count) {
             // ---- a new problem: A exponents and digits into registers ----
             const int ea = row_exponent<G::KS>(xa);
             expa[row] = ea;
-            const bool tiny = __builtin_amdgcn_ballot_w64(ea < kTinyRowExp) != 0;
+            const int sc = row_scale(ea);
+            const bool scaled = __builtin_amdgcn_ballot_w64(sc != 0) != 0;
+            const RowCut cut(ea + sc);
 #pragma unroll
             for (int h = 0; h < G::KS; ++h) {
                 u4_t f[8];
-                slice_step(xa[h], ea, tiny, f);
+                slice_step(xa[h], cut, sc, scaled, f);
 #pragma unroll
                 for (int q = 0; q < G::S; ++q) ad[q][h] = f[q];
                 __builtin_amdgcn_sched_barrier(0);
@@ -633,8 +649,8 @@ split_i8_stream_kernel(SplitArgs args, int64_t count) {
         // of the VALU work, so that the VALU issues while the MFMAs run.  Planes go in the
         // order 0, 7, 1, 6, 2, 5, 3, 4 (8, 1, 7, 2, 6, 3, 5, 4 products): any two
         // consecutive groups hold at least 9 products, and fragments are read two groups
-        // ahead.  Rows of region t + 1 with E < -960 take the scaled slicing (a scale of 2^0
-        // for the others: four ldexp per lane).
+        // ahead.  Rows of region t + 1 outside the exponent range take the scaled slicing (a
+        // scale of 2^0 for the others: four ldexp per lane).
         static_assert(G::L == G::S && G::S == 8, "eight planes, all levels below 8");
         constexpr int kOrder[8] = {0, 7, 1, 6, 2, 5, 3, 4};
         constexpr int NF = 8 * G::KS;
@@ -645,7 +661,7 @@ split_i8_stream_kernel(SplitArgs args, int64_t count) {
         fb[0] = bfrag(kOrder[0], 0);
         fb[1] = bfrag(kOrder[1], 0);
         d2_t a0, a1;
-        uint32_t c_e = 0;
+        RowCut cut(0);
         uint64_t dw[4];
         uint32_t out[8];
         auto valu_step = [&](auto s_tag) {
@@ -655,15 +671,15 @@ split_i8_stream_kernel(SplitArgs args, int64_t count) {
             } else if constexpr (s == 1) {
                 a0 = bitcast<d2_t>(x1[0]);
                 a1 = bitcast<d2_t>(x1[1]);
-                const int sc = E < kTinyRowExp ? 1000 : 0;
+                const int sc = row_scale(E);
                 a0[0] = __builtin_amdgcn_ldexp(a0[0], sc);
                 a0[1] = __builtin_amdgcn_ldexp(a0[1], sc);
                 a1[0] = __builtin_amdgcn_ldexp(a1[0], sc);
                 a1[1] = __builtin_amdgcn_ldexp(a1[1], sc);
-                c_e = (uint32_t)(1023 + E + sc);
+                cut = RowCut(E + sc);
             } else if constexpr (s >= 2 && s <= 5) {
                 const double x = s == 2 ? a0[0] : s == 3 ? a0[1] : s == 4 ? a1[0] : a1[1];
-                dw[s - 2] = digit_word(x, c_e);
+                dw[s - 2] = digit_word(x, cut);
             } else if constexpr (s == 6) {
                 transpose4(dw[0], dw[1], dw[2], dw[3], out);
             } else if constexpr (s == 7) {
