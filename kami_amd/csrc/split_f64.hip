@@ -735,27 +735,18 @@ split_pipe_kernel(SplitArgs args, int64_t count) {
     };
     auto slice = [&](const u4_t (&x)[4], int e, unsigned char* plane0) {
         unsigned char* dst = plane0 + srow * G::ROWB + 2 * sk;
-        double r[8];
+        u4_t plane[G::S];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const d2_t d = bitcast<d2_t>(x[i]);
-            r[2 * i] = __builtin_amdgcn_ldexp(d[0], G::BETA - e);
-            r[2 * i + 1] = __builtin_amdgcn_ldexp(d[1], G::BETA - e);
+            const d2_t v = bitcast<d2_t>(x[i]);
+            uint32_t d[G::S];
+            PairDigits<SAT, G::BETA, G::S>::make(__builtin_amdgcn_ldexp(v[0], 3 * G::BETA - e),
+                                                 __builtin_amdgcn_ldexp(v[1], 3 * G::BETA - e), d);
+#pragma unroll
+            for (int s = 0; s < G::S; ++s) plane[s][i] = d[s];
         }
 #pragma unroll
-        for (int s = 0; s < G::S; ++s) {
-            u4_t packed;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const double q0 = __builtin_rint(r[2 * j]), q1 = __builtin_rint(r[2 * j + 1]);
-                packed[j] = pack2<SAT>(q0, q1);
-                if (s + 1 < G::S) {
-                    r[2 * j] = (r[2 * j] - q0) * (double)(1 << G::BETA);
-                    r[2 * j + 1] = (r[2 * j + 1] - q1) * (double)(1 << G::BETA);
-                }
-            }
-            store_raw<16>(dst + s * G::PLANE, packed);
-        }
+        for (int s = 0; s < G::S; ++s) store_raw<16>(dst + s * G::PLANE, plane[s]);
     };
 
     int64_t p = blockIdx.x;  // work unit
@@ -1104,9 +1095,9 @@ static hipError_t launch_pipe_tiles(const SplitArgs& a, int64_t units, hipStream
 }
 
 // a.tiles_m x a.tiles_n counts 64 x 64 tiles of C per problem.  A tile and chunk takes a CU
-// 2.3-2.7 us in the 64-wide form, 6.8-8.9 us in the 128-wide one (four times the outputs), so
+// 2.3-2.7 us in the 64-wide form, 6.6-8.6 us in the 128-wide one (four times the outputs), so
 // the wide form is taken where its rounds over the chip, at three times the price, are
-// fewer: 128^3 x 4096 568 us against 676, but 1024^3 (64 wide tiles) 217 against 73 and
+// fewer: 128^3 x 4096 556 us against 676, but 1024^3 (64 wide tiles) 217 against 73 and
 // 1536^3 (144) 325 against 300.
 template <class SAT, int BETA, int S, int G>
 hipError_t launch_split_stream(const SplitArgs& a, int64_t count, hipStream_t s) {
