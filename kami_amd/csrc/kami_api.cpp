@@ -189,7 +189,7 @@ static const Prior kPriors[] = {
     {KAMI_PREC_F64, 128, 128, 128, KAMI_PART_2D, 4, 2},
     {KAMI_PREC_F64, 128, 128, 512, KAMI_PART_2D, 4},
     {KAMI_PREC_F16_F32, 32, 32, 32, KAMI_PART_2D, 1}, {KAMI_PREC_F16_F32, 64, 64, 64, KAMI_PART_1D, 4},
-    {KAMI_PREC_F16_F32, 128, 128, 128, KAMI_PART_2D, 4},
+    {KAMI_PREC_F16_F32, 128, 128, 128, KAMI_PART_1D, 4},
     {KAMI_PREC_F16_F32, 256, 256, 256, KAMI_PART_1D, 16},
     {KAMI_PREC_F16_F32, 128, 128, 32, KAMI_PART_1D, 8},
     {KAMI_PREC_F16_F32, 192, 192, 16, KAMI_PART_1D, 12}, {KAMI_PREC_F16_F32, 192, 192, 32, KAMI_PART_1D, 12},
@@ -201,6 +201,27 @@ static const Prior kPriors[] = {
     {KAMI_PREC_BF16_F32, 192, 192, 16, KAMI_PART_1D, 12}, {KAMI_PREC_BF16_F32, 192, 192, 32, KAMI_PART_1D, 12},
     {KAMI_PREC_BF16_F32, 256, 256, 16, KAMI_PART_1D, 16}, {KAMI_PREC_BF16_F32, 256, 256, 32, KAMI_PART_1D, 8},
 };
+
+// Forms for batches of no more problems than CUs, where AUTO would take one of the priors.
+// Every problem has a CU to itself then, and more waves on it hide its loads better, while
+// there is no next problem to load ahead (us, this form against the prior: FP64 64^3 x 64 4.5,
+// 5.1; x 256 7.2, 7.6; x 768 18.0, 15.9.  BF16 128^3 x 64 3.8, 4.6; x 512 12.5, 11.1.  FP16
+// 256^3 x 64 13.1, 15.6; x 256 28.1, 28.4; x 512 59.3, 58.0).  The same products in the same
+// order, so the bits do not depend on it; the query reports the prior.
+constexpr int64_t kSmallBatch = 256;
+static const Prior kSmallPriors[] = {
+    {KAMI_PREC_F64, 64, 64, 64, KAMI_PART_2D, 4},
+    {KAMI_PREC_F16_F32, 128, 128, 128, KAMI_PART_2D, 4}, {KAMI_PREC_F16_F32, 256, 256, 256, KAMI_PART_2D, 4},
+    {KAMI_PREC_BF16_F32, 128, 128, 128, KAMI_PART_2D, 4}, {KAMI_PREC_BF16_F32, 256, 256, 256, KAMI_PART_2D, 4},
+};
+static const Prior* small_batch_prior(const kami_gemm_desc* d, int64_t count) {
+    TuneVal tv;
+    if (count > kSmallBatch || d->partition != KAMI_PART_AUTO || d->pipeline != 0 || d->iters != 1) return nullptr;
+    for (const Prior& p : kSmallPriors)
+        if (p.prec == d->precision && p.m == d->m && p.n == d->n && p.k == d->k)
+            return get_tuned_choice(p.prec, p.m, p.n, p.k, &tv) ? nullptr : &p;
+    return nullptr;
+}
 
 // The persistent form handles the 2D partition with B stored N x K and iters = 1.
 static bool pipe_allowed(const kami_gemm_desc* d) {
@@ -409,6 +430,13 @@ kami_status kami_block_gemm(const kami_gemm_desc* d, const void* A, const void* 
     kami_status st = prepare_args(d, A, B, C, count, stride_a, stride_b, stride_c, args);
     if (st != KAMI_OK || count == 0) return st;
     if (is_split(d->precision)) return split_launch(d, args, count, (hipStream_t)stream);
+    kami_gemm_desc small = *d;
+    if (const Prior* p = small_batch_prior(d, count)) {
+        small.partition = p->part;
+        small.ranks = p->ranks;
+        small.pipeline = p->pipe;
+        d = &small;
+    }
     const BlockInstance* in = resolve_block(d, &st);
     if (!in) return st;
     // one workgroup per problem: the grid's work-items must stay below 2^32
