@@ -8,9 +8,8 @@
 //   * problems carry their own {m, n, k, lda, ldb, ldc, A, B, C} (the kami_problem array);
 //   * every problem is cut into output tiles; a tile is one 64-byte queue entry holding
 //     its own operand pointers, strides, extents and variant (WorkItem);
-//   * an entry is cut into wave tiles of up to 32 x 32 (2-byte inputs: 64 x 32; WaveUnit, 8
-//     bytes each).  A wave
-//     computes one of them alone, staged through LDS of its own, so there is no barrier
+//   * an entry is cut into wave tiles of up to 32 x 32 (2-byte inputs: 64 x 64; WaveUnit, 8
+//     bytes each).  A wave computes one of them alone, staged through LDS of its own, so there is no barrier
 //     and no shared counter: the hardware's dispatcher hands out the workgroups, longest
 //     problems first, and one wave's loads hide behind the products of the others;
 //   * units are laid out so that neighbouring tiles run on one XCD at the same time;
@@ -22,11 +21,12 @@
 // M, N and K must be multiples of 16.
 //
 // What bounds it: 20000 problems of 16 to 256 (3.58 GB FP64, 1.19 GB FP16 with FP32 C) run
-// in 810 us and 290 us, 4.4 and 4.1 TB/s of the algorithmic bytes; the matrix pipes are
-// 57 % busy in FP64, and L1 takes 10 TB/s of lines from L2 in either.  The persistent form this replaced (workgroups popping tiles of up to
-// 128 x 128 from an atomic counter, LDS stages shared by four waves, one barrier a stage, a
-// one-thread kernel to clear the counter) took 1027 us and 398 us: two workgroups a CU and
-// their barriers left too little in flight.
+// in 807 us and 275 us, 4.4 and 4.3 TB/s of the algorithmic bytes; the matrix pipes are
+// 57 % busy in FP64, whose HBM traffic (3.81 GB, 4.7 TB/s) runs near the rate of a copy (4.8).
+// The persistent form this replaced (workgroups popping tiles of up to 128 x 128 from an atomic
+// counter, LDS stages shared by four waves, one barrier a stage, a one-thread kernel to clear
+// the counter) took 1027 us and 398 us: two workgroups a CU and their barriers left too little
+// in flight.
 #include <algorithm>
 #include <cstring>
 #include <memory>
@@ -63,7 +63,7 @@ static_assert(kVariants == kBatchedVariants, "tuning-cache variant range");
 static const int kVariantTM[kVariants] = {64, 32, 64, 128, 128, 64};
 static const int kVariantTN[kVariants] = {64, 32, 64, 64, 128, 128};
 static const int kVariantSM[kVariants] = {4, 4, 1, 4, 4, 4};  // atoms of a wave tile, at most
-static const int kVariantSN[kVariants] = {2, 2, 2, 2, 2, 2};
+static const int kVariantSN[kVariants] = {4, 4, 2, 4, 4, 4};
 
 // Variants a precision offers: 4 and 5 are FP64's.
 inline int variants_of(int prec) { return prec == KAMI_PREC_F64 ? kVariants : 4; }
@@ -75,16 +75,17 @@ struct WaveUnit {
     uint8_t ra, ca, im, jn;
 };
 static_assert(sizeof(WaveUnit) == 8, "wave unit layout");
-// Wave tiles in atoms, largest first; a precision starts at first_cap.  2-byte inputs take
-// 64 x 32: the rate at which a CU's L1 takes lines bounds them, and a taller tile reads B's
-// half as often (20000 problems of 16 to 256: 284 us against 304 with 32 x 32; 64 x 64 tiles, at
-// two waves a SIMD, 273, but 109 against 102 at 128^3 x 4096 and 23.8 against 21.7 for problems
-// of 16 to 64).  FP64 takes 32 x 32: 64 x 32 at two waves a SIMD, 789 us against 808, leaves
-// 60 against 59 for problems of 16 to 64 and twice the registers.
-constexpr int kCaps = 4;
-static const int kCapM[kCaps] = {4, 2, 1, 1}, kCapN[kCaps] = {2, 2, 2, 1};
-constexpr int kMostN = 2;
-constexpr int first_cap(int elt) { return elt == 8 ? 1 : 0; }
+// Wave tiles in atoms, largest first; a precision starts at first_cap.  For 2-byte inputs the
+// rate at which a CU's L1 takes lines sets the time, and a larger tile reads them less often:
+// 64 x 64 where wide_pays (256^3 x 1024 115 us against 141 with 64 x 32, 320^3 x 1024 227
+// against 280, 20000 problems of 16 to 256 276 against 291), else 64 x 32 (20000 of 16 to 64
+// 21.7 against 23.8; the same of 16 to 256 304 with 32 x 32).  FP64 takes 32 x 32: 64 x 32 at two
+// waves a SIMD, 789 us against 808, leaves 60 against 59 for problems of 16 to 64 and twice the
+// registers.
+constexpr int kCaps = 5;
+static const int kCapM[kCaps] = {4, 4, 2, 1, 1}, kCapN[kCaps] = {4, 2, 2, 2, 1};
+constexpr int kWideCap = 0;
+constexpr int first_cap(int elt) { return elt == 8 ? 2 : 1; }
 constexpr int kWavesPerGroup = 4;
 constexpr int kXcds = 8;  // workgroup L runs on XCD L mod 8
 
@@ -98,7 +99,7 @@ struct BatchArgs {
     const WaveUnit* units;
     int64_t n_units;  // a multiple of kWavesPerGroup x kXcds
     double alpha, beta;
-    int tall;  // 1: wave tiles may be four atoms high (cap 0)
+    int cap;  // the largest wave tile is kCapM[cap] x kCapN[cap] atoms
 };
 
 __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
@@ -140,9 +141,10 @@ struct WaveTile {
     // K x N operands: FP64 fragments are loaded straight (16 lanes read 16 consecutive
     // columns); rows of 2-byte values are turned by transposing LDS reads
     static constexpr bool TURN = KN && !F64;
-    static constexpr int TROW = JN * 32 + 16;  // bytes of a staged K row
-    static constexpr int PPR = JN * 2;         // 16-byte pieces of a K row
-    static constexpr int NA = IM * 2, NB = JN * 2;  // 16-byte pieces of a lane
+    static constexpr int PPR = JN == 3 ? 8 : JN * 2;  // lanes of a K row, a 16-byte piece each
+    static constexpr int TROW = PPR * 16 + 16;        // bytes of a staged K row
+    static constexpr int NA = IM * 2, NB = TURN ? PPR : JN * 2;  // 16-byte pieces of a lane
+    static_assert(!TURN || KS == 64, "NB loads of 64 / PPR rows are a stage");
     static constexpr int A_LDS = IM * 16 * 128;
     static constexpr int LDS = A_LDS + (!KN ? JN * 16 * 128 : TURN ? KS * TROW : 0);
 
@@ -199,7 +201,8 @@ struct WaveTile {
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
                 const int r = k0 + i * RPL;
-                s.b[i] = buffer_load16(rb, r + lane / PPR < k ? boff : kBufferRange,
+                const bool live = r + lane / PPR < k && (JN != 3 || lane % PPR < 2 * JN);
+                s.b[i] = buffer_load16(rb, live ? boff : kBufferRange,
                                        (r < k ? r : 0) * ldb * ELT);
             }
         }
@@ -308,14 +311,14 @@ struct WaveTile {
     }
 };
 
-// MM: atoms of a wave tile's height, at most (a queue without taller ones keeps the smaller
-// kernel, four waves a SIMD).  One wave per unit; a workgroup is four consecutive units (neighbouring wave tiles of
-// one problem share its lines of A and B in the CU's L1).
-template <class AT, bool KN, int MM>
+// MM x NN: atoms of a wave tile, at most: the smaller the tile, the more waves a SIMD holds (2 x 2
+// four, 4 x 2 three, 4 x 4 two).  One wave per unit; a workgroup is four consecutive units
+// (neighbouring wave tiles of one problem share its lines of A and B in the CU's L1).
+template <class AT, bool KN, int MM, int NN>
 __global__ void __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(MM == 2 ? 4 : 3)))
+__attribute__((amdgpu_waves_per_eu(MM == 2 ? 4 : NN == 2 ? 3 : 2)))
 batched_wave_kernel(BatchArgs args) {
-    constexpr int LDS_WAVE = WaveTile<AT, KN, MM, kMostN>::LDS;
+    constexpr int LDS_WAVE = WaveTile<AT, KN, MM, NN>::LDS;
     __shared__ __attribute__((aligned(16))) unsigned char smem[kWavesPerGroup * LDS_WAVE];
     const int wave = uni(threadIdx.x >> 6);
     unsigned char* const lds = smem + wave * LDS_WAVE;
@@ -326,10 +329,20 @@ batched_wave_kernel(BatchArgs args) {
         WaveTile<AT, KN, decltype(im)::value, decltype(jn)::value>(w, u, lds).run(w, u, args.alpha, args.beta);
     };
     auto run_rows = [&](auto im) {
-        if (u.jn == 1)
-            run(im, std::integral_constant<int, 1>{});
-        else
-            run(im, std::integral_constant<int, 2>{});
+        // Returns leave 116 registers where branches past each other leave 160 (4 x 2: 20000
+        // problems of 16 to 64 45.0 us against 47.5), but 208 against 166 with 4 x 4 (320^3 x
+        // 1024 231 against 226).
+        if constexpr (NN == 2) {
+            if (u.jn == 1) return run(im, std::integral_constant<int, 1>{});
+            if (u.jn == 2) return run(im, std::integral_constant<int, 2>{});
+        } else {
+            if (u.jn == 1)
+                run(im, std::integral_constant<int, 1>{});
+            else if (u.jn == 2)
+                run(im, std::integral_constant<int, 2>{});
+            if (u.jn == 3) run(im, std::integral_constant<int, 3>{});
+            if (u.jn == 4) run(im, std::integral_constant<int, 4>{});
+        }
     };
     if (u.im == 1) return run_rows(std::integral_constant<int, 1>{});
     if (u.im == 2) return run_rows(std::integral_constant<int, 2>{});
@@ -368,12 +381,12 @@ static int64_t batched_groups(int64_t n_units) { return n_units / kWavesPerGroup
 // A dispatch holds fewer than 2^32 work-items; longer queues take several.
 constexpr int64_t kMaxGroups = (int64_t)1 << 23;
 
-template <class AT, int MM>
+template <class AT, int MM, int NN>
 static void launch_kernel(const BatchArgs& a, bool kn, dim3 grid, hipStream_t s) {
     if (kn)
-        hipLaunchKernelGGL((batched_wave_kernel<AT, true, MM>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((batched_wave_kernel<AT, true, MM, NN>), grid, dim3(256), 0, s, a);
     else
-        hipLaunchKernelGGL((batched_wave_kernel<AT, false, MM>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((batched_wave_kernel<AT, false, MM, NN>), grid, dim3(256), 0, s, a);
 }
 
 template <class AT>
@@ -382,12 +395,14 @@ static hipError_t launch_for(BatchArgs a, bool kn, hipStream_t s) {
     for (int64_t left = batched_groups(a.n_units); left > 0 && e == hipSuccess; left -= kMaxGroups) {
         const dim3 grid((unsigned)std::min(left, kMaxGroups));
         if constexpr (sizeof(typename AT::in_t) == 2) {
-            if (a.tall)
-                launch_kernel<AT, 4>(a, kn, grid, s);
+            if (a.cap == kWideCap)
+                launch_kernel<AT, 4, 4>(a, kn, grid, s);
+            else if (kCapM[a.cap] == 4)
+                launch_kernel<AT, 4, 2>(a, kn, grid, s);
             else
-                launch_kernel<AT, 2>(a, kn, grid, s);
+                launch_kernel<AT, 2, 2>(a, kn, grid, s);
         } else {
-            launch_kernel<AT, 2>(a, kn, grid, s);
+            launch_kernel<AT, 2, 2>(a, kn, grid, s);
         }
         e = hipGetLastError();
         a.units += kMaxGroups * kWavesPerGroup;
@@ -468,8 +483,32 @@ static int64_t count_units(const WorkItem* items, int64_t n_items, int cap) {
 // 17.2 (and 17.2 with 2048 here); FP16 is bound by the launch itself there.
 constexpr int64_t kFullUnits = 4096;
 
+// Whether 2-byte inputs take 64 x 64 wave tiles, of which there would be `wide` instead of `tall`
+// of 64 x 32: they have to fill the chip twice over (kFullUnits is four waves a SIMD, they run
+// two; 256^3 x 200 34.5 us against 32.4), be fewer by a quarter at least, or nothing is read less
+// often, and run long enough to hide their loads with two waves: the mean K by work at least
+// 128, two stages (128^3 x 8192 201 us either way, 144^3 x 4096 192 against 205).
+static bool wide_pays(const WorkItem* items, int64_t n_items, int64_t wide, int64_t tall) {
+    if (wide < kFullUnits || 4 * wide > 3 * tall) return false;
+    double work = 0, work_k = 0;
+    for (int64_t i = 0; i < n_items; ++i) {
+        const WorkItem& w = items[i];
+        const double f = (double)std::min(w.mlim, kVariantTM[w.variant]) * std::min(w.nlim, kVariantTN[w.variant]) * w.k;
+        work += f;
+        work_k += f * w.k;
+    }
+    return work_k >= 128.0 * work;
+}
+
 static int wave_cap(const WorkItem* items, int64_t n_items, int elt, int64_t* n_units) {
     int cap = first_cap(elt);
+    if (elt == 2) {
+        const int64_t wide = count_units(items, n_items, kWideCap);
+        if (wide_pays(items, n_items, wide, count_units(items, n_items, cap))) {
+            *n_units = wide;
+            return kWideCap;
+        }
+    }
     while ((*n_units = count_units(items, n_items, cap)) < kFullUnits && cap + 1 < kCaps) ++cap;
     return cap;
 }
@@ -629,7 +668,7 @@ static kami_status upload(const void* host, size_t bytes, void** dev) {
 struct DeviceQueue {
     void* mem = nullptr;
     int64_t n_items = 0, n_units = 0;
-    int tall = 0;
+    int cap = 0;
     const WorkItem* items() const { return static_cast<const WorkItem*>(mem); }
     const WaveUnit* units() const { return reinterpret_cast<const WaveUnit*>(items() + n_items); }
 };
@@ -646,7 +685,7 @@ static kami_status upload_queue(const std::vector<WorkItem>& items, int elt, Dev
     build_units(items.data(), n, cap, n_units, reinterpret_cast<WaveUnit*>(host.get() + item_bytes));
     q->n_items = n;
     q->n_units = n_units;
-    q->tall = cap == 0;
+    q->cap = cap;
     return upload(host.get(), bytes, &q->mem);
 }
 
@@ -803,7 +842,7 @@ kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count, i
                     if (q.mem) (void)hipFree(q.mem);
                     break;
                 }
-                BatchArgs a{q.items(), q.units(), q.n_units, o.alpha, 0.0, q.tall};
+                BatchArgs a{q.items(), q.units(), q.n_units, o.alpha, 0.0, q.cap};
                 e = launch_batched(precision, a, plan->b_kn, s);  // warm-up
                 if (e == hipSuccess) e = hipEventRecord(e0, s);
                 for (int rep = 0; rep < 3 && e == hipSuccess; ++rep)
@@ -854,7 +893,7 @@ kami_status kami_batched_execute(kami_batched_plan* plan, void* stream) {
     if (!plan) return KAMI_EINVAL;
     hipStream_t s = (hipStream_t)stream;
     const BatchArgs a{plan->queue.items(), plan->queue.units(), plan->queue.n_units, plan->alpha, plan->beta,
-                      plan->queue.tall};
+                      plan->queue.cap};
     const hipError_t e = launch_batched(plan->prec, a, plan->b_kn, s);
     if (e != hipSuccess) return hip_fail(e);
     return KAMI_OK;
@@ -926,7 +965,7 @@ kami_status kami_batched_gemm_static(const kami_problem* probs, int64_t count, i
                                   hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return hip_fail(e);
     const WorkItem* d_items = reinterpret_cast<const WorkItem*>(base);
-    BatchArgs a{d_items, reinterpret_cast<const WaveUnit*>(d_items + n_items), n_units, o.alpha, o.beta, cap == 0};
+    BatchArgs a{d_items, reinterpret_cast<const WaveUnit*>(d_items + n_items), n_units, o.alpha, o.beta, cap};
     e = launch_batched(precision, a, b_kn, s);
     if (e != hipSuccess) return hip_fail(e);
     return KAMI_OK;
