@@ -8,7 +8,7 @@
 //   * problems carry their own {m, n, k, lda, ldb, ldc, A, B, C} (the kami_problem array);
 //   * every problem is cut into output tiles; a tile is one 64-byte queue entry holding
 //     its own operand pointers, strides, extents and variant (WorkItem);
-//   * an entry is cut into wave tiles of up to 32 x 32 (2-byte inputs: 64 x 64; WaveUnit, 8
+//   * an entry is cut into wave tiles of up to 64 x 32 (2-byte inputs: 64 x 64; WaveUnit, 8
 //     bytes each).  A wave computes one of them alone, staged through LDS of its own, so there is no barrier
 //     and no shared counter: the hardware's dispatcher hands out the workgroups, longest
 //     problems first, and one wave's loads hide behind the products of the others;
@@ -21,8 +21,8 @@
 // M, N and K must be multiples of 16.
 //
 // What bounds it: 20000 problems of 16 to 256 (3.58 GB FP64, 1.19 GB FP16 with FP32 C) run
-// in 807 us and 275 us, 4.4 and 4.3 TB/s of the algorithmic bytes; the matrix pipes are
-// 57 % busy in FP64, whose HBM traffic (3.81 GB, 4.7 TB/s) runs near the rate of a copy (4.8).
+// in 788 us and 275 us, 4.5 and 4.3 TB/s of the algorithmic bytes; FP64 moves 3.81 GB, at the rate
+// of a copy (4.8 TB/s).
 // The persistent form this replaced (workgroups popping tiles of up to 128 x 128 from an atomic
 // counter, LDS stages shared by four waves, one barrier a stage, a one-thread kernel to clear
 // the counter) took 1027 us and 398 us: two workgroups a CU and their barriers left too little
@@ -57,7 +57,7 @@ constexpr int kQueueShift = 3;
 // Tile variants.  Index = variant id stored in the work items.
 //   0: 64 x 64 tile      1: 32 x 32 tile      2: 64 x 64 tile, wave tiles of 16 x 32
 //   3: 128 x 64 tile     4: 128 x 128 tile (FP64)     5: 64 x 128 tile (FP64)
-// Wave tiles are 32 x 32 except where noted.
+// Wave tiles are as large as kCapM and kCapN allow except where noted.
 constexpr int kVariants = 6;
 static_assert(kVariants == kBatchedVariants, "tuning-cache variant range");
 static const int kVariantTM[kVariants] = {64, 32, 64, 128, 128, 64};
@@ -75,16 +75,14 @@ struct WaveUnit {
     uint8_t ra, ca, im, jn;
 };
 static_assert(sizeof(WaveUnit) == 8, "wave unit layout");
-// Wave tiles in atoms, largest first; a precision starts at first_cap.  For 2-byte inputs the
-// rate at which a CU's L1 takes lines sets the time, and a larger tile reads them less often:
-// 64 x 64 where wide_pays (256^3 x 1024 115 us against 141 with 64 x 32, 320^3 x 1024 227
-// against 280, 20000 problems of 16 to 256 276 against 291), else 64 x 32 (20000 of 16 to 64
-// 21.7 against 23.8; the same of 16 to 256 304 with 32 x 32).  FP64 takes 32 x 32: 64 x 32 at two
-// waves a SIMD, 789 us against 808, leaves 60 against 59 for problems of 16 to 64 and twice the
-// registers.
+// Wave tiles in atoms, largest first.  A larger tile reads A's and B's lines less often, and
+// fewer of its waves fit a SIMD.  A precision starts at first_cap or, where larger_pays, at the
+// one before: 2-byte inputs at 64 x 32 or 64 x 64 (256^3 x 1024 141 us, 115; 320^3 x 1024 280, 227;
+// 20000 problems of 16 to 256 291, 276, and 304 with 32 x 32; 20000 of 16 to 64 21.7, 23.8), FP64
+// at 32 x 32 or 64 x 32 (20000 of 16 to 256 807, 788; 128^3 x 4096 387, 372; 256^3 x 1024 636, 609;
+// 64^3 x 8192 148, 155; with 64 x 64 169 there and 614 at 256^3).
 constexpr int kCaps = 5;
 static const int kCapM[kCaps] = {4, 4, 2, 1, 1}, kCapN[kCaps] = {4, 2, 2, 2, 1};
-constexpr int kWideCap = 0;
 constexpr int first_cap(int elt) { return elt == 8 ? 2 : 1; }
 constexpr int kWavesPerGroup = 4;
 constexpr int kXcds = 8;  // workgroup L runs on XCD L mod 8
@@ -360,7 +358,7 @@ static int bucket_of(const kami_problem& p) {
 // Prior variant of a bucket: the largest tile that the problem fills, following the
 // reference's choice of fewer, larger warps for larger sizes
 // (scripts/fp64_batched_GH200.sh:7-14).  The tile is what the queue counts and deals out;
-// every prior's wave tiles are 32 x 32.
+// every prior's wave tiles are the queue's largest.
 static int prior_variant(int prec, int bucket) {
     const int cm = bucket / 25, cn = (bucket / 5) % 5;
     if (cm == 0 && cn == 0) return 1;
@@ -394,15 +392,12 @@ static hipError_t launch_for(BatchArgs a, bool kn, hipStream_t s) {
     hipError_t e = hipSuccess;
     for (int64_t left = batched_groups(a.n_units); left > 0 && e == hipSuccess; left -= kMaxGroups) {
         const dim3 grid((unsigned)std::min(left, kMaxGroups));
-        if constexpr (sizeof(typename AT::in_t) == 2) {
-            if (a.cap == kWideCap)
-                launch_kernel<AT, 4, 4>(a, kn, grid, s);
-            else if (kCapM[a.cap] == 4)
-                launch_kernel<AT, 4, 2>(a, kn, grid, s);
-            else
-                launch_kernel<AT, 2, 2>(a, kn, grid, s);
-        } else {
+        if (kCapM[a.cap] <= 2) {
             launch_kernel<AT, 2, 2>(a, kn, grid, s);
+        } else if (kCapN[a.cap] == 2) {
+            launch_kernel<AT, 4, 2>(a, kn, grid, s);
+        } else if constexpr (sizeof(typename AT::in_t) == 2) {
+            launch_kernel<AT, 4, 4>(a, kn, grid, s);
         }
         e = hipGetLastError();
         a.units += kMaxGroups * kWavesPerGroup;
@@ -483,13 +478,16 @@ static int64_t count_units(const WorkItem* items, int64_t n_items, int cap) {
 // 17.2 (and 17.2 with 2048 here); FP16 is bound by the launch itself there.
 constexpr int64_t kFullUnits = 4096;
 
-// Whether 2-byte inputs take 64 x 64 wave tiles, of which there would be `wide` instead of `tall`
-// of 64 x 32: they have to fill the chip twice over (kFullUnits is four waves a SIMD, they run
-// two; 256^3 x 200 34.5 us against 32.4), be fewer by a quarter at least, or nothing is read less
-// often, and run long enough to hide their loads with two waves: the mean K by work at least
-// 128, two stages (128^3 x 8192 201 us either way, 144^3 x 4096 192 against 205).
-static bool wide_pays(const WorkItem* items, int64_t n_items, int64_t wide, int64_t tall) {
-    if (wide < kFullUnits || 4 * wide > 3 * tall) return false;
+// Whether the wave tiles one size larger than first_cap's pay, of which there would be `larger`
+// instead of `first`: they have to fill the chip twice over (two waves a SIMD for 2-byte inputs,
+// three for FP64; FP16 256^3 x 200, 3200 of them, 34.5 us against 32.4, FP64 K x N 128^3 x 600,
+// 4800 of them, 68.0 against 63.7), be fewer by a quarter at least, or little
+// is read less often, and run long enough to hide their loads with fewer waves: a mean K by work of
+// 128 for 2-byte inputs (two stages; 128^3 x 8192 201 us either way, 144^3 x 4096 192 against
+// 205), 96 for FP64 (six; 96^3 x 4096 192 against 198, 64^3 x 8192 155 against 148).
+static bool larger_pays(const WorkItem* items, int64_t n_items, int elt, int64_t larger, int64_t first) {
+    if (larger < 2 * 1024 * (elt == 8 ? 3 : 2) || 4 * larger > 3 * first) return false;
+    const double least = elt == 8 ? 96 : 128;
     double work = 0, work_k = 0;
     for (int64_t i = 0; i < n_items; ++i) {
         const WorkItem& w = items[i];
@@ -497,17 +495,15 @@ static bool wide_pays(const WorkItem* items, int64_t n_items, int64_t wide, int6
         work += f;
         work_k += f * w.k;
     }
-    return work_k >= 128.0 * work;
+    return work_k >= least * work;
 }
 
 static int wave_cap(const WorkItem* items, int64_t n_items, int elt, int64_t* n_units) {
     int cap = first_cap(elt);
-    if (elt == 2) {
-        const int64_t wide = count_units(items, n_items, kWideCap);
-        if (wide_pays(items, n_items, wide, count_units(items, n_items, cap))) {
-            *n_units = wide;
-            return kWideCap;
-        }
+    const int64_t larger = count_units(items, n_items, cap - 1);
+    if (larger_pays(items, n_items, elt, larger, count_units(items, n_items, cap))) {
+        *n_units = larger;
+        return cap - 1;
     }
     while ((*n_units = count_units(items, n_items, cap)) < kFullUnits && cap + 1 < kCaps) ++cap;
     return cap;
