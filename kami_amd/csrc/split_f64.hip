@@ -336,12 +336,21 @@ __device__ inline uint32_t low_halves(uint32_t a, uint32_t b) { return __builtin
 __device__ inline uint32_t high_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
 
 // 1024 + field per binary16 half: a 10-bit field under the exponent of 1024 (and 2048 for the
-// field 1024, by the carry); subtracting 1024 + bias leaves the digit, exactly.
-__device__ inline uint32_t half_digits(uint32_t fields, float bias) {
-    typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
-    const _Float16 off = (_Float16)(-1024.0f - bias);
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2_t, fields) + h2_t{off, off});
+// field 1024, by the carry); adding `off` = -(1024 + bias) leaves the digit, exactly.
+typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+__device__ inline uint32_t half_digits(uint32_t fields, uint32_t off) {
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2_t, fields) + __builtin_bit_cast(h2_t, off));
 }
+__device__ constexpr uint32_t half_offset(float bias) {
+    const _Float16 off = (_Float16)(-1024.0f - bias);
+    return __builtin_bit_cast(uint32_t, h2_t{off, off});
+}
+
+// The fields of a NaN or an infinity are those of no value at all.  A row's chunk that holds
+// one therefore has NaN for its first digits, which reaches every element of C that it
+// takes part in: first() is what is added to those digits; the largest upper word of |x| over the
+// chunk says which it is.
+__device__ inline bool holds_nonfinite(uint32_t upper) { return upper >= 0x7ff00000u; }
 
 template <class SAT, int BETA, int S>
 struct PairDigits;
@@ -349,49 +358,58 @@ struct PairDigits;
 template <int S>
 struct PairDigits<AtomF16x32, 9, S> {
     static_assert(S == 6 || S == 7, "two triples and at most one digit more");
-    __device__ static inline void triple(uint32_t ua, uint32_t ub, uint32_t* d) {
+    using first_t = uint32_t;
+    __device__ static inline first_t first(uint32_t upper) {
+        return half_offset(512.0f) | (uint32_t)((int32_t)(upper + 0x00100000u) >> 31);
+    }
+    __device__ static inline void triple(uint32_t ua, uint32_t ub, uint32_t off, uint32_t* d) {
         typedef uint16_t us2_t __attribute__((ext_vector_type(2)));
         const us2_t hi = __builtin_bit_cast(us2_t, high_halves(ua, ub)) >> (uint16_t)2;
-        d[0] = half_digits(__builtin_bit_cast(uint32_t, hi) + 0x64006400u, 512.0f);
-        d[1] = half_digits((low_halves(ua >> 9, ub >> 9) & 0x01FF01FFu) | 0x64006400u, 256.0f);
-        d[2] = half_digits((low_halves(ua, ub) & 0x01FF01FFu) | 0x64006400u, 256.0f);
+        d[0] = half_digits(__builtin_bit_cast(uint32_t, hi) + 0x64006400u, off);
+        d[1] = half_digits((low_halves(ua >> 9, ub >> 9) & 0x01FF01FFu) | 0x64006400u, half_offset(256.0f));
+        d[2] = half_digits((low_halves(ua, ub) & 0x01FF01FFu) | 0x64006400u, half_offset(256.0f));
     }
-    __device__ static inline void make(double a, double b, uint32_t (&d)[S]) {
+    __device__ static inline void make(double a, double b, first_t first, uint32_t (&d)[S]) {
         constexpr double M = kRound + (double)((512 << 18) + (256 << 9) + 256);
         const double ta = a + M, tb = b + M;
-        triple(low_word(ta), low_word(tb), d);
+        triple(low_word(ta), low_word(tb), first, d);
         const double ra = a - (ta - M), rb = b - (tb - M);  // exact
         constexpr double W = 134217728.0;  // 2^27
         const double sa = __builtin_fma(ra, W, M), sb = __builtin_fma(rb, W, M);
-        triple(low_word(sa), low_word(sb), d + 3);
+        triple(low_word(sa), low_word(sb), half_offset(512.0f), d + 3);
         if constexpr (S == 7) {
             constexpr double M1 = kRound + 512.0;
             const double qa = __builtin_fma(ra, W, -(sa - M)), qb = __builtin_fma(rb, W, -(sb - M));
             const uint32_t f = low_halves(low_word(__builtin_fma(qa, 512.0, M1)), low_word(__builtin_fma(qb, 512.0, M1)));
-            d[6] = half_digits(f + 0x64006400u, 512.0f);
+            d[6] = half_digits(f + 0x64006400u, half_offset(512.0f));
         }
     }
 };
 
 template <>
 struct PairDigits<AtomBF16x32, 8, 7> {
+    using first_t = float;
+    __device__ static inline first_t first(uint32_t upper) {
+        return holds_nonfinite(upper) ? __builtin_nanf("") : -128.0f;
+    }
     // |digit| <= 256 is exact in bfloat16: the upper half of its float
     __device__ static inline uint32_t pack(float a, float b) {
         return high_halves(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
     }
-    __device__ static inline void triple(uint32_t ua, uint32_t ub, uint32_t* d) {
+    // (`off` is added to the second digits: the first need no bias)
+    __device__ static inline void triple(uint32_t ua, uint32_t ub, float off, uint32_t* d) {
         d[0] = pack((float)((int32_t)ua >> 16), (float)((int32_t)ub >> 16));
-        d[1] = pack((float)((ua >> 8) & 255u) - 128.0f, (float)((ub >> 8) & 255u) - 128.0f);
+        d[1] = pack((float)((ua >> 8) & 255u) + off, (float)((ub >> 8) & 255u) + off);
         d[2] = pack((float)(ua & 255u) - 128.0f, (float)(ub & 255u) - 128.0f);
     }
-    __device__ static inline void make(double a, double b, uint32_t (&d)[7]) {
+    __device__ static inline void make(double a, double b, first_t first, uint32_t (&d)[7]) {
         constexpr double M = kRound + (double)((128 << 8) + 128);
         const double ta = a + M, tb = b + M;
-        triple(low_word(ta), low_word(tb), d);
+        triple(low_word(ta), low_word(tb), first, d);
         const double ra = a - (ta - M), rb = b - (tb - M);  // exact
         constexpr double W = 16777216.0;  // 2^24
         const double sa = __builtin_fma(ra, W, M), sb = __builtin_fma(rb, W, M);
-        triple(low_word(sa), low_word(sb), d + 3);
+        triple(low_word(sa), low_word(sb), -128.0f, d + 3);
         const double qa = __builtin_fma(ra, W, -(sa - M)), qb = __builtin_fma(rb, W, -(sb - M));
         d[6] = pack((float)(int32_t)low_word(__builtin_fma(qa, 256.0, kRound)),
                     (float)(int32_t)low_word(__builtin_fma(qb, 256.0, kRound)));
@@ -520,10 +538,13 @@ split_stream_kernel(SplitArgs args, int64_t count) {
     // Exponent e with |x| < 2^e over the row's 32 values of the chunk: the largest upper
     // word of |x| (monotonic in |x|) over the thread's 8 values and the row's 4 threads (one
     // DPP quad), completed with all-ones lower bits, so frexp also covers subnormal rows.
+    using Digits = PairDigits<SAT, G::BETA, G::S>;
+    typename Digits::first_t first_digit;  // of the chunk taken from x
     auto chunk_exp = [&]() {
         uint32_t h = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) h = max(h, max(x[i][1] & 0x7fffffffu, x[i][3] & 0x7fffffffu));
+        first_digit = Digits::first(h);  // of the thread's own values
         h = max(h, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h, 0xB1, 0xF, 0xF, false));  // quad_perm 1,0,3,2
         h = max(h, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h, 0x4E, 0xF, 0xF, false));  // quad_perm 2,3,0,1
         return __builtin_amdgcn_frexp_exp(__builtin_bit_cast(double, ((uint64_t)h << 32) | 0xffffffffu));
@@ -543,7 +564,7 @@ split_stream_kernel(SplitArgs args, int64_t count) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             uint32_t d[G::S];
-            PairDigits<SAT, G::BETA, G::S>::make(v[i][0], v[i][1], d);
+            Digits::make(v[i][0], v[i][1], first_digit, d);
 #pragma unroll
             for (int s = 0; s < G::S; ++s) plane[s][i] = d[s];
         }
@@ -725,23 +746,25 @@ split_pipe_kernel(SplitArgs args, int64_t count) {
     // Exponent e with |x| < 2^e over the row's 32 values of the chunk: the largest upper
     // word of |x| (monotonic in |x|) over the thread's 8 values and the row's 4 threads (one
     // DPP quad), completed with all-ones lower bits, so frexp also covers subnormal rows.
-    auto chunk_exp = [&](const u4_t (&x)[4]) {
+    using Digits = PairDigits<SAT, G::BETA, G::S>;
+    auto chunk_exp = [&](const u4_t (&x)[4], typename Digits::first_t& first) {
         uint32_t h = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) h = max(h, max(x[i][1] & 0x7fffffffu, x[i][3] & 0x7fffffffu));
         h = max(h, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h, 0xB1, 0xF, 0xF, false));  // quad_perm 1,0,3,2
         h = max(h, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h, 0x4E, 0xF, 0xF, false));  // quad_perm 2,3,0,1
+        first = Digits::first(h);
         return __builtin_amdgcn_frexp_exp(__builtin_bit_cast(double, ((uint64_t)h << 32) | 0xffffffffu));
     };
-    auto slice = [&](const u4_t (&x)[4], int e, unsigned char* plane0) {
+    auto slice = [&](const u4_t (&x)[4], int e, typename Digits::first_t first, unsigned char* plane0) {
         unsigned char* dst = plane0 + srow * G::ROWB + 2 * sk;
         u4_t plane[G::S];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const d2_t v = bitcast<d2_t>(x[i]);
             uint32_t d[G::S];
-            PairDigits<SAT, G::BETA, G::S>::make(__builtin_amdgcn_ldexp(v[0], 3 * G::BETA - e),
-                                                 __builtin_amdgcn_ldexp(v[1], 3 * G::BETA - e), d);
+            Digits::make(__builtin_amdgcn_ldexp(v[0], 3 * G::BETA - e),
+                         __builtin_amdgcn_ldexp(v[1], 3 * G::BETA - e), first, d);
 #pragma unroll
             for (int s = 0; s < G::S; ++s) plane[s][i] = d[s];
         }
@@ -765,13 +788,14 @@ split_pipe_kernel(SplitArgs args, int64_t count) {
 
         for (int c = 0; c < nch; ++c) {
             // ---- exponents and digit planes of this chunk ----
-            const int ea = chunk_exp(xa), eb = chunk_exp(xb);
+            typename Digits::first_t fa, fb;
+            const int ea = chunk_exp(xa, fa), eb = chunk_exp(xb, fb);
             if ((tid & 3) == 0) {
                 expo[srow] = ea;
                 expo[G::BM + srow] = eb;
             }
-            slice(xa, ea, smem);
-            slice(xb, eb, smem + G::SA_BYTES);
+            slice(xa, ea, fa, smem);
+            slice(xb, eb, fb, smem + G::SA_BYTES);
             // the next chunk is in flight during the products
             if (c + 1 < nch) {
                 pa += G::KC;
