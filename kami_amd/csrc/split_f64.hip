@@ -346,10 +346,10 @@ __device__ constexpr uint32_t half_offset(float bias) {
     return __builtin_bit_cast(uint32_t, h2_t{off, off});
 }
 
-// The fields of a NaN or an infinity are those of no value at all.  A row's chunk that holds
-// one therefore has NaN for its first digits, which reaches every element of C that it
-// takes part in: first() is what is added to those digits; the largest upper word of |x| over the
-// chunk says which it is.
+// The fields of a NaN or an infinity are those of no value at all, so where one is among the
+// values that a thread slices, the first (BF16: second) digits of them are NaN, which reaches
+// every element of C that they take part in: first() is what is added to those digits, and the
+// largest upper word of |x| over the values says which it is.
 __device__ inline bool holds_nonfinite(uint32_t upper) { return upper >= 0x7ff00000u; }
 
 template <class SAT, int BETA, int S>
@@ -360,7 +360,7 @@ struct PairDigits<AtomF16x32, 9, S> {
     static_assert(S == 6 || S == 7, "two triples and at most one digit more");
     using first_t = uint32_t;
     __device__ static inline first_t first(uint32_t upper) {
-        return half_offset(512.0f) | (uint32_t)((int32_t)(upper + 0x00100000u) >> 31);
+        return holds_nonfinite(upper) ? 0x7E007E00u : half_offset(512.0f);
     }
     __device__ static inline void triple(uint32_t ua, uint32_t ub, uint32_t off, uint32_t* d) {
         typedef uint16_t us2_t __attribute__((ext_vector_type(2)));
@@ -751,9 +751,9 @@ split_pipe_kernel(SplitArgs args, int64_t count) {
         uint32_t h = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) h = max(h, max(x[i][1] & 0x7fffffffu, x[i][3] & 0x7fffffffu));
+        first = Digits::first(h);  // of the thread's own values
         h = max(h, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h, 0xB1, 0xF, 0xF, false));  // quad_perm 1,0,3,2
         h = max(h, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)h, 0x4E, 0xF, 0xF, false));  // quad_perm 2,3,0,1
-        first = Digits::first(h);
         return __builtin_amdgcn_frexp_exp(__builtin_bit_cast(double, ((uint64_t)h << 32) | 0xffffffffu));
     };
     auto slice = [&](const u4_t (&x)[4], int e, typename Digits::first_t first, unsigned char* plane0) {
