@@ -34,6 +34,7 @@ struct SpmmArgs {
     const void* B;
     void* C;
     double alpha, beta;
+    uint32_t first;  // tile of the dispatch's first workgroup
 };
 
 // One workgroup per (block row i, tile of WN x 16 CT columns of C): wave (wk, wn) multiplies
@@ -96,7 +97,7 @@ spmm_kernel(SpmmArgs a) {
     // order, q = total / 8, r = total mod 8 (a bijection of [0, total)).
     const uint32_t L = blockIdx.x, total = gridDim.x;
     const uint32_t x = L % 8, q8 = total / 8, r8 = total % 8;
-    const uint32_t P = x * q8 + (x < r8 ? x : r8) + L / 8;
+    const uint32_t P = a.first + x * q8 + (x < r8 ? x : r8) + L / 8;
     const int i = (int)(P % (uint32_t)a.mb);             // block row of A and C
     const int nt = (int)(P / (uint32_t)a.mb) * G::TN;    // first column of the C tile
     const int wk = wave / G::WN, wn = wave % G::WN;
@@ -306,16 +307,23 @@ spmm_kernel(SpmmArgs a) {
     }
 }
 
+// A dispatch holds fewer than 2^32 work-items; more tiles take several.
 template <int BS, class AT, int WK, int WN, int CT>
-static hipError_t launch_form(const SpmmArgs& a, hipStream_t s) {
+static hipError_t launch_form(SpmmArgs a, hipStream_t s) {
     using G = SpmmGeom<BS, AT, false, WK, WN, CT>;
+    constexpr int64_t kMost = ((int64_t)1 << 31) / G::NT;
     const int64_t total = (int64_t)a.mb * (((int64_t)a.n + G::TN - 1) / G::TN);
-    const dim3 grid((unsigned)total), block(G::NT);
-    if (a.b_kn)
-        hipLaunchKernelGGL((spmm_kernel<BS, AT, true, WK, WN, CT>), grid, block, 0, s, a);
-    else
-        hipLaunchKernelGGL((spmm_kernel<BS, AT, false, WK, WN, CT>), grid, block, 0, s, a);
-    return hipGetLastError();
+    hipError_t e = hipSuccess;
+    for (int64_t first = 0; first < total && e == hipSuccess; first += kMost) {
+        const dim3 grid((unsigned)std::min(total - first, kMost)), block(G::NT);
+        a.first = (uint32_t)first;
+        if (a.b_kn)
+            hipLaunchKernelGGL((spmm_kernel<BS, AT, true, WK, WN, CT>), grid, block, 0, s, a);
+        else
+            hipLaunchKernelGGL((spmm_kernel<BS, AT, false, WK, WN, CT>), grid, block, 0, s, a);
+        e = hipGetLastError();
+    }
+    return e;
 }
 
 // Which form: enough workgroups share a row's stages among four waves; FP64 blocks of 32 as
@@ -373,6 +381,7 @@ kami_status kami_bsr_spmm(const kami_bsr* A, const void* B, int32_t n, int64_t l
         return KAMI_EINVAL;
     if ((ldb * ei) % 16 || ((uintptr_t)B % 16) || ((uintptr_t)C % eo)) return KAMI_EINVAL;
     if (A->nnzb > 0 && ((uintptr_t)A->vals % 16)) return KAMI_EINVAL;
+    // (fewer than 2^26 tiles of any form)
     if ((int64_t)A->mb * (((int64_t)n + 63) / 64) >= ((int64_t)1 << 24)) return KAMI_ENOTSUP;
     kami_status st = device_check();
     if (st != KAMI_OK) return st;
