@@ -160,7 +160,7 @@ def block_gemm(A, B, C=None, *, precision=None, partition="auto", ranks=0, b_lay
     """
     if stream is None:
         out = (_FAST or _fast()).block_gemm(
-            A, B, C, -1 if precision is None else precision, _part(partition), ranks,
+            A, B, C, precision, _part(partition), ranks,
             _layout(b_layout), iters, alpha, beta, slices, pipeline, 0)
         if out is not None:
             return out
@@ -517,7 +517,7 @@ def bsr_spgemm(A: BsrMatrix, B: BsrMatrix, *, precision=None, alpha=1.0, stream=
     if stream is None and type(A) is BsrMatrix and type(B) is BsrMatrix:
         out = (_FAST or _fast()).bsr_spgemm(
             A.mb, A.nb, A.bs, A.rowptr, A.colidx, A.vals, B.mb, B.nb, B.bs, B.rowptr, B.colidx,
-            B.vals, -1 if precision is None else precision, alpha)
+            B.vals, precision, alpha)
         if out is not None:
             return BsrMatrix(A.mb, B.nb, A.bs, *out)
     ws = spgemm_workspace(A, B)
@@ -537,7 +537,7 @@ def bsr_spmm(A: BsrMatrix, B, C=None, *, b_layout="nk", precision=None, alpha=1.
     if stream is None and type(A) is BsrMatrix:
         out = (_FAST or _fast()).bsr_spmm(
             A.mb, A.nb, A.bs, A.rowptr, A.colidx, A.vals, B, C, B_KN if b_layout == "kn" else B_NK,
-            -1 if precision is None else precision, alpha, beta)
+            precision, alpha, beta)
         if out is not None:
             return out
     import torch

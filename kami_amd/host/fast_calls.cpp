@@ -64,6 +64,18 @@ int precision_of(const at::Tensor& t) {
     }
 }
 
+// The wrapper's `precision` argument for a call on `t`; false when it is no precision
+bool precision_arg(PyObject* o, const at::Tensor& t, int* prec) {
+    if (o == Py_None) {
+        *prec = precision_of(t);
+        return true;
+    }
+    const long v = PyLong_AsLong(o);
+    if ((v == -1 && PyErr_Occurred()) || v < KAMI_PREC_F64 || v > KAMI_PREC_F64_SPLIT_I8) return false;
+    *prec = (int)v;
+    return true;
+}
+
 // Runs `f`; a torch error (no storage, out of memory) leaves the call to the wrapper
 template <class F>
 PyObject* plain(F f) {
@@ -78,7 +90,7 @@ PyObject* plain(F f) {
 
 PyObject* wrap(const at::Tensor& t) { return THPVariable_Wrap(t); }
 
-// block_gemm(A, B, C or None, precision or -1, partition, ranks, b_layout, iters, alpha, beta,
+// block_gemm(A, B, C or None, precision or None, partition, ranks, b_layout, iters, alpha, beta,
 //            slices, pipeline, tiled)
 PyObject* block_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return plain([&]() -> PyObject* {
@@ -88,9 +100,11 @@ PyObject* block_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t dim = A->dim();
         if ((dim != 2 && dim != 3) || B->dim() != dim) return nullptr;
         kami_gemm_desc d = {};
-        long v[8];
-        const int at_[8] = {3, 4, 5, 6, 7, 10, 11, 12};
-        for (int i = 0; i < 8; ++i) {
+        int prec;
+        if (!precision_arg(a[3], *A, &prec)) return nullptr;
+        long v[7];
+        const int at_[7] = {4, 5, 6, 7, 10, 11, 12};
+        for (int i = 0; i < 7; ++i) {
             v[i] = PyLong_AsLong(a[at_[i]]);
             if (v[i] == -1 && PyErr_Occurred()) return nullptr;
             if (v[i] < INT32_MIN || v[i] > INT32_MAX) return nullptr;
@@ -98,12 +112,11 @@ PyObject* block_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         d.alpha = PyFloat_AsDouble(a[8]);
         d.beta = PyFloat_AsDouble(a[9]);
         if (PyErr_Occurred()) return nullptr;
-        const int prec = v[0] == -1 ? precision_of(*A) : (int)v[0];
         at::ScalarType in, out;
         if (!types_of(prec, &in, &out)) return nullptr;
         const int64_t count = dim == 3 ? A->size(0) : 1;
         const int64_t m = A->size(dim - 2), k = A->size(dim - 1);
-        const bool kn = v[3] == KAMI_B_KN;
+        const bool kn = v[2] == KAMI_B_KN;
         const int64_t nn = B->size(kn ? dim - 1 : dim - 2);
         if (B->size(kn ? dim - 2 : dim - 1) != k || (dim == 3 && B->size(0) != count)) return nullptr;
         if (m > INT32_MAX || nn > INT32_MAX || k > INT32_MAX) return nullptr;
@@ -123,13 +136,13 @@ PyObject* block_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         d.n = (int32_t)nn;
         d.k = (int32_t)k;
         d.precision = prec;
-        d.partition = (int32_t)v[1];
-        d.ranks = (int32_t)v[2];
-        d.b_layout = (int32_t)v[3];
-        d.iters = (int32_t)v[4];
-        d.slices = (int32_t)v[5];
-        d.pipeline = (int32_t)v[6];
-        const kami_status st = (v[7] ? g_lib.split_gemm : g_lib.block_gemm)(
+        d.partition = (int32_t)v[0];
+        d.ranks = (int32_t)v[1];
+        d.b_layout = (int32_t)v[2];
+        d.iters = (int32_t)v[3];
+        d.slices = (int32_t)v[4];
+        d.pipeline = (int32_t)v[5];
+        const kami_status st = (v[6] ? g_lib.split_gemm : g_lib.block_gemm)(
             &d, A->data_ptr(), B->data_ptr(), C.data_ptr(), count, 0, 0, 0, current_stream());
         if (st != KAMI_OK) return nullptr;
         if (a[2] == Py_None) return wrap(C);
@@ -166,17 +179,17 @@ bool bsr_of(PyObject* const* a, kami_bsr* X, const at::Tensor* (&t)[3]) {
     return true;
 }
 
-// bsr_spmm(6 of A, B, C or None, b_layout, precision or -1, alpha, beta)
+// bsr_spmm(6 of A, B, C or None, b_layout, precision or None, alpha, beta)
 PyObject* bsr_spmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return plain([&]() -> PyObject* {
         kami_bsr A;
         const at::Tensor* t[3];
         if (n != 12 || !bsr_of(a, &A, t)) return nullptr;
         const at::Tensor* B = gpu_tensor(a[6]);
-        const long lay = PyLong_AsLong(a[8]), p = PyLong_AsLong(a[9]);
+        const long lay = PyLong_AsLong(a[8]);
         const double alpha = PyFloat_AsDouble(a[10]), beta = PyFloat_AsDouble(a[11]);
-        if (PyErr_Occurred()) return nullptr;
-        const int prec = p == -1 ? precision_of(*t[2]) : (int)p;
+        int prec;
+        if (PyErr_Occurred() || !precision_arg(a[9], *t[2], &prec)) return nullptr;
         at::ScalarType in, out;
         if ((prec != KAMI_PREC_F64 && prec != KAMI_PREC_F16_F32 && prec != KAMI_PREC_BF16_F32) ||
             !types_of(prec, &in, &out))
@@ -203,16 +216,15 @@ PyObject* bsr_spmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
-// bsr_spgemm(6 of A, 6 of B, precision or -1, alpha) -> (rowptr, colidx, vals)
+// bsr_spgemm(6 of A, 6 of B, precision or None, alpha) -> (rowptr, colidx, vals)
 PyObject* bsr_spgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return plain([&]() -> PyObject* {
         kami_bsr A, B;
         const at::Tensor *ta[3], *tb[3];
         if (n != 14 || !bsr_of(a, &A, ta) || !bsr_of(a + 6, &B, tb)) return nullptr;
-        const long p = PyLong_AsLong(a[12]);
         const double alpha = PyFloat_AsDouble(a[13]);
-        if (PyErr_Occurred()) return nullptr;
-        const int prec = p == -1 ? precision_of(*ta[2]) : (int)p;
+        int prec;
+        if (PyErr_Occurred() || !precision_arg(a[12], *ta[2], &prec)) return nullptr;
         at::ScalarType in, out;
         if ((prec != KAMI_PREC_F64 && prec != KAMI_PREC_F16_F32 && prec != KAMI_PREC_BF16_F32) ||
             !types_of(prec, &in, &out))
