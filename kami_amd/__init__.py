@@ -141,13 +141,18 @@ def _fast():
                                "(or __graft_entry__.build())")
         import torch  # noqa: F401  (the extension links against it)
         from . import _fast_calls
-        L = lib()
-        _fast_calls.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (
-            L.kami_block_gemm, L.kami_split_gemm, L.kami_batched_execute, L.kami_bsr_spgemm_symbolic,
-            L.kami_bsr_spgemm_fill, L.kami_bsr_spgemm_numeric, L.kami_bsr_spmm,
-            L.kami_bsr_spgemm_structure)))
+        _fast_calls.bind(check, *_fast_entry_points())
         _FAST = _fast_calls
     return _FAST
+
+
+def _fast_entry_points():
+    """Addresses of the library's entry points in the order that bind takes them."""
+    L = lib()
+    return [ctypes.cast(f, ctypes.c_void_p).value for f in (
+        L.kami_block_gemm, L.kami_split_gemm, L.kami_batched_execute, L.kami_bsr_spgemm_symbolic,
+        L.kami_bsr_spgemm_fill, L.kami_bsr_spgemm_numeric, L.kami_bsr_spmm,
+        L.kami_bsr_spgemm_structure)]
 
 
 def block_gemm(A, B, C=None, *, precision=None, partition="auto", ranks=0, b_layout="nk",

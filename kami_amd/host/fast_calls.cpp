@@ -3,9 +3,11 @@
 //
 // Every function takes the call only when it is plain -- exact torch.Tensor objects on the
 // GPU, contiguous (or with unit column stride where the wrapper asks no more), of the right
-// types and shapes -- and returns None otherwise, also when the library refuses the call or
-// torch cannot give an address: the wrapper then runs its own checks, which name what is
-// wrong, and its own call.  Nothing is remembered between calls.
+// types and shapes -- and returns None otherwise, also when the library refuses the call
+// before it launches anything or torch cannot give an address: the wrapper then runs its own
+// checks, which name what is wrong, and its own call.  An error of the HIP runtime is raised
+// from here: work may have been enqueued by then, and a second call would do it twice
+// (with beta != 0, add twice).  Nothing is remembered between calls.
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
@@ -27,7 +29,20 @@ struct Lib {
     decltype(&kami_bsr_spmm) spmm;
     decltype(&kami_bsr_spgemm_structure) structure;
 } g_lib;
+PyObject* g_check = nullptr;  // check(status, what), raises for a status that is no success
 bool g_bound = false;
+
+// What a library call's status means for the native call
+struct Refused : std::exception {};      // left to the wrapper
+struct PythonError : std::exception {};  // raised: a Python error is set
+
+void done(kami_status st, const char* what) {
+    if (st == KAMI_OK) return;
+    if (st != KAMI_EHIP) throw Refused();
+    PyObject* r = PyObject_CallFunction(g_check, "is", (int)st, what);
+    Py_XDECREF(r);
+    throw PythonError();
+}
 
 void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
@@ -82,6 +97,8 @@ PyObject* plain(F f) {
     if (!g_bound) Py_RETURN_NONE;
     try {
         if (PyObject* r = f()) return r;
+    } catch (const PythonError&) {
+        if (PyErr_Occurred()) return nullptr;
     } catch (const std::exception&) {
     }
     if (PyErr_Occurred()) PyErr_Clear();
@@ -144,7 +161,7 @@ PyObject* block_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         d.pipeline = (int32_t)v[5];
         const kami_status st = (v[6] ? g_lib.split_gemm : g_lib.block_gemm)(
             &d, A->data_ptr(), B->data_ptr(), C.data_ptr(), count, 0, 0, 0, current_stream());
-        if (st != KAMI_OK) return nullptr;
+        done(st, v[6] ? "kami_split_gemm" : "kami_block_gemm");
         if (a[2] == Py_None) return wrap(C);
         Py_INCREF(a[2]);
         return a[2];
@@ -155,8 +172,8 @@ PyObject* block_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* batched_execute(PyObject*, PyObject* arg) {
     return plain([&]() -> PyObject* {
         void* plan = PyLong_AsVoidPtr(arg);
-        if (!plan || g_lib.batched_execute(static_cast<kami_batched_plan*>(plan), current_stream()) != KAMI_OK)
-            return nullptr;
+        if (!plan) return nullptr;
+        done(g_lib.batched_execute(static_cast<kami_batched_plan*>(plan), current_stream()), "kami_batched_execute");
         Py_RETURN_TRUE;
     });
 }
@@ -207,9 +224,8 @@ PyObject* bsr_spmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
                 return nullptr;
             C = *c;
         }
-        if (g_lib.spmm(&A, B->data_ptr(), (int32_t)nn, B->stride(0), (int32_t)lay, C.data_ptr(), C.stride(0),
-                       prec, alpha, beta, current_stream()) != KAMI_OK)
-            return nullptr;
+        done(g_lib.spmm(&A, B->data_ptr(), (int32_t)nn, B->stride(0), (int32_t)lay, C.data_ptr(), C.stride(0),
+                        prec, alpha, beta, current_stream()), "kami_bsr_spmm");
         if (a[7] == Py_None) return wrap(C);
         Py_INCREF(a[7]);
         return a[7];
@@ -250,7 +266,7 @@ PyObject* bsr_spgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                      ws.data_ptr(), ws_bytes, stream)
                    : g_lib.symbolic(&A, &B, rp, &nnz, ws.data_ptr(), ws_bytes, stream);
         Py_END_ALLOW_THREADS
-        if (st != KAMI_OK) return nullptr;
+        done(st, "kami_bsr_spgemm_symbolic");
         if (fused) {  // the storage's size too, so that a saved C holds its own blocks only
             colidx.unsafeGetTensorImpl()->set_sizes_contiguous({nnz > 0 ? nnz : 1});
             colidx.storage().unsafeGetStorageImpl()->set_nbytes((size_t)(nnz > 0 ? nnz : 1) * 4);
@@ -258,10 +274,10 @@ PyObject* bsr_spgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
             colidx = at::empty({nnz > 0 ? nnz : 1}, ints);
         }
         int32_t* const ci = static_cast<int32_t*>(colidx.data_ptr());
-        if (!fused && g_lib.fill(&A, &B, rp, ci, ws.data_ptr(), ws_bytes, stream) != KAMI_OK) return nullptr;
+        if (!fused) done(g_lib.fill(&A, &B, rp, ci, ws.data_ptr(), ws_bytes, stream), "kami_bsr_spgemm_fill");
         at::Tensor vals = at::empty({nnz > 0 ? nnz : 1, A.bs, A.bs}, ta[2]->options().dtype(out));
-        if (nnz > 0 && g_lib.numeric(&A, &B, rp, ci, nnz, vals.data_ptr(), prec, alpha, stream) != KAMI_OK)
-            return nullptr;
+        if (nnz > 0)
+            done(g_lib.numeric(&A, &B, rp, ci, nnz, vals.data_ptr(), prec, alpha, stream), "kami_bsr_spgemm_numeric");
         if (nnz == 0) {
             colidx = colidx.slice(0, 0, 0);
             vals = vals.slice(0, 0, 0);
@@ -275,15 +291,15 @@ PyObject* bsr_spgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
-// bind(addresses of the eight entry points, in Lib's order)
+// bind(check, addresses of the eight entry points, in Lib's order)
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void* p[8];
-    if (n != 8) {
-        PyErr_SetString(PyExc_TypeError, "bind expects eight addresses");
+    if (n != 9 || !PyCallable_Check(a[0])) {
+        PyErr_SetString(PyExc_TypeError, "bind expects a callable and eight addresses");
         return nullptr;
     }
     for (int i = 0; i < 8; ++i) {
-        p[i] = PyLong_AsVoidPtr(a[i]);
+        p[i] = PyLong_AsVoidPtr(a[1 + i]);
         if (!p[i]) {
             if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "null entry point");
             return nullptr;
@@ -293,6 +309,8 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
                 (decltype(Lib::batched_execute))p[2], (decltype(Lib::symbolic))p[3],
                 (decltype(Lib::fill))p[4], (decltype(Lib::numeric))p[5], (decltype(Lib::spmm))p[6],
                 (decltype(Lib::structure))p[7]};
+    Py_INCREF(a[0]);
+    Py_XSETREF(g_check, a[0]);
     g_bound = true;
     Py_RETURN_NONE;
 }
