@@ -32,6 +32,15 @@ struct Lib {
 PyObject* g_check = nullptr;  // check(status, what), raises for a status that is no success
 bool g_bound = false;
 
+// Other Python threads run while the library is in a call or torch allocates: a launch waits
+// where a stream's queue is full.
+struct NoGil {
+    PyThreadState* const state = PyEval_SaveThread();
+    NoGil() = default;
+    NoGil(const NoGil&) = delete;
+    ~NoGil() { PyEval_RestoreThread(state); }
+};
+
 // What a library call's status means for the native call
 struct Refused : std::exception {};      // left to the wrapper
 struct PythonError : std::exception {};  // raised: a Python error is set
@@ -139,10 +148,7 @@ PyObject* block_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (m > INT32_MAX || nn > INT32_MAX || k > INT32_MAX) return nullptr;
         if (!is(*A, in, *A) || !is(*B, in, *A) || !A->is_contiguous() || !B->is_contiguous()) return nullptr;
         at::Tensor C;
-        if (a[2] == Py_None) {
-            C = dim == 3 ? at::empty({count, m, nn}, A->options().dtype(out))
-                         : at::empty({m, nn}, A->options().dtype(out));
-        } else {
+        if (a[2] != Py_None) {
             const at::Tensor* c = gpu_tensor(a[2]);
             if (!c || c->dim() != dim || !is(*c, out, *A) || !c->is_contiguous()) return nullptr;
             if (c->size(dim - 2) != m || c->size(dim - 1) != nn || (dim == 3 && c->size(0) != count))
@@ -159,8 +165,15 @@ PyObject* block_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         d.iters = (int32_t)v[3];
         d.slices = (int32_t)v[4];
         d.pipeline = (int32_t)v[5];
-        const kami_status st = (v[6] ? g_lib.split_gemm : g_lib.block_gemm)(
-            &d, A->data_ptr(), B->data_ptr(), C.data_ptr(), count, 0, 0, 0, current_stream());
+        kami_status st;
+        {
+            const NoGil released;
+            if (!C.defined())
+                C = dim == 3 ? at::empty({count, m, nn}, A->options().dtype(out))
+                             : at::empty({m, nn}, A->options().dtype(out));
+            st = (v[6] ? g_lib.split_gemm : g_lib.block_gemm)(
+                &d, A->data_ptr(), B->data_ptr(), C.data_ptr(), count, 0, 0, 0, current_stream());
+        }
         done(st, v[6] ? "kami_split_gemm" : "kami_block_gemm");
         if (a[2] == Py_None) return wrap(C);
         Py_INCREF(a[2]);
@@ -173,7 +186,12 @@ PyObject* batched_execute(PyObject*, PyObject* arg) {
     return plain([&]() -> PyObject* {
         void* plan = PyLong_AsVoidPtr(arg);
         if (!plan) return nullptr;
-        done(g_lib.batched_execute(static_cast<kami_batched_plan*>(plan), current_stream()), "kami_batched_execute");
+        kami_status st;
+        {
+            const NoGil released;
+            st = g_lib.batched_execute(static_cast<kami_batched_plan*>(plan), current_stream());
+        }
+        done(st, "kami_batched_execute");
         Py_RETURN_TRUE;
     });
 }
@@ -216,16 +234,20 @@ PyObject* bsr_spmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t nn = B->size(kn ? 1 : 0), rows = (int64_t)A.mb * A.bs;
         if (B->size(kn ? 0 : 1) != (int64_t)A.nb * A.bs || nn > INT32_MAX) return nullptr;
         at::Tensor C;
-        if (a[7] == Py_None) {
-            C = at::zeros({rows, nn}, B->options().dtype(out));
-        } else {
+        if (a[7] != Py_None) {
             const at::Tensor* c = gpu_tensor(a[7]);
             if (!c || c->dim() != 2 || !is(*c, out, *B) || c->size(0) != rows || c->size(1) != nn || c->stride(1) != 1)
                 return nullptr;
             C = *c;
         }
-        done(g_lib.spmm(&A, B->data_ptr(), (int32_t)nn, B->stride(0), (int32_t)lay, C.data_ptr(), C.stride(0),
-                        prec, alpha, beta, current_stream()), "kami_bsr_spmm");
+        kami_status st;
+        {
+            const NoGil released;
+            if (!C.defined()) C = at::zeros({rows, nn}, B->options().dtype(out));
+            st = g_lib.spmm(&A, B->data_ptr(), (int32_t)nn, B->stride(0), (int32_t)lay, C.data_ptr(), C.stride(0),
+                            prec, alpha, beta, current_stream());
+        }
+        done(st, "kami_bsr_spmm");
         if (a[7] == Py_None) return wrap(C);
         Py_INCREF(a[7]);
         return a[7];
@@ -253,31 +275,37 @@ PyObject* bsr_spgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const bool fused = A.mb <= kStructureRows && most <= (1 << 18);
         if (fused) ws_bytes += (size_t)A.mb * 4;
         const auto ints = ta[0]->options();
-        at::Tensor ws = at::empty({(int64_t)ws_bytes / 4}, ints);
-        at::Tensor rowptr = at::empty({(int64_t)A.mb + 1}, ints);
-        int32_t* const rp = static_cast<int32_t*>(rowptr.data_ptr());
-        void* const stream = current_stream();
+        at::Tensor rowptr, colidx, vals;
         int64_t nnz = 0;
         kami_status st;
-        at::Tensor colidx;
-        if (fused) colidx = at::empty({most}, ints);
-        Py_BEGIN_ALLOW_THREADS  // waits for the device
-        st = fused ? g_lib.structure(&A, &B, rp, static_cast<int32_t*>(colidx.data_ptr()), most, &nnz,
-                                     ws.data_ptr(), ws_bytes, stream)
-                   : g_lib.symbolic(&A, &B, rp, &nnz, ws.data_ptr(), ws_bytes, stream);
-        Py_END_ALLOW_THREADS
-        done(st, "kami_bsr_spgemm_symbolic");
-        if (fused) {  // the storage's size too, so that a saved C holds its own blocks only
-            colidx.unsafeGetTensorImpl()->set_sizes_contiguous({nnz > 0 ? nnz : 1});
-            colidx.storage().unsafeGetStorageImpl()->set_nbytes((size_t)(nnz > 0 ? nnz : 1) * 4);
-        } else {
-            colidx = at::empty({nnz > 0 ? nnz : 1}, ints);
+        const char* phase = "kami_bsr_spgemm_symbolic";
+        {
+            const NoGil released;
+            at::Tensor ws = at::empty({(int64_t)ws_bytes / 4}, ints);
+            rowptr = at::empty({(int64_t)A.mb + 1}, ints);
+            int32_t* const rp = static_cast<int32_t*>(rowptr.data_ptr());
+            void* const stream = current_stream();
+            if (fused) colidx = at::empty({most}, ints);
+            st = fused ? g_lib.structure(&A, &B, rp, static_cast<int32_t*>(colidx.data_ptr()), most, &nnz,
+                                         ws.data_ptr(), ws_bytes, stream)
+                       : g_lib.symbolic(&A, &B, rp, &nnz, ws.data_ptr(), ws_bytes, stream);
+            if (st == KAMI_OK && fused) {  // the storage's size too, so that a saved C holds its own blocks only
+                colidx.unsafeGetTensorImpl()->set_sizes_contiguous({nnz > 0 ? nnz : 1});
+                colidx.storage().unsafeGetStorageImpl()->set_nbytes((size_t)(nnz > 0 ? nnz : 1) * 4);
+            } else if (st == KAMI_OK) {
+                colidx = at::empty({nnz > 0 ? nnz : 1}, ints);
+                phase = "kami_bsr_spgemm_fill";
+                st = g_lib.fill(&A, &B, rp, static_cast<int32_t*>(colidx.data_ptr()), ws.data_ptr(), ws_bytes, stream);
+            }
+            if (st == KAMI_OK) {
+                vals = at::empty({nnz > 0 ? nnz : 1, A.bs, A.bs}, ta[2]->options().dtype(out));
+                phase = "kami_bsr_spgemm_numeric";
+                if (nnz > 0)
+                    st = g_lib.numeric(&A, &B, rp, static_cast<const int32_t*>(colidx.data_ptr()), nnz,
+                                       vals.data_ptr(), prec, alpha, stream);
+            }
         }
-        int32_t* const ci = static_cast<int32_t*>(colidx.data_ptr());
-        if (!fused) done(g_lib.fill(&A, &B, rp, ci, ws.data_ptr(), ws_bytes, stream), "kami_bsr_spgemm_fill");
-        at::Tensor vals = at::empty({nnz > 0 ? nnz : 1, A.bs, A.bs}, ta[2]->options().dtype(out));
-        if (nnz > 0)
-            done(g_lib.numeric(&A, &B, rp, ci, nnz, vals.data_ptr(), prec, alpha, stream), "kami_bsr_spgemm_numeric");
+        done(st, phase);
         if (nnz == 0) {
             colidx = colidx.slice(0, 0, 0);
             vals = vals.slice(0, 0, 0);
