@@ -130,19 +130,35 @@ def _stream_ptr(stream):
 _FAST = None
 
 
+class _NoFast:
+    """Stands in for the native call path where it cannot be loaded: every call is the
+    wrapper's own (ctypes), through the same library."""
+
+    @staticmethod
+    def _to_wrapper(*args):
+        return None
+
+    block_gemm = batched_execute = bsr_spmm = bsr_spgemm = _to_wrapper
+
+
 def _fast():
     """The native call path (host/fast_calls.cpp), bound to the loaded library.  Its functions
-    answer None to any call that is not plain, and the wrapper then checks and calls itself."""
+    answer None to any call that is not plain, and the wrapper then checks and calls itself.
+    Without the extension, or with one built against another torch, a warning says so once
+    and the wrappers make every call themselves."""
     global _FAST
     if _FAST is None:
-        path = os.path.join(_abi.HERE, "_fast_calls.so")
-        if not os.path.exists(path):
-            raise RuntimeError(f"{path} is missing: build it with `make -C kami_amd/csrc` "
-                               "(or __graft_entry__.build())")
         import torch  # noqa: F401  (the extension links against it)
-        from . import _fast_calls
-        _fast_calls.bind(check, *_fast_entry_points())
-        _FAST = _fast_calls
+        try:
+            from . import _fast_calls
+        except ImportError as e:
+            import warnings
+            warnings.warn(f"kami_amd: the native call path could not be loaded ({e}); small calls take "
+                          "longer. Build it with `make -C kami_amd/csrc`.", RuntimeWarning, stacklevel=3)
+            _FAST = _NoFast
+        else:
+            _fast_calls.bind(check, *_fast_entry_points())
+            _FAST = _fast_calls
     return _FAST
 
 
