@@ -29,14 +29,23 @@ namespace kami {
 constexpr int cmin(int a, int b) { return a < b ? a : b; }
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
-// KN_: B is stored K x N.  Its K rows go to LDS as they are and the reads turn them.  (Turning
+// B_: B is stored N x K, or K x N.  Then its K rows go to LDS as they are and the reads turn them.  (Turning
 // them in the writes instead cost eight 2-byte or two 8-byte conflicting stores a piece:
 // FP16 256^3 x 1024 183 us against 114.5, 224^3 x 2048 246 against 177, FP64 128^3 x 4096 431
 // against 376, 64 x 64 x 512 x 2048 273 against 226; N x K 111, 187, 335 and 209.)
-template <class AT, int BM_, int BN_, int BK_, int PM_, int PN_, int PK_, int KS_, bool KN_ = false>
+// Repeated products on one stage of 2-byte values are another matter: the reads are repeated
+// and the writes are not, and a turned fragment is two reads of half a row where a row of K
+// is one.  They turn the rows in the writes (TURNED): 64^3 x 1024, 400 times, BF16 104 us
+// against 164, 128 x 128 x 32 x 1024, 279 times, 158 against 238, 256^3 x 1024, 8 times, 318
+// against 403.
+enum BStage : int { kStageNK, kStageRows, kStageTurned };
+template <class AT, int BM_, int BN_, int BK_, int PM_, int PN_, int PK_, int KS_, int B_ = kStageNK>
 struct BlockGeom {
-    static constexpr bool KN = KN_;
-    using AsKN = BlockGeom<AT, BM_, BN_, BK_, PM_, PN_, PK_, KS_, true>;
+    static constexpr bool SRC_KN = B_ != kStageNK;    // K rows in memory
+    static constexpr bool KN = B_ == kStageRows;      // K rows in LDS
+    static constexpr bool TURNED = B_ == kStageTurned;
+    using AsKN = BlockGeom<AT, BM_, BN_, BK_, PM_, PN_, PK_, KS_, kStageRows>;
+    using AsTurned = BlockGeom<AT, BM_, BN_, BK_, PM_, PN_, PK_, KS_, kStageTurned>;
     static constexpr int BM = BM_, BN = BN_, BK = BK_;
     static constexpr int PM = PM_, PN = PN_, PK = PK_, KS = KS_;
     static constexpr int WAVES = PM * PN * PK;
@@ -96,17 +105,19 @@ struct BlockArgs {
 };
 
 // B fragment of column atom jn at K step ks of the K slice of wave (pn, pk), from the stage at
-// bb.  K x N: a lane's values are AT::KV rows of one column.  K step 8: the upper lane groups'
+// bb; kk is the lane's byte offset in a row of K.  (The address is formed as the fragments of A
+// are: with the row's part first, the 256^3 resident forms kept an address per fragment and
+// spilled 60 registers, FP16 x 1024, 8 times, 246 -> 596 us.)  K x N rows: a lane's values are AT::KV rows of one column.  K step 8: the upper lane groups'
 // values are not used, and they read the lower groups' rows so as to stay in the stage.
 template <class AT, class G>
 __device__ __forceinline__ typename AT::frag_t stage_b_fragment(const unsigned char* bb, int lane, int pn,
-                                                                int pk, int jn, int ks) {
+                                                                int pk, int jn, int ks, int kk) {
     using frag_t = typename AT::frag_t;
-    const int col = pn * G::TN + lane % G::DIM, grp = lane / G::DIM;
     if constexpr (!G::KN) {
-        const int kk = (pk * G::KSW + AT::KV * grp + ks * AT::KSTEP) * G::ELT;
-        return bitcast<frag_t>(load_raw<AT::FRAG_BYTES>(bb + (col + jn * G::DIM) * G::ROWB + kk));
+        return bitcast<frag_t>(load_raw<AT::FRAG_BYTES>(
+            bb + (pn * G::TN + jn * G::DIM + (lane % G::DIM)) * G::ROWB + kk));
     } else {
+        const int col = pn * G::TN + lane % G::DIM, grp = lane / G::DIM;
         constexpr int GROUPS = cmin(64 / G::DIM, AT::KSTEP / AT::KV);
         const unsigned char* q = bb + G::krow(pk * G::KSW + AT::KV * (grp % GROUPS));
         const int step = G::krow(ks * AT::KSTEP) + jn * G::DIM * G::ELT;
@@ -135,14 +146,17 @@ __device__ __forceinline__ typename AT::frag_t stage_b_fragment(const unsigned c
 // 4.2 us, 4.5 with 3), and so do the 2D instances (BF16 64^3 51 us, 58).
 template <class AT, class G>
 constexpr int waves_per_simd() {
-    if (G::ELT == 8 || G::PN > 1 || G::PK > 1 || G::BM < 64) return 8;
+    if (G::ELT == 8 || G::PN > 1 || G::PK > 1 || G::BM < 64 || G::TURNED) return 8;
     const int want = G::IM * G::JN * G::NACC >= 128 ? 2 : 3, own = (G::WAVES + 3) / 4;
     return (want + own - 1) / own * own;  // whole workgroups
 }
 
 // KFENCE > 0: a scheduling fence after every KFENCE K steps of a stage, so the
 // compiler does not hoist the B fragment loads of a whole long stage ahead of the MFMAs
-// (used by the resident forms, whose single stage covers all of K).
+// (used by the resident forms, whose single stage covers all of K).  With 2 the wave's rows of A
+// are loaded once B's have arrived: the address unit takes their fragments four lanes a
+// clock, and B, which every wave waits for, would queue behind them (256^3 x 1024, twice,
+// 119 us against 127; 192^3 x 2048 113 against 116).
 //
 // SP > 1: the wave tiles of the full BN columns do not fit the register file, so the
 // problem's columns are computed in SP passes of G::BN = BN / SP columns each (B rows and
@@ -175,7 +189,7 @@ block_gemm_kernel(BlockArgs args) {
     for (int sp = 0; sp < SP; ++sp) {
     if (sp > 0) __syncthreads();  // the previous pass is done with LDS
     const in_t* __restrict__ B = reinterpret_cast<const in_t*>(args.B) + prob * args.sb +
-                                 (int64_t)sp * G::BN * (G::KN ? 1 : ldb);
+                                 (int64_t)sp * G::BN * (G::SRC_KN ? 1 : ldb);
     out_t* __restrict__ C = reinterpret_cast<out_t*>(args.C) + prob * args.sc + sp * G::BN;
 
     accv_t acc[G::IM][G::JN];
@@ -202,7 +216,7 @@ block_gemm_kernel(BlockArgs args) {
                 }
             }
         }
-        if constexpr (!G::KN) {
+        if constexpr (!G::SRC_KN) {
             constexpr int CPR = G::KS / G::VE;
 #pragma unroll
             for (int i = 0; i < G::NBC; ++i) {
@@ -238,13 +252,20 @@ block_gemm_kernel(BlockArgs args) {
             }
         }
         unsigned char* bb = base + G::A_LDS;
-        constexpr int CPR = (G::KN ? G::BN : G::KS) / G::VE;
+        constexpr int CPR = (G::SRC_KN ? G::BN : G::KS) / G::VE;
 #pragma unroll
         for (int i = 0; i < G::NBC; ++i) {
             const int c = tid + i * G::NT;
             if (c < G::CB) {
                 const int r = c / CPR, cc = c % CPR;
-                store_raw<16>(bb + (G::KN ? G::krow(r) : r * G::ROWB) + cc * 16, stB[i]);
+                if constexpr (G::TURNED) {
+                    const in_t* e = reinterpret_cast<const in_t*>(&stB[i]);
+#pragma unroll
+                    for (int q = 0; q < G::VE; ++q)
+                        *reinterpret_cast<in_t*>(bb + (cc * G::VE + q) * G::ROWB + r * G::ELT) = e[q];
+                } else {
+                    store_raw<16>(bb + (G::KN ? G::krow(r) : r * G::ROWB) + cc * 16, stB[i]);
+                }
             }
         }
     };
@@ -289,7 +310,7 @@ block_gemm_kernel(BlockArgs args) {
             if constexpr (AT::NSUB == 1) {
 #pragma unroll
                 for (int jn = 0; jn < G::JN; ++jn) {
-                    const frag_t bf = stage_b_fragment<AT, G>(bb, lane, pn, pk, jn, ks);
+                    const frag_t bf = stage_b_fragment<AT, G>(bb, lane, pn, pk, jn, ks, kk);
 #pragma unroll
                     for (int im = 0; im < G::IM; ++im) AT::mma(acc[im][jn], af[im], bf);
                 }
@@ -299,7 +320,7 @@ block_gemm_kernel(BlockArgs args) {
                 frag_t bf[G::JN];
 #pragma unroll
                 for (int jn = 0; jn < G::JN; ++jn)
-                    bf[jn] = stage_b_fragment<AT, G>(bb, lane, pn, pk, jn, ks);
+                    bf[jn] = stage_b_fragment<AT, G>(bb, lane, pn, pk, jn, ks, kk);
 #pragma unroll
                 for (int e = 0; e < AT::NSUB; ++e)
 #pragma unroll
@@ -313,10 +334,12 @@ block_gemm_kernel(BlockArgs args) {
     };
 
     // ---- main loop ----
+    constexpr bool A_LATE = KFENCE == 2;
     load_stage(0);
-    load_a(0, a_cur);
+    if constexpr (!A_LATE) load_a(0, a_cur);
     write_stage(0);
     __syncthreads();
+    if constexpr (A_LATE) load_a(0, a_cur);
     if constexpr (G::NS == 1) {
         for (int it = 0; it < args.iters; ++it) compute(0);
     } else {
@@ -414,15 +437,35 @@ block_gemm_kernel(BlockArgs args) {
     }  // column passes
 }
 
+template <class AT, class G, int KFENCE, int SP>
+hipError_t launch_block_gemm_as(const BlockArgs& args, int64_t count, hipStream_t stream) {
+    hipLaunchKernelGGL((block_gemm_kernel<AT, G, KFENCE, SP>), dim3((unsigned)count), dim3(G::NT), 0, stream,
+                       args);
+    return hipGetLastError();
+}
+
+// Repetitions from which 2-byte K x N rows in one stage are turned in the writes (64^3 x 2048
+// in 1D, 8 times 0.93 of the time with rows turned by the reads, 16 times 0.76; 128^3 x 2048
+// 8 times 1.07, 16 times 0.89; several stages are written again for every repetition and stay
+// rows: 128 x 128 x 512 x 256, 64 times, 0.41 of the time with turned writes).
+constexpr int kTurnIters = 8;
+
 template <class AT, class G, int KFENCE = 0, int SP = 1>
 hipError_t launch_block_gemm(const BlockArgs& args, int64_t count, hipStream_t stream) {
-    if (args.b_kn)
-        hipLaunchKernelGGL((block_gemm_kernel<AT, typename G::AsKN, KFENCE, SP>), dim3((unsigned)count),
-                           dim3(G::NT), 0, stream, args);
-    else
-        hipLaunchKernelGGL((block_gemm_kernel<AT, G, KFENCE, SP>), dim3((unsigned)count), dim3(G::NT), 0,
-                           stream, args);
-    return hipGetLastError();
+    if constexpr (G::ELT == 2 && G::NS == 1)
+        if (args.b_kn && args.iters >= kTurnIters)
+            return launch_block_gemm_as<AT, typename G::AsTurned, KFENCE, SP>(args, count, stream);
+    if (args.b_kn) return launch_block_gemm_as<AT, typename G::AsKN, KFENCE, SP>(args, count, stream);
+    return launch_block_gemm_as<AT, G, KFENCE, SP>(args, count, stream);
+}
+
+// A resident form, which is taken for iters > 1 only, and turns in the writes for any: with
+// rows in LDS the instances of 16 waves and FP64's spill (FP16 256^3 x 2048 in 16 waves, 4 times,
+// 0.91 of the time with rows; in 8 waves 1.34, but 16 waves are the faster form).
+template <class AT, class G>
+hipError_t launch_resident(const BlockArgs& args, int64_t count, hipStream_t stream) {
+    if (args.b_kn) return launch_block_gemm_as<AT, typename G::AsTurned, 2, 1>(args, count, stream);
+    return launch_block_gemm_as<AT, G, 2, 1>(args, count, stream);
 }
 
 }  // namespace kami

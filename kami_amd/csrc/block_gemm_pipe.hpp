@@ -94,7 +94,7 @@ block_gemm_pipe_kernel(BlockArgs args, int64_t count) {
             frag_t bf[G::JN];
 #pragma unroll
             for (int jn = 0; jn < G::JN; ++jn)
-                bf[jn] = stage_b_fragment<AT, G>(bb, lane, pn, 0, jn, ks);
+                bf[jn] = stage_b_fragment<AT, G>(bb, lane, pn, 0, jn, ks, kk);
 #pragma unroll
             for (int e = 0; e < AT::NSUB; ++e)
 #pragma unroll

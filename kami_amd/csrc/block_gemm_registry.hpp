@@ -85,7 +85,7 @@ void add_resident_instance(std::vector<BlockInstance>& v, int ranks) {
     using G = BlockGeom<AT, BM, BN, BK, PM, PN, 1, BK>;
     static_assert(G::NS == 1, "whole K in one stage");
     v.push_back(BlockInstance{PREC, BM, BN, BK, PN == 1 ? 1 : 2, ranks, PM, PN, 1, BK, G::NT,
-                              G::LDS, AT::KSTEP, &launch_block_gemm<AT, G, 2>, 1, 1, 1});
+                              G::LDS, AT::KSTEP, &launch_resident<AT, G>, 1, 1, 1});
 }
 
 // Largest prefetch depth <= want that divides the stage count.
