@@ -61,6 +61,10 @@ struct BlockGeom {
     static constexpr int VE = 16 / ELT;  // elements per 16-byte staging chunk
     static constexpr bool A_PRIV = (PN == 1);
     static constexpr int NBUF = (NS == 1) ? 1 : 2;
+    // FP64 over several stages: the bound of a piece that is always within it is left out, since
+    // the loads and writes of a stage are otherwise a branch each (3D 128^3 x 1024 115 us with
+    // the branches, 102 without; a single stage is faster with them, 64^3 in 1D 26.2, 27.6)
+    static constexpr bool WHOLE = ELT == 8 && NS > 1;
     static constexpr int ROWB = lds_row_bytes(KS * ELT, AT::FRAG_BYTES);  // conflict-free reads
     static constexpr int A_LDS = A_PRIV ? 0 : BM * ROWB;
     // K x N: bytes between staged K rows, and the extra bytes after every eight of 2-byte
@@ -210,7 +214,7 @@ block_gemm_kernel(BlockArgs args) {
 #pragma unroll
             for (int i = 0; i < G::NA; ++i) {
                 const int c = tid + i * G::NT;
-                if (c < G::CA) {
+                if ((G::WHOLE && G::CA % G::NT == 0) || c < G::CA) {
                     const int r = c / CPR, cc = c % CPR;
                     stA[i] = load_raw<16>(A + r * lda + k0 + cc * G::VE);
                 }
@@ -221,7 +225,7 @@ block_gemm_kernel(BlockArgs args) {
 #pragma unroll
             for (int i = 0; i < G::NBC; ++i) {
                 const int c = tid + i * G::NT;
-                if (c < G::CB) {
+                if ((G::WHOLE && G::CB % G::NT == 0) || c < G::CB) {
                     const int r = c / CPR, cc = c % CPR;
                     stB[i] = load_raw<16>(B + r * ldb + k0 + cc * G::VE);
                 }
@@ -231,7 +235,7 @@ block_gemm_kernel(BlockArgs args) {
 #pragma unroll
             for (int i = 0; i < G::NBC; ++i) {
                 const int c = tid + i * G::NT;
-                if (c < G::CB) {
+                if ((G::WHOLE && G::CB % G::NT == 0) || c < G::CB) {
                     const int kr = c / CPR, jc = c % CPR;
                     stB[i] = load_raw<16>(B + (int64_t)(k0 + kr) * ldb + jc * G::VE);
                 }
@@ -245,7 +249,7 @@ block_gemm_kernel(BlockArgs args) {
 #pragma unroll
             for (int i = 0; i < G::NA; ++i) {
                 const int c = tid + i * G::NT;
-                if (c < G::CA) {
+                if ((G::WHOLE && G::CA % G::NT == 0) || c < G::CA) {
                     const int r = c / CPR, cc = c % CPR;
                     store_raw<16>(base + r * G::ROWB + cc * 16, stA[i]);
                 }
@@ -256,7 +260,7 @@ block_gemm_kernel(BlockArgs args) {
 #pragma unroll
         for (int i = 0; i < G::NBC; ++i) {
             const int c = tid + i * G::NT;
-            if (c < G::CB) {
+            if ((G::WHOLE && G::CB % G::NT == 0) || c < G::CB) {
                 const int r = c / CPR, cc = c % CPR;
                 if constexpr (G::TURNED) {
                     const in_t* e = reinterpret_cast<const in_t*>(&stB[i]);
@@ -452,8 +456,12 @@ constexpr int kTurnIters = 8;
 
 template <class AT, class G, int KFENCE = 0, int SP = 1>
 hipError_t launch_block_gemm(const BlockArgs& args, int64_t count, hipStream_t stream) {
-    if constexpr (G::ELT == 2 && G::NS == 1)
-        if (args.b_kn && args.iters >= kTurnIters)
+    // FP64 in one stage on a wave grid: a fragment's two rows are two reads, by every wave row
+    // (2D 64^3 x 1024 23.8 us turned in the writes, 25.8 in the reads; 1D, where a wave reads
+    // all of B either way, 29.2 and 26.3)
+    constexpr bool grid64 = G::ELT == 8 && G::PN > 1;
+    if constexpr (G::NS == 1 && (G::ELT == 2 || grid64))
+        if (args.b_kn && (grid64 || args.iters >= kTurnIters))
             return launch_block_gemm_as<AT, typename G::AsTurned, KFENCE, SP>(args, count, stream);
     if (args.b_kn) return launch_block_gemm_as<AT, typename G::AsKN, KFENCE, SP>(args, count, stream);
     return launch_block_gemm_as<AT, G, KFENCE, SP>(args, count, stream);
