@@ -223,13 +223,31 @@ static const Prior* small_batch_prior(const kami_gemm_desc* d, int64_t count) {
     return nullptr;
 }
 
-// The persistent form handles the 2D partition with B stored N x K and iters = 1.
+// The persistent form can be asked for with the 2D partition, B stored N x K and iters = 1.
 static bool pipe_allowed(const kami_gemm_desc* d) {
     return d->b_layout == KAMI_B_NK && d->iters == 1;
 }
 
+// FP64 has it for B stored K x N too, where no form is asked for.
+static bool pipe_chosen_kn(const kami_gemm_desc* d) {
+    return d->b_layout == KAMI_B_KN && d->precision == KAMI_PREC_F64 && d->iters == 1 && d->pipeline == 0;
+}
+
+// FP64 with B stored K x N and neither a form asked for nor one measured: the partition's
+// persistent form, where one is compiled and the problem is not small (128^3 x 4096 346 us
+// against 380, 64^3 x 1024 20.6 against 27.0; but 32^3 x 4096 19.3 against 18.1, x 64 4.4 against 3.9).
+static const BlockInstance* untuned_form(const kami_gemm_desc* d, bool tuned, const BlockInstance& in) {
+    if (tuned || !pipe_chosen_kn(d) || in.m < 64) return &in;
+    for (const auto& o : registry())
+        if (o.pipe == 2 && o.prec == in.prec && o.m == in.m && o.n == in.n && o.k == in.k &&
+            o.part == in.part && o.ranks == in.ranks)
+            return &o;
+    return &in;
+}
+
 const BlockInstance* resolve_block(const kami_gemm_desc* d, kami_status* st) {
     int part = d->partition, ranks = d->ranks, pipe = d->pipeline;
+    bool tuned = false;
     if (pipe < 0 || pipe > 2) {
         *st = KAMI_EINVAL;
         return nullptr;
@@ -240,6 +258,7 @@ const BlockInstance* resolve_block(const kami_gemm_desc* d, kami_status* st) {
         ranks = 0;
         int ppipe = 1;
         if (get_tuned_choice(d->precision, d->m, d->n, d->k, &tv)) {
+            tuned = true;
             part = tv.part;
             ranks = tv.ranks;
             ppipe = tv.pipe;
@@ -258,7 +277,7 @@ const BlockInstance* resolve_block(const kami_gemm_desc* d, kami_status* st) {
             *st = KAMI_ENOTSUP;
             return nullptr;
         }
-        pipe = 1;
+        if (!(tuned && pipe_chosen_kn(d))) pipe = 1;
     }
     const bool ranks_defaulted = ranks == 0;
     if (ranks_defaulted) ranks = default_ranks(d->precision, part, d->m, d->n, d->k);
@@ -288,7 +307,7 @@ const BlockInstance* resolve_block(const kami_gemm_desc* d, kami_status* st) {
     for (const auto& in : registry()) {
         if (!in.resident && same_key(in, pipe)) {
             *st = KAMI_OK;
-            return &in;
+            return untuned_form(d, tuned, in);
         }
     }
     // a defaulted wave count that has no compiled instance of this shape: the first
@@ -298,7 +317,7 @@ const BlockInstance* resolve_block(const kami_gemm_desc* d, kami_status* st) {
             if (!in.resident && in.prec == d->precision && in.m == d->m && in.n == d->n &&
                 in.k == d->k && in.part == part && in.pipe == pipe) {
                 *st = KAMI_OK;
-                return &in;
+                return untuned_form(d, tuned, in);
             }
     }
     // AUTO falls back to any compiled per-problem instance of the shape
@@ -307,7 +326,7 @@ const BlockInstance* resolve_block(const kami_gemm_desc* d, kami_status* st) {
             if (!in.resident && in.prec == d->precision && in.m == d->m && in.n == d->n &&
                 in.k == d->k && in.pipe == 1) {
                 *st = KAMI_OK;
-                return &in;
+                return untuned_form(d, tuned, in);
             }
     }
     *st = KAMI_ENOTSUP;
@@ -444,17 +463,6 @@ kami_status kami_block_gemm(const kami_gemm_desc* d, const void* A, const void* 
         return KAMI_ENOTSUP;
     st = device_check();
     if (st != KAMI_OK) return st;
-    // FP64 with B stored K x N and no form asked for: the partition's persistent form, where one
-    // is compiled and the problem is not small (128^3 x 4096 346 us against 380, 64^3 x 1024
-    // 20.6 against 27.0; but 32^3 x 4096 19.3 against 18.1, x 64 4.4 against 3.9).  The query goes
-    // on reporting the partition's plain form.
-    if (args.b_kn && d->precision == KAMI_PREC_F64 && d->pipeline == 0 && d->iters == 1 && in->m >= 64)
-        for (const auto& o : registry())
-            if (o.pipe == 2 && o.prec == in->prec && o.m == in->m && o.n == in->n && o.k == in->k &&
-                o.part == in->part && o.ranks == in->ranks) {
-                in = &o;
-                break;
-            }
     hipError_t e = in->launch(args, count, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e);
     return KAMI_OK;
@@ -489,20 +497,31 @@ kami_status kami_block_gemm_autotune(const kami_gemm_desc* d, const void* A, con
     }
     float best_ms = 1e30f;
     int best_part = 0, best_ranks = 0, best_pipe = 1;
+    kami_gemm_desc untold = *d;
+    untold.pipeline = 0;  // every form is timed, whichever the caller asks for
     st = KAMI_ENOTSUP;
     for (const auto& in : registry()) {
         if (in.prec != d->precision || in.m != d->m || in.n != d->n || in.k != d->k) continue;
-        if (in.pipe == 2 && !pipe_allowed(d)) continue;
+        const bool kn_form = in.pipe == 2 && pipe_chosen_kn(&untold);  // not to be had by asking
+        if (in.pipe == 2 && !pipe_allowed(d) && !kn_form) continue;
         if (in.resident) continue;  // dispatched by iters under its streaming form's key
         kami_gemm_desc t = *d;
         t.partition = in.part;
         t.ranks = in.ranks;
         t.pipeline = in.pipe;
         t.beta = 0.0;  // repeated runs must not feed back into C
-        kami_status r = kami_block_gemm(&t, A, B, C, count, 0, 0, 0, stream);  // warm-up
+        BlockArgs args;
+        auto run = [&]() -> kami_status {
+            if (!kn_form) return kami_block_gemm(&t, A, B, C, count, 0, 0, 0, stream);
+            const kami_status r = prepare_args(&t, A, B, C, count, 0, 0, 0, args);
+            if (r != KAMI_OK) return r;
+            const hipError_t e = in.launch(args, count, s);
+            return e == hipSuccess ? KAMI_OK : hip_fail(e);
+        };
+        kami_status r = run();  // warm-up
         if (r != KAMI_OK) { st = r; break; }
         (void)hipEventRecord(e0, s);
-        for (int rep = 0; rep < 3; ++rep) (void)kami_block_gemm(&t, A, B, C, count, 0, 0, 0, stream);
+        for (int rep = 0; rep < 3; ++rep) (void)run();
         (void)hipEventRecord(e1, s);
         he = hipEventSynchronize(e1);
         if (he != hipSuccess) { st = hip_fail(he); break; }
