@@ -8,6 +8,8 @@
 // checks, which name what is wrong, and its own call.  An error of the HIP runtime is raised
 // from here: work may have been enqueued by then, and a second call would do it twice
 // (with beta != 0, add twice).  Nothing is remembered between calls.
+#include <algorithm>
+
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
@@ -254,6 +256,9 @@ PyObject* bsr_spmm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
+// Columns that may be allocated before nnzb(C) is known whatever C will have: 64 KiB.
+constexpr int64_t kRoom = 1 << 14;
+
 // bsr_spgemm(6 of A, 6 of B, precision or None, alpha) -> (rowptr, colidx, vals)
 PyObject* bsr_spgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return plain([&]() -> PyObject* {
@@ -269,10 +274,13 @@ PyObject* bsr_spgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
             return nullptr;
         if (A.nb != B.mb || A.bs != B.bs || !is(*ta[2], in, *ta[0]) || !is(*tb[2], in, *ta[0])) return nullptr;
         size_t ws_bytes = (size_t)A.mb * (((size_t)B.nb + 31) / 32) * 4;
-        // Up to 1 MiB for every block C could have: the columns are written before the count is
-        // known here, and the scan is not a launch of its own.
+        // Up to 2^18 blocks that C could have: the columns are written before the count is known
+        // here, and the scan is not a launch of its own.  There is room for all of them up to
+        // kRoom, else for twice the products that equal rows would give (8192^2, 2 % of 32 x 32
+        // blocks: 13000 of 65536; C has 6606).
         const int64_t most = (int64_t)A.mb * B.nb;
         const bool fused = A.mb <= kStructureRows && most <= (1 << 18);
+        const int64_t room = std::min(most, std::max<int64_t>(kRoom, 2 * (int64_t)A.nnzb * B.nnzb / B.mb));
         if (fused) ws_bytes += (size_t)A.mb * 4;
         const auto ints = ta[0]->options();
         at::Tensor rowptr, colidx, vals;
@@ -285,11 +293,15 @@ PyObject* bsr_spgemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
             rowptr = at::empty({(int64_t)A.mb + 1}, ints);
             int32_t* const rp = static_cast<int32_t*>(rowptr.data_ptr());
             void* const stream = current_stream();
-            if (fused) colidx = at::empty({most}, ints);
-            st = fused ? g_lib.structure(&A, &B, rp, static_cast<int32_t*>(colidx.data_ptr()), most, &nnz,
+            if (fused) colidx = at::empty({room}, ints);
+            st = fused ? g_lib.structure(&A, &B, rp, static_cast<int32_t*>(colidx.data_ptr()), room, &nnz,
                                          ws.data_ptr(), ws_bytes, stream)
                        : g_lib.symbolic(&A, &B, rp, &nnz, ws.data_ptr(), ws_bytes, stream);
-            if (st == KAMI_OK && fused) {  // the storage's size too, so that a saved C holds its own blocks only
+            // kept where C, for as long as it lives, holds no more than kRoom columns or an eighth
+            // of its own size too much; written again otherwise, as where the room did not do
+            const int64_t block_bytes = (int64_t)A.bs * A.bs * at::elementSize(out) + 4;
+            const bool keep = fused && nnz <= room && room - nnz <= std::max(kRoom, nnz * block_bytes / 32);
+            if (st == KAMI_OK && keep) {  // the storage's size too, so that a saved C holds its own blocks only
                 colidx.unsafeGetTensorImpl()->set_sizes_contiguous({nnz > 0 ? nnz : 1});
                 colidx.storage().unsafeGetStorageImpl()->set_nbytes((size_t)(nnz > 0 ? nnz : 1) * 4);
             } else if (st == KAMI_OK) {
