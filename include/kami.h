@@ -159,8 +159,8 @@ kami_status kami_device_check(void);     /* KAMI_OK when the current device is g
 kami_status kami_gemm_desc_init(kami_gemm_desc* d, int32_t m, int32_t n, int32_t k,
                                 int32_t precision);
 /* Validate a descriptor and report the instance it resolves to. Touches no device.  It
- * knows no problem count: with KAMI_PART_AUTO a call of 256 problems or fewer may take a form
- * of more waves (the same products in the same order).  The tiles that the persistent split
+ * knows no problem count: with KAMI_PART_AUTO a call of few problems may take a form of
+ * another wave count (the same products in the same order).  The tiles that the persistent split
  * forms cut a problem into depend on the count too; 64 x 64 ones are reported. */
 kami_status kami_block_gemm_query(const kami_gemm_desc* d, kami_gemm_config* out);
 /* count independent problems; problem p uses A + p*stride_a, B + p*stride_b,

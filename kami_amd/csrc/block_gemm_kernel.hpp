@@ -33,11 +33,11 @@ constexpr int cmax(int a, int b) { return a > b ? a : b; }
 // them in the writes instead cost eight 2-byte or two 8-byte conflicting stores a piece:
 // FP16 256^3 x 1024 183 us against 114.5, 224^3 x 2048 246 against 177, FP64 128^3 x 4096 431
 // against 376, 64 x 64 x 512 x 2048 273 against 226; N x K 111, 187, 335 and 209.)
-// Repeated products on one stage of 2-byte values are another matter: the reads are repeated
-// and the writes are not, and a turned fragment is two reads of half a row where a row of K
-// is one.  They turn the rows in the writes (TURNED): 64^3 x 1024, 400 times, BF16 104 us
-// against 164, 128 x 128 x 32 x 1024, 279 times, 158 against 238, 256^3 x 1024, 8 times, 318
-// against 403.
+// Many repeated products on one stage of 2-byte values are another matter: the reads are
+// repeated and the writes are not, and a turned fragment is two reads of half a row where a row of
+// K is one.  They turn the rows in the writes (TURNED, from turn_iters on): 64^3 x 1024, 400 times,
+// BF16 104 us against 164, 128 x 128 x 32 x 1024, 279 times, 158 against 238, 256^3 x 1024, 8
+// times, 318 against 403.
 enum BStage : int { kStageNK, kStageRows, kStageTurned };
 template <class AT, int BM_, int BN_, int BK_, int PM_, int PN_, int PK_, int KS_, int B_ = kStageNK>
 struct BlockGeom {
@@ -109,10 +109,11 @@ struct BlockArgs {
 };
 
 // B fragment of column atom jn at K step ks of the K slice of wave (pn, pk), from the stage at
-// bb; kk is the lane's byte offset in a row of K.  (The address is formed as the fragments of A
-// are: with the row's part first, the 256^3 resident forms kept an address per fragment and
-// spilled 60 registers, FP16 x 1024, 8 times, 246 -> 596 us.)  K x N rows: a lane's values are AT::KV rows of one column.  K step 8: the upper lane groups'
-// values are not used, and they read the lower groups' rows so as to stay in the stage.
+// bb; kk is the lane's byte offset in a row of K.  The address is formed as the fragments of A
+// are: with the row's part first, the 256^3 resident forms keep an address per fragment and
+// spill 60 registers (FP16 x 1024, 8 times, 596 us against 246).  K x N rows: a lane's values
+// are AT::KV rows of one column.  K step 8: the upper lane groups' values are not used, and they
+// read the lower groups' rows so as to stay in the stage.
 template <class AT, class G>
 __device__ __forceinline__ typename AT::frag_t stage_b_fragment(const unsigned char* bb, int lane, int pn,
                                                                 int pk, int jn, int ks, int kk) {
@@ -142,17 +143,31 @@ __device__ __forceinline__ typename AT::frag_t stage_b_fragment(const unsigned c
     }
 }
 
-// Waves a SIMD is to hold, at most.  1D instances of 2-byte values write more than they read,
-// and with fewer problems in flight and the registers spent on longer runs of loads the writes
-// go faster: 64 x 64 x 32 x 8192 43.5 us uncapped, 39.6 with 3 waves; 128 x 128 x 32 x 8192
-// 131 (K x N 145), 124.5; 64 x 64 x 16 39.2, 37.1; 64^3 49.0, 47.6; 192 x 192 x 32 x 2048
-// 141 (K x N 145) and 141 with 2.  Smaller problems want all the waves they can have (16^3
-// 4.2 us, 4.5 with 3), and so do the 2D instances (BF16 64^3 51 us, 58).
+// Waves a SIMD is to hold, at most, where a call moves more than the caches hold.  1D instances
+// of 2-byte values write more than they read, and with fewer problems in flight and the registers
+// spent on longer runs of loads the writes to memory go faster: operands not in the caches, 64 x
+// 64 x 32 x 4096 with 4 waves 23.2 us uncapped, 20.0 with 3 a SIMD; 128 x 128 x 16 x 2048 with 8
+// 35.4, 30.8; 64^3 x 4096 25.8, 24.8; 128 x 128 x 32 x 4096 with 4 (K x N) 72.8, 64.1.  8: no
+// such form.  Smaller problems want all the waves they can have (16^3 4.2 us, 4.5 with 3), and so
+// do the 2D instances (BF16 64^3 51 us, 58).
 template <class AT, class G>
 constexpr int waves_per_simd() {
     if (G::ELT == 8 || G::PN > 1 || G::PK > 1 || G::BM < 64 || G::TURNED) return 8;
     const int want = G::IM * G::JN * G::NACC >= 128 ? 2 : 3, own = (G::WAVES + 3) / 4;
     return (want + own - 1) / own * own;  // whole workgroups
+}
+// Below that the writes stay in the caches and every wave helps (64 x 64 x 16 x 2048 with 4 waves
+// 9.3 us, capped 11.1; 128 x 128 x 16 x 1024 14.0, 15.1; 84 MB of 64 x 64 x 16 16.6, 17.6, but 100
+// MB of 64 x 64 x 32 24.2, 21.3, and 84 MB of 128 x 128 x 32 with eight waves 20.6, 18.8).  From many repetitions on the products bound it: their fragments
+// want the registers whatever the size (64^3 x 2048, 32 times, 29.4 us, capped 24.5), as long as
+// two workgroups fit a CU (192 x 192 x 16 x 8192 with 12 waves, 32 times, 324 us, 412 capped to
+// one).  Where LDS holds no second workgroup anyway the cap takes no waves away.
+constexpr int64_t cap_bytes(int waves) { return waves >= 8 ? 80000000 : 100000000; }
+constexpr int kCapIters = 8;
+template <class AT, class G>
+bool cap_pays(int64_t bytes, int iters) {
+    if (2 * G::LDS > 160 * 1024) return true;
+    return iters > kCapIters ? waves_per_simd<AT, G>() >= 2 * ((G::WAVES + 3) / 4) : bytes >= cap_bytes(G::WAVES);
 }
 
 // KFENCE > 0: a scheduling fence after every KFENCE K steps of a stage, so the
@@ -165,9 +180,9 @@ constexpr int waves_per_simd() {
 // SP > 1: the wave tiles of the full BN columns do not fit the register file, so the
 // problem's columns are computed in SP passes of G::BN = BN / SP columns each (B rows and
 // C columns of pass sp start at sp * G::BN); A is read again in every pass.
-template <class AT, class G, int KFENCE = 0, int SP = 1>
-__global__ void __launch_bounds__(G::NT)
-__attribute__((amdgpu_waves_per_eu((G::WAVES + 3) / 4, waves_per_simd<AT, G>())))
+// MOST: waves a SIMD holds, at most (waves_per_simd).
+template <class AT, class G, int KFENCE = 0, int SP = 1, int MOST = 8>
+__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu((G::WAVES + 3) / 4, MOST)))
 block_gemm_kernel(BlockArgs args) {
     using in_t = typename AT::in_t;
     using acc_t = typename AT::acc_t;
@@ -341,6 +356,9 @@ block_gemm_kernel(BlockArgs args) {
     constexpr bool A_LATE = KFENCE == 2;
     load_stage(0);
     if constexpr (!A_LATE) load_a(0, a_cur);
+    // the arguments that products and stores need, while the loads are on their way (fetched
+    // where they are used they are waited for behind those: 128 x 128 x 32 x 512 8.1 us, 7.7)
+    asm volatile("" ::"s"(args.iters), "s"(args.alpha), "s"(args.beta));
     write_stage(0);
     __syncthreads();
     if constexpr (A_LATE) load_a(0, a_cur);
@@ -441,35 +459,42 @@ block_gemm_kernel(BlockArgs args) {
     }  // column passes
 }
 
-template <class AT, class G, int KFENCE, int SP>
+template <class AT, class G, int KFENCE, int SP, int MOST = 8>
 hipError_t launch_block_gemm_as(const BlockArgs& args, int64_t count, hipStream_t stream) {
-    hipLaunchKernelGGL((block_gemm_kernel<AT, G, KFENCE, SP>), dim3((unsigned)count), dim3(G::NT), 0, stream,
+    if constexpr (MOST == 8 && KFENCE < 2 && waves_per_simd<AT, G>() < 8) {  // (resident forms repeat)
+        constexpr int64_t problem = (int64_t)(G::BM + G::BN * SP) * G::BK * G::ELT + (int64_t)G::BM * G::BN * SP * 4;
+        if (cap_pays<AT, G>(count * problem, args.iters))
+            return launch_block_gemm_as<AT, G, KFENCE, SP, waves_per_simd<AT, G>()>(args, count, stream);
+    }
+    hipLaunchKernelGGL((block_gemm_kernel<AT, G, KFENCE, SP, MOST>), dim3((unsigned)count), dim3(G::NT), 0, stream,
                        args);
     return hipGetLastError();
 }
 
-// Repetitions from which 2-byte K x N rows in one stage are turned in the writes (64^3 x 2048
-// in 1D, 8 times 0.93 of the time with rows turned by the reads, 16 times 0.76; 128^3 x 2048
-// 8 times 1.07, 16 times 0.89; several stages are written again for every repetition and stay
-// rows: 128 x 128 x 512 x 256, 64 times, 0.41 of the time with turned writes).
-constexpr int kTurnIters = 8;
+// Repetitions from which 2-byte K x N rows in one stage are turned in the writes, once, and not
+// in the reads, every time; the conflicting writes cost more the more columns there are (turned in
+// the writes against the reads, 4096 problems: 64^3 8 times 28.1 us, 26.8, 16 times 35.1, 36.5;
+// 128^3 8 times 125, 110, 16 times 172, 195, 32 times 313, 358; 256 x 256 x 32 16 times 302, 265,
+// x 1024 128 times 321, 343).  Several stages are written again for every repetition and stay
+// rows (128 x 128 x 512 x 256, 64 times, 0.41 of the time with turned writes).
+constexpr int turn_iters(int columns) { return columns / 8; }
 
 template <class AT, class G, int KFENCE = 0, int SP = 1>
 hipError_t launch_block_gemm(const BlockArgs& args, int64_t count, hipStream_t stream) {
-    // FP64 in one stage on a wave grid: a fragment's two rows are two reads, by every wave row
-    // (2D 64^3 x 1024 23.8 us turned in the writes, 25.8 in the reads; 1D, where a wave reads
-    // all of B either way, 29.2 and 26.3)
-    constexpr bool grid64 = G::ELT == 8 && G::PN > 1;
+    // FP64 in one stage on a wave grid: a fragment's two rows are two reads, by every wave row, which
+    // costs more than the conflicting writes once the CUs hold several problems of 64 columns (2D
+    // 64^3 x 1024 23.8 us turned in the writes, 25.8 in the reads, x 64 5.2, 4.8; 32^3 x 1024 4.9,
+    // 4.5; 1D, where a wave reads all of B either way, 64^3 x 1024 29.2 and 26.3)
+    constexpr bool grid64 = G::ELT == 8 && G::PN > 1 && G::BN >= 64;
     if constexpr (G::NS == 1 && (G::ELT == 2 || grid64))
-        if (args.b_kn && (grid64 || args.iters >= kTurnIters))
+        if (args.b_kn && (grid64 ? count > 512 : args.iters >= turn_iters(G::BN * SP)))
             return launch_block_gemm_as<AT, typename G::AsTurned, KFENCE, SP>(args, count, stream);
     if (args.b_kn) return launch_block_gemm_as<AT, typename G::AsKN, KFENCE, SP>(args, count, stream);
     return launch_block_gemm_as<AT, G, KFENCE, SP>(args, count, stream);
 }
 
-// A resident form, which is taken for iters > 1 only, and turns in the writes for any: with
-// rows in LDS the instances of 16 waves and FP64's spill (FP16 256^3 x 2048 in 16 waves, 4 times,
-// 0.91 of the time with rows; in 8 waves 1.34, but 16 waves are the faster form).
+// A resident form, which is taken for repeated products only (2-byte K x N: three or more), and
+// turns in the writes for any: with rows in LDS the instances of 16 waves and FP64's spill.
 template <class AT, class G>
 hipError_t launch_resident(const BlockArgs& args, int64_t count, hipStream_t stream) {
     if (args.b_kn) return launch_block_gemm_as<AT, typename G::AsTurned, 2, 1>(args, count, stream);

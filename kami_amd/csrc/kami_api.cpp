@@ -192,34 +192,52 @@ static const Prior kPriors[] = {
     {KAMI_PREC_F16_F32, 128, 128, 128, KAMI_PART_1D, 4},
     {KAMI_PREC_F16_F32, 256, 256, 256, KAMI_PART_1D, 16},
     {KAMI_PREC_F16_F32, 128, 128, 32, KAMI_PART_1D, 8},
-    {KAMI_PREC_F16_F32, 192, 192, 16, KAMI_PART_1D, 12}, {KAMI_PREC_F16_F32, 192, 192, 32, KAMI_PART_1D, 12},
+    {KAMI_PREC_F16_F32, 192, 192, 16, KAMI_PART_1D, 12},
     {KAMI_PREC_F16_F32, 256, 256, 16, KAMI_PART_1D, 16}, {KAMI_PREC_F16_F32, 256, 256, 32, KAMI_PART_1D, 8},
     {KAMI_PREC_BF16_F32, 32, 32, 32, KAMI_PART_2D, 1}, {KAMI_PREC_BF16_F32, 64, 64, 64, KAMI_PART_1D, 4},
     {KAMI_PREC_BF16_F32, 128, 128, 128, KAMI_PART_1D, 4},
     {KAMI_PREC_BF16_F32, 256, 256, 256, KAMI_PART_1D, 16},
     {KAMI_PREC_BF16_F32, 128, 128, 32, KAMI_PART_1D, 8},
-    {KAMI_PREC_BF16_F32, 192, 192, 16, KAMI_PART_1D, 12}, {KAMI_PREC_BF16_F32, 192, 192, 32, KAMI_PART_1D, 12},
+    {KAMI_PREC_BF16_F32, 192, 192, 16, KAMI_PART_1D, 12},
     {KAMI_PREC_BF16_F32, 256, 256, 16, KAMI_PART_1D, 16}, {KAMI_PREC_BF16_F32, 256, 256, 32, KAMI_PART_1D, 8},
 };
 
-// Forms for batches of no more problems than CUs, where AUTO would take one of the priors.
-// Every problem has a CU to itself then, and more waves on it hide its loads better, while
+// Forms for batches of a few problems, where AUTO would take one of the priors.  Up to as many
+// problems as CUs every one has a CU to itself, and more waves on it hide its loads better, while
 // there is no next problem to load ahead (us, this form against the prior: FP64 64^3 x 64 4.5,
 // 5.1; x 256 7.2, 7.6; x 768 18.0, 15.9.  BF16 128^3 x 64 3.8, 4.6; x 512 12.5, 11.1.  FP16
-// 256^3 x 64 13.1, 15.6; x 256 28.1, 28.4; x 512 59.3, 58.0).  The same products in the same
-// order, so the bits do not depend on it; the query reports the prior.
-constexpr int64_t kSmallBatch = 256;
-static const Prior kSmallPriors[] = {
-    {KAMI_PREC_F64, 64, 64, 64, KAMI_PART_2D, 4},
-    {KAMI_PREC_F16_F32, 128, 128, 128, KAMI_PART_2D, 4}, {KAMI_PREC_F16_F32, 256, 256, 256, KAMI_PART_2D, 4},
-    {KAMI_PREC_BF16_F32, 128, 128, 128, KAMI_PART_2D, 4}, {KAMI_PREC_BF16_F32, 256, 256, 256, KAMI_PART_2D, 4},
+// 256^3 x 64 13.1, 15.6; x 256 28.1, 28.4; x 512 59.3, 58.0).  128 x 128 x 32 between two
+// workgroups of eight waves a CU and the size that caps them wants four waves (x 512 9.6, 9.1;
+// x 1024 16.4, 20.2; x 2048 34.9, 33.6), 192 x 192 x 32 twelve only while there is one workgroup
+// or two a CU (x 64 4.8, 6.2; x 512 17.4, 17.4; x 8192, 32 times, 392, 384).  The same products in
+// the same order, so the bits do not depend on it; the query reports the prior.
+struct BatchPrior {
+    int64_t first, last;  // problems
+    Prior form;
 };
-static const Prior* small_batch_prior(const kami_gemm_desc* d, int64_t count) {
+static const BatchPrior kBatchPriors[] = {
+    {1, 256, {KAMI_PREC_F64, 64, 64, 64, KAMI_PART_2D, 4}},
+    {1, 256, {KAMI_PREC_F16_F32, 128, 128, 128, KAMI_PART_2D, 4}},
+    {1, 256, {KAMI_PREC_F16_F32, 256, 256, 256, KAMI_PART_2D, 4}},
+    {1, 256, {KAMI_PREC_BF16_F32, 128, 128, 128, KAMI_PART_2D, 4}},
+    {1, 256, {KAMI_PREC_BF16_F32, 256, 256, 256, KAMI_PART_2D, 4}},
+    {513, 1228, {KAMI_PREC_F16_F32, 128, 128, 32, KAMI_PART_1D, 4}},
+    {513, 1228, {KAMI_PREC_BF16_F32, 128, 128, 32, KAMI_PART_1D, 4}},
+    {1, 512, {KAMI_PREC_F16_F32, 192, 192, 32, KAMI_PART_1D, 12}},
+    {1, 512, {KAMI_PREC_BF16_F32, 192, 192, 32, KAMI_PART_1D, 12}},
+};
+static const Prior* batch_prior(const kami_gemm_desc* d, int64_t count) {
     TuneVal tv;
-    if (count > kSmallBatch || d->partition != KAMI_PART_AUTO || d->pipeline != 0 || d->iters != 1) return nullptr;
-    for (const Prior& p : kSmallPriors)
-        if (p.prec == d->precision && p.m == d->m && p.n == d->n && p.k == d->k)
-            return get_tuned_choice(p.prec, p.m, p.n, p.k, &tv) ? nullptr : &p;
+    if (d->partition != KAMI_PART_AUTO || d->pipeline != 0) return nullptr;
+    for (const BatchPrior& b : kBatchPriors) {
+        const Prior& p = b.form;
+        if (p.prec != d->precision || p.m != d->m || p.n != d->n || p.k != d->k) continue;
+        if (count < b.first || count > b.last) continue;
+        if (d->iters > 1)  // a resident form is the better one for those
+            for (const auto& in : registry())
+                if (in.resident && in.prec == p.prec && in.m == p.m && in.n == p.n && in.k == p.k) return nullptr;
+        return get_tuned_choice(p.prec, p.m, p.n, p.k, &tv) ? nullptr : &p;
+    }
     return nullptr;
 }
 
@@ -282,12 +300,15 @@ const BlockInstance* resolve_block(const kami_gemm_desc* d, kami_status* st) {
     const bool ranks_defaulted = ranks == 0;
     if (ranks_defaulted) ranks = default_ranks(d->precision, part, d->m, d->n, d->k);
     // repeated products (iters > 1) use a key's resident form (all of K in one LDS stage)
-    // where one is compiled; a single product uses the streaming form
+    // where one is compiled; a single product uses the streaming form.  The resident forms turn
+    // K x N rows of 2-byte values as they write them, all of K before the first product, which
+    // two repetitions do not pay for (256^3 x 512 twice 115 us, streamed 83).
+    const int resident_from = d->b_layout == KAMI_B_KN && d->precision != KAMI_PREC_F64 ? 3 : 2;
     auto same_key = [&](const BlockInstance& in, int want_pipe) {
         return in.prec == d->precision && in.m == d->m && in.n == d->n && in.k == d->k &&
                in.part == part && in.ranks == ranks && in.pipe == want_pipe;
     };
-    if (d->iters > 1 && (pipe == 0 || pipe == 1))
+    if (d->iters >= resident_from && (pipe == 0 || pipe == 1))
         for (const auto& in : registry())
             if (in.resident && same_key(in, 1)) {
                 *st = KAMI_OK;
@@ -450,7 +471,7 @@ kami_status kami_block_gemm(const kami_gemm_desc* d, const void* A, const void* 
     if (st != KAMI_OK || count == 0) return st;
     if (is_split(d->precision)) return split_launch(d, args, count, (hipStream_t)stream);
     kami_gemm_desc small = *d;
-    if (const Prior* p = small_batch_prior(d, count)) {
+    if (const Prior* p = batch_prior(d, count)) {
         small.partition = p->part;
         small.ranks = p->ranks;
         small.pipeline = p->pipe;
