@@ -284,7 +284,7 @@ kami_status kami_bsr_spmm(const kami_bsr* A, const void* B, int32_t n, int64_t l
                           double alpha, double beta, void* stream);
 
 /* ---------------------------------------------------------------- slicing, generators */
-/* The digit slicing of the split-precision path, standalone: X (rows x k FP64, row-major,
+/* A digit slicing for the split-precision path, standalone: X (rows x k FP64, row-major,
  * ldx >= k, 0 = packed) is written as
  *     X(i, j) ~= 2^(e(i, c) - BETA) * sum_{s < slices} d_s(i, j) 2^(-BETA s),   c = j / 32,
  * with e(i, c) the exponent of the largest |X(i, j)| of the 32-wide chunk c of row i
@@ -294,9 +294,11 @@ kami_status kami_bsr_spmm(const kami_bsr* A, const void* B, int32_t n, int64_t l
  * (BETA = 8, bfloat16 digits); 1 <= slices <= 8.  digits (device): `slices` planes of
  * rows x k 16-bit values, plane s at digits + s * rows * k; exps (device): int32
  * rows x ceil(k / 32).  The error per element is at most 2^(e - BETA * slices - 1);
- * finite inputs.  No counterpart in the reference (it has no split-precision path): the
- * slicing step of kami_block_gemm / kami_split_gemm, for callers that run the slice
- * products with a GEMM of their own. */
+ * finite inputs.  No counterpart in the reference (it has no split-precision path): for
+ * callers that run the slice products with a GEMM of their own.  kami_block_gemm and
+ * kami_split_gemm form digits within the same bounds and with the same error, but not always
+ * the same ones: their default forms round once for three digits (0.5 in base 256 is 1, -128
+ * there and 0, 128 here). */
 kami_status kami_split_slices(const double* X, int64_t rows, int64_t k, int64_t ldx,
                               int32_t precision, int32_t slices, uint16_t* digits,
                               int32_t* exps, void* stream);

@@ -251,8 +251,9 @@ __all__ += ["split_gemm"]
 
 
 def split_slices(X, *, precision=PREC_F64_SPLIT_F16, slices=6, stream=None):
-    """Digit slices of an FP64 matrix as the split-precision path forms them
-    (kami_split_slices): returns (digits, exps) with digits a uint16 tensor of shape
+    """Digit slices of an FP64 matrix for slice products with a GEMM of one's own
+    (kami_split_slices; the split-precision path's digits have the same bounds and error, but
+    differ at ties): returns (digits, exps) with digits a uint16 tensor of shape
     (slices, rows, k) holding binary16 (FP16 precision) or bfloat16 (BF16) bits and exps
     an int32 tensor (rows, ceil(k / 32)), so that
     X[i, j] ~= sum_s digits[s, i, j] * 2^(exps[i, j // 32] - BETA * (s + 1)).

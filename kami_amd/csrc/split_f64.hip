@@ -11,9 +11,10 @@
 //   1. exponents: e_i = exponent of max_k |A(i,k)| for every row of A and f_j of every
 //      row of B (B is stored N x K), so |A(i,k)| < 2^e_i;
 //   2. slicing, per 32-wide K chunk: A(i,k) 2^(BETA - e_i) = sum_s a_s 2^(-BETA (s-1))
-//      with integer digits a_s chosen by round-to-nearest (|a_1| <= 2^BETA,
-//      |a_s| <= 2^(BETA-1) after that), exactly representable in FP16 (BETA = 9) or
-//      BF16 (BETA = 8); the digits go to LDS, one plane per slice;
+//      with integer digits a_s (|a_1| <= 2^BETA, |a_s| <= 2^(BETA-1) after that), exactly
+//      representable in FP16 (BETA = 9) or BF16 (BETA = 8): the form with a workgroup per
+//      problem rounds them to nearest one by one, the persistent forms round once for three and
+//      cut the fields of the integer (PairDigits); the digits go to LDS, one plane per slice;
 //   3. products: for every level g = s + t <= G the FP32 MFMA sum
 //      T_g = sum_{s+t=g} a_s b_t^T over the 32-wide chunk is an integer of magnitude
 //      <= 2^24 (checked at compile time for the levels that matter), hence exact in
@@ -21,7 +22,8 @@
 //      2^(-BETA g) after each chunk;
 //   4. C(i,j) = alpha 2^(e_i + f_j) acc(i,j) + beta C(i,j).
 // The error relative to 2^(e_i + f_j) is about K 2^(-BETA S - 1) from the truncated
-// digits plus the dropped levels g > G; finite inputs are required.
+// digits plus the dropped levels g > G.  A NaN or an infinity makes the elements of C that
+// it takes part in NaN.
 #include <cmath>
 #include <cstdint>
 
@@ -440,6 +442,14 @@ struct SplitStreamGeom {
                   "the two smallest levels are combined in FP32");
 };
 
+// Digit products of levels g <= G with S digits per operand
+constexpr int products_of(int S, int G) {
+    int n = 0;
+    for (int s = 1; s <= S; ++s)
+        for (int t = 1; t <= S; ++t) n += s + t <= G;
+    return n;
+}
+
 // Persistent form.  A workgroup walks work units blockIdx.x, + gridDim.x, ... -- one unit
 // is a BT x BT tile of C of one problem, K any multiple of 32 -- as one stream of 32-wide
 // K chunks.  The exponents are taken per row and per chunk, from the registers that hold
@@ -457,14 +467,6 @@ struct SplitStreamGeom {
 // beside 56 matrix instructions).  1024^3 with seven FP16 digits: 217 us with 128 x 128
 // tiles (64 of them on 256 CUs, slicing and products across barriers), 87 with 64 x 64
 // tiles and two buffers, 78 with PairDigits, 73 with the schedule.
-// Digit products of levels g <= G with S digits per operand
-constexpr int products_of(int S, int G) {
-    int n = 0;
-    for (int s = 1; s <= S; ++s)
-        for (int t = 1; t <= S; ++t) n += s + t <= G;
-    return n;
-}
-
 template <class SAT, class G>
 __global__ void __launch_bounds__(G::NT)
 split_stream_kernel(SplitArgs args, int64_t count) {

@@ -1,9 +1,10 @@
-// Entry points beside the GEMM paths: the digit slicing of the split-precision path as a
+// Entry points beside the GEMM paths: a digit slicing for the split-precision path as a
 // standalone kernel, and the reference programs' known-answer inputs generated in device
 // memory.
 //
-// kami_split_slices writes the same digits the split GEMM kernels form in LDS
-// (split_f64.hip): per row and per 32-wide chunk of K an exponent e with every |x| of the
+// kami_split_slices writes digits of the bounds and the error of those that the split GEMM kernels
+// form in LDS (split_f64.hip; the default forms round once for three digits, so theirs may
+// differ at ties): per row and per 32-wide chunk of K an exponent e with every |x| of the
 // chunk below 2^e (0 for an all-zero chunk), then r = x 2^(BETA - e) and, slice by slice,
 // d = rint(r) (round to nearest, ties to even), r = (r - d) 2^BETA.
 //
