@@ -21,8 +21,8 @@
 // M, N and K must be multiples of 16.
 //
 // What bounds it: 20000 problems of 16 to 256 (3.58 GB FP64, 1.19 GB FP16 with FP32 C) run
-// in 788 us and 275 us, 4.5 and 4.3 TB/s of the algorithmic bytes; FP64 moves 3.81 GB, at the rate
-// of a copy (4.8 TB/s).
+// in 788 us and 275 us, 4.5 and 4.3 TB/s of the algorithmic bytes; FP64 moves 3.97 GB, at the rate
+// of a copy (5 TB/s).
 // The persistent form this replaced (workgroups popping tiles of up to 128 x 128 from an atomic
 // counter, LDS stages shared by four waves, one barrier a stage, a one-thread kernel to clear
 // the counter) took 1027 us and 398 us: two workgroups a CU and their barriers left too little
@@ -174,11 +174,12 @@ struct WaveTile {
         roff = (lane & 15) * 128 + ((grp ^ (((lane >> 2) & 3) << 1)) << 4);
     }
 
+    // Stage c of K's (k + KS - 1) / KS
     __device__ __forceinline__ void load(Stage& s, int c) const {
-        // pieces past K lie out of the descriptor's range; the scalar offsets stay inside
-        // the operand
-        const int k0 = c * KS, kb = k0 < k ? k0 : 0;
-        const bool ok = F64 ? k0 < k : k0 + (lane & 7) * VE < k;  // K is a multiple of 16
+        // pieces past K (a multiple of 16, which FP64 stages do not pass) lie out of the
+        // descriptor's range; the scalar offsets stay inside the operand
+        const int kb = c * KS;
+        const bool ok = F64 || kb + (lane & 7) * VE < k;
         const int ao = ok ? aoff : kBufferRange, bo = ok ? boff : kBufferRange;
 #pragma unroll
         for (int i = 0; i < NA; ++i) s.a[i] = buffer_load16(ra, ao, (i * 8 * lda + kb) * ELT);
@@ -198,7 +199,7 @@ struct WaveTile {
             constexpr int RPL = 64 / PPR;  // K rows of one load instruction
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
-                const int r = k0 + i * RPL;
+                const int r = kb + i * RPL;
                 const bool live = r + lane / PPR < k && (JN != 3 || lane % PPR < 2 * JN);
                 s.b[i] = buffer_load16(rb, live ? boff : kBufferRange,
                                        (r < k ? r : 0) * ldb * ELT);
@@ -273,10 +274,9 @@ struct WaveTile {
         for (int i = 0; i < IM; ++i)
 #pragma unroll
             for (int j = 0; j < JN; ++j) acc[i][j] = accv_t{0, 0, 0, 0};
-        // Stage c in LDS, stage c + 1 in registers or on its way.  Straight-line stages: a
-        // branch around a load would make the compiler wait for every load in flight where
-        // the paths meet, so the stage past the last one is loaded too, out of range (no
-        // memory traffic).
+        // Stage c - 1 in LDS, stage c in registers or on its way; the last one after the loop.
+        // (Straight-line stages: a branch around a load would make the compiler wait for every
+        // load in flight where the paths meet.)
         Stage s;
         const int n = (k + KS - 1) / KS;
         load(s, 0);
@@ -628,7 +628,7 @@ static kami_status check_problem(kami_problem& p, int b_layout, int ei, int eo) 
         ((uintptr_t)p.C % eo))
         return KAMI_EINVAL;
     // Operand pieces are addressed by 32-bit byte offsets from the tile's origin
-    // (stream_load): the farthest piece of any tile must end below kBufferRange.
+    // (WaveTile::load): the farthest piece of any tile must end below kBufferRange.
     const int64_t a_span = ((int64_t)(std::min(p.m, 128) - 1) * p.lda + p.k) * ei;
     const int64_t b_span = b_layout == KAMI_B_NK
                                ? ((int64_t)(std::min(p.n, 128) - 1) * p.ldb + p.k) * ei
