@@ -356,9 +356,12 @@ block_gemm_kernel(BlockArgs args) {
     constexpr bool A_LATE = KFENCE == 2;
     load_stage(0);
     if constexpr (!A_LATE) load_a(0, a_cur);
-    // the arguments that products and stores need, while the loads are on their way (fetched
-    // where they are used they are waited for behind those: 128 x 128 x 32 x 512 8.1 us, 7.7)
-    asm volatile("" ::"s"(args.iters), "s"(args.alpha), "s"(args.beta));
+    // the arguments that products and stores need, while the loads are on their way: fetched where
+    // they are used they are waited for behind those (128 x 128 x 32 x 512 in four waves 8.1 us,
+    // 7.9; 192 x 192 x 16 x 64 in 2D 0.96 of the time).  Smaller tiles on wave grids lose by it
+    // (32^3 in 2 x 2 waves, 1000 times, 1.07), FP64 neither way.
+    if constexpr (G::ELT == 2 && (G::PN == 1 ? G::BM >= 64 : G::BM >= 192))
+        asm volatile("" ::"s"(args.iters), "s"(args.alpha), "s"(args.beta));
     write_stage(0);
     __syncthreads();
     if constexpr (A_LATE) load_a(0, a_cur);
