@@ -303,7 +303,11 @@ struct SpNumGeom {
     static constexpr int LDS = A_LDS + (F64 ? 0 : BS * TROW);
 };
 
-constexpr int kNumWaves = 4;  // waves (output blocks) of a workgroup
+// Waves (output blocks) of a workgroup: four, or one from kAloneIters repetitions of 2-byte products
+// on, where the waves of a workgroup end far apart and their room waits for the last (8 % of 256
+// x 256 blocks of 16, 1000 times, 973 us with four, 920 with one; 8 times 38.2 and 36.1, but 1024 copies
+// of 8 x 8 blocks of 32, 8 times, 125 and 137; FP64 16 x 16, 64 times, 65.6 and 72.3).
+constexpr int kNumWaves = 4, kAloneIters = 64;
 
 __device__ inline int find_col(const int32_t* ci, int lo, int hi, int j) {
     // index in [lo, hi) with ci[idx] == j, or -1 (ci ascending within the row)
@@ -315,30 +319,36 @@ __device__ inline int find_col(const int32_t* ci, int lo, int hi, int j) {
     return (lo < end && ci[lo] == j) ? lo : -1;
 }
 
-// Block row of output block cb: the last row with rpC[row] <= cb, found by a 256-way search
-// (each round a lane probes four of 256 evenly spaced row pointers).
-__device__ inline int row_of(const int32_t* rpC, int mb, int64_t cb, int lane) {
+// Block row of output block cb: the last row with rpC[row] <= cb.  Each round a lane probes Q of
+// 64 Q evenly spaced row pointers.  Up to 256 rows four probes find it in one round; beyond that
+// they cost more lines than the rounds they save (16384 copies of 8 x 8 blocks of 16 side by
+// side, 131072 rows: 741 us with one probe, 885 with four; 1024 of 8 x 8 blocks of 32 118, 138).
+template <int Q>
+__device__ inline int row_search(const int32_t* rpC, int mb, int64_t cb, int lane) {
     int lo = 0, hi = mb;
     while (hi - lo > 1) {
-        const int64_t step = ((int64_t)hi - lo + 255) / 256;
+        const int64_t step = ((int64_t)hi - lo + 64 * Q - 1) / (64 * Q);
         int c = 0;
-        bool le[4];
+        bool le[Q];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < Q; ++q) {
             const int64_t idx = lo + (lane + 64 * q + 1) * step;
             le[q] = idx < hi && (int64_t)rpC[idx] <= cb;
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) c += __popcll(__ballot(le[q]));  // probes are monotone
+        for (int q = 0; q < Q; ++q) c += __popcll(__ballot(le[q]));  // probes are monotone
         const int64_t nlo = lo + c * step;
         hi = (int)min((int64_t)hi, nlo + step);
         lo = (int)nlo;
     }
     return __builtin_amdgcn_readfirstlane(lo);
 }
+__device__ inline int row_of(const int32_t* rpC, int mb, int64_t cb, int lane) {
+    return mb <= 256 ? row_search<4>(rpC, mb, cb, lane) : row_search<1>(rpC, mb, cb, lane);
+}
 
-template <int BS, class AT>
-__global__ void __launch_bounds__(64 * kNumWaves)
+template <int BS, class AT, int W>
+__global__ void __launch_bounds__(64 * W)
 spgemm_numeric_kernel(int mb, int64_t nnzc, const int32_t* rpA, const int32_t* ciA,
                       const void* vA_, const int32_t* rpB, const int32_t* ciB, const void* vB_,
                       const int32_t* rpC, const int32_t* ciC, void* vC_, double alpha_d,
@@ -350,7 +360,7 @@ spgemm_numeric_kernel(int mb, int64_t nnzc, const int32_t* rpA, const int32_t* c
     using frag_t = typename AT::frag_t;
     using accv_t = typename AT::accv_t;
     constexpr int FB = AT::FRAG_BYTES, IM = G::IM, KSTEPS = G::KSTEPS;
-    __shared__ __attribute__((aligned(16))) unsigned char smem[kNumWaves * G::LDS];
+    __shared__ __attribute__((aligned(16))) unsigned char smem[W * G::LDS];
     const in_t* vA = reinterpret_cast<const in_t*>(vA_);
     const in_t* vB = reinterpret_cast<const in_t*>(vB_);
     out_t* vC = reinterpret_cast<out_t*>(vC_);
@@ -363,7 +373,7 @@ spgemm_numeric_kernel(int mb, int64_t nnzc, const int32_t* rpA, const int32_t* c
     const uint32_t L = blockIdx.x, x8 = L % 8, q8 = gridDim.x / 8, r8 = gridDim.x % 8;
     const int64_t P = x8 * q8 + (x8 < r8 ? x8 : r8) + L / 8;
 
-    for (int64_t cb = P * kNumWaves + wave; cb < nnzc; cb += (int64_t)gridDim.x * kNumWaves) {
+    for (int64_t cb = P * W + wave; cb < nnzc; cb += (int64_t)gridDim.x * W) {
         const int j = load_uniform(ciC + cb);
         const int i = row_of(rpC, mb, cb, lane);
         accv_t acc[IM][IM];
@@ -660,11 +670,16 @@ kami_status kami_bsr_spgemm_numeric_repeat(const kami_bsr* A, const kami_bsr* B,
     st = device_check();
     if (st != KAMI_OK) return st;
     hipStream_t s = (hipStream_t)stream;
-    const unsigned grid = (unsigned)std::min<int64_t>((nnzbC + kNumWaves - 1) / kNumWaves, 1 << 20);
-#define KAMI_SPNUM(BS, AT)                                                                      \
-    hipLaunchKernelGGL((spgemm_numeric_kernel<BS, AT>), dim3(grid), dim3(64 * kNumWaves), 0, s, A->mb,       \
+    const int waves = iters >= kAloneIters && precision != KAMI_PREC_F64 ? 1 : kNumWaves;
+    const unsigned grid = (unsigned)std::min<int64_t>((nnzbC + waves - 1) / waves, 1 << 20);
+#define KAMI_SPNUM_W(BS, AT, W)                                                                  \
+    hipLaunchKernelGGL((spgemm_numeric_kernel<BS, AT, W>), dim3(grid), dim3(64 * W), 0, s, A->mb, \
                        nnzbC, A->rowptr, A->colidx, A->vals, B->rowptr, B->colidx, B->vals,      \
                        rowptrC, colidxC, valC, alpha, (int)iters)
+#define KAMI_SPNUM(BS, AT)                                                                       \
+    do {                                                                                         \
+        if (waves == 1) KAMI_SPNUM_W(BS, AT, 1); else KAMI_SPNUM_W(BS, AT, kNumWaves);           \
+    } while (0)
     if (precision == KAMI_PREC_F16_F32) {
         if (A->bs == 16) KAMI_SPNUM(16, AtomF16x16); else KAMI_SPNUM(32, AtomF16x32);
     } else if (precision == KAMI_PREC_BF16_F32) {
@@ -675,6 +690,7 @@ kami_status kami_bsr_spgemm_numeric_repeat(const kami_bsr* A, const kami_bsr* B,
         return KAMI_ENOTSUP;
     }
 #undef KAMI_SPNUM
+#undef KAMI_SPNUM_W
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e);
     return KAMI_OK;
