@@ -326,14 +326,24 @@ static hipError_t launch_form(SpmmArgs a, hipStream_t s) {
     return e;
 }
 
-// Which form: enough workgroups share a row's stages among four waves; FP64 blocks of 32 as
-// two K groups x two column groups (a row's two stages per block go to one wave each, and
-// the column groups read A's lines together: 23.5 us against 26.2 for four K groups at
-// 8192^2, 2 % of 32 x 32 blocks, n = 256), the others as four K groups (FP64 blocks of 16
-// at 4800^2, 20 %, n = 128: 31.7 us against 36.3).  Where the tiles leave the chip idle
-// and the rows are long, one row's stages go to 16 or 8 waves: 20 block rows of 80 blocks of
-// 32, n = 48: FP64 28.6 us against 43.5 with four (and 135 with the earlier kernel), FP16
-// 11.2 against 13.6; 100 rows of 20, n = 64: FP64 15.1 against 17.0.
+// Which form.  Four K groups of waves share a row's stages; FP64 blocks of 32 two K groups x two
+// column groups (a row's two stages per block go to one wave each, and the column groups read
+// A's lines together: 23.5 us against 26.2 for four K groups at 8192^2, 2 % of 32 x 32
+// blocks, n = 256).  Where the tiles leave the chip idle and the rows are long, one row's stages
+// go to 16 or 8 waves: 20 block rows of 80 blocks of 32, n = 48: FP64 28.6 us against 43.5 with
+// four, FP16 11.2 against 13.6; 100 rows of 20, n = 64: FP64 15.1 against 17.0.
+// 16 columns are one atom (4096 rows of 2 blocks of 16: FP64 10.4 us with the tiles of
+// more columns, 6.1; FP16 5.9 and 4.0).
+// FP64 with tiles enough to fill the chip shares a row's A among four column groups, so that no
+// partial tiles are summed: blocks of 16, 4096 rows of 1, n = 1024 291 us with four K groups, 194;
+// rows of 16, n = 256 407 and 323; but with few tiles for the rows' length four K groups: 256
+// rows of 51, n = 1024 142 and 154, 4800^2, 20 %, n = 128 31.7 and 36.3.  Columns of one atom a wave
+// (64 a workgroup) where there are no more, or rows and tiles are few (1000 rows of 1, n = 256 16.9
+// us, 11.8; with 128 a workgroup 12.7).  Blocks of 32 split K of their own block two ways already, and
+// uneven rows want that (512 rows of 3.2, n = 256 27 us, 30 with column groups); rows of 1 (4096, n
+// = 256 112 and 104) and long ones (16, n = 256 941 and 820) do not.
+// 2-byte blocks of 16 whose B, stored N x K, has more than an XCD's L2 (4 MiB) under 64 columns take 32 (4096
+// rows of 4, n = 256 57 us, 41; rows of 1 27 and 29; K x N 28 and 47).
 template <int BS, class AT, int CT>
 static hipError_t launch_spmm(const SpmmArgs& a, hipStream_t s) {
     using G = SpmmGeom<BS, AT, false, 4, 1, CT>;
@@ -341,10 +351,22 @@ static hipError_t launch_spmm(const SpmmArgs& a, hipStream_t s) {
     const int64_t stages = a.nnzb * G::HS / a.mb;  // of an average row
     if (tiles <= 256 && stages >= 32) return launch_form<BS, AT, 16, 1, CT>(a, s);
     if (tiles <= 512 && stages >= 16) return launch_form<BS, AT, 8, 1, CT>(a, s);
-    if constexpr (G::F64 && BS == 32)
+    if (a.n <= 16) return tiles <= 512 ? launch_form<BS, AT, 4, 1, 1>(a, s) : launch_form<BS, AT, 2, 1, 1>(a, s);
+    const bool many = tiles > std::max<int64_t>(1024, 400 * stages);
+    if constexpr (G::F64 && BS == 32) {
+        if (many && stages <= 2 && a.n > 32 && a.n <= 64) return launch_form<BS, AT, 1, 4, 1>(a, s);
+        if (many && (stages <= 2 || stages >= 24) && a.n >= 128) return launch_form<BS, AT, 1, 4, 2>(a, s);
         return launch_form<BS, AT, 2, 2, CT>(a, s);
-    else
-        return launch_form<BS, AT, 4, 1, CT>(a, s);
+    } else if constexpr (G::F64) {
+        if (a.n <= 32 && stages <= 2) return launch_form<BS, AT, 1, 2, 1>(a, s);
+        if (many && a.n > 32) {
+            if (a.n < 128 || (stages <= 6 && tiles < 8192)) return launch_form<BS, AT, 1, 4, 1>(a, s);
+            return launch_form<BS, AT, 1, 4, 2>(a, s);
+        }
+    } else if constexpr (BS == 16) {
+        if (!a.b_kn && stages >= 3 && (int64_t)a.nb * BS * 64 * G::ELT > (4 << 20)) return launch_form<BS, AT, 4, 1, 2>(a, s);
+    }
+    return launch_form<BS, AT, 4, 1, CT>(a, s);
 }
 
 }  // namespace kami
