@@ -485,24 +485,29 @@ constexpr int64_t kFullUnits = 4096;
 // 4800 of them, 68.0 against 63.7), be fewer by a quarter at least, or little
 // is read less often, and run long enough to hide their loads with fewer waves: a mean K by work of
 // 128 for 2-byte inputs (two stages; 128^3 x 8192 201 us either way, 144^3 x 4096 192 against
-// 205), 96 for FP64 (six; 96^3 x 4096 192 against 198, 64^3 x 8192 155 against 148).
-static bool larger_pays(const WorkItem* items, int64_t n_items, int elt, int64_t larger, int64_t first) {
+// 205), 96 for FP64 (six; 96^3 x 4096 192 against 198, 64^3 x 8192 155 against 148).  FP64 K x N
+// reads B eight bytes a lane, again for every row of tiles: in long queues of wide problems the
+// larger ones pay whatever K (256 x 256 x 16 x 2000 217 against 254, 1024 x 256 x 32 x 500 285 against
+// 343; but x 100 50 against 47, 128 x 128 x 32 x 2000 86 against 81).
+static bool larger_pays(const WorkItem* items, int64_t n_items, int elt, bool b_kn, int64_t larger, int64_t first) {
     if (larger < 2 * 1024 * (elt == 8 ? 3 : 2) || 4 * larger > 3 * first) return false;
     const double least = elt == 8 ? 96 : 128;
-    double work = 0, work_k = 0;
+    double work = 0, work_k = 0, work_n = 0;
     for (int64_t i = 0; i < n_items; ++i) {
         const WorkItem& w = items[i];
         const double f = (double)std::min(w.mlim, kVariantTM[w.variant]) * std::min(w.nlim, kVariantTN[w.variant]) * w.k;
         work += f;
         work_k += f * w.k;
+        work_n += f * w.nlim;  // columns to the problem's edge
     }
-    return work_k >= least * work;
+    const bool wide_kn = elt == 8 && b_kn && larger >= 14 * 1024 && work_n > 160 * work;
+    return wide_kn || work_k >= least * work;
 }
 
-static int wave_cap(const WorkItem* items, int64_t n_items, int elt, int64_t* n_units) {
+static int wave_cap(const WorkItem* items, int64_t n_items, int elt, bool b_kn, int64_t* n_units) {
     int cap = first_cap(elt);
     const int64_t larger = count_units(items, n_items, cap - 1);
-    if (larger_pays(items, n_items, elt, larger, count_units(items, n_items, cap))) {
+    if (larger_pays(items, n_items, elt, b_kn, larger, count_units(items, n_items, cap))) {
         *n_units = larger;
         return cap - 1;
     }
@@ -670,11 +675,11 @@ struct DeviceQueue {
     const WaveUnit* units() const { return reinterpret_cast<const WaveUnit*>(items() + n_items); }
 };
 
-static kami_status upload_queue(const std::vector<WorkItem>& items, int elt, DeviceQueue* q) {
+static kami_status upload_queue(const std::vector<WorkItem>& items, int elt, bool b_kn, DeviceQueue* q) {
     const int64_t n = (int64_t)items.size();
     if (n > UINT32_MAX) return KAMI_ENOMEM;  // 256 GiB of entries
     int64_t n_units = 0;
-    const int cap = wave_cap(items.data(), n, elt, &n_units);
+    const int cap = wave_cap(items.data(), n, elt, b_kn, &n_units);
     const size_t item_bytes = (size_t)n * sizeof(WorkItem), bytes = item_bytes + (size_t)n_units * sizeof(WaveUnit);
     std::unique_ptr<unsigned char[]> host(new (std::nothrow) unsigned char[bytes]);
     if (!host) return KAMI_ENOMEM;
@@ -834,7 +839,7 @@ kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count, i
                 std::vector<WorkItem> items;
                 build_items(sample, sb, vb, ei, eo, plan->b_kn, items);
                 DeviceQueue q;
-                st = upload_queue(items, ei, &q);
+                st = upload_queue(items, ei, plan->b_kn, &q);
                 if (st != KAMI_OK) {
                     if (q.mem) (void)hipFree(q.mem);
                     break;
@@ -871,7 +876,7 @@ kami_status kami_batched_plan_create(const kami_problem* probs, int64_t count, i
     std::vector<WorkItem> items;
     build_items(hp, bucket, variant_of_bucket, ei, eo, plan->b_kn, items);
     plan->n_items = (int64_t)items.size();
-    st = upload_queue(items, ei, &plan->queue);
+    st = upload_queue(items, ei, plan->b_kn, &plan->queue);
     if (st != KAMI_OK) {
         free_plan(plan);
         return st;
@@ -952,7 +957,7 @@ kami_status kami_batched_gemm_static(const kami_problem* probs, int64_t count, i
     build_items(g_static.probs, count, g_static.bucket, variant_of_bucket, ei, eo, b_kn,
                 g_static.order, items);
     int64_t n_units = 0;
-    const int cap = wave_cap(items, n_items, ei, &n_units);
+    const int cap = wave_cap(items, n_items, ei, b_kn, &n_units);
     build_units(items, n_items, cap, n_units, units);
     hipStream_t s = (hipStream_t)stream;
     // From pageable memory the copy has consumed the staging array when the call returns,
