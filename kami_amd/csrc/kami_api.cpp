@@ -251,11 +251,12 @@ static bool pipe_chosen_kn(const kami_gemm_desc* d) {
     return d->b_layout == KAMI_B_KN && d->precision == KAMI_PREC_F64 && d->iters == 1 && d->pipeline == 0;
 }
 
-// FP64 with B stored K x N and neither a form asked for nor one measured: the partition's
-// persistent form, where one is compiled and the problem is not small (128^3 x 4096 346 us
-// against 380, 64^3 x 1024 20.6 against 27.0; but 32^3 x 4096 19.3 against 18.1, x 64 4.4 against 3.9).
+// FP64 with B stored K x N and neither a form asked for nor one measured: the persistent form of
+// 4 x 4 waves, where one is compiled and the problem is not small (128^3 x 4096 346 us against
+// 380, 64^3 x 1024 20.6 against 27.0; but 32^3 x 4096 19.3 against 18.1, x 64 4.4 against 3.9, and 2 x 2
+// waves 64^3 x 8192 152 against 138, x 64 6.7 against 5.2).
 static const BlockInstance* untuned_form(const kami_gemm_desc* d, bool tuned, const BlockInstance& in) {
-    if (tuned || !pipe_chosen_kn(d) || in.m < 64) return &in;
+    if (tuned || !pipe_chosen_kn(d) || in.m < 64 || in.ranks < 4) return &in;
     for (const auto& o : registry())
         if (o.pipe == 2 && o.prec == in.prec && o.m == in.m && o.n == in.n && o.k == in.k &&
             o.part == in.part && o.ranks == in.ranks)
