@@ -29,8 +29,8 @@ namespace kami {
 constexpr int cmin(int a, int b) { return a < b ? a : b; }
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
-// B_: B is stored N x K, or K x N.  Then its K rows go to LDS as they are and the reads turn them.  (Turning
-// them in the writes instead cost eight 2-byte or two 8-byte conflicting stores a piece:
+// B_: B is stored N x K, or K x N.  Then its K rows go to LDS as they are and the reads turn
+// them.  (Turning them in the writes instead cost eight 2-byte or two 8-byte conflicting stores a piece:
 // FP16 256^3 x 1024 183 us against 114.5, 224^3 x 2048 246 against 177, FP64 128^3 x 4096 431
 // against 376, 64 x 64 x 512 x 2048 273 against 226; N x K 111, 187, 335 and 209.)
 // Many repeated products on one stage of 2-byte values are another matter: the reads are
@@ -158,10 +158,11 @@ constexpr int waves_per_simd() {
 }
 // Below that the writes stay in the caches and every wave helps (64 x 64 x 16 x 2048 with 4 waves
 // 9.3 us, capped 11.1; 128 x 128 x 16 x 1024 14.0, 15.1; 84 MB of 64 x 64 x 16 16.6, 17.6, but 100
-// MB of 64 x 64 x 32 24.2, 21.3, and 84 MB of 128 x 128 x 32 with eight waves 20.6, 18.8).  From many repetitions on the products bound it: their fragments
-// want the registers whatever the size (64^3 x 2048, 32 times, 29.4 us, capped 24.5), as long as
-// two workgroups fit a CU (192 x 192 x 16 x 8192 with 12 waves, 32 times, 324 us, 412 capped to
-// one).  Where LDS holds no second workgroup anyway the cap takes no waves away.
+// MB of 64 x 64 x 32 24.2, 21.3, and 84 MB of 128 x 128 x 32 with eight waves 20.6, 18.8).  From
+// many repetitions on the products bound it: their fragments want the registers whatever the size
+// (64^3 x 2048, 32 times, 29.4 us, capped 24.5), as long as two workgroups fit a CU (192 x 192 x 16
+// x 8192 with 12 waves, 32 times, 324 us, 412 capped to one).  Where LDS holds no second workgroup
+// anyway the cap takes no waves away.
 constexpr int64_t cap_bytes(int waves) { return waves >= 8 ? 80000000 : 100000000; }
 constexpr int kCapIters = 8;
 template <class AT, class G>
